@@ -39,17 +39,29 @@ void launch_f16_gemv(hipStream_t stream, const uint16_t *w_f16, long n_out, int 
                      const GemvFuse *fuse = nullptr);
 
 /* Scratch of the double-accumulation projection, for one pass of up to F64_M_MAX rows. */
-struct F64Scratch {
-    double *xd;        /* [F64_M_MAX][n_in] the activations in double */
-    double *xs;        /* [F64_M_MAX][ceil(n_in / 64)] their norms per stage of 64 columns */
-    int    *amb_count; /* outputs whose rounding depends on the order of the sum ... */
-    int2   *amb_list;  /* ... [n_out * F64_M_MAX] (weight row, activation row) */
+struct F64Lists { /* outputs (weight row, activation row), n_out * F64_M_MAX at most: */
+    int2 *near;   /* so close to a rounding boundary that the order of the sum may matter */
+    int2 *open;   /* ... that it does, as far as the bounds tell */
+    int  *n_near, *n_open;
 };
+struct F64Scratch {
+    void    *act; /* f16_linear_act_bytes(n_in): the activations as digits */
+    F64Lists list;
+};
+constexpr int F16_XROW_BYTES    = 32;
+constexpr int F16_DIGITS_MAX_IN = 65536; /* columns whose digit products the integer sums hold */
+size_t f16_linear_act_bytes(int n_in);    /* a multiple of 16 */
 /* The portable kernel (cpu_scalar_w_quant_mN for F16): y[m][r] = (float) sum_i (double) x[m][i] *
  * (double) f16(W[r][i]), the sum as if in index order; n_m <= F64_M_MAX, n_in a multiple of 8. */
 void launch_f16_linear_f64(hipStream_t stream, const uint16_t *w_f16, long n_out, int n_in,
                            const float *x, long ld_x, int n_m, const F64Scratch &ws, float *y,
                            long ld_y);
+/* launch_rmsnorm_rows of the rows h into normed and that projection of them, the norm in the
+ * launch that cuts the activations. */
+void launch_rmsnorm_f16_linear_f64(hipStream_t stream, const float *h, long ld_h, const float *wn,
+                                   float eps, float *normed, long ld_n, const uint16_t *w_f16,
+                                   long n_out, int n_in, int n_m, const F64Scratch &ws, float *y,
+                                   long ld_y);
 
 /* Scratch of the Q6_K projection, for one pass of up to Q6K_M_MAX rows. */
 constexpr int Q6K_M_MAX = 4;

@@ -1227,8 +1227,8 @@ int geist_hip_f16_gemv_rows(geist_hip_sampler *s, const uint16_t *d_w_f16, size_
     return after_launch(s, "f16 gemv");
 }
 
-/* Scratch of the f64 projection: activations in double, their stage norms, the list of outputs
- * for the second kernel. */
+/* Scratch of the f64 projection: the activations as digits, the list of outputs for the second
+ * kernel. */
 static int f64_scratch(geist_hip_sampler *s, size_t n_out, size_t n_in, F64Scratch &ws) {
     if (s->f64_in < n_in || s->f64_out < n_out) {
         if (s->f64_ws) {
@@ -1238,8 +1238,7 @@ static int f64_scratch(geist_hip_sampler *s, size_t n_out, size_t n_in, F64Scrat
         }
         const size_t in = n_in > s->f64_in ? n_in : s->f64_in;
         const size_t out = n_out > s->f64_out ? n_out : s->f64_out;
-        const size_t bytes = (size_t) F64_M_MAX * (in + in / 64 + 2) * sizeof(double) + 16 +
-                             out * F64_M_MAX * sizeof(int2);
+        const size_t bytes = f16_linear_act_bytes((int) in) + 16 + 2 * out * F64_M_MAX * sizeof(int2);
         if (hipMalloc(&s->f64_ws, bytes) != hipSuccess) {
             s->f64_ws = nullptr;
             return fail(s, GEIST_HIP_E_OOM, "f64 projection: scratch");
@@ -1247,10 +1246,11 @@ static int f64_scratch(geist_hip_sampler *s, size_t n_out, size_t n_in, F64Scrat
         s->f64_in = in, s->f64_out = out;
     }
     char *p      = static_cast<char *>(s->f64_ws);
-    ws.xd        = reinterpret_cast<double *>(p);
-    ws.xs        = ws.xd + (size_t) F64_M_MAX * s->f64_in;
-    ws.amb_count = reinterpret_cast<int *>(ws.xs + (size_t) F64_M_MAX * (s->f64_in / 64 + 2));
-    ws.amb_list  = reinterpret_cast<int2 *>(reinterpret_cast<char *>(ws.amb_count) + 16);
+    ws.act       = p;
+    int *n       = reinterpret_cast<int *>(p + f16_linear_act_bytes((int) s->f64_in));
+    ws.list.n_near = n, ws.list.n_open = n + 1;
+    ws.list.near   = reinterpret_cast<int2 *>(n + 4);
+    ws.list.open   = ws.list.near + s->f64_out * F64_M_MAX;
     return GEIST_HIP_OK;
 }
 
@@ -1892,7 +1892,7 @@ static int project_sample_impl(geist_hip_sampler *s, const float *d_hidden, size
             launch_rmsnorm_q8k_row_rows(s->stream, d_hidden, (long) ld_hidden, d_norm_weight,
                                         rms_eps, (int) rows, (int) d_model, d_normed,
                                         (long) d_model, q4k_kx4, q6ws.act8);
-    } else {
+    } else if (!f64) { /* (the projection in double norms its rows itself) */
         launch_rmsnorm_rows(s->stream, d_hidden, (long) ld_hidden, d_norm_weight, rms_eps,
                             (int) rows, (int) d_model, d_normed, (long) d_model);
     }
@@ -1944,10 +1944,17 @@ static int project_sample_impl(geist_hip_sampler *s, const float *d_hidden, size
     } else if (f64) {
         /* more than one row: the reference's batch kernel (cpu_scalar_w_quant_mN), its x86
          * kernels being decode-only; or the portable backend asked for */
-        rc = f16_linear_impl(s, d_embed_f16, n_vocab, d_model, d_normed, d_model, rows, d_logits,
-                             ld_logits);
-        if (rc)
+        F64Scratch ws;
+        if ((rc = f64_scratch(s, n_vocab, d_model, ws)) != GEIST_HIP_OK)
             return rc;
+        for (size_t m0 = 0; m0 < rows; m0 += F64_M_MAX) {
+            const size_t m = rows - m0 < (size_t) F64_M_MAX ? rows - m0 : (size_t) F64_M_MAX;
+            launch_rmsnorm_f16_linear_f64(s->stream, d_hidden + m0 * ld_hidden, (long) ld_hidden,
+                                          d_norm_weight, rms_eps, d_normed + m0 * d_model,
+                                          (long) d_model, d_embed_f16, (long) n_vocab,
+                                          (int) d_model, (int) m, ws, d_logits + m0 * ld_logits,
+                                          (long) ld_logits);
+        }
     } else {
         for (size_t m0 = 0; m0 < rows; m0 += GEMV_M_MAX) {
             const size_t m = rows - m0 < (size_t) GEMV_M_MAX ? rows - m0 : (size_t) GEMV_M_MAX;

@@ -453,3 +453,27 @@ def test_f16_linear_in_double_on_order_sensitive_rows(hs, oracle, m):
     other = (x.astype(np.float64) @ w.astype(np.float64).T).astype(np.float32)
     assert (other != want).any()          # the case does hang on the order
     assert (got.view(np.uint32) == want.view(np.uint32)).all(), int((got != want).sum())
+
+
+@pytest.mark.parametrize("n_out,n_in,m,scale", [
+    (1, 8, 2, 0.05), (15, 56, 4, 0.05), (17, 64, 5, 0.05), (33, 72, 8, 0.05), (4113, 256, 9, 0.05),
+    (50, 3520, 8, 0.05), (50, 1768, 13, 0.05), (31, 264, 16, 40.0), (64, 4096, 3, 2.5), (9, 65544, 2, 0.05)])
+def test_f16_linear_digit_edges(hs, oracle, n_out, n_in, m, scale):
+    """The int8-digit kernel at the edges of its tiles (16 weight rows, 64 columns, 4 / 8 / 16
+    activation rows), of what LDS holds of the activations (3413 columns of 8 rows, 1706 of 16), of
+    the weights' range (rows of magnitudes beyond 127, or of ||w|| that could hold one) and of the
+    integer sums (65536 columns): equal to the oracle in every bit."""
+    print(f"f16 digits n_out={n_out} n_in={n_in} m={m} scale={scale}", flush=True)
+    g = np.random.default_rng(n_out + n_in + m)
+    w16 = (g.standard_normal((n_out, n_in)) * scale).astype(np.float16)
+    w16[0, :8] = [127.0, -127.5, 0.5, -0.5, 6e-8, -6e-8, 0.25, -0.0]
+    w16[-1] = g.choice(np.array([2.0 ** -24, -2.0 ** -14, 0.498, -0.4990234375], np.float16), n_in)
+    x = g.standard_normal((m, n_in)).astype(np.float32)
+    x *= np.exp2(g.integers(-40, 3, x.shape)).astype(np.float32)   # remainders beyond six digits
+    x[0] = np.where(g.random(n_in) < 0.5, np.float32(1.0), np.float32(-1.0))   # partial sums near 0
+    y = torch.full((m, n_out), 7.0, dtype=torch.float32, device="cuda")
+    hs.f16_linear(to_dev(w16.view(np.int16), torch), to_dev(x, torch), y)
+    hs.sync()
+    want = oracle.f16_linear_f64(w16.view(np.uint16), x)
+    got = y.cpu().numpy()
+    assert (bits(got) == bits(want)).all(), np.argwhere(bits(got) != bits(want))[:5]
