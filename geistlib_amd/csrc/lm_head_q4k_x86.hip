@@ -20,7 +20,8 @@
  * table row; a dword holds the 4-bit values of eight consecutive elements, one mask gives the
  * even ones as bytes and a shift and a mask the odd ones, and two v_dot4_i32_i8 multiply them
  * with the activations, which the quantiser lays out to match (per eight elements a dword of the
- * even ones and a dword of the odd ones) and which are scalar operands.
+ * even ones and a dword of the odd ones) and which are scalar operands. Batches of decode rows go
+ * to the matrix cores (k_q4k_packed_linear_x86_mfma).
  */
 #include "lm_head_kernels.h"
 #include "rmsnorm_device.h"
@@ -153,7 +154,7 @@ __device__ __forceinline__ void q4x_load(const uint32_t *__restrict__ base, int 
     k.dd    = __builtin_nontemporal_load(base + 2304 + r);
 }
 
-/* M activation rows share a pass over the table. PAIRS: the binary32 accumulators are joined once
+/* M activation rows share a pass over the table (1 or 2, and 8 with PAIRS). PAIRS: the binary32 accumulators are joined once
  * per pair of sub-blocks (the reference's 16 x 16 AVX-512 tiles,
  * kernel_q4kx8_gemm_avx512_full.c:94, 729-778) instead of once per super-block. */
 template <int M, bool PAIRS>
@@ -281,6 +282,132 @@ __global__ __launch_bounds__(Q4X_TPB, PAIRS && M > 2 ? 3 : 4) void k_q4k_packed_
     }
 }
 
+/* The same for 2 to 8 activation rows on the int8 matrix cores. A block's scale has 6 bits and a
+ * table value 4: with the scale cut into two digits of 3 bits, value x digit is at most 105, an
+ * int8, and v_pk_mul_lo_u16 forms four of them at once (105 x 257 fits 16 bits: no carry from one
+ * byte into the next). I = sum (q * low digit) a + 8 sum (q * high digit) a is then two
+ * 16 x 16 x 64 products per 64 elements, and M, the minima spread over their sub-blocks' elements,
+ * a third. The operands: activation rows (lane & 15; there are n_m, the others repeat the last and
+ * are not stored) by table rows. A lane's 16 elements of K are half of what one 16-byte load of its
+ * table row holds, so that lane group kg takes sub-block 4 h + kg whole, in two products, and the
+ * even and odd elements stay in the order in which the activations' dwords have them.
+ *
+ * What bounds it: the pass over the table, 5 TB/s at 262144 x 1536 (the vector kernel's dot
+ * products and their scalar operands took 3.4 at 8 rows and 4 us more per row). Quantiser and
+ * projection of 8 rows, us, from HBM: 262144 x 1536 73.4 -> 56.4, 128256 x 2560 87.1 -> 47.7,
+ * 32000 x 4096 114 -> 38.0. A wavefront owns 32 table rows (two tiles; 128 registers, four
+ * wavefronts per SIMD): a tile's loads for the next block are issued as soon as its values are
+ * cut, into the registers that those leave. Four tiles at three wavefronts took 59.0 / 48.0 /
+ * 46.0, one tile at six (spilled) 81 / 69 / 43. */
+typedef int            q4x_i4 __attribute__((ext_vector_type(4)));
+typedef unsigned short q4x_us2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ int q4x_times(uint32_t bytes, uint32_t digit2) {
+    return (int) __builtin_bit_cast(uint32_t, __builtin_bit_cast(q4x_us2, bytes) *
+                                                  __builtin_bit_cast(q4x_us2, digit2));
+}
+
+template <int NT, int WAVES>
+__global__ __launch_bounds__(Q4X_TPB, WAVES) void k_q4k_packed_linear_x86_mfma(
+    const uint32_t *__restrict__ packed, long n_out, int nb, const uint32_t *__restrict__ act,
+    int n_m, float *__restrict__ y, long ld_y) {
+    const int  lane = threadIdx.x & 63, j = lane & 15, kg = lane >> 4;
+    const long unit = (long) blockIdx.x * (Q4X_TPB / 64) + threadIdx.x / 64;
+    const long row0 = unit * (16 * NT); /* NT tiles of 16 rows, of one group of 64 */
+    if (row0 >= n_out)
+        return;
+    const int       r0     = (int) (row0 & 63);
+    const uint32_t *base   = packed + (row0 >> 6) * nb * Q4X_PACK_DWORDS;
+    const long      act_ld = (long) nb * Q4X_ACT_DWORDS + Q4X_ACT_TAIL;
+    const uint32_t *arow   = act + (long) (j < n_m ? j : n_m - 1) * act_ld + 8 * kg;
+    /* byte kg of a dword, into the low byte of both halves / into all four bytes */
+    const uint32_t sel_half = 0x0c000c00u | (uint32_t) kg * 0x00010001u;
+    const uint32_t sel_all  = (uint32_t) kg * 0x01010101u;
+
+    float d_a[4], acc[NT][4], acc_min[NT][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int m = 4 * kg + i;
+        d_a[i] = __uint_as_float(act[(m < n_m ? m : n_m - 1) * act_ld + (long) nb * Q4X_ACT_DWORDS]);
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+            acc[t][i] = 0.0f, acc_min[t][i] = 0.0f;
+    }
+    q4x_u4   q[NT][2], sm[NT]; /* values of sub-blocks kg and 4 + kg; scales, minima */
+    uint32_t dd[NT];
+    q4x_i4   a[2][2], an[2][2];
+    auto load_tile = [&](const uint32_t *blk, int t) {
+        const uint32_t *p = blk + 4 * (r0 + 16 * t + j);
+        q[t][0] = __builtin_nontemporal_load(reinterpret_cast<const q4x_u4 *>(p + kg * 256));
+        q[t][1] = __builtin_nontemporal_load(reinterpret_cast<const q4x_u4 *>(p + (4 + kg) * 256));
+        sm[t]   = __builtin_nontemporal_load(reinterpret_cast<const q4x_u4 *>(p + 8 * 256));
+        dd[t]   = __builtin_nontemporal_load(blk + 2304 + r0 + 16 * t + j);
+    };
+    auto load_act = [&](int b, q4x_i4 (&v)[2][2]) {
+        const uint32_t *p = arow + (long) b * Q4X_ACT_DWORDS;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            v[h][0] = *reinterpret_cast<const q4x_i4 *>(p + 32 * h);
+            v[h][1] = *reinterpret_cast<const q4x_i4 *>(p + 32 * h + 4);
+        }
+    };
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+        load_tile(base, t);
+    load_act(0, a);
+    for (int b = 0; b < nb; ++b) {
+        /* (the last block loads itself again: no branch between the loads and their waits) */
+        const int       bn   = b + 1 < nb ? b + 1 : b;
+        const uint32_t *next = base + (long) bn * Q4X_PACK_DWORDS;
+        load_act(bn, an);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            q4x_i4      lo = {0, 0, 0, 0}, hi = {0, 0, 0, 0}, mi = {0, 0, 0, 0};
+            const float d    = __half2float(__ushort_as_half((unsigned short) (dd[t] & 0xffffu)));
+            const float dmin = __half2float(__ushort_as_half((unsigned short) (dd[t] >> 16)));
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const uint32_t sc = __builtin_amdgcn_perm(0u, h ? sm[t].y : sm[t].x, sel_half);
+                const uint32_t sl = sc & 0x00070007u, sh = (sc >> 3) & 0x00070007u;
+                const int      mn = (int) __builtin_amdgcn_perm(0u, h ? sm[t].w : sm[t].z, sel_all);
+                const q4x_i4   mv = {mn, mn, mn, mn};
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const uint32_t w0 = k ? q[t][h].z : q[t][h].x, w1 = k ? q[t][h].w : q[t][h].y;
+                    const uint32_t e0 = w0 & 0x0f0f0f0fu, o0 = (w0 >> 4) & 0x0f0f0f0fu;
+                    const uint32_t e1 = w1 & 0x0f0f0f0fu, o1 = (w1 >> 4) & 0x0f0f0f0fu;
+                    const q4x_i4   wl = {q4x_times(e0, sl), q4x_times(o0, sl), q4x_times(e1, sl),
+                                         q4x_times(o1, sl)};
+                    const q4x_i4   wh = {q4x_times(e0, sh), q4x_times(o0, sh), q4x_times(e1, sh),
+                                         q4x_times(o1, sh)};
+                    lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[h][k], wl, lo, 0, 0, 0);
+                    hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[h][k], wh, hi, 0, 0, 0);
+                    mi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[h][k], mv, mi, 0, 0, 0);
+                }
+            }
+            load_tile(next, t);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                acc[t][i] = __builtin_fmaf((float) (lo[i] + 8 * hi[i]), __fmul_rn(d, d_a[i]), acc[t][i]);
+                acc_min[t][i] =
+                    __builtin_fmaf((float) mi[i], __fmul_rn(dmin, d_a[i]), acc_min[t][i]);
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            a[h][0] = an[h][0], a[h][1] = an[h][1];
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const long row = row0 + 16 * t + j;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (row < n_out && 4 * kg + i < n_m)
+                y[(4 * kg + i) * ld_y + row] = __fsub_rn(acc[t][i], acc_min[t][i]);
+    }
+}
+
 size_t q4k_x86_act_dwords(int n_in) {
     return (size_t) (n_in / 256) * Q4X_ACT_DWORDS + Q4X_ACT_TAIL;
 }
@@ -297,31 +424,25 @@ void launch_rmsnorm_q8k_row_rows(hipStream_t stream, const float *x, long ld_x, 
                                                                       ties_even, act);
 }
 
-template <int M>
-static void q4x_launch(hipStream_t stream, const uint32_t *packed, long n_out, int nb,
-                       const uint32_t *act, bool pairs, float *y, long ld_y) {
-    const long groups = (n_out + 63) / 64;
-    const dim3 grid((unsigned) ((groups + 3) / 4)), block(Q4X_TPB);
-    if (pairs)
-        k_q4k_packed_gemv_x86<M, true><<<grid, block, 0, stream>>>(packed, n_out, nb, act, y, ld_y);
-    else
-        k_q4k_packed_gemv_x86<M, false><<<grid, block, 0, stream>>>(packed, n_out, nb, act, y, ld_y);
-}
-
 void launch_q4k_packed_gemv_q8k(hipStream_t stream, const void *packed, long n_out, int n_in,
                                 const uint32_t *act, int n_m, bool pairs, float *y, long ld_y) {
     const uint32_t *p  = static_cast<const uint32_t *>(packed);
     const int       nb = n_in / 256;
-    switch (n_m) {
-    case 1: q4x_launch<1>(stream, p, n_out, nb, act, pairs, y, ld_y); break;
-    case 2: q4x_launch<2>(stream, p, n_out, nb, act, pairs, y, ld_y); break;
-    case 3: q4x_launch<3>(stream, p, n_out, nb, act, pairs, y, ld_y); break;
-    case 4: q4x_launch<4>(stream, p, n_out, nb, act, pairs, y, ld_y); break;
-    case 5: q4x_launch<5>(stream, p, n_out, nb, act, pairs, y, ld_y); break;
-    case 6: q4x_launch<6>(stream, p, n_out, nb, act, pairs, y, ld_y); break;
-    case 7: q4x_launch<7>(stream, p, n_out, nb, act, pairs, y, ld_y); break;
-    default: q4x_launch<8>(stream, p, n_out, nb, act, pairs, y, ld_y); break;
-    }
+    const long      groups = (n_out + 63) / 64;
+    const dim3      grid((unsigned) ((groups + 3) / 4)), block(Q4X_TPB);
+    /* One row leaves the matrix cores 15/16 idle and the vector kernel streams at the same rate; two
+     * rows of at most six super-blocks, 48.9 us by it and 50.2 by the matrix cores (262144 x 1536),
+     * of ten 48.8 and 45.6 (128256 x 2560), of sixteen 57.5 and 36.5. pairs: a tile of sixteen
+     * rows' order of accumulation, which comes in eights. */
+    if (pairs)
+        k_q4k_packed_gemv_x86<Q4X_M_MAX, true><<<grid, block, 0, stream>>>(p, n_out, nb, act, y, ld_y);
+    else if (n_m == 1)
+        k_q4k_packed_gemv_x86<1, false><<<grid, block, 0, stream>>>(p, n_out, nb, act, y, ld_y);
+    else if (n_m == 2 && nb <= 6)
+        k_q4k_packed_gemv_x86<2, false><<<grid, block, 0, stream>>>(p, n_out, nb, act, y, ld_y);
+    else
+        k_q4k_packed_linear_x86_mfma<2, 4><<<dim3((unsigned) ((groups + 1) / 2)), block, 0, stream>>>(
+            p, n_out, nb, act, n_m, y, ld_y);
 }
 
 } // namespace gs

@@ -144,6 +144,30 @@ def test_q4k_batch_equals_the_x86_backend(hs, oracle, n_out, n_in, m):
         hs.set_projection(0)
 
 
+@pytest.mark.parametrize("n_out,n_in,m", [(8, 256, 3), (40, 1792, 2), (72, 512, 8), (136, 256, 5),
+                                          (200, 1536, 2), (1000, 768, 6)])
+def test_q4k_batch_at_the_edges_of_the_matrix_tiles(hs, oracle, n_out, n_in, m):
+    """Table rows that fill half a tile or a few, every row count up to 8, and the largest integers
+    the operands can hold: values 15, scales and minima 63, activations of +-127 in runs. The sums
+    are integers, so the logits are the decode kernel's bit for bit; rows beyond the batch and
+    columns beyond the table stay untouched."""
+    print(f"q4k matrix tiles {n_out} x {n_in}, {m} rows", flush=True)
+    g = np.random.default_rng(n_out + n_in + m)
+    w = random_q4k_table(g, n_out, n_in)
+    w.reshape(n_out, -1, 144)[::2, :, 4:] = 0xFF
+    packed = packed_copy(hs, w, n_in)
+    x = tie_rows(g, m, n_in, 1.0)
+    x[0] = np.where(np.arange(n_in) % 96 < 64, 5.0, -5.0)
+    x[m - 1] = 0.0
+    y = torch.full((m + 1, n_out + 3), np.nan, dtype=torch.float32, device="cuda")
+    hs.q4k_packed_linear_x86(packed, n_out, n_in, torch.from_numpy(x).cuda(), y[:m, :n_out])
+    hs.sync()
+    got = y.cpu().numpy()
+    assert np.isnan(got[m:]).all() and np.isnan(got[:, n_out:]).all()
+    want = oracle_q4k_linear_x86(oracle.lib, w, x, n_in, avx512=True)
+    assert np.array_equal(got[:m, :n_out].view(np.uint32), want.view(np.uint32))
+
+
 def test_q4k_decode_refuses_shapes_the_x86_kernel_does_not_take(hs):
     from geistlib_amd.binding import GeistHipError
     packed = torch.zeros((hs.q4k_packed_bytes(12, 256),), dtype=torch.uint8, device="cuda")
