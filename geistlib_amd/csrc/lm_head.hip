@@ -407,22 +407,26 @@ __global__ __launch_bounds__(LM_TPB) void k_f16_gemv_batched(const uint16_t *__r
  * a double sum only shows in the binary32 result when 1 / sqrt(mean + eps) lies within the
  * sum's error of the middle between two binary32 values. The workgroup adds in a fixed parallel
  * order and, in that rare case, one thread repeats the sum in the reference's order. */
-__global__ __launch_bounds__(LM_TPB) void k_rmsnorm_rows(const float *__restrict__ x, long ld_x,
-                                                         const float *__restrict__ w, float eps,
-                                                         int n, float *__restrict__ y, long ld_y) {
-    __shared__ double s_part[LM_TPB];
-    __shared__ float  s_inv;
+__global__ __launch_bounds__(NORM_TPB) void k_rmsnorm_rows(const float *__restrict__ x, long ld_x,
+                                                           const float *__restrict__ w, float eps,
+                                                           int n, float *__restrict__ y, long ld_y) {
+    __shared__ NormShared s_norm;
     const int    tid = threadIdx.x;
     const float *xr  = x + (long) blockIdx.x * ld_x;
     float       *yr  = y + (long) blockIdx.x * ld_y;
-    const float inv = block_rms_inv<LM_TPB>(xr, n, eps, s_part, &s_inv);
-    for (int i = tid; i < n; i += LM_TPB)
+    float        v[NORM_PER];
+    const float  inv = block_rmsnorm(xr, w, n, eps, v, s_norm);
+#pragma unroll
+    for (int k = 0; k < NORM_PER; ++k)
+        if (k * NORM_TPB + tid < n)
+            yr[k * NORM_TPB + tid] = v[k];
+    for (int i = NORM_PER * NORM_TPB + tid; i < n; i += NORM_TPB)
         yr[i] = __fmul_rn(__fmul_rn(xr[i], inv), w[i]);
 }
 
 void launch_rmsnorm_rows(hipStream_t stream, const float *x, long ld_x, const float *w, float eps,
                          int n_rows, int n, float *y, long ld_y) {
-    k_rmsnorm_rows<<<dim3(n_rows), dim3(LM_TPB), 0, stream>>>(x, ld_x, w, eps, n, y, ld_y);
+    k_rmsnorm_rows<<<dim3(n_rows), dim3(NORM_TPB), 0, stream>>>(x, ld_x, w, eps, n, y, ld_y);
 }
 
 bool f16_gemv_can_fuse(int n_m) { return n_m >= 1 && n_m <= 2; }

@@ -36,11 +36,11 @@ constexpr int Q4X_TPB         = 256;
 constexpr int Q4X_ROW_DWORDS  = 37;
 constexpr int Q4X_PACK_DWORDS = Q4X_ROW_DWORDS * 64; /* the packed copy's dwords per (64 rows, block) */
 
-/* Thread t's element of a super-block, given the reciprocal of the row's scale: its int8 value
+/* Element t of a super-block, held by thread t modulo 256, given the reciprocal of the row's scale: its int8 value
  * into the block's dwords (ob), the sums per sub-block of 32 behind them. */
 __device__ __forceinline__ void q4x_quantize_block(float xv, float inv, bool ties_even,
                                                    uint32_t *__restrict__ ob) {
-    const int   t = threadIdx.x;
+    const int   t = threadIdx.x & 255;
     const float v = __fmul_rn(xv, inv);
     /* the decode kernel's quantiser rounds half away from zero by truncation and clamps; the
      * batch quantiser is lrintf (|v| <= 127 up to rounding: nothing to clamp) */
@@ -93,44 +93,47 @@ __global__ __launch_bounds__(Q4X_TPB) void k_q8k_row_quantize(const float *__res
 }
 
 /* The output norm (cpu_scalar_rmsnorm, as k_rmsnorm_rows computes it) and that quantiser in one
- * launch, one workgroup per row: the normed row goes to y and, as int8, to act. A thread reads
- * back what it wrote itself. n a multiple of 256. */
-__global__ __launch_bounds__(Q4X_TPB) void k_rmsnorm_q8k_row_rows(const float *__restrict__ x,
-                                                                 long ld_x,
-                                                                 const float *__restrict__ w,
-                                                                 float eps, int n,
-                                                                 float *__restrict__ y, long ld_y,
-                                                                 bool ties_even,
-                                                                 uint32_t *__restrict__ act) {
-    __shared__ double s_part[Q4X_TPB];
-    __shared__ float  s_inv;
-    __shared__ float  s_max[Q4X_TPB / 64];
+ * launch, one workgroup per row, four super-blocks at a time: the normed row goes to y and, as
+ * int8, to act. Elements that are not held are read back by the thread that wrote them. n a
+ * multiple of 256. */
+__global__ __launch_bounds__(NORM_TPB) void k_rmsnorm_q8k_row_rows(const float *__restrict__ x,
+                                                                  long ld_x,
+                                                                  const float *__restrict__ w,
+                                                                  float eps, int n,
+                                                                  float *__restrict__ y, long ld_y,
+                                                                  bool ties_even,
+                                                                  uint32_t *__restrict__ act) {
+    __shared__ NormShared s_norm;
+    __shared__ float      s_max[NORM_TPB / 64];
     const int    nb = n / 256, m = blockIdx.x, t = threadIdx.x;
     const float *xr = x + (long) m * ld_x;
     float       *yr = y + (long) m * ld_y;
     uint32_t    *o  = act + (long) m * ((long) nb * Q4X_ACT_DWORDS + Q4X_ACT_TAIL);
-    const float  rinv = block_rms_inv<Q4X_TPB>(xr, n, eps, s_part, &s_inv);
-    float        ax = 0.0f;
-    for (int b = 0; b < nb; ++b) {
-        const int   i = 256 * b + t;
-        const float v = __fmul_rn(__fmul_rn(xr[i], rinv), w[i]);
-        yr[i]         = v;
-        ax            = __builtin_fmaxf(ax, __builtin_fabsf(v));
-    }
+    float        v[NORM_PER], ax = 0.0f;
+    const float  rinv = block_rmsnorm(xr, w, n, eps, v, s_norm);
 #pragma unroll
-    for (int s = 32; s >= 1; s >>= 1)
-        ax = __builtin_fmaxf(ax, __shfl_xor(ax, s));
-    if ((t & 63) == 0)
-        s_max[t >> 6] = ax;
-    __syncthreads();
-    const float amax  = __builtin_fmaxf(__builtin_fmaxf(s_max[0], s_max[1]),
-                                        __builtin_fmaxf(s_max[2], s_max[3]));
+    for (int k = 0; k < NORM_PER; ++k) {
+        if (k * NORM_TPB + t < n)
+            yr[k * NORM_TPB + t] = v[k];
+        ax = __builtin_fmaxf(ax, __builtin_fabsf(v[k]));
+    }
+    for (int i = NORM_PER * NORM_TPB + t; i < n; i += NORM_TPB) {
+        const float e = __fmul_rn(__fmul_rn(xr[i], rinv), w[i]);
+        yr[i]         = e;
+        ax            = __builtin_fmaxf(ax, __builtin_fabsf(e));
+    }
+    const float amax  = block_norm_max(ax, s_max);
     const float scale = amax == 0.0f ? 1.0f : __fdiv_rn(amax, 127.0f);
     const float inv   = __fdiv_rn(1.0f, scale);
     if (t == 0)
         o[(long) nb * Q4X_ACT_DWORDS] = __float_as_uint(scale);
-    for (int b = 0; b < nb; ++b)
-        q4x_quantize_block(yr[256 * b + t], inv, ties_even, o + (long) b * Q4X_ACT_DWORDS);
+#pragma unroll
+    for (int k = 0; k < NORM_PER; ++k)
+        if (k * NORM_TPB + t < n) /* (whole blocks) */
+            q4x_quantize_block(v[k], inv, ties_even,
+                               o + (long) ((k * NORM_TPB + t) >> 8) * Q4X_ACT_DWORDS);
+    for (int i = NORM_PER * NORM_TPB + t; i < n; i += NORM_TPB)
+        q4x_quantize_block(yr[i], inv, ties_even, o + (long) (i >> 8) * Q4X_ACT_DWORDS);
 }
 
 typedef uint32_t q4x_u4 __attribute__((ext_vector_type(4)));
@@ -420,7 +423,7 @@ void launch_q8k_row_quantize(hipStream_t stream, const float *x, long ld_x, int 
 void launch_rmsnorm_q8k_row_rows(hipStream_t stream, const float *x, long ld_x, const float *w,
                                  float eps, int n_rows, int n, float *y, long ld_y, bool ties_even,
                                  uint32_t *act) {
-    k_rmsnorm_q8k_row_rows<<<dim3(n_rows), dim3(Q4X_TPB), 0, stream>>>(x, ld_x, w, eps, n, y, ld_y,
+    k_rmsnorm_q8k_row_rows<<<dim3(n_rows), dim3(NORM_TPB), 0, stream>>>(x, ld_x, w, eps, n, y, ld_y,
                                                                       ties_even, act);
 }
 

@@ -38,13 +38,14 @@ namespace gs {
 constexpr int Q6X_TPB         = 256;
 constexpr int Q6X_PACK_DWORDS = 53 * 64; /* the packed copy's dwords per (64 rows, block) */
 
-/* One super-block's 256 activations, one to a thread of the workgroup, as int8 (64 dwords, four
- * to a dword in element order), their sixteen sums per group of sixteen as int32, and d_a, written
- * to o[0 .. Q8K_ACT_DWORDS). s_max: four floats that no thread still reads from an earlier call
- * (the callers alternate between two). */
-__device__ __forceinline__ void q8k_quantize_block(float xv, uint32_t *__restrict__ o,
-                                                   float *s_max) {
-    const int t  = threadIdx.x;
+/* One super-block's 256 activations, one to a thread modulo 256, as int8 (64 dwords, four to a
+ * dword in element order), their sixteen sums per group of sixteen as int32, and d_a, written to
+ * o[0 .. Q8K_ACT_DWORDS) (store: the block is there; every thread of the workgroup calls). s_max:
+ * the four floats of these 256 threads, which none of them still reads from an earlier call (the
+ * callers alternate between two). */
+__device__ __forceinline__ void q8k_quantize_block(float xv, uint32_t *__restrict__ o, float *s_max,
+                                                   bool store) {
+    const int t  = threadIdx.x & 255;
     float     ax = __builtin_fabsf(xv);
     /* the reference keeps the running maximum when a comparison with a NaN fails; fmaxf drops
      * the NaN in the same way */
@@ -66,6 +67,8 @@ __device__ __forceinline__ void q8k_quantize_block(float xv, uint32_t *__restric
     const uint32_t b1 = (uint32_t) __shfl_down(q, 1) & 0xffu;
     const uint32_t b2 = (uint32_t) __shfl_down(q, 2) & 0xffu;
     const uint32_t b3 = (uint32_t) __shfl_down(q, 3) & 0xffu;
+    if (!store)
+        return;
     if ((t & 3) == 0)
         o[t >> 2] = b0 | (b1 << 8) | (b2 << 16) | (b3 << 24);
     if ((t & 15) == 0)
@@ -80,29 +83,40 @@ __global__ __launch_bounds__(Q6X_TPB) void k_q8k_quantize(const float *__restric
     __shared__ float s_max[Q6X_TPB / 64];
     const int        b = blockIdx.x, m = blockIdx.y;
     q8k_quantize_block(x[(long) m * ld_x + (long) b * 256 + threadIdx.x],
-                       act + ((long) m * nb + b) * Q8K_ACT_DWORDS, s_max);
+                       act + ((long) m * nb + b) * Q8K_ACT_DWORDS, s_max, true);
 }
 
 /* The output norm (cpu_scalar_rmsnorm, src/backends/cpu_scalar/elementwise.c:241-280, as
- * k_rmsnorm_rows computes it) and the quantiser in one launch, one workgroup per row: the normed
- * row goes to y and, as int8 super-blocks, to act. n a multiple of 256. */
-__global__ __launch_bounds__(Q6X_TPB) void k_rmsnorm_q8k_rows(const float *__restrict__ x,
-                                                             long ld_x,
-                                                             const float *__restrict__ w,
-                                                             float eps, int n,
-                                                             float *__restrict__ y, long ld_y,
-                                                             uint32_t *__restrict__ act) {
-    __shared__ double s_part[Q6X_TPB];
-    __shared__ float  s_inv;
-    __shared__ float  s_max[2][Q6X_TPB / 64];
-    const int    nb = n / 256, m = blockIdx.x, t = threadIdx.x;
+ * k_rmsnorm_rows computes it) and the quantiser in one launch, one workgroup per row, four
+ * super-blocks at a time: the normed row goes to y and, as int8 super-blocks, to act. n a multiple
+ * of 256. */
+__global__ __launch_bounds__(NORM_TPB) void k_rmsnorm_q8k_rows(const float *__restrict__ x,
+                                                              long ld_x,
+                                                              const float *__restrict__ w,
+                                                              float eps, int n,
+                                                              float *__restrict__ y, long ld_y,
+                                                              uint32_t *__restrict__ act) {
+    __shared__ NormShared s_norm;
+    __shared__ float      s_max[2][NORM_TPB / 64];
+    const int    nb = n / 256, m = blockIdx.x, t = threadIdx.x, grp = t >> 8;
     const float *xr = x + (long) m * ld_x;
-    const float  inv = block_rms_inv<Q6X_TPB>(xr, n, eps, s_part, &s_inv);
-    for (int b = 0; b < nb; ++b) {
-        const int   i = 256 * b + t;
-        const float v = __fmul_rn(__fmul_rn(xr[i], inv), w[i]);
-        y[(long) m * ld_y + i] = v;
-        q8k_quantize_block(v, act + ((long) m * nb + b) * Q8K_ACT_DWORDS, s_max[b & 1]);
+    float        v[NORM_PER];
+    const float  inv = block_rmsnorm(xr, w, n, eps, v, s_norm);
+    /* (trips are uniform over the workgroup: the quantiser has barriers) */
+    auto block = [&](int k, float e) {
+        const int i = k * NORM_TPB + t, b = 4 * k + grp;
+        if (b < nb)
+            y[(long) m * ld_y + i] = e;
+        q8k_quantize_block(e, act + ((long) m * nb + b) * Q8K_ACT_DWORDS, s_max[k & 1] + 4 * grp,
+                           b < nb);
+    };
+#pragma unroll
+    for (int k = 0; k < NORM_PER; ++k)
+        if (k * NORM_TPB < n)
+            block(k, v[k]);
+    for (int k = NORM_PER; k * NORM_TPB < n; ++k) {
+        const int i = k * NORM_TPB + t;
+        block(k, i < n ? __fmul_rn(__fmul_rn(xr[i], inv), w[i]) : 0.0f);
     }
 }
 
@@ -302,7 +316,7 @@ __global__ __launch_bounds__(Q6X_TPB) void k_q6k_gemv_x86(const uint8_t *__restr
 constexpr int Q8S_ACT_TAIL = 8;
 
 __device__ __forceinline__ void q8s_quantize_block(float xv, float inv, uint32_t *__restrict__ ob) {
-    const int t = threadIdx.x;
+    const int t = threadIdx.x & 255;
     const int q = __float2int_rn(__fmul_rn(xv, inv)); /* lrintf; |x * inv| <= 127 up to rounding */
     int       sum = q;
 #pragma unroll
@@ -322,17 +336,9 @@ __device__ __forceinline__ void q8s_quantize_block(float xv, float inv, uint32_t
 }
 
 /* the reciprocal of the row's scale from the row's largest magnitude, the scale to *o_scale */
-__device__ __forceinline__ float q8s_row_inv(float ax, float *s_max, uint32_t *o_scale) {
+__device__ __forceinline__ float q8s_row_inv(float amax, uint32_t *o_scale) {
     const int t = threadIdx.x;
-#pragma unroll
-    for (int s = 32; s >= 1; s >>= 1)
-        ax = __builtin_fmaxf(ax, __shfl_xor(ax, s));
-    if ((t & 63) == 0)
-        s_max[t >> 6] = ax;
-    __syncthreads();
-    const float amax = __builtin_fmaxf(__builtin_fmaxf(s_max[0], s_max[1]),
-                                       __builtin_fmaxf(s_max[2], s_max[3]));
-    float scale = __fdiv_rn(amax, 127.0f);
+    float     scale = __fdiv_rn(amax, 127.0f);
     if (scale == 0.0f)
         scale = 1.0f;
     if (t == 0)
@@ -350,35 +356,52 @@ __global__ __launch_bounds__(Q6X_TPB) void k_q8s_row_quantize(const float *__res
     float            ax = 0.0f;
     for (int b = 0; b < nb; ++b)
         ax = __builtin_fmaxf(ax, __builtin_fabsf(xr[256 * b + t])); /* (a NaN is passed over) */
-    const float inv = q8s_row_inv(ax, s_max, o + (long) nb * Q8K_ACT_DWORDS);
+#pragma unroll
+    for (int s = 32; s >= 1; s >>= 1)
+        ax = __builtin_fmaxf(ax, __shfl_xor(ax, s));
+    if ((t & 63) == 0)
+        s_max[t >> 6] = ax;
+    __syncthreads();
+    const float amax = __builtin_fmaxf(__builtin_fmaxf(s_max[0], s_max[1]),
+                                       __builtin_fmaxf(s_max[2], s_max[3]));
+    const float inv  = q8s_row_inv(amax, o + (long) nb * Q8K_ACT_DWORDS);
     for (int b = 0; b < nb; ++b)
         q8s_quantize_block(xr[256 * b + t], inv, o + (long) b * Q8K_ACT_DWORDS);
 }
 
 /* The output norm (as k_rmsnorm_rows computes it) and that quantiser in one launch, one workgroup
- * per row; a thread reads back what it wrote itself. n a multiple of 256. */
-__global__ __launch_bounds__(Q6X_TPB) void k_rmsnorm_q8s_rows(const float *__restrict__ x, long ld_x,
-                                                             const float *__restrict__ w, float eps,
-                                                             int n, float *__restrict__ y, long ld_y,
-                                                             uint32_t *__restrict__ act) {
-    __shared__ double s_part[Q6X_TPB];
-    __shared__ float  s_inv;
-    __shared__ float  s_max[Q6X_TPB / 64];
+ * per row, four super-blocks at a time; elements that are not held are read back by the thread that
+ * wrote them. n a multiple of 256. */
+__global__ __launch_bounds__(NORM_TPB) void k_rmsnorm_q8s_rows(const float *__restrict__ x, long ld_x,
+                                                              const float *__restrict__ w, float eps,
+                                                              int n, float *__restrict__ y, long ld_y,
+                                                              uint32_t *__restrict__ act) {
+    __shared__ NormShared s_norm;
+    __shared__ float      s_max[NORM_TPB / 64];
     const int    nb = n / 256, m = blockIdx.x, t = threadIdx.x;
     const float *xr = x + (long) m * ld_x;
     float       *yr = y + (long) m * ld_y;
     uint32_t    *o  = act + (long) m * ((long) nb * Q8K_ACT_DWORDS + Q8S_ACT_TAIL);
-    const float  rinv = block_rms_inv<Q6X_TPB>(xr, n, eps, s_part, &s_inv);
-    float        ax = 0.0f;
-    for (int b = 0; b < nb; ++b) {
-        const int   i = 256 * b + t;
-        const float v = __fmul_rn(__fmul_rn(xr[i], rinv), w[i]);
-        yr[i]         = v;
-        ax            = __builtin_fmaxf(ax, __builtin_fabsf(v));
+    float        v[NORM_PER], ax = 0.0f;
+    const float  rinv = block_rmsnorm(xr, w, n, eps, v, s_norm);
+#pragma unroll
+    for (int k = 0; k < NORM_PER; ++k) {
+        if (k * NORM_TPB + t < n)
+            yr[k * NORM_TPB + t] = v[k];
+        ax = __builtin_fmaxf(ax, __builtin_fabsf(v[k]));
     }
-    const float inv = q8s_row_inv(ax, s_max, o + (long) nb * Q8K_ACT_DWORDS);
-    for (int b = 0; b < nb; ++b)
-        q8s_quantize_block(yr[256 * b + t], inv, o + (long) b * Q8K_ACT_DWORDS);
+    for (int i = NORM_PER * NORM_TPB + t; i < n; i += NORM_TPB) {
+        const float e = __fmul_rn(__fmul_rn(xr[i], rinv), w[i]);
+        yr[i]         = e;
+        ax            = __builtin_fmaxf(ax, __builtin_fabsf(e));
+    }
+    const float inv = q8s_row_inv(block_norm_max(ax, s_max), o + (long) nb * Q8K_ACT_DWORDS);
+#pragma unroll
+    for (int k = 0; k < NORM_PER; ++k)
+        if (k * NORM_TPB + t < n) /* (whole blocks) */
+            q8s_quantize_block(v[k], inv, o + (long) ((k * NORM_TPB + t) >> 8) * Q8K_ACT_DWORDS);
+    for (int i = NORM_PER * NORM_TPB + t; i < n; i += NORM_TPB)
+        q8s_quantize_block(yr[i], inv, o + (long) (i >> 8) * Q8K_ACT_DWORDS);
 }
 
 typedef uint32_t q8s_u8v __attribute__((ext_vector_type(8), aligned(16)));
@@ -585,7 +608,7 @@ void launch_q8s_row_quantize(hipStream_t stream, const float *x, long ld_x, int 
 
 void launch_rmsnorm_q8s_rows(hipStream_t stream, const float *x, long ld_x, const float *w,
                              float eps, int n_rows, int n, float *y, long ld_y, uint32_t *act) {
-    k_rmsnorm_q8s_rows<<<dim3(n_rows), dim3(Q6X_TPB), 0, stream>>>(x, ld_x, w, eps, n, y, ld_y,
+    k_rmsnorm_q8s_rows<<<dim3(n_rows), dim3(NORM_TPB), 0, stream>>>(x, ld_x, w, eps, n, y, ld_y,
                                                                   act);
 }
 
@@ -639,7 +662,7 @@ void launch_q8k_quantize(hipStream_t stream, const float *x, long ld_x, int n_m,
 
 void launch_rmsnorm_q8k_rows(hipStream_t stream, const float *x, long ld_x, const float *w,
                              float eps, int n_rows, int n, float *y, long ld_y, uint32_t *act) {
-    k_rmsnorm_q8k_rows<<<dim3(n_rows), dim3(Q6X_TPB), 0, stream>>>(x, ld_x, w, eps, n, y, ld_y,
+    k_rmsnorm_q8k_rows<<<dim3(n_rows), dim3(NORM_TPB), 0, stream>>>(x, ld_x, w, eps, n, y, ld_y,
                                                                   act);
 }
 

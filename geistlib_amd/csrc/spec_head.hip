@@ -214,49 +214,49 @@ __global__ __launch_bounds__(SP_TPB) void k_spec_sketch_rows(SpecHeadDev d) {
  * runs in front: h = (x * inv_rms) * norm_w, written to h_out for the finalist kernel, in the
  * arithmetic of the norm kernel of the dense head. */
 template <bool NORM>
-__global__ __launch_bounds__(SP_TPB) void k_spec_act(SpecHeadDev d, const float *__restrict__ h_in,
-                                                     const float *__restrict__ norm_w, float eps,
-                                                     float *__restrict__ h_out) {
-    __shared__ float  s_max[SP_TPB / SP_WAVE];
-    __shared__ double s_sum[3][SP_TPB / SP_WAVE];
-    __shared__ double s_part[NORM ? SP_TPB : 1];
-    __shared__ float  s_inv;
-    __shared__ float  s_h[NORM ? SPEC_D_MODEL_MAX : 1];
+__global__ __launch_bounds__(NORM_TPB) void k_spec_act(SpecHeadDev d, const float *__restrict__ h_in,
+                                                       const float *__restrict__ norm_w, float eps,
+                                                       float *__restrict__ h_out) {
+    __shared__ NormShared s_norm;
+    __shared__ float      s_max[NORM_TPB / SP_WAVE];
+    __shared__ double     s_sum[3][NORM_TPB / SP_WAVE];
+    __shared__ float      s_h[SPEC_D_MODEL_MAX];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const float *h = h_in;
+    /* the thread's first kept dimension: asked for with the row */
+    const int dim0 = tid < d.sketch_dim ? d.dims[tid] : 0;
+    float     v[NORM_PER], inv = 0.0f;
     if (NORM) {
-        const float inv = block_rms_inv<SP_TPB>(h_in, d.d_model, eps, s_part, &s_inv);
-        for (int i = tid; i < d.d_model; i += SP_TPB) {
-            const float y = __fmul_rn(__fmul_rn(h_in[i], inv), norm_w[i]);
-            s_h[i]        = y;
-            h_out[i]      = y;
-        }
-        __syncthreads();
-        h = s_h;
+        inv = block_rmsnorm(h_in, norm_w, d.d_model, eps, v, s_norm);
+    } else {
+#pragma unroll
+        for (int k = 0; k < NORM_PER; ++k)
+            v[k] = k * NORM_TPB + tid < d.d_model ? h_in[k * NORM_TPB + tid] : 0.0f;
     }
-    float     amax = 0.0f;
-    double    all2 = 0.0;
-    for (int i = tid; i < d.d_model; i += SP_TPB) {
-        const float v = h[i];
-        amax          = __builtin_fmaxf(amax, __builtin_fabsf(v));
-        all2 += (double) v * (double) v;
-    }
-    amax = wave_max(amax);
-    if (lane == 0)
-        s_max[wv] = amax;
-    __syncthreads();
-    amax = 1e-8f;
-    for (int i = 0; i < SP_TPB / SP_WAVE; ++i)
-        amax = __builtin_fmaxf(amax, s_max[i]);
+    float  amax = 0.0f;
+    double all2 = 0.0;
+    auto   take = [&](int i, float y) {
+        s_h[i] = y;
+        if (NORM)
+            h_out[i] = y;
+        amax = __builtin_fmaxf(amax, __builtin_fabsf(y));
+        all2 += (double) y * (double) y;
+    };
+#pragma unroll
+    for (int k = 0; k < NORM_PER; ++k)
+        if (k * NORM_TPB + tid < d.d_model)
+            take(k * NORM_TPB + tid, v[k]);
+    for (int i = NORM_PER * NORM_TPB + tid; i < d.d_model; i += NORM_TPB)
+        take(i, NORM ? __fmul_rn(__fmul_rn(h_in[i], inv), norm_w[i]) : h_in[i]);
+    amax = __builtin_fmaxf(block_norm_max(amax, s_max), 1e-8f); /* (its barrier is s_h's too) */
     const float x_q = __fdiv_rn(127.0f, amax);
     double      l1 = 0.0, kept2 = 0.0;
-    for (int s = tid; s < d.sketch_dim; s += SP_TPB) {
-        const float v = h[d.dims[s]];
-        float       q = __builtin_rintf(__fmul_rn(v, x_q));
+    for (int s = tid; s < d.sketch_dim; s += NORM_TPB) {
+        const float e = s_h[s == tid ? dim0 : d.dims[s]];
+        float       q = __builtin_rintf(__fmul_rn(e, x_q));
         q             = __builtin_fminf(__builtin_fmaxf(q, -127.0f), 127.0f);
         d.act[s]      = q;
-        l1 += fabs((double) v);
-        kept2 += (double) v * (double) v;
+        l1 += fabs((double) e);
+        kept2 += (double) e * (double) e;
     }
     all2  = wave_sum(all2);
     l1    = wave_sum(l1);
@@ -266,7 +266,7 @@ __global__ __launch_bounds__(SP_TPB) void k_spec_act(SpecHeadDev d, const float 
     __syncthreads();
     if (tid == 0) {
         double a = 0.0, b = 0.0, c = 0.0;
-        for (int i = 0; i < SP_TPB / SP_WAVE; ++i)
+        for (int i = 0; i < NORM_TPB / SP_WAVE; ++i)
             a += s_sum[0][i], b += s_sum[1][i], c += s_sum[2][i];
         const double drop = a - c > 0.0 ? a - c : 0.0;
         d.sc->inv_xq      = __fdiv_rn(1.0f, x_q);
@@ -594,10 +594,10 @@ void launch_spec_try(hipStream_t stream, const SpecHeadDev &d, const float *h, b
     const dim3 one(1), block(SP_TPB), sel(SP_SEL_TPB);
     const dim3 rows((unsigned) ((d.vocab + SP_TPB - 1) / SP_TPB));
     if (norm_w != nullptr) {
-        k_spec_act<true><<<one, block, 0, stream>>>(d, h, norm_w, eps, h_normed);
+        k_spec_act<true><<<one, dim3(NORM_TPB), 0, stream>>>(d, h, norm_w, eps, h_normed);
         h = h_normed;
     } else {
-        k_spec_act<false><<<one, block, 0, stream>>>(d, h, nullptr, 0.0f, nullptr);
+        k_spec_act<false><<<one, dim3(NORM_TPB), 0, stream>>>(d, h, nullptr, 0.0f, nullptr);
     }
     GemvFuse f{};
     f.gmax = d.gmax;

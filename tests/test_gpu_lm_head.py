@@ -477,3 +477,47 @@ def test_f16_linear_digit_edges(hs, oracle, n_out, n_in, m, scale):
     want = oracle.f16_linear_f64(w16.view(np.uint16), x)
     got = y.cpu().numpy()
     assert (bits(got) == bits(want)).all(), np.argwhere(bits(got) != bits(want))[:5]
+
+
+@pytest.mark.parametrize("n", [1, 1023, 1025, 4095, 4097, 6000])
+def test_rmsnorm_at_the_edges_of_what_a_workgroup_holds(hs, oracle, n):
+    """A workgroup of 1024 threads holds four elements each; beyond 4096 it reads the row again."""
+    g = np.random.default_rng(n)
+    x = (g.standard_normal((3, n)) * 3).astype(np.float32)
+    w = (1.0 + 0.2 * g.standard_normal(n)).astype(np.float32)
+    d_x = to_dev(x, torch)
+    for y in (torch.empty_like(d_x), d_x):                                 # and in place
+        hs.rmsnorm(d_x, to_dev(w, torch), 1e-6, y)
+        hs.sync()
+        assert (bits(y.cpu().numpy()) == bits(oracle.rmsnorm(x, w, 1e-6))).all()
+
+
+@pytest.mark.parametrize("table", ["q6k", "q4k"])
+@pytest.mark.parametrize("d_model", [256, 1024, 1792, 4096, 4352, 6144])
+def test_norm_and_quantiser_in_one_launch(hs, oracle, table, d_model):
+    """The norm that quantises on the way (four super-blocks at a time, from 4096 elements on
+    reading back) against the norm and the quantiser as launches of their own: bit for bit."""
+    from geistlib_amd import SampleParams
+    from oracle_lib import random_q4k_table, random_q6k_table
+    g = np.random.default_rng(d_model)
+    vocab = 72
+    w = (random_q6k_table if table == "q6k" else random_q4k_table)(g, vocab, d_model)
+    size, pack, run, linear = ((hs.q6k_packed_bytes, hs.q6k_pack, hs.project_sample_q6k_packed,
+                                hs.q6k_packed_linear_x86) if table == "q6k" else
+                               (hs.q4k_packed_bytes, hs.q4k_pack, hs.project_sample_q4k_packed,
+                                hs.q4k_packed_linear_x86))
+    packed = torch.empty(size(vocab, d_model), dtype=torch.uint8, device="cuda")
+    pack(to_dev(w, torch), d_model, packed)
+    norm_w = (1.0 + 0.2 * g.standard_normal(d_model)).astype(np.float32)
+    for rows in (1, 3, 4):
+        h = (g.standard_normal((rows, d_model)) * 3).astype(np.float32)
+        logits = torch.empty((rows, vocab), device="cuda")
+        normed = torch.empty((rows, d_model), device="cuda")
+        out = torch.empty(rows, dtype=torch.int32, device="cuda")
+        run(to_dev(h, torch), to_dev(norm_w, torch), 1e-6, packed, vocab, logits,
+            SampleParams.make(temperature=0.0), None, out, normed)
+        want = torch.empty((rows, vocab), device="cuda")
+        linear(packed, vocab, d_model, normed, want)
+        hs.sync()
+        assert (bits(normed.cpu().numpy()) == bits(oracle.rmsnorm(h, norm_w, 1e-6))).all()
+        assert (bits(logits.cpu().numpy()) == bits(want.cpu().numpy())).all(), rows
