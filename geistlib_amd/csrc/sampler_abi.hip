@@ -557,7 +557,7 @@ static MeetSpace meet_space(geist_hip_sampler *s, const Launch &L, uint32_t word
 
 static int sample_impl(geist_hip_sampler *s, const struct geist_hip_rows *rows,
                        const struct geist_hip_sample_params *params, const float *d_uniforms,
-                       geist_hip_token_t *d_out) {
+                       geist_hip_token_t *d_out, const gs_host::Generators &rng = {}) {
     if (s) {
         s->epoch_by_kernel = false;
         s->tell = false;
@@ -569,7 +569,8 @@ static int sample_impl(geist_hip_sampler *s, const struct geist_hip_rows *rows,
                       capture != hipStreamCaptureStatusActive;
         }
     }
-    const int rc = gs_host::sample_stages(s, rows, params, d_uniforms, d_out, gs_host::STAGE_ALL, nullptr);
+    const int rc = gs_host::sample_stages(s, rows, params, d_uniforms, d_out, gs_host::STAGE_ALL, nullptr,
+                                          rng);
     if (rc == GEIST_HIP_OK && s->tell) {
         /* the ids of this call are written when the word holds this epoch */
         const Notify nt = {s->h_done, s->epoch + 1, s->rows_done};
@@ -629,7 +630,8 @@ static int reserve_sorted_workspace(geist_hip_sampler *s) {
  * follows it per row. geist_hip_sample_rows runs both. */
 int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *rows,
                            const struct geist_hip_sample_params *params, const float *d_uniforms,
-                           geist_hip_token_t *d_out, unsigned stages, const char **stream_kernel) {
+                           geist_hip_token_t *d_out, unsigned stages, const char **stream_kernel,
+                           const gs_host::Generators &rng) {
     const bool do_stream = stages & gs_host::STAGE_STREAM,
                do_tail = stages & gs_host::STAGE_TAIL;
     const char *unused_name;
@@ -651,6 +653,13 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
         return fail(s, GEIST_HIP_E_INVALID_ARG, "stochastic configuration without uniforms");
     HIPCHK(s, hipSetDevice(s->device));
 
+    /* a generator per row: the one-launch kernels take the draw themselves (a launch of its own is
+     * 4.7 us of a step of 13 to 19); every other path has the draws written in front of it */
+    const bool own_rng = rng.states && s->row_arrive && (!rng.shared || rows->rows == 1);
+    auto       draws   = [&] {
+        if (rng.states)
+            launch_rng_units(s->stream, rng.states, rng.shared, (int) rows->rows, s->uniforms);
+    };
     FinalLaunch f{};
     f.inv_t      = rs.inv_t;
     f.top_p      = rs.top_p;
@@ -675,6 +684,7 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
     }
     if (rs.use_k) {
         if (rs.k > TOPK_FAST_MAX) {
+            draws();
             f.mode         = FINAL_TOPK;
             f.k            = rs.k;
             *stream_kernel = "k_topk_general";
@@ -753,12 +763,17 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
                 nt                 = Notify{s->h_done, s->epoch + 1, s->rows_done};
                 s->epoch_by_kernel = true;
             }
+            if (own_rng)
+                f.rng = rng.states;
+            else
+                draws();
             if (do_stream)
                 launch_cand_scan_final(scan, L, f, s->tmax, wg_cands_at(s->wcands, rows->rows, wgs_row),
                                        r_w, r_last, reinterpret_cast<uint32_t *>(s->row_arrive),
                                        s->handoff_far, nt, (int) wgs_row, halves ? 4 : 8);
             return after_launch(s, "top-k");
         }
+        draws();
         if (m) {
             const WaveCands wc = wave_cands_at(s->wcands, row_waves);
             f.row_flag         = s->row_flag;
@@ -788,11 +803,17 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
              * faster form, their workgroups being smaller and gone sooner). The measuring
              * stages cannot split it: the streaming stage is the whole step. */
             *stream_kernel = "k_temperature_draw";
+            RowGenerators gen = {};
+            if (own_rng)
+                gen = RowGenerators{rng.states, reinterpret_cast<uint32_t *>(s->row_arrive)};
+            else
+                draws();
             if (do_stream)
-                launch_temperature_draw(scan, rs.inv_t, d_uniforms, d_out,
+                launch_temperature_draw(scan, rs.inv_t, d_uniforms, gen, d_out,
                                         meet_space(s, scan, 2, true));
             return after_launch(s, "temperature");
         }
+        draws();
         *stream_kernel = "k_scan_expsum";
         if (do_stream &&
             launch_scan_expsum(scan, rs.inv_t, nullptr, s->chunk_best, s->chunk_sum, nullptr, 0,
@@ -815,6 +836,7 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
     if (L.rv.n_chunks > s->max_chunks)
         return fail(s, GEIST_HIP_E_UNSUPPORTED, "n_vocab %zu needs more than %d chunks",
                     rows->n_vocab, s->max_chunks);
+    draws();
     /* min-p bounds the kept prefix by the row maximum alone, so the exp-sum pass can list the
      * candidates on its way; rows whose list overflows fall back to the bound of the row-final
      * kernel and a third pass */
@@ -1076,10 +1098,9 @@ int geist_hip_sample_rows_rng(geist_hip_sampler *s, const struct geist_hip_rows 
     if (!greedy) {
         if (!d_rng_states)
             return fail(s, GEIST_HIP_E_INVALID_ARG, "null rng states");
-        HIPCHK(s, hipSetDevice(s->device));
-        launch_rng_units(s->stream, d_rng_states, shared, (int) rows->rows, s->uniforms);
     }
-    return sample_impl(s, rows, params, greedy ? nullptr : s->uniforms, d_out_tokens);
+    return sample_impl(s, rows, params, greedy ? nullptr : s->uniforms, d_out_tokens,
+                       {greedy ? nullptr : d_rng_states, shared});
 }
 
 int geist_hip_argmax_f32(geist_hip_sampler *s, const float *d_logits, size_t n,
@@ -1968,12 +1989,12 @@ static int project_sample_impl(geist_hip_sampler *s, const float *d_hidden, size
                                 d_logits + m0 * ld_logits, (long) ld_logits);
         }
     }
-    if (!rs.greedy && d_rng_states) {
-        launch_rng_units(s->stream, d_rng_states, shared, (int) rows, s->uniforms);
+    const bool rng = !rs.greedy && d_rng_states;
+    if (rng)
         d_uniforms = s->uniforms;
-    }
     s->tmax_ready = topk_scan;
-    rc            = sample_impl(s, &r, params, rs.greedy ? nullptr : d_uniforms, d_out_tokens);
+    rc            = sample_impl(s, &r, params, rs.greedy ? nullptr : d_uniforms, d_out_tokens,
+                                {rng ? d_rng_states : nullptr, shared});
     s->tmax_ready = false;
     return rc;
 }

@@ -137,7 +137,7 @@ __device__ __forceinline__ float group_maxima(const float4 (&v)[NG], float (&gm)
 
 /* NG: float4 groups a lane holds, 8 (a workgroup scans 32768 logits) or, for launches of few
  * rows, 4 (16384: twice the workgroups to a row, so that twice the compute units fetch it). */
-template <bool PEN, bool STREAM, int NG>
+template <bool PEN, bool STREAM, int NG, bool RNG>
 __global__ __launch_bounds__(OL_THREADS) void k_cand_scan_final(RowView rvs, RowView rv,
                                                                 WgCands wc, int r_w, int r_last,
                                                                 FinalArgs a,
@@ -185,7 +185,7 @@ __global__ __launch_bounds__(OL_THREADS) void k_cand_scan_final(RowView rvs, Row
         if (tid + OL_THREADS < rv.hist_ld)
             hid1 = hrow[tid + OL_THREADS];
     }
-    const float u_row = a.uniforms[row + vz];
+    const float u_row = RNG ? 0.0f : a.uniforms[row + vz];
     uint64_t    tabv  = 0;
     if (tid < 32)
         tabv = g_expf_tab[tid];
@@ -408,6 +408,11 @@ __global__ __launch_bounds__(OL_THREADS) void k_cand_scan_final(RowView rvs, Row
     const long sw0 = (long) row * W;
     float4     gv[2];
     uint32_t   gi[2], cw[2];
+    /* the state of the row's generator where the draw comes from it: this workgroup alone reads it
+     * and, at the end, writes the advanced state (4.7 us as a launch of its own in front) */
+    uint64_t state = 0;
+    if (RNG)
+        state = a.rng[row + vz];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const bool on = h == 0 || G > 4;
@@ -595,8 +600,11 @@ __global__ __launch_bounds__(OL_THREADS) void k_cand_scan_final(RowView rvs, Row
     }
     if (tid < WAVE) {
         /* (k <= CAND_K_MAX = 64 on this path) */
-        const int tok = finish_sorted_lanes(k, s_pack, a.inv_t, a.top_p, a.min_p, u_row, s_tab);
+        const float u   = RNG ? xorshift_unit(state) : u_row;
+        const int   tok = finish_sorted_lanes(k, s_pack, a.inv_t, a.top_p, a.min_p, u, s_tab);
         if (tid == 0) {
+            if (RNG) /* (through to memory, as the id below: it is there when the host is told) */
+                __hip_atomic_store(a.rng + row, state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             if (!nt.h_done) {
                 a.out[row] = tok;
             } else {

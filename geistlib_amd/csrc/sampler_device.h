@@ -605,5 +605,16 @@ __device__ __forceinline__ float zbin_threshold(int b) {
     return -(float) (b + 1) / (float) ZBIN_PER_NAT;
 }
 
+/* xorshift64* (sampler.c:35-48): one step of a generator, and the uniform of its 24 leading bits */
+__device__ __forceinline__ uint64_t xorshift_step(uint64_t &s) {
+    s ^= s >> 12;
+    s ^= s << 25;
+    s ^= s >> 27;
+    return s * 0x2545F4914F6CDD1DULL;
+}
+__device__ __forceinline__ float xorshift_unit(uint64_t &s) {
+    return (float) (uint32_t) (xorshift_step(s) >> 40) * (1.0f / 16777216.0f);
+}
+
 } // namespace gs
 #endif

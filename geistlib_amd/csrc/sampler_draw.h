@@ -147,6 +147,7 @@ template <int NV, bool PEN, bool PLAIN>
 __device__ __forceinline__ void draw_chunk(const RowView &rv, int row, int chunk, int n_rows,
                                            int base, int end, float inv_t,
                                            const float *__restrict__ uniforms,
+                                           const RowGenerators &rng,
                                            int32_t *__restrict__ out, uint64_t *sum_slots,
                                            uint32_t *s_cnt16, double *s_sum, uint64_t *s_tab,
                                            uint64_t tabv, double *s_tr, DrawShared &sh,
@@ -154,7 +155,13 @@ __device__ __forceinline__ void draw_chunk(const RowView &rv, int row, int chunk
     const int tid = threadIdx.x, C = rv.n_chunks;
     if (PEN)
         __builtin_amdgcn_s_setprio(3); /* see expsum_chunk */
-    const float u_row = uniforms[row];
+    /* the row's draw, for the first wavefront: given, or the next of the row's generator */
+    float    u_row = 0.0f;
+    uint64_t state = 0;
+    if (rng.states == nullptr)
+        u_row = uniforms[row];
+    else if (tid < WAVE)
+        state = __hip_atomic_load(rng.states + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     HistPrefetch pf;
     if (PEN)
         pf = history_prefetch(rv, row, n_rows);
@@ -243,8 +250,20 @@ __device__ __forceinline__ void draw_chunk(const RowView &rv, int row, int chunk
         }
         __syncthreads();
     }
-    /* where the draw falls: the same arithmetic in every workgroup of the row */
+    /* where the draw falls: the same arithmetic in every workgroup of the row. One that has read
+     * the generator's state is counted; whichever is counted last writes the advanced state (which
+     * workgroups met does not matter: none can read it any more). The count comes after the
+     * meetings, whose polls would wait for its answer. */
+    uint32_t counted = 0;
     if (tid < WAVE) {
+        if (rng.states != nullptr) {
+            uint32_t one = 1u;
+            asm volatile("" : "+v"(one) : "v"(state)); /* not before the state has arrived */
+            if (tid == 0)
+                counted = __hip_atomic_fetch_add(rng.arrive + (long) row * ARRIVE_STRIDE_INTS, one,
+                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            u_row = xorshift_unit(state);
+        }
         double    run, target;
         const int at = walk_locate_chunk(sh.csum, C, u_row, &run, &target);
         int       js = 0;
@@ -260,6 +279,11 @@ __device__ __forceinline__ void draw_chunk(const RowView &rv, int row, int chunk
         }
     }
     __syncthreads();
+    if (rng.states != nullptr && tid == 0 && counted == (uint32_t) (C - 1)) {
+        __hip_atomic_store(rng.arrive + (long) row * ARRIVE_STRIDE_INTS, 0u, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+        rng.states[row] = state;
+    }
     if (sh.walk.chunk != chunk)
         return; /* another workgroup's */
     const double target = sh.walk.target;
@@ -299,6 +323,7 @@ __device__ __forceinline__ void draw_chunk(const RowView &rv, int row, int chunk
 template <int NV, bool PEN>
 __global__ __launch_bounds__(TPB) void k_temperature_draw(RowView rv, int n_rows, float inv_t,
                                                           const float *__restrict__ uniforms,
+                                                          RowGenerators rng,
                                                           int32_t *__restrict__ out,
                                                           MeetSpace meet) {
     __shared__ __align__(16) uint32_t s_cnt16[PEN ? NV * TPB * 2 : 1];
@@ -337,10 +362,10 @@ __global__ __launch_bounds__(TPB) void k_temperature_draw(RowView rv, int n_rows
     const bool plain = rv.vec_ok && end - base == NV * TPB * 4 && !(rv.softcap > 0.0f) &&
                        rv.allowed == nullptr;
     if (plain)
-        draw_chunk<NV, PEN, true>(rv, row, chunk, n_rows, base, end, inv_t, uniforms, out,
+        draw_chunk<NV, PEN, true>(rv, row, chunk, n_rows, base, end, inv_t, uniforms, rng, out,
                                   sum_slots, s_cnt16, s_sum, s_tab, tabv, s_tr, s_draw, fs);
     else
-        draw_chunk<NV, PEN, false>(rv, row, chunk, n_rows, base, end, inv_t, uniforms, out,
+        draw_chunk<NV, PEN, false>(rv, row, chunk, n_rows, base, end, inv_t, uniforms, rng, out,
                                    sum_slots, s_cnt16, s_sum, s_tab, tabv, s_tr, s_draw, fs);
 }
 

@@ -180,6 +180,7 @@ struct FinalLaunch {
                                   applies it to what it keeps */
     float           inv_t, top_p, min_p;
     const float    *uniforms;
+    uint64_t       *rng; /* launch_cand_scan_final: the rows' generators in place of uniforms, or NULL */
     const uint64_t *chunk_best;
     const double   *chunk_sum;
     const double   *slab_sum;
@@ -210,8 +211,15 @@ int launch_scan_expsum(const Launch &L, float inv_t, float *tmax, uint64_t *chun
 /* The temperature draw in one kernel (sampler_draw.h): out[row] = the id drawn with
  * uniforms[row]. For L.nv == 2. `meet.slots` holds 2 * rows * n_chunks zeroed words: the
  * workgroups of a row meet twice. */
-void launch_temperature_draw(const Launch &L, float inv_t, const float *uniforms, int32_t *out,
-                             const MeetSpace &meet);
+/* The rows' generators, when a kernel takes its draws from them itself: states[row] is read by the
+ * row's workgroups and advanced by the last of them; arrive: a zeroed counter per row, ARRIVE_STRIDE_INTS
+ * apart, left zeroed. states == NULL: the draws are in `uniforms`. */
+struct RowGenerators {
+    uint64_t *states;
+    uint32_t *arrive;
+};
+void launch_temperature_draw(const Launch &L, float inv_t, const float *uniforms,
+                             const RowGenerators &rng, int32_t *out, const MeetSpace &meet);
 /* last z bin that can hold an entry passing min_p (with slack); ZBINS - 1 when min_p is off or
  * that deep */
 int zbin_of_min_p(float min_p);

@@ -1207,6 +1207,7 @@ struct FinalArgs {
                                   * logits to the same value: only entries whose capped value lies
                                   * strictly above the capped bound are certain to be all there
                                   * is, and k of those are needed. */
+    uint64_t       *rng; /* k_cand_scan_final<..., true>: the rows' own generators */
 };
 
 /* ============================================================================================
@@ -1865,26 +1866,20 @@ __global__ __launch_bounds__(TPB) void k_penalties(RowView rv, float *__restrict
 /* ============================================================================================
  * k_rng_units: xorshift64* (sampler.c:35-48). shared: one state, row r takes draw r+1.
  * ========================================================================================== */
-__device__ __forceinline__ uint64_t xorshift_step(uint64_t &s) {
-    s ^= s >> 12;
-    s ^= s << 25;
-    s ^= s >> 27;
-    return s * 0x2545F4914F6CDD1DULL;
-}
 __global__ void k_rng_units(uint64_t *states, int shared, int rows, float *uniforms) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (shared) {
         if (r == 0) {
             uint64_t s = states[0];
             for (int i = 0; i < rows; ++i)
-                uniforms[i] = (float) (uint32_t) (xorshift_step(s) >> 40) * (1.0f / 16777216.0f);
+                uniforms[i] = xorshift_unit(s);
             states[0] = s;
         }
         return;
     }
     if (r < rows) {
         uint64_t s  = states[r];
-        uniforms[r] = (float) (uint32_t) (xorshift_step(s) >> 40) * (1.0f / 16777216.0f);
+        uniforms[r] = xorshift_unit(s);
         states[r]   = s;
     }
 }
@@ -1964,16 +1959,16 @@ int zbin_of_min_p(float min_p) {
     return z_m * ZBIN_PER_NAT < (double) (ZBINS - 1) ? (int) (z_m * ZBIN_PER_NAT) : ZBINS - 1;
 }
 
-void launch_temperature_draw(const Launch &L, float inv_t, const float *uniforms, int32_t *out,
-                             const MeetSpace &meet) {
+void launch_temperature_draw(const Launch &L, float inv_t, const float *uniforms,
+                             const RowGenerators &rng, int32_t *out, const MeetSpace &meet) {
     /* for launches of a few rows: the geometry of 2048 elements per workgroup only. Rows in
      * eights, so that the workgroups of a row have linear ids equal modulo 8 and share an XCD
      * (xcd_row_chunk); the workgroups of the rows that are not there leave at once. */
     const dim3 grid(L.rv.n_chunks, (L.rows + 7) & ~7), block(TPB);
     if (L.pen)
-        k_temperature_draw<2, true><<<grid, block, 0, L.stream>>>(L.rv, L.rows, inv_t, uniforms, out, meet);
+        k_temperature_draw<2, true><<<grid, block, 0, L.stream>>>(L.rv, L.rows, inv_t, uniforms, rng, out, meet);
     else
-        k_temperature_draw<2, false><<<grid, block, 0, L.stream>>>(L.rv, L.rows, inv_t, uniforms, out, meet);
+        k_temperature_draw<2, false><<<grid, block, 0, L.stream>>>(L.rv, L.rows, inv_t, uniforms, rng, out, meet);
 }
 
 void launch_spec(const Launch &L, const SpecLaunch &sp, const MeetSpace *meet) {
@@ -2038,6 +2033,7 @@ static FinalArgs final_args(const FinalLaunch &f) {
     a.top_p      = f.top_p;
     a.min_p      = f.min_p;
     a.uniforms   = f.uniforms;
+    a.rng        = f.rng;
     a.chunk_best = f.chunk_best;
     a.chunk_sum  = f.chunk_sum;
     a.slab_sum   = f.slab_sum;
@@ -2121,17 +2117,25 @@ void launch_cand_scan_final(const Launch &scan, const Launch &L, const FinalLaun
         kernel<<<grid, block, 0, L.stream>>>(scan.rv, L.rv, wc, r_w, r_last, a, tmax, arrive,
                                              far_always ? 1 : 0, nt);
     };
-    if (groups == 4) { /* launches of few rows: half the logits to a workgroup */
+    /* PEN, STREAM, float4 groups a lane, RNG. (The draw's source as a run-time choice cost every
+     * call with given draws 0.16 us of 13.2 at 64 rows of 128256.) */
+    auto pick = [&](auto ng, auto rng) {
+        constexpr int  NG  = decltype(ng)::value;
+        constexpr bool RNG = decltype(rng)::value;
         if (L.pen)
-            scan.rv.stream_loads ? go(k_cand_scan_final<true, true, 4>) : go(k_cand_scan_final<true, false, 4>);
+            scan.rv.stream_loads ? go(k_cand_scan_final<true, true, NG, RNG>)
+                                 : go(k_cand_scan_final<true, false, NG, RNG>);
         else
-            scan.rv.stream_loads ? go(k_cand_scan_final<false, true, 4>) : go(k_cand_scan_final<false, false, 4>);
-        return;
-    }
-    if (L.pen)
-        scan.rv.stream_loads ? go(k_cand_scan_final<true, true, 8>) : go(k_cand_scan_final<true, false, 8>);
+            scan.rv.stream_loads ? go(k_cand_scan_final<false, true, NG, RNG>)
+                                 : go(k_cand_scan_final<false, false, NG, RNG>);
+    };
+    using std::integral_constant;
+    using std::true_type;
+    using std::false_type;
+    if (groups == 4) /* launches of few rows: half the logits to a workgroup */
+        f.rng ? pick(integral_constant<int, 4>{}, true_type{}) : pick(integral_constant<int, 4>{}, false_type{});
     else
-        scan.rv.stream_loads ? go(k_cand_scan_final<false, true, 8>) : go(k_cand_scan_final<false, false, 8>);
+        f.rng ? pick(integral_constant<int, 8>{}, true_type{}) : pick(integral_constant<int, 8>{}, false_type{});
 }
 
 __global__ __launch_bounds__(TPB) void k_zero_words(uint64_t *__restrict__ p, uint32_t n) {

@@ -713,6 +713,44 @@ def test_device_rng_matches_reference_stream(hs, oracle):
     assert out.cpu().tolist() == want
 
 
+@pytest.mark.parametrize("rows,n", [(1, 32000), (1, 128256), (3, 50257), (8, 30000), (16, 32000),
+                                    (40, 9000), (5, 2049)])
+@pytest.mark.parametrize("options", [dict(temperature=0.8), dict(temperature=0.7, top_k=40, top_p=0.9),
+                                     dict(temperature=0.7, top_k=100), dict(temperature=1.0, top_p=0.9),
+                                     dict(temperature=0.9, min_p=0.05)])
+def test_rows_own_generators_give_the_draws_of_their_units(hs, rows, n, options):
+    """A call that takes its draws from a generator per row -- in the kernel that draws where one
+    launch serves the row, in a launch in front elsewhere -- against the same call on the units
+    computed on the host, several calls in a row, also where the row's workgroups do not meet
+    (wait limit 0) or are taken not to share a cache: tokens and states are whole numbers."""
+    from geistlib_amd import HipSampler
+    from geistlib_amd.workloads import xorshift_units
+    print(f"own generators {rows} x {n} {options}", flush=True)
+    x, _ = rows_rng(rows + n, rows, n)
+    d = to_dev(x, torch)
+    view, prm = HipSampler.rows(d), P(**options)
+    seeds = [(r + 1) * 0x9E3779B97F4A7C15 % 2 ** 64 for r in range(rows)]
+    st = torch.from_numpy(np.array(seeds, dtype=np.uint64).view(np.int64)).cuda()
+    out, want = (torch.empty(rows, dtype=torch.int32, device="cuda") for _ in range(2))
+    try:
+        for step in range(4):
+            if step == 2:
+                hs.set_wait_limit(0)
+                hs.handoff_scope(True)
+            hs.sample_rng(view, prm, st, rows == 1 and step == 1, out)
+            drawn = [xorshift_units(s, 1) for s in seeds]
+            seeds = [int(d[1]) for d in drawn]
+            u = np.array([d[0][0] for d in drawn], dtype=np.float32)
+            units = to_dev(u, torch)
+            hs.sample(view, prm, units, want)
+            hs.sync()
+            assert out.cpu().tolist() == want.cpu().tolist(), step
+            assert st.cpu().numpy().view(np.uint64).tolist() == seeds, step
+    finally:
+        hs.set_wait_limit(65536)
+        hs.handoff_scope(False)
+
+
 # ------------------------------------------------------------------- strided / unaligned
 def test_row_stride_and_unaligned_rows(hs, oracle):
     g = np.random.default_rng(3)
