@@ -487,7 +487,7 @@ def bench_lm_head(args, m_rows, q8=False):
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
                      "kernel": ("k_q8w_gemv" if q8 else
-                                "k_f16_linear_f64 (+ activations to double, listed outputs)"
+                                "k_f16_linear_digits (+ activations cut into digits, near and open outputs)"
                                 if f64_batch else "k_f16_gemv"),
                      "kernel_us": round(kernel_us, 3),
                      "kernel_algorithmic_bytes": w_bytes,
