@@ -22,6 +22,7 @@
  * run while the next stages' loads, four per wavefront, are under way. With the products in
  * double (v_mfma_f64_4x4x4, half of whose rate eight rows could use) the same pass took 189 us.
  */
+#include "f32_rounding.h"
 #include "lm_head_kernels.h"
 #include "rmsnorm_device.h"
 #include "sampler_device.h"
@@ -204,14 +205,6 @@ __global__ __launch_bounds__(XD_TPB) void k_x_digits(const float *__restrict__ x
         o.norm = finite ? sqrt(sq) * (1.0 + 0x1p-40) : (double) __builtin_inff();
         o.rest = rest * unit * (1.0 + 0x1p-40);
     }
-}
-
-/* (float) s, and whether every value within err of s rounds to the same binary32. */
-__device__ __forceinline__ bool f32_rounding_is_safe(double s, double err, float &f) {
-    f = (float) s;
-    const double up = 0.5 * ((double) f + (double) nextafterf(f, __builtin_inff()));
-    const double dn = 0.5 * ((double) f + (double) nextafterf(f, -__builtin_inff()));
-    return up - s > err && s - dn > err;
 }
 
 /* The digits of a lane's sixteen weights (eight dwords q): a weight times 2^24 is a whole number,

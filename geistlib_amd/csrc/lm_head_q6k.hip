@@ -32,6 +32,7 @@
  * aligned dwords that hold it and shifted into place. The activations are uniform over the
  * wavefront and come as scalar operands.
  */
+#include "f32_rounding.h"
 #include "lm_head_kernels.h"
 #include "lm_head_q6k_block.h"
 
@@ -47,15 +48,14 @@ constexpr int Q6K_TPB         = 256;
 
 /* (float) s, and whether every value within err of s rounds to the same binary32. */
 __device__ __forceinline__ bool q6k_rounding_is_safe(double s, double err, float &f) {
-    f = (float) s;
     /* Not finite: with an infinite or NaN activation the sum's terms are infinities and NaNs,
      * and this kernel's split into t - 32 * sum x can meet inf - inf where the reference's sum in
      * index order does not. The kernel that adds in the reference's order decides. */
-    if (!(__builtin_fabsf(f) < __builtin_inff()))
+    if (!(__builtin_fabs(s) < __builtin_inf())) {
+        f = (float) s;
         return false;
-    const double up = 0.5 * ((double) f + (double) nextafterf(f, __builtin_inff()));
-    const double dn = 0.5 * ((double) f + (double) nextafterf(f, -__builtin_inff()));
-    return up - s > err && s - dn > err;
+    }
+    return f32_rounding_is_safe(s, err, f);
 }
 
 /* xd[m][k] = (double) x[m][k]; per group of 16 elements xsum = sum x and xabs = sum |x| (rounded

@@ -329,6 +329,42 @@ def test_f16_linear_in_double_at_the_ends_of_the_range(hs, oracle, m):
     assert np.isinf(want).any() and nan.any() and (np.abs(want[0, 5:]) < 1.2e-38).any()
 
 
+def sums_at_the_end_of_binary32(n_in, rng):
+    """Activations against weights of 1 (or -1) whose sums lie around 2^128 - 2^103, where binary32
+    ends: the exact sum below it and the sum in index order above it (17 additions that each round
+    up by half a step of the double sum), the other way round, and well on either side."""
+    top = np.float32(np.finfo(np.float32).max)
+    x = np.zeros((6, n_in), dtype=np.float32)
+    step = np.float32(2.0 ** 74)
+    up, down = step * np.float32(1 + 2.0 ** -10), step * np.float32(1 - 2.0 ** -10)
+    near = np.float32((2.0 ** 24 - 1) * 2.0 ** 79)          # 2^103 - 2^79
+    x[0, :2], x[0, 2:19] = (top, near), up                  # exact: finite; in order: infinite
+    x[1, :2], x[1, 2:40] = (top, near), down                # exact: infinite; in order: finite
+    x[2, :2] = top, near                                    # finite either way
+    x[3, :3] = top, near, np.float32(2.0 ** 80)             # infinite either way
+    x[4] = rng.standard_normal(n_in) * 3e38 / np.sqrt(n_in) # about one row in three infinite
+    x[5, :2] = top, top
+    return x
+
+
+def test_f16_linear_in_double_sums_at_the_end_of_binary32(hs, oracle):
+    """Where the order of the additions decides whether a sum is the largest binary32 or infinite,
+    the order is the reference's."""
+    g = np.random.default_rng(77)
+    n_out, n_in = 300, 64
+    w16 = g.choice([-1.0, 1.0], (n_out, n_in)).astype(np.float16)
+    w16[:8], w16[8:16] = 1.0, -1.0
+    x = sums_at_the_end_of_binary32(n_in, g)
+    want = oracle.f16_linear_f64(w16.view(np.uint16), x)
+    assert np.isinf(want[0, :16]).all() and np.isfinite(want[1, :16]).all()
+    for m0, m1 in ((0, 6), (0, 1), (1, 2)):
+        y = torch.full((m1 - m0, n_out), 7.0, dtype=torch.float32, device="cuda")
+        hs.f16_linear(to_dev(w16.view(np.int16), torch), to_dev(x[m0:m1], torch), y)
+        hs.sync()
+        got = y.cpu().numpy()
+        assert (bits(got) == bits(want[m0:m1])).all(), np.argwhere(bits(got) != bits(want[m0:m1]))[:8]
+
+
 @pytest.mark.parametrize("m", [2, 9, 19])
 def test_f16_linear_in_double_with_row_strides(hs, oracle, m):
     """Padded rows on both sides (row strides above the row lengths), 19 rows in two passes of the

@@ -10,6 +10,7 @@ import pytest
 from oracle_lib import (oracle_q6k_gemv_x86, oracle_q6k_linear, oracle_q6k_linear_x86,
                         oracle_q8k_quantize, random_q6k_table)
 from test_gpu_host_layer import SessionOpts, host, make_head  # noqa: F401 (fixture)
+from test_gpu_lm_head import sums_at_the_end_of_binary32
 
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
@@ -205,6 +206,31 @@ def test_q6k_linear_with_activations_that_are_not_finite(hs, oracle):
         assert np.array_equal(np.isnan(got), np.isnan(want)), name
         ok = ~np.isnan(want)
         assert np.array_equal(got.view(np.uint32)[ok], want.view(np.uint32)[ok]), name
+
+
+def test_q6k_linear_sums_at_the_end_of_binary32(hs, oracle):
+    """Sums around 2^128 - 2^103 over weights of 1 and -1: whether one is the largest binary32 or
+    infinite is up to the order of the additions, which is the reference's."""
+    g = np.random.default_rng(78)
+    n_out, n_in = 130, 256
+    w = np.zeros((n_out, 210), dtype=np.uint8)
+    w[:, :128], w[:, 128:192], w[:, 192:208] = 0x11, 0xAA, 1    # q - 32 = 1, scales 1, d = 1
+    w[:, 209] = 0x3C
+    w[60:, 209] = 0xBC                                          # d = -1
+    x = sums_at_the_end_of_binary32(n_in, g)
+    want = oracle_q6k_linear(oracle.lib, w, x, n_in)
+    assert np.isinf(want[0]).all() and np.isfinite(want[1]).all()
+    d_w, d_x = torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda()
+    packed = torch.zeros((hs.q6k_packed_bytes(n_out, n_in),), dtype=torch.uint8, device="cuda")
+    hs.q6k_pack(d_w, n_in, packed)
+    for call in (lambda y: hs.q6k_linear(d_w, n_in, d_x, y),
+                 lambda y: hs.q6k_packed_linear(packed, n_out, n_in, d_x, y)):
+        y = torch.full((len(x), n_out), 7.0, dtype=torch.float32, device="cuda")
+        call(y)
+        hs.sync()
+        got = y.cpu().numpy()
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), \
+            np.argwhere(got.view(np.uint32) != want.view(np.uint32))[:8]
 
 
 def test_q6k_argument_errors(hs):
