@@ -50,7 +50,8 @@ constexpr int LDS_STAGES = 160; /* LDS, in KiB: stages times tiles of activation
 
 /* What the projection needs to know of a cut activation row. */
 struct XRow {
-    double unit; /* the value of one unit of the integer sum: 2^-24 times the activations' unit */
+    double unit; /* the value of one unit of the integer sum: 2^-24 times the activations' unit; NaN
+                  * for a row that holds a NaN, and so is every output of it */
     double norm; /* ||x||, rounded up; infinite for a row that is not finite */
     double rest; /* the sum of what the cut left over of each activation, rounded up */
     double pad;
@@ -201,10 +202,20 @@ __global__ __launch_bounds__(XD_TPB) void k_x_digits(const float *__restrict__ x
     if (t == 0) {
         XRow &o = rows[m];
         const double unit = __longlong_as_double((long long) (1023 - 46 + e) << 52);
-        o.unit = unit * 0x1p-24;
+        o.unit = top > 0x7f800000u ? __builtin_nan("") : unit * 0x1p-24;
         o.norm = finite ? sqrt(sq) * (1.0 + 0x1p-40) : (double) __builtin_inff();
         o.rest = rest * unit * (1.0 + 0x1p-40);
     }
+}
+
+/* (float) s, and whether every order of the additions leads there, err bounding what they round
+ * away. Products are exact and their sums far within double's range: a sum that is not finite had
+ * a product that is not, and is the same in any order. */
+__device__ __forceinline__ bool order_is_free(double s, double err, float &f) {
+    if (fabs(s) < __builtin_inf())
+        return f32_rounding_is_safe(s, err, f);
+    f = (float) s;
+    return true;
 }
 
 /* The digits of a lane's sixteen weights (eight dwords q): a weight times 2^24 is a whole number,
@@ -372,7 +383,7 @@ __device__ __forceinline__ void digits_tile(const Rows &rows, const Rows &rows_n
         if (!(w2 < 16000.0f)) /* a weight could be out of the digits' range */
             err = (double) __builtin_inff();
         float f;
-        if (!f32_rounding_is_safe(sum, err, f))
+        if (!order_is_free(sum, err, f))
             list.near[atomicAdd(list.n_near, 1)] = make_int2((int) row_id, m);
         y[m * ld_y + row_id] = f;
         __builtin_amdgcn_sched_barrier(0);
@@ -491,7 +502,7 @@ __global__ __launch_bounds__(LOOK_TPB) void k_f16_linear_look(const uint16_t *__
          * are this sum's error, all the reference's */
         const double rounds = (double) ((n_in + LOOK_COLS - 1) / LOOK_COLS);
         float        f;
-        const bool   ok = f32_rounding_is_safe(
+        const bool   ok = order_is_free(
             base, (own + all + 160.0 * rounds * top) * 0x1p-53 * (1.0 + 0x1p-20), f);
         if (lane == 0) {
             if (ok)

@@ -365,6 +365,64 @@ def test_f16_linear_in_double_sums_at_the_end_of_binary32(hs, oracle):
         assert (bits(got) == bits(want[m0:m1])).all(), np.argwhere(bits(got) != bits(want[m0:m1]))[:8]
 
 
+def f16_linear_us(hs, w16, x, calls=20):
+    """Microseconds of a call of f16_linear, the least of three runs."""
+    y = torch.empty((x.shape[0], w16.shape[0]), dtype=torch.float32, device="cuda")
+    hs.f16_linear(w16, x, y)
+    best = float("inf")
+    for _ in range(3):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        for _ in range(calls):
+            hs.f16_linear(w16, x, y)
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3 / calls)
+    return best
+
+
+@pytest.mark.parametrize("m", [1, 5, 8, 16, 19])
+def test_f16_linear_in_double_with_activations_that_are_not_finite(hs, oracle, m):
+    """A NaN, an infinity, infinities of either sign, all of them, among rows that are finite: each
+    output as the oracle has it, against weights that are zero, NaN and infinite among others."""
+    g = np.random.default_rng(60 + m)
+    n_out, n_in = 900, 264
+    w16 = (g.standard_normal((n_out, n_in)) * 0.05).astype(np.float16)
+    w16[0] = 0
+    w16[1, 3], w16[2, 5], w16[3, 7] = np.nan, np.inf, -np.inf
+    w16[4:200, 9] = 0
+    w16[200:300] *= 100
+    x = (g.standard_normal((m, n_in)) * 3).astype(np.float32)
+    broken = ([(17, np.nan)], [(9, np.inf)], [(9, -np.inf)], [(9, np.inf), (100, -np.inf)],
+              [(5, np.inf), (100, np.inf), (200, np.inf)], [(9, np.inf), (17, np.nan)], [(0, np.nan)])
+    for r in range(m):
+        if m == 1 or r % 2:
+            for at, v in broken[(r // 2) % len(broken)]:
+                x[r, at] = v
+    want = oracle.f16_linear_f64(w16.view(np.uint16), x)
+    y = torch.full((m, n_out), 7.0, dtype=torch.float32, device="cuda")
+    hs.f16_linear(to_dev(w16.view(np.int16), torch), to_dev(x, torch), y)
+    hs.sync()
+    got = y.cpu().numpy()
+    nan = np.isnan(want)
+    assert (np.isnan(got) == nan).all(), np.argwhere(np.isnan(got) != nan)[:5]
+    assert (bits(got)[~nan] == bits(want)[~nan]).all(), np.argwhere(bits(got) != bits(want))[:5]
+
+
+def test_f16_linear_in_double_takes_rows_that_are_not_finite_in_its_stride(hs):
+    """One broken row of a batch does not hold the others up: with a NaN nothing is looked at
+    again (1.0 times the time of finite rows), with an infinity each output of the row once (2.4
+    times). Sent through the sums in index order they took 37 times as long."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    w = torch.empty((64000, 2048), dtype=torch.float16, device="cuda").normal_(0, 0.05, generator=g)
+    w, x = w.view(torch.int16), torch.randn((8, 2048), device="cuda", generator=g)
+    finite = f16_linear_us(hs, w, x)
+    for value, most in ((float("nan"), 2.0), (float("inf"), 6.0)):
+        x[3, 100] = value
+        assert f16_linear_us(hs, w, x) < most * finite, value
+
+
 @pytest.mark.parametrize("m", [2, 9, 19])
 def test_f16_linear_in_double_with_row_strides(hs, oracle, m):
     """Padded rows on both sides (row strides above the row lengths), 19 rows in two passes of the
