@@ -218,20 +218,28 @@ __device__ __forceinline__ bool order_is_free(double s, double err, float &f) {
     return true;
 }
 
+/* v_cvt_i32_f32: towards zero, NaN to 0, what int does not hold to its ends (as a cast, undefined) */
+__device__ __forceinline__ uint32_t to_int(float f) {
+    uint32_t r;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(f));
+    return r;
+}
+
 /* The digits of a lane's sixteen weights (eight dwords q): a weight times 2^24 is a whole number,
  * and adding 0x808080 moves the carries of the three lower signed bytes to their left neighbours, so
  * that each byte less 128 is a digit. The sum is exact in binary32 below 127: a weight of 2^-6 or
  * more has its eleven bits above the 2^7 that the constant ends on. Byte n of four weights then goes
- * to dword i of operand n. */
-__device__ __forceinline__ void weight_digits(const uint32_t (&q)[8], i4v (&d)[4]) {
+ * to dword i of operand n. far: bit 7 of a byte is set if a leading digit lies outside -65 .. 63, for
+ * a weight of 64 or more (a carry from the byte below makes -65 one of the others). */
+__device__ __forceinline__ void weight_digits(const uint32_t (&q)[8], i4v (&d)[4], uint32_t &far) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         uint32_t t[4];
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
             const h2v w  = __builtin_bit_cast(h2v, q[2 * i + k]);
-            t[2 * k]     = (uint32_t) (int) __builtin_fmaf((float) w[0], 0x1p24f, (float) 0x808080);
-            t[2 * k + 1] = (uint32_t) (int) __builtin_fmaf((float) w[1], 0x1p24f, (float) 0x808080);
+            t[2 * k]     = to_int(__builtin_fmaf((float) w[0], 0x1p24f, (float) 0x808080));
+            t[2 * k + 1] = to_int(__builtin_fmaf((float) w[1], 0x1p24f, (float) 0x808080));
         }
         const uint32_t a01 = __builtin_amdgcn_perm(t[1], t[0], 0x05010400u); /* bytes 0, 0, 1, 1 */
         const uint32_t a23 = __builtin_amdgcn_perm(t[3], t[2], 0x05010400u);
@@ -242,6 +250,9 @@ __device__ __forceinline__ void weight_digits(const uint32_t (&q)[8], i4v (&d)[4
         d[2][i] = (int) (__builtin_amdgcn_perm(b23, b01, 0x05040100u) ^ 0x80808080u);
         d[3][i] = (int) __builtin_amdgcn_perm(b23, b01, 0x07060302u);
     }
+#pragma unroll
+    for (int i = 0; i < 4; i += 2)
+        far |= ((uint32_t) d[3][i] + 0x40404040u) | ((uint32_t) d[3][i + 1] + 0x40404040u);
 }
 
 /* A wavefront's weights under way, as they are read: lane l gets columns 8 (l / 8) .. + 7 of a
@@ -280,8 +291,8 @@ __device__ __forceinline__ void ring_take(const uint32_t (&q)[8], uint32_t (&o)[
 }
 
 /* One tile of 16 weight rows against the cut activations. A lane of column group kg holds the sums
- * of its weight row l % 16 and the activation rows kg, kg + 4, ... The outputs of a weight row
- * that could hold a magnitude of 127 or more (||w|| of 126) go to the second kernel. */
+ * of its weight row l % 16 and the activation rows kg, kg + 4, ... The outputs of a weight row with
+ * a magnitude of 64 or more, which the digits may not hold, go to the second kernel. */
 template <int NT, int TPB, bool LDSX, bool FULL>
 __device__ __forceinline__ void digits_tile(const Rows &rows, const Rows &rows_next, long row_id,
                                             long n_out, int n_in, i4v *s_x,
@@ -294,6 +305,7 @@ __device__ __forceinline__ void digits_tile(const Rows &rows, const Rows &rows_n
     constexpr int TURN_X = AHEAD * NT * 64; /* operands of a turn of the ring */
     i4v       acc[WDIGITS][NT];
     f4v       nrm = {0.0f, 0.0f, 0.0f, 0.0f};
+    uint32_t  far = 0;
 #pragma unroll
     for (int d = 0; d < WDIGITS; ++d)
 #pragma unroll
@@ -322,7 +334,7 @@ __device__ __forceinline__ void digits_tile(const Rows &rows, const Rows &rows_n
                 i4v      d[WDIGITS];
                 uint32_t q[8];
                 ring_take(ring.q[u], q);
-                weight_digits(q, d);
+                weight_digits(q, d, far);
                 /* ||w||^2 on the diagonal of the tile times itself */
                 const h8v h0 = __builtin_bit_cast(h8v, (u4v){q[0], q[1], q[2], q[3]});
                 const h8v h1 = __builtin_bit_cast(h8v, (u4v){q[4], q[5], q[6], q[7]});
@@ -353,6 +365,9 @@ __device__ __forceinline__ void digits_tile(const Rows &rows, const Rows &rows_n
     const int   j  = lane & 15;
     const float v0 = (j & 2) ? ((j & 1) ? nrm[3] : nrm[2]) : ((j & 1) ? nrm[1] : nrm[0]);
     const float w2 = __shfl(v0, (j >> 2) * 16 + j);
+    far |= (uint32_t) __shfl_xor((int) far, 16);
+    far |= (uint32_t) __shfl_xor((int) far, 32);
+    const bool digits_hold = (far & 0x80808080u) == 0 && w2 < __builtin_inff(); /* (no NaN either) */
     /* rounded up by more than the binary32 sum's error and than what subnormal weights, were the
      * matrix cores to drop them, could add */
     const double wn = (double) __builtin_sqrtf(w2) * (1.0 + 1e-4 + (double) n_in * 0x1p-22) +
@@ -379,11 +394,9 @@ __device__ __forceinline__ void digits_tile(const Rows &rows, const Rows &rows_n
         const double mid = (double) ((T[3] << 8) + T[2]);
         const double lo  = (double) ((T[1] << 8) + T[0]);
         const double sum = __builtin_fma(hi, 0x1p32, __builtin_fma(mid, 0x1p16, lo)) * xr.unit;
-        double       err = (double) (n_in + 16) * 0x1p-53 * 1.01 * wn * xr.norm + 128.0 * xr.rest;
-        if (!(w2 < 16000.0f)) /* a weight could be out of the digits' range */
-            err = (double) __builtin_inff();
-        float f;
-        if (!order_is_free(sum, err, f))
+        const double err = (double) (n_in + 16) * 0x1p-53 * 1.01 * wn * xr.norm + 128.0 * xr.rest;
+        float        f;
+        if (!order_is_free(sum, err, f) || !digits_hold)
             list.near[atomicAdd(list.n_near, 1)] = make_int2((int) row_id, m);
         y[m * ld_y + row_id] = f;
         __builtin_amdgcn_sched_barrier(0);

@@ -423,6 +423,44 @@ def test_f16_linear_in_double_takes_rows_that_are_not_finite_in_its_stride(hs):
         assert f16_linear_us(hs, w, x) < most * finite, value
 
 
+@pytest.mark.parametrize("m,n_in", [(2, 520), (8, 256), (16, 72), (6, 3528)])
+def test_f16_linear_in_double_with_large_weights(hs, oracle, m, n_in):
+    """Weights around the ends of what the leading digit and the conversion hold (64, 127, 2^7),
+    alone in their rows and in each column of a group of sixteen, and rows of a large norm."""
+    g = np.random.default_rng(90 + m)
+    ends = np.array([62.5, 63.0, 63.47, 63.5, 63.97, 64.0, 64.5, 65.0, 65.47, 65.5, 66.0, 126.9,
+                     127.0, 127.44, 127.5, 127.94, 128.0, 128.5, 129.0, 255.9, 1000.0, 65504.0])
+    ends = np.concatenate([ends, -ends])
+    n_out = 3 * len(ends) + 200
+    w16 = (g.standard_normal((n_out, n_in)) * 0.05).astype(np.float16)
+    for i, e in enumerate(ends):
+        w16[i, g.integers(0, n_in)] = e
+        w16[len(ends) + i, i % 16 + 16 * g.integers(0, n_in // 16)] = e
+        w16[2 * len(ends) + i, ::3] = e
+    w16[-200:] = (g.standard_normal((200, n_in)) * g.choice([3.0, 10.0, 30.0], (200, 1))).astype(np.float16)
+    x = (g.standard_normal((m, n_in)) * 3).astype(np.float32)
+    y = torch.full((m, n_out), 7.0, dtype=torch.float32, device="cuda")
+    hs.f16_linear(to_dev(w16.view(np.int16), torch), to_dev(x, torch), y)
+    hs.sync()
+    want = oracle.f16_linear_f64(w16.view(np.uint16), x)
+    got = y.cpu().numpy()
+    assert (bits(got) == bits(want)).all(), np.argwhere(bits(got) != bits(want))[:5]
+
+
+def test_f16_linear_in_double_takes_rows_of_a_large_norm_in_its_stride(hs):
+    """It is a single weight's magnitude that the digits are bound by, not a row's norm: a table
+    of standard deviation 4 takes what one of 0.05 takes (8 times as long when rows of a norm
+    above 126 were left to the second kernel)."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(4)
+    x = torch.randn((8, 2048), device="cuda", generator=g)
+    us = []
+    for std in (0.05, 4.0):
+        w = torch.empty((64000, 2048), dtype=torch.float16, device="cuda").normal_(0, std, generator=g)
+        us.append(f16_linear_us(hs, w.view(torch.int16), x))
+    assert us[1] < 2 * us[0], us
+
+
 @pytest.mark.parametrize("m", [2, 9, 19])
 def test_f16_linear_in_double_with_row_strides(hs, oracle, m):
     """Padded rows on both sides (row strides above the row lengths), 19 rows in two passes of the
