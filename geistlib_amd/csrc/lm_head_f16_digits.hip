@@ -229,9 +229,8 @@ __device__ __forceinline__ uint32_t to_int(float f) {
  * and adding 0x808080 moves the carries of the three lower signed bytes to their left neighbours, so
  * that each byte less 128 is a digit. The sum is exact in binary32 below 127: a weight of 2^-6 or
  * more has its eleven bits above the 2^7 that the constant ends on. Byte n of four weights then goes
- * to dword i of operand n. far: bit 7 of a byte is set if a leading digit lies outside -65 .. 63, for
- * a weight of 64 or more (a carry from the byte below makes -65 one of the others). */
-__device__ __forceinline__ void weight_digits(const uint32_t (&q)[8], i4v (&d)[4], uint32_t &far) {
+ * to dword i of operand n. */
+__device__ __forceinline__ void weight_digits(const uint32_t (&q)[8], i4v (&d)[4]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         uint32_t t[4];
@@ -250,9 +249,6 @@ __device__ __forceinline__ void weight_digits(const uint32_t (&q)[8], i4v (&d)[4
         d[2][i] = (int) (__builtin_amdgcn_perm(b23, b01, 0x05040100u) ^ 0x80808080u);
         d[3][i] = (int) __builtin_amdgcn_perm(b23, b01, 0x07060302u);
     }
-#pragma unroll
-    for (int i = 0; i < 4; i += 2)
-        far |= ((uint32_t) d[3][i] + 0x40404040u) | ((uint32_t) d[3][i + 1] + 0x40404040u);
 }
 
 /* A wavefront's weights under way, as they are read: lane l gets columns 8 (l / 8) .. + 7 of a
@@ -291,8 +287,9 @@ __device__ __forceinline__ void ring_take(const uint32_t (&q)[8], uint32_t (&o)[
 }
 
 /* One tile of 16 weight rows against the cut activations. A lane of column group kg holds the sums
- * of its weight row l % 16 and the activation rows kg, kg + 4, ... The outputs of a weight row with
- * a magnitude of 64 or more, which the digits may not hold, go to the second kernel. */
+ * of its weight row l % 16 and the activation rows kg, kg + 4, ... The outputs of a weight row that
+ * could hold a magnitude of 127 or more go to the second kernel: one with a norm of 126 or more in
+ * some turn of the ring (256 columns). */
 template <int NT, int TPB, bool LDSX, bool FULL>
 __device__ __forceinline__ void digits_tile(const Rows &rows, const Rows &rows_next, long row_id,
                                             long n_out, int n_in, i4v *s_x,
@@ -304,8 +301,8 @@ __device__ __forceinline__ void digits_tile(const Rows &rows, const Rows &rows_n
     const int n_stage = (n_in + STAGE_K - 1) / STAGE_K;
     constexpr int TURN_X = AHEAD * NT * 64; /* operands of a turn of the ring */
     i4v       acc[WDIGITS][NT];
-    f4v       nrm = {0.0f, 0.0f, 0.0f, 0.0f};
-    uint32_t  far = 0;
+    const int j  = lane & 15;
+    float     w2 = 0.0f, turn_w2 = 0.0f; /* ||w||^2 of row j of the tile, and the largest of a turn */
 #pragma unroll
     for (int d = 0; d < WDIGITS; ++d)
 #pragma unroll
@@ -321,6 +318,7 @@ __device__ __forceinline__ void digits_tile(const Rows &rows, const Rows &rows_n
         /* the activations of this turn, and the next turn's on their way */
         const i4v *xd = LDSX ? s_x + s0 * NT * 64 : s_x + buf * TURN_X;
         i4v        xn[LDSX ? 1 : (TURN_X + TPB - 1) / TPB];
+        f4v        nrm = {0.0f, 0.0f, 0.0f, 0.0f};
         if (!LDSX) {
 #pragma unroll
             for (int i = 0; i < (TURN_X + TPB - 1) / TPB; ++i) {
@@ -334,7 +332,7 @@ __device__ __forceinline__ void digits_tile(const Rows &rows, const Rows &rows_n
                 i4v      d[WDIGITS];
                 uint32_t q[8];
                 ring_take(ring.q[u], q);
-                weight_digits(q, d, far);
+                weight_digits(q, d);
                 /* ||w||^2 on the diagonal of the tile times itself */
                 const h8v h0 = __builtin_bit_cast(h8v, (u4v){q[0], q[1], q[2], q[3]});
                 const h8v h1 = __builtin_bit_cast(h8v, (u4v){q[4], q[5], q[6], q[7]});
@@ -352,6 +350,10 @@ __device__ __forceinline__ void digits_tile(const Rows &rows, const Rows &rows_n
                 ring_load<FULL>(src, u, last - s1 * STAGE_K, ring.q[u]);
             __builtin_amdgcn_sched_barrier(0); /* (stages mixed together would not fit the registers) */
         }
+        /* the lane of column group j / 4 holds, in register j % 4, the square of row j */
+        const float v0 = (j & 2) ? ((j & 1) ? nrm[3] : nrm[2]) : ((j & 1) ? nrm[1] : nrm[0]);
+        w2 += v0;
+        turn_w2 = __builtin_fmaxf(turn_w2, v0);
         if (!LDSX) {
             buf ^= 1;
 #pragma unroll
@@ -361,13 +363,9 @@ __device__ __forceinline__ void digits_tile(const Rows &rows, const Rows &rows_n
             lds_barrier();
         }
     }
-    /* the lane of column group j / 4 holds, in register j % 4, the square of row j */
-    const int   j  = lane & 15;
-    const float v0 = (j & 2) ? ((j & 1) ? nrm[3] : nrm[2]) : ((j & 1) ? nrm[1] : nrm[0]);
-    const float w2 = __shfl(v0, (j >> 2) * 16 + j);
-    far |= (uint32_t) __shfl_xor((int) far, 16);
-    far |= (uint32_t) __shfl_xor((int) far, 32);
-    const bool digits_hold = (far & 0x80808080u) == 0 && w2 < __builtin_inff(); /* (no NaN either) */
+    w2      = __shfl(w2, (j >> 2) * 16 + j);
+    turn_w2 = __shfl(turn_w2, (j >> 2) * 16 + j);
+    const bool digits_hold = turn_w2 < 16000.0f && w2 < __builtin_inff(); /* (no NaN either) */
     /* rounded up by more than the binary32 sum's error and than what subnormal weights, were the
      * matrix cores to drop them, could add */
     const double wn = (double) __builtin_sqrtf(w2) * (1.0 + 1e-4 + (double) n_in * 0x1p-22) +
