@@ -54,7 +54,9 @@ struct XRow {
                   * for a row that holds a NaN, and so is every output of it */
     double norm; /* ||x||, rounded up; infinite for a row that is not finite */
     double rest; /* the sum of what the cut left over of each activation, rounded up */
-    double pad;
+    double exact_to; /* products whose magnitudes add up to less add without rounding, in any order:
+                      * they are multiples of 2^-24 times the largest power of two that the
+                      * activations are multiples of, and this is 2^53 of that */
 };
 static_assert(sizeof(XRow) == F16_XROW_BYTES, "the scratch is sized by the caller");
 
@@ -104,6 +106,7 @@ __global__ __launch_bounds__(XD_TPB) void k_x_digits(const float *__restrict__ x
                                                      F64Lists list) {
     __shared__ double   s_d[3][XD_TPB / 64];
     __shared__ uint32_t s_u[XD_TPB / 64];
+    __shared__ uint32_t s_z[XD_TPB / 64];
     __shared__ float    s_inv;
     const int    m = blockIdx.x, t = threadIdx.x;
     const float *xr = x + (long) m * ld_x;
@@ -146,11 +149,7 @@ __global__ __launch_bounds__(XD_TPB) void k_x_digits(const float *__restrict__ x
             top              = b > top ? b : top;
         }
     }
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) {
-        const uint32_t o = (uint32_t) __shfl_xor((int) top, d);
-        top              = o > top ? o : top;
-    }
+    top = wave_max_u32(top);
     if ((t & 63) == 0)
         s_u[t >> 6] = top;
     sq = xd_block_sum(sq, s_d[1]); /* (its barrier is s_u's too) */
@@ -163,6 +162,7 @@ __global__ __launch_bounds__(XD_TPB) void k_x_digits(const float *__restrict__ x
     const double scale = __longlong_as_double((long long) (1023 + 46 - e) << 52);
     const int    g = m & 3, p0 = XDIGITS * (m >> 2);
     double       rest = 0.0;
+    long long    any  = 0; /* the integers' bits */
     for (int i = t; i < n_group; i += XD_TPB) {
         uint32_t lo[XDIGITS] = {}, hi[XDIGITS] = {};
         if (i < n8 && finite) {
@@ -179,6 +179,7 @@ __global__ __launch_bounds__(XD_TPB) void k_x_digits(const float *__restrict__ x
                 const double r = f + 0x1.8p52; /* the integer, in the low bits */
                 rest += fabs(f - (r - 0x1.8p52));
                 long long k = __double_as_longlong(r) - __double_as_longlong(0x1.8p52);
+                any |= k;
 #pragma unroll
                 for (int d = 0; d < XDIGITS; ++d) {
                     const int b = (int) (int8_t) k;
@@ -198,13 +199,21 @@ __global__ __launch_bounds__(XD_TPB) void k_x_digits(const float *__restrict__ x
             *reinterpret_cast<uint2 *>(o) = make_uint2(lo[d], hi[d]);
         }
     }
-    rest = xd_block_sum(rest, s_d[2]);
+    /* 64 less the number of bits that are zero at the end of all integers; 0 if they are zeros */
+    const uint32_t ends = wave_max_u32(any ? 64u - (uint32_t) __builtin_ctzll((unsigned long long) any) : 0u);
+    if ((t & 63) == 0)
+        s_z[t >> 6] = ends;
+    rest = xd_block_sum(rest, s_d[2]); /* (its barrier is s_z's too) */
     if (t == 0) {
+        uint32_t z = s_z[0];
+        for (int i = 1; i < XD_TPB / 64; ++i)
+            z = s_z[i] > z ? s_z[i] : z;
         XRow &o = rows[m];
         const double unit = __longlong_as_double((long long) (1023 - 46 + e) << 52);
         o.unit = top > 0x7f800000u ? __builtin_nan("") : unit * 0x1p-24;
         o.norm = finite ? sqrt(sq) * (1.0 + 0x1p-40) : (double) __builtin_inff();
         o.rest = rest * unit * (1.0 + 0x1p-40);
+        o.exact_to = rest == 0.0 ? ldexp(unit, 53 - 24 + 64 - (int) z) : 0.0;
     }
 }
 
@@ -457,14 +466,19 @@ __global__ void k_f16_linear_list_all(long n_out, int n_m, F64Lists list) {
  * on average. Here the lanes add eight products each per 512 columns, a scan puts their sums
  * together, and u sum |S_k| over all partial sums S_k, which the lanes then know, bounds what the
  * reference's additions round away; of 2850 listed outputs (8 x 128256, 2560 columns) about 30
- * stay open. 14.6 MB in rows scattered over the table: five loads of a row in flight at once. */
+ * stay open. 14.6 MB in rows scattered over the table: five loads of a row in flight at once.
+ * Activations of few bits, an int8's or a bfloat16's, put many sums right on a boundary, but their
+ * additions round nothing away (XRow::exact_to): left open all the same, they made a batch of
+ * integers up to 127 take 1300 us (8 x 128256 x 2560), now 240. */
 constexpr int LOOK_TPB   = 256;
 constexpr int LOOK_COLS  = 8 * 64; /* of a row per round of the wavefront */
 constexpr int LOOK_AHEAD = 5;      /* rounds whose loads are requested together */
 __global__ __launch_bounds__(LOOK_TPB) void k_f16_linear_look(const uint16_t *__restrict__ w,
                                                               int n_in, const float *__restrict__ x,
-                                                              long ld_x, float *__restrict__ y,
-                                                              long ld_y, F64Lists list) {
+                                                              long ld_x,
+                                                              const XRow *__restrict__ xrow,
+                                                              float *__restrict__ y, long ld_y,
+                                                              F64Lists list) {
     const int lane = threadIdx.x & 63, count = *list.n_near;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     for (int it = (int) blockIdx.x * (LOOK_TPB / 64) + wave; it < count;
@@ -473,6 +487,7 @@ __global__ __launch_bounds__(LOOK_TPB) void k_f16_linear_look(const uint16_t *__
         const uint16_t *wr = w + (long) mine.x * n_in;
         const float    *xm = x + (long) mine.y * ld_x;
         const bool      vx = ((uintptr_t) xm & 15) == 0;
+        const double    exact_to = xrow ? xrow[mine.y].exact_to : 0.0;
         double          base = 0.0, own = 0.0, all = 0.0, top = 0.0;
         for (int k0 = 0; k0 < n_in; k0 += LOOK_COLS * LOOK_AHEAD) {
             h8v   h[LOOK_AHEAD];
@@ -510,11 +525,13 @@ __global__ __launch_bounds__(LOOK_TPB) void k_f16_linear_look(const uint16_t *__
             top = fmax(top, __shfl_xor(top, d));
         }
         /* own and the scans' additions (63 and one per round, of values up to twice the largest)
-         * are this sum's error, all the reference's */
+         * are this sum's error, all the reference's. (A product is at most the sums in front of and
+         * behind it: their magnitudes add up to 2 own at most.) */
         const double rounds = (double) ((n_in + LOOK_COLS - 1) / LOOK_COLS);
         float        f;
         const bool   ok = order_is_free(
-            base, (own + all + 160.0 * rounds * top) * 0x1p-53 * (1.0 + 0x1p-20), f);
+                              base, (own + all + 160.0 * rounds * top) * 0x1p-53 * (1.0 + 0x1p-20), f) ||
+                          2.0 * own * (1.0 + 0x1p-30) < exact_to;
         if (lane == 0) {
             if (ok)
                 y[mine.y * ld_y + mine.x] = f;
@@ -665,7 +682,8 @@ static void f16_linear_pass(hipStream_t stream, const uint16_t *w_f16, long n_ou
         launch_digits<3, 768>(stream, w_f16, n_out, n_in, xdig, xrow, n_m, y, ld_y, ws.list);
     else
         launch_digits<6, 512>(stream, w_f16, n_out, n_in, xdig, xrow, n_m, y, ld_y, ws.list);
-    k_f16_linear_look<<<dim3(1024), dim3(LOOK_TPB), 0, stream>>>(w_f16, n_in, x, ld_x, y, ld_y, ws.list);
+    k_f16_linear_look<<<dim3(1024), dim3(LOOK_TPB), 0, stream>>>(
+        w_f16, n_in, x, ld_x, n_in > F16_DIGITS_MAX_IN ? nullptr : xrow, y, ld_y, ws.list);
     k_f16_linear_listed<<<dim3(128), dim3(LISTED_TPB), 0, stream>>>(w_f16, n_in, x, ld_x, y, ld_y, ws.list);
 }
 
