@@ -143,7 +143,7 @@ __device__ __forceinline__ void row_sums_meet(uint64_t *row_slots, int chunk, in
     __syncthreads();
 }
 
-template <int NV, bool PEN, bool PLAIN>
+template <int NV, bool PEN, bool RNG, bool PLAIN>
 __device__ __forceinline__ void draw_chunk(const RowView &rv, int row, int chunk, int n_rows,
                                            int base, int end, float inv_t,
                                            const float *__restrict__ uniforms,
@@ -158,7 +158,7 @@ __device__ __forceinline__ void draw_chunk(const RowView &rv, int row, int chunk
     /* the row's draw, for the first wavefront: given, or the next of the row's generator */
     float    u_row = 0.0f;
     uint64_t state = 0;
-    if (rng.states == nullptr)
+    if (!RNG)
         u_row = uniforms[row];
     else if (tid < WAVE)
         state = __hip_atomic_load(rng.states + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -256,12 +256,16 @@ __device__ __forceinline__ void draw_chunk(const RowView &rv, int row, int chunk
      * meetings, whose polls would wait for its answer. */
     uint32_t counted = 0;
     if (tid < WAVE) {
-        if (rng.states != nullptr) {
-            uint32_t one = 1u;
-            asm volatile("" : "+v"(one) : "v"(state)); /* not before the state has arrived */
+        if (RNG) {
+            uint32_t most = (uint32_t) (C - 1);
+            /* counted when the state has arrived, which is waited for here and not before */
+            asm volatile("" : "+v"(most), "+v"(state));
+            /* (an increment that wraps to 0 behind the last: nothing to reset, and the compiler leaves
+             * it alone; of an addition it makes one for the wavefront that waits for its answer,
+             * 0.35 us) */
             if (tid == 0)
-                counted = __hip_atomic_fetch_add(rng.arrive + (long) row * ARRIVE_STRIDE_INTS, one,
-                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                counted = __builtin_amdgcn_atomic_inc32(rng.arrive + (long) row * ARRIVE_STRIDE_INTS, most,
+                                                        __ATOMIC_RELAXED, "agent");
             u_row = xorshift_unit(state);
         }
         double    run, target;
@@ -279,11 +283,8 @@ __device__ __forceinline__ void draw_chunk(const RowView &rv, int row, int chunk
         }
     }
     __syncthreads();
-    if (rng.states != nullptr && tid == 0 && counted == (uint32_t) (C - 1)) {
-        __hip_atomic_store(rng.arrive + (long) row * ARRIVE_STRIDE_INTS, 0u, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
+    if (RNG && tid == 0 && counted == (uint32_t) (C - 1))
         rng.states[row] = state;
-    }
     if (sh.walk.chunk != chunk)
         return; /* another workgroup's */
     const double target = sh.walk.target;
@@ -320,7 +321,9 @@ __device__ __forceinline__ void draw_chunk(const RowView &rv, int row, int chunk
         out[row] = tok;
 }
 
-template <int NV, bool PEN>
+/* RNG: the draws come from the rows' generators, else from `uniforms`. (As a run-time choice it cost
+ * calls with given draws 0.2-0.3 us: one row of 32000 with penalties 6.98 -> 7.17, two 6.96 -> 7.29.) */
+template <int NV, bool PEN, bool RNG>
 __global__ __launch_bounds__(TPB) void k_temperature_draw(RowView rv, int n_rows, float inv_t,
                                                           const float *__restrict__ uniforms,
                                                           RowGenerators rng,
@@ -362,10 +365,10 @@ __global__ __launch_bounds__(TPB) void k_temperature_draw(RowView rv, int n_rows
     const bool plain = rv.vec_ok && end - base == NV * TPB * 4 && !(rv.softcap > 0.0f) &&
                        rv.allowed == nullptr;
     if (plain)
-        draw_chunk<NV, PEN, true>(rv, row, chunk, n_rows, base, end, inv_t, uniforms, rng, out,
+        draw_chunk<NV, PEN, RNG, true>(rv, row, chunk, n_rows, base, end, inv_t, uniforms, rng, out,
                                   sum_slots, s_cnt16, s_sum, s_tab, tabv, s_tr, s_draw, fs);
     else
-        draw_chunk<NV, PEN, false>(rv, row, chunk, n_rows, base, end, inv_t, uniforms, rng, out,
+        draw_chunk<NV, PEN, RNG, false>(rv, row, chunk, n_rows, base, end, inv_t, uniforms, rng, out,
                                    sum_slots, s_cnt16, s_sum, s_tab, tabv, s_tr, s_draw, fs);
 }
 

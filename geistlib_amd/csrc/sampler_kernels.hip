@@ -1965,10 +1965,13 @@ void launch_temperature_draw(const Launch &L, float inv_t, const float *uniforms
      * eights, so that the workgroups of a row have linear ids equal modulo 8 and share an XCD
      * (xcd_row_chunk); the workgroups of the rows that are not there leave at once. */
     const dim3 grid(L.rv.n_chunks, (L.rows + 7) & ~7), block(TPB);
-    if (L.pen)
-        k_temperature_draw<2, true><<<grid, block, 0, L.stream>>>(L.rv, L.rows, inv_t, uniforms, rng, out, meet);
+    auto go = [&](auto kernel) {
+        kernel<<<grid, block, 0, L.stream>>>(L.rv, L.rows, inv_t, uniforms, rng, out, meet);
+    };
+    if (rng.states != nullptr)
+        L.pen ? go(k_temperature_draw<2, true, true>) : go(k_temperature_draw<2, false, true>);
     else
-        k_temperature_draw<2, false><<<grid, block, 0, L.stream>>>(L.rv, L.rows, inv_t, uniforms, rng, out, meet);
+        L.pen ? go(k_temperature_draw<2, true, false>) : go(k_temperature_draw<2, false, false>);
 }
 
 void launch_spec(const Launch &L, const SpecLaunch &sp, const MeetSpace *meet) {
