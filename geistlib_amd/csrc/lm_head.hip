@@ -407,26 +407,41 @@ __global__ __launch_bounds__(LM_TPB) void k_f16_gemv_batched(const uint16_t *__r
  * a double sum only shows in the binary32 result when 1 / sqrt(mean + eps) lies within the
  * sum's error of the middle between two binary32 values. The workgroup adds in a fixed parallel
  * order and, in that rare case, one thread repeats the sum in the reference's order. */
-__global__ __launch_bounds__(NORM_TPB) void k_rmsnorm_rows(const float *__restrict__ x, long ld_x,
-                                                           const float *__restrict__ w, float eps,
-                                                           int n, float *__restrict__ y, long ld_y) {
+template <int TPB, int PER>
+__global__ __launch_bounds__(TPB) void k_rmsnorm_rows(const float *__restrict__ x, long ld_x,
+                                                      const float *__restrict__ w, float eps, int n,
+                                                      float *__restrict__ y, long ld_y) {
     __shared__ NormShared s_norm;
     const int    tid = threadIdx.x;
     const float *xr  = x + (long) blockIdx.x * ld_x;
     float       *yr  = y + (long) blockIdx.x * ld_y;
-    float        v[NORM_PER];
-    const float  inv = block_rmsnorm(xr, w, n, eps, v, s_norm);
+    float        v[PER];
+    const float  inv = block_rmsnorm<TPB, PER>(xr, w, n, eps, v, s_norm);
 #pragma unroll
-    for (int k = 0; k < NORM_PER; ++k)
-        if (k * NORM_TPB + tid < n)
-            yr[k * NORM_TPB + tid] = v[k];
-    for (int i = NORM_PER * NORM_TPB + tid; i < n; i += NORM_TPB)
+    for (int k = 0; k < PER; ++k)
+        if (k * TPB + tid < n)
+            yr[k * TPB + tid] = v[k];
+    for (int i = PER * TPB + tid; i < n; i += TPB)
         yr[i] = __fmul_rn(__fmul_rn(xr[i], inv), w[i]);
 }
 
 void launch_rmsnorm_rows(hipStream_t stream, const float *x, long ld_x, const float *w, float eps,
                          int n_rows, int n, float *y, long ld_y) {
-    k_rmsnorm_rows<<<dim3(n_rows), dim3(NORM_TPB), 0, stream>>>(x, ld_x, w, eps, n, y, ld_y);
+    auto go = [&](auto kernel, int tpb) {
+        kernel<<<dim3(n_rows), dim3(tpb), 0, stream>>>(x, ld_x, w, eps, n, y, ld_y);
+    };
+    /* No more threads than hold a short row, and beyond the 512 rows that are at work at a time with
+     * 1024 threads each, 256: many rows want many workgroups, few long ones all threads. 4096 rows
+     * of 64 elements 4.9 us (16.6 with 1024 threads), of 1024 6.9 (18.0), of 2560 13.4 (20.7); 512
+     * rows of 2560 4.8 (5.5 with 256), of 4096 4.9 (7.2). */
+    if (n <= 256)
+        go(k_rmsnorm_rows<64, 4>, 64);
+    else if (n <= 1024)
+        go(k_rmsnorm_rows<256, 4>, 256);
+    else if (n_rows > 512 && n <= 4096)
+        go(k_rmsnorm_rows<256, 16>, 256);
+    else
+        go(k_rmsnorm_rows<NORM_TPB, NORM_PER>, NORM_TPB);
 }
 
 bool f16_gemv_can_fuse(int n_m) { return n_m >= 1 && n_m <= 2; }

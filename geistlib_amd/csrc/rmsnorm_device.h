@@ -25,7 +25,7 @@ __device__ __forceinline__ float rms_inv_sequential(const float *__restrict__ xr
     return (float) (1.0 / sqrt(sumsq / (double) n + (double) eps));
 }
 
-/* The threads that norm one row. One row is one workgroup's work, and it is latency that it takes:
+/* The threads that norm one row where there are few rows. One row is one workgroup's work, and it is latency that it takes:
  * the row's and the weights' elements are asked for at once, four of each per thread, and stay in
  * registers. 256 threads that looped over memory twice, and added their sums through LDS in eight
  * barriers, took 10.7 us of a cold step for the norm of 2560 elements where this takes 4.7 (4.6 is
@@ -39,28 +39,29 @@ struct NormShared {
     float  inv;
 };
 
-/* The inverse RMS of xr[0..n) for a workgroup of NORM_TPB threads, every thread gets it, and in
- * v[k] the normed element (x inv) w at k NORM_TPB + tid (0 from n on); elements from
- * NORM_PER NORM_TPB on are the caller's. The squares are added in double in a fixed parallel order
+/* The inverse RMS of xr[0..n) for a workgroup of TPB threads, every thread gets it, and in
+ * v[k] the normed element (x inv) w at k TPB + tid (0 from n on); elements from PER TPB on are the
+ * caller's. The squares are added in double in a fixed parallel order
  * (a thread's elements ascending, then a butterfly over the lanes and over the wavefronts) and,
  * where the binary32 result could depend on the order, once more by one thread in the reference's
  * order. One call per launch (s is not given free for another). */
+template <int TPB = NORM_TPB, int PER = NORM_PER>
 __device__ __forceinline__ float block_rmsnorm(const float *__restrict__ xr,
                                                const float *__restrict__ w, int n, float eps,
-                                               float (&v)[NORM_PER], NormShared &s) {
+                                               float (&v)[PER], NormShared &s) {
     const int tid = threadIdx.x;
-    float     wv[NORM_PER];
+    float     wv[PER];
 #pragma unroll
-    for (int k = 0; k < NORM_PER; ++k) {
-        const int i = k * NORM_TPB + tid;
+    for (int k = 0; k < PER; ++k) {
+        const int i = k * TPB + tid;
         v[k]        = i < n ? xr[i] : 0.0f;
         wv[k]       = i < n ? w[i] : 0.0f;
     }
     double a = 0.0;
 #pragma unroll
-    for (int k = 0; k < NORM_PER; ++k)
+    for (int k = 0; k < PER; ++k)
         a += (double) v[k] * (double) v[k];
-    for (int i = NORM_PER * NORM_TPB + tid; i < n; i += NORM_TPB)
+    for (int i = PER * TPB + tid; i < n; i += TPB)
         a += (double) xr[i] * (double) xr[i];
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1)
@@ -69,9 +70,9 @@ __device__ __forceinline__ float block_rmsnorm(const float *__restrict__ xr,
         s.part[tid >> 6] = a;
     __syncthreads();
     if (tid < 64) {
-        a = s.part[tid & (NORM_TPB / 64 - 1)];
+        a = s.part[tid & (TPB / 64 - 1)];
 #pragma unroll
-        for (int d = NORM_TPB / 128; d >= 1; d >>= 1)
+        for (int d = TPB / 128; d >= 1; d >>= 1)
             a += __shfl_xor(a, d);
         if (tid == 0) {
             float f;
@@ -83,7 +84,7 @@ __device__ __forceinline__ float block_rmsnorm(const float *__restrict__ xr,
     __syncthreads();
     const float inv = s.inv;
 #pragma unroll
-    for (int k = 0; k < NORM_PER; ++k)
+    for (int k = 0; k < PER; ++k)
         v[k] = __fmul_rn(__fmul_rn(v[k], inv), wv[k]);
     return inv;
 }

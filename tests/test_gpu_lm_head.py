@@ -25,6 +25,21 @@ def bits(a):
     return np.ascontiguousarray(a, dtype=np.float32).view(np.uint32)
 
 
+def call_us(call, calls):
+    """Microseconds of a call among others, the least of three runs."""
+    call()
+    best = float("inf")
+    for _ in range(3):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        for _ in range(calls):
+            call()
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3 / calls)
+    return best
+
+
 def run_gemv(hs, w16, x):
     d_w = to_dev(w16.view(np.int16), torch)
     d_x = to_dev(x, torch)
@@ -86,6 +101,30 @@ def test_f16_gemv_strides_and_errors(hs, oracle):
     bad = torch.zeros((4, 20), dtype=torch.float16, device="cuda")        # n_in % 8 != 0
     with pytest.raises(GeistHipError):
         hs.f16_gemv(bad, torch.zeros((1, 20), device="cuda"), torch.zeros((1, 4), device="cuda"))
+
+
+@pytest.mark.parametrize("rows,n", [(3, 1), (2, 255), (2, 256), (2, 257), (2, 1024), (2, 1025),
+                                    (512, 1030), (513, 1030), (513, 4095), (513, 4096), (513, 4097),
+                                    (2, 4097), (700, 40)])
+def test_rmsnorm_rows_at_the_edges_of_the_workgroup_sizes(hs, oracle, rows, n):
+    """Rows on both sides of what 64, 256 and 1024 threads hold, and of the number of rows that
+    chooses between the latter two: every bit as the oracle has it."""
+    g = np.random.default_rng(rows + n)
+    x = (g.standard_normal((rows, n)) * 3).astype(np.float32)
+    w = (1 + 0.1 * g.standard_normal(n)).astype(np.float32)
+    y = torch.full((rows, n), 7.0, dtype=torch.float32, device="cuda")
+    hs.rmsnorm(to_dev(x, torch), to_dev(w, torch), 1e-6, y)
+    hs.sync()
+    assert (bits(y.cpu().numpy()) == bits(oracle.rmsnorm(x, w, 1e-6))).all()
+
+
+def test_rmsnorm_of_many_short_rows_is_a_launch(hs):
+    """4096 rows of 256 elements take what 512 take (3.5 times that with 1024 threads a row)."""
+    w = torch.ones(256, device="cuda")
+    x = [torch.randn((rows, 256), device="cuda") for rows in (512, 4096)]
+    y = [torch.empty_like(t) for t in x]
+    us = [call_us(lambda: hs.rmsnorm(a, w, 1e-6, b), 200) for a, b in zip(x, y)]
+    assert us[1] < 2 * us[0], us
 
 
 @pytest.mark.parametrize("rows,n", [(1, 2560), (5, 1536), (17, 4096), (3, 7), (2, 300)])
@@ -365,20 +404,9 @@ def test_f16_linear_in_double_sums_at_the_end_of_binary32(hs, oracle):
         assert (bits(got) == bits(want[m0:m1])).all(), np.argwhere(bits(got) != bits(want[m0:m1]))[:8]
 
 
-def f16_linear_us(hs, w16, x, calls=20):
-    """Microseconds of a call of f16_linear, the least of three runs."""
+def f16_linear_us(hs, w16, x):
     y = torch.empty((x.shape[0], w16.shape[0]), dtype=torch.float32, device="cuda")
-    hs.f16_linear(w16, x, y)
-    best = float("inf")
-    for _ in range(3):
-        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
-        a.record()
-        for _ in range(calls):
-            hs.f16_linear(w16, x, y)
-        b.record()
-        torch.cuda.synchronize()
-        best = min(best, a.elapsed_time(b) * 1e3 / calls)
-    return best
+    return call_us(lambda: hs.f16_linear(w16, x, y), 20)
 
 
 @pytest.mark.parametrize("m", [1, 5, 8, 16, 19])
