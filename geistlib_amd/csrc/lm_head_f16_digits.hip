@@ -461,6 +461,23 @@ __global__ void k_f16_linear_list_all(long n_out, int n_m, F64Lists list) {
         *list.n_near = (int) (n_out * n_m), *list.n_open = 0;
 }
 
+/* One output's products added in index order by a wavefront: its lanes form 64 products at a time and
+ * every lane runs the chain. */
+__device__ __forceinline__ float sum_in_order(const uint16_t *__restrict__ wr,
+                                              const float *__restrict__ xm, int n_in) {
+    const int lane = threadIdx.x & 63;
+    double    acc  = 0.0; /* (never -0: the zeros behind the row's end change nothing) */
+    for (int k0 = 0; k0 < n_in; k0 += 64) {
+        const int    k = k0 + lane < n_in ? k0 + lane : 0;
+        const double w = (double) (float) __builtin_bit_cast(_Float16, wr[k]);
+        const uint2  p = __builtin_bit_cast(uint2, k0 + lane < n_in ? (double) xm[k] * w : 0.0);
+#pragma unroll
+        for (int i = 0; i < 64; ++i)
+            acc += __builtin_bit_cast(double, make_uint2(readlane_u32(p.x, i), readlane_u32(p.y, i)));
+    }
+    return (float) acc;
+}
+
 /* A closer look at the outputs near a rounding boundary, a wavefront each. The bound that listed
  * them is cheap, not tight: it takes every partial sum for ||w|| ||x||, which is 95 times what it is
  * on average. Here the lanes add eight products each per 512 columns, a scan puts their sums
@@ -469,7 +486,11 @@ __global__ void k_f16_linear_list_all(long n_out, int n_m, F64Lists list) {
  * stay open. 14.6 MB in rows scattered over the table: five loads of a row in flight at once.
  * Activations of few bits, an int8's or a bfloat16's, put many sums right on a boundary, but their
  * additions round nothing away (XRow::exact_to): left open all the same, they made a batch of
- * integers up to 127 take 1300 us (8 x 128256 x 2560), now 240. */
+ * integers up to 127 take 1300 us (8 x 128256 x 2560), now 213. What is open goes on a list for the
+ * kernel behind this one, but of short rows, whose chain takes less than that launch, and beyond the
+ * list's end: 256 outputs are two rounds of that kernel, 18 us, and a chain of 2560 additions here
+ * is 30, 4096 of them side by side (every one of 16 x 20000 x 2560 open: 5800 us, with a list that holds
+ * all 20300). */
 constexpr int LOOK_TPB   = 256;
 constexpr int LOOK_COLS  = 8 * 64; /* of a row per round of the wavefront */
 constexpr int LOOK_AHEAD = 5;      /* rounds whose loads are requested together */
@@ -478,7 +499,7 @@ __global__ __launch_bounds__(LOOK_TPB) void k_f16_linear_look(const uint16_t *__
                                                               long ld_x,
                                                               const XRow *__restrict__ xrow,
                                                               float *__restrict__ y, long ld_y,
-                                                              F64Lists list) {
+                                                              F64Lists list, int open_max) {
     const int lane = threadIdx.x & 63, count = *list.n_near;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     for (int it = (int) blockIdx.x * (LOOK_TPB / 64) + wave; it < count;
@@ -487,6 +508,9 @@ __global__ __launch_bounds__(LOOK_TPB) void k_f16_linear_look(const uint16_t *__
         const uint16_t *wr = w + (long) mine.x * n_in;
         const float    *xm = x + (long) mine.y * ld_x;
         const bool      vx = ((uintptr_t) xm & 15) == 0;
+        /* (a list that is full is left alone: additions to one word by the ten thousand take their
+         * time. Asked for here, where nothing waits for it) */
+        const int       seen = __hip_atomic_load(list.n_open, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const double    exact_to = xrow ? xrow[mine.y].exact_to : 0.0;
         double          base = 0.0, own = 0.0, all = 0.0, top = 0.0;
         for (int k0 = 0; k0 < n_in; k0 += LOOK_COLS * LOOK_AHEAD) {
@@ -532,12 +556,20 @@ __global__ __launch_bounds__(LOOK_TPB) void k_f16_linear_look(const uint16_t *__
         const bool   ok = order_is_free(
                               base, (own + all + 160.0 * rounds * top) * 0x1p-53 * (1.0 + 0x1p-20), f) ||
                           2.0 * own * (1.0 + 0x1p-30) < exact_to;
-        if (lane == 0) {
-            if (ok)
-                y[mine.y * ld_y + mine.x] = f;
-            else
-                list.open[atomicAdd(list.n_open, 1)] = mine;
+        if (!ok) { /* (uniform) */
+            int at = open_max;
+            if (seen < open_max && lane == 0)
+                at = atomicAdd(list.n_open, 1);
+            at = __builtin_amdgcn_readfirstlane(at);
+            if (at < open_max) {
+                if (lane == 0)
+                    list.open[at] = mine;
+                continue;
+            }
+            f = sum_in_order(wr, xm, n_in);
         }
+        if (lane == 0)
+            y[mine.y * ld_y + mine.x] = f;
     }
 }
 
@@ -561,7 +593,7 @@ __global__ __launch_bounds__(LISTED_TPB) void k_f16_linear_listed(
     __shared__ double s_end[LISTED_PARTS][64 * LISTED_CAND];
     __shared__ double s_sum[LISTED_PARTS];
     const int lane = threadIdx.x & 63, part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int count = *list.n_open;
+    const int count = *list.n_open < F64_OPEN_MAX ? *list.n_open : F64_OPEN_MAX;
     for (int it = blockIdx.x; it < count; it += gridDim.x) { /* (uniform over the workgroup) */
         const int2      mine = list.open[it];
         const uint16_t *wr   = w + (long) mine.x * n_in;
@@ -653,8 +685,10 @@ void launch_digits(hipStream_t stream, const uint16_t *w, long n_out, int n_in, 
     }
     const size_t lds = (size_t) n_stage * NT * 1024;
     auto k = full ? k_f16_linear_digits<NT, TPB, true, true> : k_f16_linear_digits<NT, TPB, true, false>;
-    (void) hipFuncSetAttribute(reinterpret_cast<const void *>(k),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, LDS_STAGES * 1024);
+    /* (more than a launch gets unasked; where it is refused so is the launch, which the caller sees) */
+    if (lds > 64 * 1024)
+        (void) hipFuncSetAttribute(reinterpret_cast<const void *>(k),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, LDS_STAGES * 1024);
     k<<<grid, block, lds, stream>>>(w, n_out, n_in, xdig, xrow, n_m, y, ld_y, list);
 }
 
@@ -682,8 +716,14 @@ static void f16_linear_pass(hipStream_t stream, const uint16_t *w_f16, long n_ou
         launch_digits<3, 768>(stream, w_f16, n_out, n_in, xdig, xrow, n_m, y, ld_y, ws.list);
     else
         launch_digits<6, 512>(stream, w_f16, n_out, n_in, xdig, xrow, n_m, y, ld_y, ws.list);
+    /* A wavefront's chain of 512 additions takes 6 us, a launch 4 and the parts 2 at least: rows of up
+     * to 512 columns are done with the closer look (16 x 64, 2 rows, called from Python: 12.5 us, with the third
+     * kernel 15.6). */
+    const int open_max = n_in <= 512 ? 0 : F64_OPEN_MAX;
     k_f16_linear_look<<<dim3(1024), dim3(LOOK_TPB), 0, stream>>>(
-        w_f16, n_in, x, ld_x, n_in > F16_DIGITS_MAX_IN ? nullptr : xrow, y, ld_y, ws.list);
+        w_f16, n_in, x, ld_x, n_in > F16_DIGITS_MAX_IN ? nullptr : xrow, y, ld_y, ws.list, open_max);
+    if (open_max == 0)
+        return;
     k_f16_linear_listed<<<dim3(128), dim3(LISTED_TPB), 0, stream>>>(w_f16, n_in, x, ld_x, y, ld_y, ws.list);
 }
 

@@ -39,9 +39,12 @@ void launch_f16_gemv(hipStream_t stream, const uint16_t *w_f16, long n_out, int 
                      const GemvFuse *fuse = nullptr);
 
 /* Scratch of the double-accumulation projection, for one pass of up to F64_M_MAX rows. */
-struct F64Lists { /* outputs (weight row, activation row), n_out * F64_M_MAX at most: */
-    int2 *near;   /* so close to a rounding boundary that the order of the sum may matter */
-    int2 *open;   /* ... that it does, as far as the bounds tell */
+constexpr int F64_OPEN_MAX = 256;
+struct F64Lists { /* outputs (weight row, activation row): */
+    int2 *near;   /* so close to a rounding boundary that the order of the sum may matter: n_out *
+                   * F64_M_MAX at most */
+    int2 *open;   /* ... that it does, as far as the bounds tell: the first F64_OPEN_MAX (of 8 x
+                   * 128256 about 30; the others are added where they were found) */
     int  *n_near, *n_open;
 };
 struct F64Scratch {

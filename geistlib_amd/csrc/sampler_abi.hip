@@ -1248,8 +1248,8 @@ int geist_hip_f16_gemv_rows(geist_hip_sampler *s, const uint16_t *d_w_f16, size_
     return after_launch(s, "f16 gemv");
 }
 
-/* Scratch of the f64 projection: the activations as digits, the list of outputs for the second
- * kernel. */
+/* Scratch of the f64 projection: the activations as digits, the lists of outputs for the kernels
+ * behind the first. */
 static int f64_scratch(geist_hip_sampler *s, size_t n_out, size_t n_in, F64Scratch &ws) {
     if (s->f64_in < n_in || s->f64_out < n_out) {
         if (s->f64_ws) {
@@ -1259,7 +1259,8 @@ static int f64_scratch(geist_hip_sampler *s, size_t n_out, size_t n_in, F64Scrat
         }
         const size_t in = n_in > s->f64_in ? n_in : s->f64_in;
         const size_t out = n_out > s->f64_out ? n_out : s->f64_out;
-        const size_t bytes = f16_linear_act_bytes((int) in) + 16 + 2 * out * F64_M_MAX * sizeof(int2);
+        const size_t bytes = f16_linear_act_bytes((int) in) + 16 +
+                             (out * F64_M_MAX + F64_OPEN_MAX) * sizeof(int2);
         if (hipMalloc(&s->f64_ws, bytes) != hipSuccess) {
             s->f64_ws = nullptr;
             return fail(s, GEIST_HIP_E_OOM, "f64 projection: scratch");
@@ -1270,8 +1271,8 @@ static int f64_scratch(geist_hip_sampler *s, size_t n_out, size_t n_in, F64Scrat
     ws.act       = p;
     int *n       = reinterpret_cast<int *>(p + f16_linear_act_bytes((int) s->f64_in));
     ws.list.n_near = n, ws.list.n_open = n + 1;
-    ws.list.near   = reinterpret_cast<int2 *>(n + 4);
-    ws.list.open   = ws.list.near + s->f64_out * F64_M_MAX;
+    ws.list.open   = reinterpret_cast<int2 *>(n + 4);
+    ws.list.near   = ws.list.open + F64_OPEN_MAX;
     return GEIST_HIP_OK;
 }
 

@@ -527,6 +527,50 @@ def test_f16_linear_in_double_takes_activations_of_few_bits_in_its_stride(hs):
     assert us[1] < 4 * us[0], us
 
 
+def sums_open_to_the_end(n_in):
+    """An activation row whose sum over weights of 1 or -1 lies on a rounding boundary but for terms
+    that its additions round away: 2^30 + 1 + 2^-24 - 2^30 and a few of 2^-60."""
+    x = np.zeros(n_in, dtype=np.float32)
+    x[[0, 1, 2, n_in - 2]] = 2.0 ** 30, 1.0, 2.0 ** -24, -2.0 ** 30
+    x[[3, n_in - 1]] = 2.0 ** -60, 2.0 ** -62
+    return x
+
+
+@pytest.mark.parametrize("n_out,n_in,m", [(2100, 520, 16), (2100, 512, 16), (3, 8, 1), (20, 2568, 2),
+                                          (1100, 1032, 16)])
+def test_f16_linear_in_double_with_every_sum_in_index_order(hs, oracle, n_out, n_in, m):
+    """Every output is left to the sum in index order: more than the list for that holds (2100 x
+    16), fewer, and rows of up to 512 columns, which are not listed."""
+    g = np.random.default_rng(n_out + n_in)
+    w16 = g.choice([-1.0, 1.0], (n_out, n_in)).astype(np.float16)
+    w16[: n_out // 2] = 1.0
+    x = np.tile(sums_open_to_the_end(n_in), (m, 1)) * (2.0 ** np.arange(m))[:, None].astype(np.float32)
+    y = torch.full((m, n_out), 7.0, dtype=torch.float32, device="cuda")
+    hs.f16_linear(to_dev(w16.view(np.int16), torch), to_dev(x, torch), y)
+    hs.sync()
+    want = oracle.f16_linear_f64(w16.view(np.uint16), x)
+    got = y.cpu().numpy()
+    assert (bits(got) == bits(want)).all(), np.argwhere(bits(got) != bits(want))[:5]
+
+
+def test_f16_linear_in_double_scratch_is_one_list(hs):
+    """The scratch of a table of 400000 rows: 16 entries of eight bytes a row, one list of them."""
+    from geistlib_amd import HipSampler
+    w = torch.zeros((400000, 8), dtype=torch.int16, device="cuda")
+    x = torch.zeros((2, 8), device="cuda")
+    y = torch.empty((2, 400000), device="cuda")
+    hs.f16_linear(w[:100], x, y[:, :100])              # (the kernels are loaded)
+    s = HipSampler(max_rows=2, max_vocab=1000)
+    s.f16_linear(w[:8], x, y[:, :8])
+    s.sync()
+    free = torch.cuda.mem_get_info()[0]
+    s.f16_linear(w, x, y)
+    s.sync()
+    used = free - torch.cuda.mem_get_info()[0]
+    s.close()
+    assert used < 1.25 * 400000 * 16 * 8, used
+
+
 @pytest.mark.parametrize("m", [2, 9, 19])
 def test_f16_linear_in_double_with_row_strides(hs, oracle, m):
     """Padded rows on both sides (row strides above the row lengths), 19 rows in two passes of the
