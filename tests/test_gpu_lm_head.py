@@ -340,8 +340,7 @@ def test_f16_linear_in_double_bit_exact(hs, oracle, n_out, n_in, m):
 @pytest.mark.parametrize("m", [1, 3, 7])
 def test_f16_linear_in_double_at_the_ends_of_the_range(hs, oracle, m):
     """Sums that overflow binary32, sums in its subnormal range, zero rows, weights that are
-    binary16 subnormals and infinities: the vector kernels (m <= 4) and the matrix-core kernel
-    agree with the oracle in every bit (NaN where it has NaN)."""
+    binary16 subnormals and infinities: every bit as the oracle has it (NaN where it has NaN)."""
     g = np.random.default_rng(m)
     n_out, n_in = 700, 512
     w16 = (g.standard_normal((n_out, n_in)) * 0.05).astype(np.float16)
@@ -487,6 +486,60 @@ def test_f16_linear_in_double_takes_rows_of_a_large_norm_in_its_stride(hs):
         w = torch.empty((64000, 2048), dtype=torch.float16, device="cuda").normal_(0, std, generator=g)
         us.append(f16_linear_us(hs, w.view(torch.int16), x))
     assert us[1] < 2 * us[0], us
+
+
+@pytest.mark.parametrize("n_out,n_in,m", [
+    (50001, 72, 8), (50001, 256, 3), (33000, 264, 16), (33000, 72, 9),   # LDS-resident
+    (49500, 3400, 5), (49500, 3656, 8), (49300, 5128, 2), (33000, 1672, 16),   # through LDS
+    (40, 3392, 8), (40, 3400, 8), (40, 1664, 16), (40, 1672, 16), (40, 5120, 4), (40, 5128, 4)])
+def test_f16_linear_in_double_beyond_a_wavefronts_first_tile(hs, oracle, n_out, n_in, m):
+    """Tables that give some wavefronts a second tile of sixteen rows (49152 rows on 256 compute
+    units, 32768 of more than 8 activation rows): weights of the next tile asked for across the end of
+    one, activations in LDS or passing through it in an even (54, 27) and odd (58) number of stages;
+    and the widest rows that LDS holds, with the next wider ones. Rows of both tiles are compared."""
+    print(f"f16 linear second tile {n_out} x {n_in}, {m} rows", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n_out + n_in + m)
+    w = torch.empty((n_out, n_in), dtype=torch.float16, device="cuda").normal_(0, 0.05, generator=g)
+    x = torch.randn((m, n_in), device="cuda", generator=g) * 3
+    y = torch.full((m, n_out), 7.0, dtype=torch.float32, device="cuda")
+    hs.f16_linear(w.view(torch.int16), x, y)
+    hs.sync()
+    rows = np.unique(np.concatenate([np.arange(min(n_out, 40)), np.arange(max(0, n_out - 400), n_out),
+                                     np.random.default_rng(m).integers(0, n_out, 300)]))
+    at = torch.from_numpy(rows).cuda()
+    want = oracle.f16_linear_f64(w[at].cpu().numpy().view(np.uint16), x.cpu().numpy())
+    got = y[:, at].cpu().numpy()
+    assert (bits(got) == bits(want)).all(), rows[np.argwhere(bits(got) != bits(want))[:5, 1]]
+    # the rest of the outputs, all below 256: within a step of binary32 (2^-16) of a plain product in
+    # double; a lost or doubled tile is off by the outputs themselves
+    plain = x.double() @ w.double().T
+    assert plain.abs().max().item() < 256 and (y.double() - plain).abs().max().item() < 2.0 ** -16
+
+
+@pytest.mark.parametrize("rows,vocab,d_model", [(9, 33000, 72), (16, 900, 1672), (19, 700, 1672),
+                                                (8, 1000, 3400), (3, 500, 5128), (7, 130, 8)])
+def test_project_sample_of_many_hidden_rows(hs, oracle, rows, vocab, d_model):
+    """The norm in the launch that cuts the activations: more than 8 rows, more than 16 (two passes),
+    row lengths on both sides of what LDS holds. Normed rows and logits bit for bit, greedy tokens."""
+    from geistlib_amd import SampleParams
+    print(f"project rows={rows} vocab={vocab} d_model={d_model}", flush=True)
+    g = np.random.default_rng(rows + vocab + d_model)
+    w16 = (g.standard_normal((vocab, d_model)) * 0.05).astype(np.float16).view(np.uint16)
+    hidden = (g.standard_normal((rows, d_model)) * 3).astype(np.float32)
+    norm_w = (1.0 + 0.1 * g.standard_normal(d_model)).astype(np.float32)
+    normed = torch.full((rows, d_model), 7.0, dtype=torch.float32, device="cuda")
+    logits = torch.full((rows, vocab), 7.0, dtype=torch.float32, device="cuda")
+    out = torch.full((rows,), -3, dtype=torch.int32, device="cuda")
+    hs.project_sample(to_dev(hidden, torch), to_dev(norm_w, torch), 1e-6,
+                      to_dev(w16.view(np.int16), torch), logits, SampleParams.make(temperature=0.0),
+                      None, out, normed=normed)
+    hs.sync()
+    normed_want = oracle.rmsnorm(hidden, norm_w, 1e-6)
+    want = oracle.f16_linear_f64(w16, normed_want)
+    assert (bits(normed.cpu().numpy()) == bits(normed_want)).all()
+    assert (bits(logits.cpu().numpy()) == bits(want)).all()
+    assert out.cpu().tolist() == [oracle.argmax(row) for row in want]
 
 
 def few_bits(kind, shape, g):
@@ -702,7 +755,7 @@ def test_f16_linear_in_double_on_order_sensitive_rows(hs, oracle, m):
     (50, 3520, 8, 0.05), (50, 1768, 13, 0.05), (31, 264, 16, 40.0), (64, 4096, 3, 2.5), (9, 65544, 2, 0.05)])
 def test_f16_linear_digit_edges(hs, oracle, n_out, n_in, m, scale):
     """The int8-digit kernel at the edges of its tiles (16 weight rows, 64 columns, 4 / 8 / 16
-    activation rows), of what LDS holds of the activations (3413 columns of 8 rows, 1706 of 16), of
+    activation rows), of what LDS holds of the activations (3392 columns of 8 rows, 1664 of 16), of
     the weights' range (rows of magnitudes beyond 127, or of ||w|| that could hold one) and of the
     integer sums (65536 columns): equal to the oracle in every bit."""
     print(f"f16 digits n_out={n_out} n_in={n_in} m={m} scale={scale}", flush=True)
