@@ -95,9 +95,9 @@ __device__ __forceinline__ void xd_load8(const float *__restrict__ p, bool vec, 
  * consecutive columns at a time, the bytes one lane of the projection feeds per digit.
  *
  * Digits: the operand of tile t (of NT) of stage s holds, for lane l of a wavefront, row l % 16
- * and the sixteen columns from 64 s + 16 (l / 16) on. Row 4 g + r of tile t is digit (4 t + r) % 6 of activation
- * row g + 4 ((4 t + r) / 6): the result tile then leaves all digits of an activation row in one
- * lane. */
+ * and the sixteen columns from 64 s + 16 (l / 16) on. Row 4 g + r of tile t is digit (4 t + r) % 6
+ * of activation row g + 4 ((4 t + r) / 6): the result tile then leaves all digits of an activation
+ * row in one lane. */
 template <bool NORM>
 __global__ __launch_bounds__(XD_TPB) void k_x_digits(const float *__restrict__ x, long ld_x,
                                                      const float *__restrict__ wn, float eps, int n,
@@ -158,7 +158,8 @@ __global__ __launch_bounds__(XD_TPB) void k_x_digits(const float *__restrict__ x
         top = s_u[i] > top ? s_u[i] : top;
     const bool finite = top < 0x7f800000u;
     /* |x| < 2^e; an activation becomes the integer nearest to x 2^(46 - e), below 2^46 */
-    const int    e = top ? (int) ((__double_as_longlong((double) __uint_as_float(top)) >> 52) & 0x7ff) - 1022 : 0;
+    const long long tb = __double_as_longlong((double) __uint_as_float(top));
+    const int    e = top ? (int) ((tb >> 52) & 0x7ff) - 1022 : 0;
     const double scale = __longlong_as_double((long long) (1023 + 46 - e) << 52);
     const int    g = m & 3, p0 = XDIGITS * (m >> 2);
     double       rest = 0.0;
@@ -195,7 +196,8 @@ __global__ __launch_bounds__(XD_TPB) void k_x_digits(const float *__restrict__ x
 #pragma unroll
         for (int d = 0; d < XDIGITS; ++d) {
             const int p = p0 + d;
-            uint8_t  *o = digits + ((((long) s * NT + (p >> 2)) * 64 + kg * 16 + 4 * g + (p & 3)) * 16 + 8 * half);
+            uint8_t  *o = digits + ((((long) s * NT + (p >> 2)) * 64 + kg * 16 + 4 * g + (p & 3)) * 16 +
+                                   8 * half);
             *reinterpret_cast<uint2 *>(o) = make_uint2(lo[d], hi[d]);
         }
     }
@@ -411,12 +413,13 @@ __device__ __forceinline__ void digits_tile(const Rows &rows, const Rows &rows_n
 }
 
 /* One workgroup per compute unit, its wavefronts taking tiles of 16 weight rows in turn (tile by
- * tile over the workgroups first, so that a table of any size uses every compute unit). The weights come straight to the registers,
- * four stages ahead of the arithmetic, the activations' operands from LDS, which holds them all for the life of the workgroup (LDSX), and no wavefront
- * waits for another behind the one barrier. Rows too long for that (3413 columns of 5 to 8
- * activation rows) have theirs pass through LDS, a turn of the ring at a time, in two buffers, for
- * the wavefronts of the workgroup in step; read from the caches instead, they took 240 us for 8 x
- * 65536 x 4096 and 380 us for 16 x 128256 x 2560. */
+ * tile over the workgroups first, so that a table of any size uses every compute unit). The weights
+ * come straight to the registers, four stages ahead of the arithmetic, the activations' operands from
+ * LDS, which holds them all for the life of the workgroup (LDSX), and no wavefront waits for another
+ * behind the one barrier. Rows too long for that (more than 5120 columns of up to 4 activation
+ * rows, 3392 of up to 8, 1664 of up to 16) have theirs pass through LDS, a turn of the ring at a
+ * time, in two buffers, for the wavefronts of the workgroup in step; read from the caches instead,
+ * they took 240 us for 8 x 65536 x 4096 and 380 us for 16 x 128256 x 2560 (now 205 and 264). */
 template <int NT, int TPB, bool LDSX, bool FULL>
 __global__ __launch_bounds__(TPB) void k_f16_linear_digits(
     const uint16_t *__restrict__ w, long n_out, int n_in, const i4v *__restrict__ xdig,
@@ -717,8 +720,8 @@ static void f16_linear_pass(hipStream_t stream, const uint16_t *w_f16, long n_ou
     else
         launch_digits<6, 512>(stream, w_f16, n_out, n_in, xdig, xrow, n_m, y, ld_y, ws.list);
     /* A wavefront's chain of 512 additions takes 6 us, a launch 4 and the parts 2 at least: rows of up
-     * to 512 columns are done with the closer look (16 x 64, 2 rows, called from Python: 12.5 us, with the third
-     * kernel 15.6). */
+     * to 512 columns are done with the closer look (16 x 64, 2 rows, called from Python: 12.5 us, with
+     * the third kernel 15.6). */
     const int open_max = n_in <= 512 ? 0 : F64_OPEN_MAX;
     k_f16_linear_look<<<dim3(1024), dim3(LOOK_TPB), 0, stream>>>(
         w_f16, n_in, x, ld_x, n_in > F16_DIGITS_MAX_IN ? nullptr : xrow, y, ld_y, ws.list, open_max);

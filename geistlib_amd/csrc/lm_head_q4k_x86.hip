@@ -36,8 +36,8 @@ constexpr int Q4X_TPB         = 256;
 constexpr int Q4X_ROW_DWORDS  = 37;
 constexpr int Q4X_PACK_DWORDS = Q4X_ROW_DWORDS * 64; /* the packed copy's dwords per (64 rows, block) */
 
-/* Element t of a super-block, held by thread t modulo 256, given the reciprocal of the row's scale: its int8 value
- * into the block's dwords (ob), the sums per sub-block of 32 behind them. */
+/* Element t of a super-block, held by thread t modulo 256, given the reciprocal of the row's scale:
+ * its int8 value into the block's dwords (ob), the sums per sub-block of 32 behind them. */
 __device__ __forceinline__ void q4x_quantize_block(float xv, float inv, bool ties_even,
                                                    uint32_t *__restrict__ ob) {
     const int   t = threadIdx.x & 255;
@@ -157,8 +157,8 @@ __device__ __forceinline__ void q4x_load(const uint32_t *__restrict__ base, int 
     k.dd    = __builtin_nontemporal_load(base + 2304 + r);
 }
 
-/* M activation rows share a pass over the table (1 or 2, and 8 with PAIRS). PAIRS: the binary32 accumulators are joined once
- * per pair of sub-blocks (the reference's 16 x 16 AVX-512 tiles,
+/* M activation rows share a pass over the table (1 or 2, and 8 with PAIRS). PAIRS: the binary32
+ * accumulators are joined once per pair of sub-blocks (the reference's 16 x 16 AVX-512 tiles,
  * kernel_q4kx8_gemm_avx512_full.c:94, 729-778) instead of once per super-block. */
 template <int M, bool PAIRS>
 __global__ __launch_bounds__(Q4X_TPB, PAIRS && M > 2 ? 3 : 4) void k_q4k_packed_gemv_x86(
