@@ -25,12 +25,12 @@ __device__ __forceinline__ float rms_inv_sequential(const float *__restrict__ xr
     return (float) (1.0 / sqrt(sumsq / (double) n + (double) eps));
 }
 
-/* The threads that norm one row where there are few rows. One row is one workgroup's work, and it is latency that it takes:
- * the row's and the weights' elements are asked for at once, four of each per thread, and stay in
- * registers. 256 threads that looped over memory twice, and added their sums through LDS in eight
- * barriers, took 10.7 us of a cold step for the norm of 2560 elements where this takes 4.7 (4.6 is
- * what any launch takes), with the Q6_K quantiser 11.3 against 5.4, with the Q4_K one for 8 rows of
- * 1536 9.9 against 5.0, with the sketch head's activations 13.6 against 6.5. */
+/* The threads that norm one row where there are few rows. One row is one workgroup's work, and it is
+ * latency that it takes: the row's and the weights' elements are asked for at once, four of each per
+ * thread, and stay in registers. 256 threads that looped over memory twice, and added their sums
+ * through LDS in eight barriers, took 11.2 us of a cold step for the norm of 2560 elements where this
+ * takes 5.3 (4.6 is what any launch takes), with the Q6_K quantiser 11.5 against 5.8, with the Q4_K
+ * one for 8 rows of 1536 9.5 against 5.5, with the sketch head's activations 13.8 against 6.0. */
 constexpr int NORM_TPB = 1024;
 constexpr int NORM_PER = 4;
 
