@@ -70,9 +70,7 @@ static_assert(sizeof(XRow) == F16_XROW_BYTES, "the scratch is sized by the calle
 /* Sum over a workgroup of XD_TPB threads, every thread gets it; s: XD_TPB / 64 entries that no
  * thread still reads. */
 __device__ __forceinline__ double xd_block_sum(double v, double *s) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1)
-        v += __shfl_xor(v, d);
+    v = wave_sum_f64(v);
     if ((threadIdx.x & 63) == 0)
         s[threadIdx.x >> 6] = v;
     __syncthreads();
