@@ -17,12 +17,12 @@
  * what is then still open (about 30) a third one adds in index order.
  *
  * What bounds it. The pass over the table: 2 bytes per weight, 657 MB at 128256 x 2560, 104 us at
- * the rate the memory gives a stream that is read once; it takes 113 to 123. Cutting the weights
+ * the rate the memory gives a stream that is read once; it takes 111 to 119. Cutting the weights
  * keeps the vector units busy half of that time (106 instructions per 64 columns and tile), the
  * matrix cores are busy a quarter; both run while the next stages' loads, four per wavefront, are
- * under way. The launches around it are the rest: 8 us for the cut, 12 and 15 for the two behind. With
+ * under way. The launches around it are the rest: 7 us for the cut, 11 and 14 for the two behind. With
  * the products in double (v_mfma_f64_4x4x4, half of whose rate eight rows could use) the same pass
- * took 205 us.
+ * took 200 us.
  *
  * What a call's data can cost. Rows that are not finite, sums beyond binary32 and activations of few
  * bits are settled on the way. Weight rows of a norm of 126 or more in 256 columns are left to the
