@@ -83,6 +83,8 @@ struct geist_hip_sampler {
     float    *probs      = nullptr; /* [max_rows][max_vocab], allocated on first use by the
                                      * full-vocabulary top-p / min-p path */
     gs::CandSpace cand   = {};      /* candidate lists of that path, allocated with probs */
+    void     *sorted_base = nullptr; /* the allocation that holds probs, cand, win and walk_rows */
+    gs::WinSpace win     = {};
     void     *walk_rows  = nullptr; /* workspace of the whole-row walk spread over the row's
                                      * chunks (sampler_walk_coop.h), allocated with probs */
     uint32_t *walk_hint  = nullptr; /* pinned, two words: the number of the last call in which
@@ -91,6 +93,7 @@ struct geist_hip_sampler {
     uint32_t  walk_calls = 0;       /* calls of the top-p / min-p path so far */
     uint32_t  walk_cleared = 0;     /* ... the one before which the workspace was last cleared */
     int       walk_mode  = 0;       /* geist_hip_sampler_set_whole_row_walk */
+    bool      walk_spread = false;  /* the last call of that path sends the spread walk */
     bool      walk_clear = false;   /* clear the workspace before its next use */
     void    *q6k_ws      = nullptr; /* scratch of the Q6_K projection, sized like f64_ws */
     size_t   q6k_in = 0, q6k_out = 0;
@@ -401,19 +404,11 @@ void geist_hip_sampler_destroy(geist_hip_sampler *s) {
     (void) hipFree(s->uniforms);
     (void) hipFree(s->probe_p);
     (void) hipFree(s->scalar_out);
-    (void) hipFree(s->probs);
-    (void) hipFree(s->walk_rows);
+    (void) hipFree(s->sorted_base);
     if (s->walk_hint)
         (void) hipHostFree(s->walk_hint);
     (void) hipFree(s->f64_ws);
     (void) hipFree(s->q6k_ws);
-    (void) hipFree(s->cand.row_bound);
-    (void) hipFree(s->cand.out_key);
-    (void) hipFree(s->cand.key);
-    (void) hipFree(s->cand.idx);
-    (void) hipFree(s->cand.count);
-    (void) hipFree(s->cand.row_sum);
-    (void) hipFree(s->cand.path);
     if (s->h_scalar)
         (void) hipHostFree(s->h_scalar);
     delete s;
@@ -586,40 +581,51 @@ static int sample_impl(geist_hip_sampler *s, const struct geist_hip_rows *rows,
 static int reserve_sorted_workspace(geist_hip_sampler *s) {
     if (s->probs)
         return GEIST_HIP_OK;
-    const size_t  R = s->max_rows;
-    gs::CandSpace c = {};
-    float        *probs = nullptr;
-    hipError_t    e = hipSetDevice(s->device);
-    if (e == hipSuccess) e = hipMalloc((void **) &c.row_bound, R * sizeof(int32_t));
-    if (e == hipSuccess) e = hipMalloc((void **) &c.out_key, R * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc((void **) &c.key, R * CAND_CAP * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc((void **) &c.idx, R * CAND_CAP * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc((void **) &c.count, R * gs::CAND_COUNT_STRIDE * sizeof(int32_t));
-    if (e == hipSuccess) e = hipMalloc((void **) &c.row_sum, R * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc((void **) &c.path, R * sizeof(int32_t));
-    if (e == hipSuccess) e = hipMalloc((void **) &probs, R * s->max_vocab * sizeof(float));
-    void     *walk_rows = nullptr;
-    uint32_t *walk_hint = nullptr;
-    if (e == hipSuccess) e = hipMalloc(&walk_rows, gs::walk_coop_bytes(R));
-    if (e == hipSuccess) e = hipMemsetAsync(walk_rows, 0, gs::walk_coop_bytes(R), s->stream);
+    const size_t R = s->max_rows;
+    /* chunks of 8192 logits, or, in small batches, of 2048 */
+    size_t wgs = R * ((s->max_vocab + 8191) / 8192);
+    if (wgs < (size_t) gs::WIN_SMALL)
+        wgs = (size_t) gs::WIN_SMALL;
+    /* one allocation, cut into parts of whole cache lines; those that start at zero come first */
+    size_t size = 0;
+    auto   part = [&](size_t bytes) {
+        const size_t at = size;
+        size += (bytes + 255) & ~(size_t) 255;
+        return at;
+    };
+    const size_t win_row = part(R * gs::WIN_ROW_BYTES), walk = part(gs::walk_coop_bytes(R)), zeroed = size;
+    const size_t win_list = part(R * gs::WIN_CAP * sizeof(uint64_t));
+    const size_t win_chunk = part(wgs * gs::WIN_CHUNK_BYTES);
+    const size_t win_hist = part(wgs * gs::WIN_BINS * sizeof(float));
+    const size_t key = part(R * CAND_CAP * sizeof(uint32_t)), idx = part(R * CAND_CAP * sizeof(uint32_t));
+    const size_t count = part(R * gs::CAND_COUNT_STRIDE * sizeof(int32_t));
+    const size_t path = part(R * sizeof(int32_t)), probs = part(R * s->max_vocab * sizeof(float));
+    char        *base = nullptr;
+    uint32_t    *walk_hint = nullptr;
+    hipError_t   e = hipSetDevice(s->device);
+    if (e == hipSuccess) e = hipMalloc((void **) &base, size);
+    if (e == hipSuccess) e = hipMemsetAsync(base, 0, zeroed, s->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
     if (e == hipSuccess) e = hipHostMalloc((void **) &walk_hint, 64, hipHostMallocDefault);
     if (e != hipSuccess) {
-        void *ptrs[] = {c.row_bound, c.out_key, c.key, c.idx, c.count, c.row_sum, c.path, probs,
-                        walk_rows};
-        for (void *q : ptrs)
-            if (q)
-                (void) hipFree(q);
-        if (walk_hint)
-            (void) hipHostFree(walk_hint);
+        if (base)
+            (void) hipFree(base);
         return fail(s, e == hipErrorOutOfMemory ? GEIST_HIP_E_OOM : GEIST_HIP_E_BACKEND,
                     "workspace of the top-p / min-p path: %s", hipGetErrorString(e));
     }
-    s->cand  = c;
-    s->probs = probs;
     walk_hint[0] = walk_hint[1] = 0u;
-    s->walk_rows = walk_rows;
-    s->walk_hint = walk_hint;
+    s->sorted_base = base;
+    s->win.row     = base + win_row;
+    s->win.list    = reinterpret_cast<uint64_t *>(base + win_list);
+    s->win.chunk   = base + win_chunk;
+    s->win.hist    = reinterpret_cast<float *>(base + win_hist);
+    s->cand.key    = reinterpret_cast<uint32_t *>(base + key);
+    s->cand.idx    = reinterpret_cast<uint32_t *>(base + idx);
+    s->cand.count  = reinterpret_cast<int32_t *>(base + count);
+    s->cand.path   = reinterpret_cast<int32_t *>(base + path);
+    s->walk_rows   = base + walk;
+    s->walk_hint   = walk_hint;
+    s->probs       = reinterpret_cast<float *>(base + probs);
     return GEIST_HIP_OK;
 }
 
@@ -836,61 +842,33 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
     if (L.rv.n_chunks > s->max_chunks)
         return fail(s, GEIST_HIP_E_UNSUPPORTED, "n_vocab %zu needs more than %d chunks",
                     rows->n_vocab, s->max_chunks);
-    draws();
-    /* min-p bounds the kept prefix by the row maximum alone, so the exp-sum pass can list the
-     * candidates on its way; rows whose list overflows fall back to the bound of the row-final
-     * kernel and a third pass */
-    const int zb_m    = zbin_of_min_p(rs.min_p);
-    f.cand            = s->cand;
-    f.minp_listed     = rs.use_m && zb_m < ZBINS - 1;
-    /* A min-p of a few percent keeps the list short on any plausible row, and the walk can follow
-     * the exp-sum pass at once. Below that a flat row may overflow the list, and the row-final
-     * kernel should get the chance to bound it by top-p instead. */
-    f.minp_direct     = f.minp_listed && rs.min_p >= 0.02f;
-    *stream_kernel = "k_scan_expsum";
-    Launch scan          = L;
-    scan.rv.stream_loads = s->logits_streamed; /* the one pass over whole rows */
-    if (do_stream &&
-        /* (the thread maxima are the row-final kernel's; with the list walk coming first and
-         * alone nobody reads them) */
-        launch_scan_expsum(scan, rs.inv_t, f.minp_direct ? nullptr : s->tmax, s->chunk_best,
-                           s->chunk_sum, nullptr, 0, nullptr, f.minp_listed ? &f.cand : nullptr,
-                           zb_m, nullptr, meet_space(s, scan, 1, (scan.rows & 7) == 0), s->fast_sums))
-        return fail(s, GEIST_HIP_E_BACKEND, "no launch geometry for the exp-sum pass");
-    if (!do_tail)
-        return after_launch(s, "exp-sum scan");
-    f.mode     = FINAL_SORTED;
-    f.row_flag = s->row_flag;
-    /* rows whose kept prefix is too wide for the shortcut of the row-final kernel flag themselves
-     * 1: their candidates are listed and walked; what that cannot serve either takes the
-     * whole-row walk inside the list-walk kernel. Each of these kernels returns at once for every
-     * row not flagged for it. With the candidates already listed by the exp-sum pass the list
-     * walk comes first and alone. */
-    if (!f.minp_direct)
-        launch_row_final(L, f);
-    /* Rows that neither shortcut nor list can serve are walked in full: by their one workgroup
-     * inside the list-walk kernel, or spread over the workgroups of their chunks by a kernel
-     * behind it. That kernel is a launch more for every call, so it is sent only while such rows
-     * keep turning up: the kernels say so in a page-locked word, which is looked at here without
-     * waiting for anything (a stale value costs time, never a token). */
+    /* Rows that nothing shorter can serve are walked in full: by one workgroup each, or spread over
+     * the workgroups of their chunks by a kernel of its own. That kernel is a launch more for every
+     * call, so it is sent only while such rows keep turning up: the kernels say so in a page-locked
+     * word, which is looked at here without waiting for anything (a stale value costs time, never a
+     * token). */
     WalkCoop wc = {};
     wc.rows       = s->walk_rows;
     wc.hint       = s->walk_hint;
     wc.wait_limit = s->wait_limit;
+    if (do_stream)
+        s->walk_calls += 1;
     if (s->walk_rows && s->walk_hint) {
         /* (calls are numbered from 1; a hint from one of the last 64 calls counts: with
          * several calls in flight the kernels' word lags behind) */
-        const uint32_t call   = ++s->walk_calls;
+        const uint32_t call   = s->walk_calls;
         const uint32_t walked = __atomic_load_n(&s->walk_hint[0], __ATOMIC_RELAXED);
         const uint32_t ranout = __atomic_load_n(&s->walk_hint[1], __ATOMIC_RELAXED);
         wc.call   = call;
         /* the spread form holds two workgroups per compute unit: beyond a few rounds of them the
          * rows' own workgroups, all at once, are the faster way */
         const bool fits = rows->rows * (size_t) L.rv.n_chunks <= 1280;
-        wc.spread = s->walk_mode == GEIST_HIP_WHOLE_ROW_WALK_SPREAD ||
-                    (s->walk_mode == GEIST_HIP_WHOLE_ROW_WALK_ADAPTIVE && fits && walked != 0u &&
-                     call - walked <= 64u);
-        if (wc.spread) {
+        if (do_stream)
+            s->walk_spread = s->walk_mode == GEIST_HIP_WHOLE_ROW_WALK_SPREAD ||
+                             (s->walk_mode == GEIST_HIP_WHOLE_ROW_WALK_ADAPTIVE && fits &&
+                              walked != 0u && call - walked <= 64u);
+        wc.spread = s->walk_spread;
+        if (wc.spread && do_tail) {
             wc.clear = (ranout != 0u && (int32_t) (ranout - s->walk_cleared) >= 0) ||
                        s->walk_clear;
             if (wc.clear)
@@ -900,6 +878,50 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
             s->walk_steps += 16u;
         }
     }
+    draws();
+    /* A min-p of a few percent bounds the kept prefix to a short list on any plausible row, by the
+     * row maximum alone: the exp-sum pass lists the candidates on its way and the list walk
+     * follows it at once. Otherwise the pass leaves histograms of the masses. */
+    const int zb_m = zbin_of_min_p(rs.min_p);
+    f.cand         = s->cand;
+    f.minp_direct  = rs.use_m && zb_m < ZBINS - 1 && rs.min_p >= 0.02f;
+    f.win          = s->win;
+    f.win_bins     = win_bins_for(rs.use_p ? rs.top_p : 0.0f, rs.min_p, rows->n_vocab);
+    /* A small batch is a chain of waits, not of bytes: chunks of 2048 logits put four times the
+     * workgroups to work on it, and reading the rows again costs less than the launch of the
+     * row-final kernel that spares most rows the reading. (The spread walk wants chunks of 8192.) */
+    const size_t small_chunks = (rows->n_vocab + 2047) / 2048;
+    f.win_locate = !f.minp_direct && !wc.spread && small_chunks <= (size_t) s->max_chunks &&
+                   small_chunks <= (size_t) MAX_CHUNKS &&
+                   rows->rows * small_chunks <= (size_t) WIN_SMALL &&
+                   rows->rows * small_chunks * small_chunks <= (size_t) WIN_SMALL_READS;
+    /* (a shallower min-p still makes a list that holds for most rows; the others have histograms) */
+    f.minp_listed = rs.use_m && zb_m < ZBINS - 1 && !f.minp_direct && !f.win_locate;
+    if (f.win_locate) {
+        L.nv           = 2;
+        L.rv.per_chunk = 2048;
+        L.rv.n_chunks  = (int) small_chunks;
+    }
+    *stream_kernel = "k_scan_expsum";
+    Launch scan          = L;
+    scan.rv.stream_loads = s->logits_streamed; /* the one pass over whole rows */
+    if (do_stream &&
+        /* (the thread maxima are the row-final kernel's: not wanted where none follows) */
+        launch_scan_expsum(scan, rs.inv_t, f.minp_direct || f.win_locate ? nullptr : s->tmax,
+                           s->chunk_best, s->chunk_sum, nullptr, 0, nullptr,
+                           f.minp_direct || f.minp_listed ? &f.cand : nullptr, zb_m, nullptr,
+                           meet_space(s, scan, 1, (scan.rows & 7) == 0), s->fast_sums,
+                           f.minp_direct ? nullptr : f.win.hist, f.win_bins))
+        return fail(s, GEIST_HIP_E_BACKEND, "no launch geometry for the exp-sum pass");
+    if (!do_tail)
+        return after_launch(s, "exp-sum scan");
+    f.mode     = FINAL_SORTED;
+    f.row_flag = s->row_flag;
+    /* rows whose kept prefix is too wide for the shortcut of the row-final kernel flag themselves 1
+     * for k_window; what that cannot serve either takes the whole-row walk. Each of these kernels
+     * returns at once for every row not flagged for it. */
+    if (!f.minp_direct && !f.win_locate)
+        launch_row_final(L, f);
     launch_candidates(L, f, s->probs, (long) s->max_vocab, wc);
     return after_launch(s, "top-p / min-p");
 }

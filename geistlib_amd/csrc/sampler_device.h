@@ -103,6 +103,16 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
 #undef GS_STEP
     return readlane_u32(v, WAVE - 1);
 }
+/* inclusive prefix sum over the lanes; lane 63 receives the total */
+__device__ __forceinline__ uint64_t wave_scan_u64(uint64_t v) {
+    v += dpp_fetch_u64<0x111, 0xf>(v);
+    v += dpp_fetch_u64<0x112, 0xf>(v);
+    v += dpp_fetch_u64<0x114, 0xf>(v);
+    v += dpp_fetch_u64<0x118, 0xf>(v);
+    v += dpp_fetch_u64<0x142, 0xa>(v);
+    v += dpp_fetch_u64<0x143, 0xc>(v);
+    return v;
+}
 __device__ __forceinline__ double wave_scan_f64_dpp(double v);
 __device__ __forceinline__ int    wave_scan_i32_dpp(int v);
 __device__ __forceinline__ double wave_sum_f64(double v) {
@@ -603,6 +613,21 @@ __device__ __forceinline__ int zbin(float arg) {
  * as zbin's last bin is). */
 __device__ __forceinline__ float zbin_threshold(int b) {
     return -(float) (b + 1) / (float) ZBIN_PER_NAT;
+}
+
+/* The bins of the mass histogram (sampler_window.h): WIN_SHIFT trailing bits of the binary32 p are
+ * dropped, counted down from p = 1, which shares bin 0 with its neighbours. */
+constexpr uint32_t WIN_TOP = 0x3f800000u;
+__device__ __forceinline__ int      win_bin(uint32_t key) { return (int) ((WIN_TOP - key) >> WIN_SHIFT); }
+__device__ __forceinline__ uint32_t win_key_hi(int d) { return WIN_TOP - ((uint32_t) d << WIN_SHIFT); }
+__device__ __forceinline__ uint32_t win_key_lo(int d) { return win_key_hi(d) - ((1u << WIN_SHIFT) - 1u); }
+
+/* A p's weight in its bin: the significand of its predecessor (all of a bin's share an exponent:
+ * a power of two belongs to the octave below), cut to 19 bits so that a chunk's 8192 fit a word.
+ * t = WIN_TOP - key. win_scale(d): what a weight in bin d stands for; relative error below 2^-17. */
+__device__ __forceinline__ uint32_t win_weight(uint32_t t) { return 0x7ffffu - ((t >> 5) & 0x3ffffu); }
+__device__ __forceinline__ float win_scale(int d) {
+    return __uint_as_float((((win_key_hi(d) - 1u) >> 23) - 18u) << 23);
 }
 
 /* xorshift64* (sampler.c:35-48): one step of a generator, and the uniform of its 24 leading bits */

@@ -81,27 +81,44 @@ struct Launch {
     hipStream_t stream;
 };
 
-/* Workspace of the candidate path of the full-vocabulary top-p / min-p modes. Elements are
- * binned by z = (max - l) * inv_t in steps of 1/ZBIN_PER_NAT; a row the thread-maxima shortcut
- * cannot serve derives (from the binned mass of its thread maxima and from min_p) the last bin
- * that can hold an element of its kept prefix, a third pass over the row lists the elements up
- * to that bin with their normalised probabilities, and a row-final kernel works on the list. */
+/* Workspace of the candidate lists of the min-p modes. Elements are binned by z = (max - l) * inv_t
+ * in steps of 1/ZBIN_PER_NAT; min_p bounds the last bin that can hold an element of the kept
+ * prefix, the exp-sum pass lists the elements up to that bin with their softmax arguments, and a
+ * row-final kernel works on the list. */
 constexpr int ZBINS        = 128;
 constexpr int ZBIN_PER_NAT = 4;
 constexpr int CAND_CAP     = 16384; /* list entries per row */
 constexpr int CAND_LDS     = 4096;  /* lists up to this length are staged in LDS */
 constexpr int CAND_COUNT_STRIDE = 32;
 struct CandSpace {
-    int32_t  *row_bound; /* [rows] last z bin listed */
-    uint32_t *out_key;   /* [rows] bits of a pn no element past that bin can exceed */
-    uint32_t *key;       /* [rows][CAND_CAP] bits of pn */
+    uint32_t *key;       /* [rows][CAND_CAP] bits of the softmax argument */
     uint32_t *idx;       /* [rows][CAND_CAP] vocabulary ids */
     int32_t  *count;     /* [rows * CAND_COUNT_STRIDE]: a row's counter has a cache line to itself
                           * (the appending wavefronts' atomic adds to one line serialise) */
-    double   *row_sum;   /* [rows] the row's exp-sum, for lists that hold p instead of pn */
-    int32_t  *path;      /* [rows] which walk served the row: 1 thread-maxima shortcut, 2 list,
-                          * 3 whole row */
+    int32_t  *path;      /* [rows] which walk served the row (geist_hip_sampler_row_paths) */
 };
+
+/* Workspace of the rows of the top-p / min-p modes that the thread-maxima shortcut does not serve
+ * (sampler_window.h): per chunk a histogram of the masses and what the chunk's workgroup reports,
+ * per row a record and the list of the entries around its nucleus edge and its draw. */
+constexpr int WIN_SHIFT = 19;   /* a bin of the histogram spans 2^19 neighbouring binary32 p: ... */
+constexpr int WIN_BINS  = 512;  /* ... 16 bins to a factor of two, down from 1 to 2^-32 */
+constexpr int WIN_CAP   = 16384; /* list entries per row */
+/* Launches of up to WIN_SMALL chunks of 2048, and of so many chunks' histograms read (every
+ * workgroup reads all of its row's), find their plans in k_window. One row of 128256 (63 x 63) 22.5
+ * us against 38 by chunks of 8192 with a row-final kernel, one of 262144 26 / 35, 16 x 128256 (16 x
+ * 63 x 63 reads) 39.3 / 43.5; 8 x 262144 (8 x 128 x 128) 58 / 54, 48 x 100000 (2352 chunks) 48 / 21. */
+constexpr int WIN_SMALL       = 1024;
+constexpr int WIN_SMALL_READS = 65536;
+struct WinSpace {
+    float    *hist;  /* [rows][chunks][WIN_BINS], by the launch's chunks */
+    uint64_t *list;  /* [rows][WIN_CAP] */
+    void     *chunk; /* [rows][chunks] x WIN_CHUNK_BYTES */
+    void     *row;   /* [rows] x WIN_ROW_BYTES, zero before the first use */
+};
+constexpr size_t WIN_CHUNK_BYTES = 32, WIN_ROW_BYTES = 128;
+/* how many bins can hold an element of a kept prefix (a multiple of four) */
+int win_bins_for(float top_p, float min_p, size_t n_vocab);
 
 /* Workspace of the candidate path of the top-k modes: what each scanning wavefront hands on to
  * the row-final kernel. A row is scanned by n_chunks * 4 wavefronts; wavefront w of row r owns
@@ -171,10 +188,15 @@ int cand_lanes_for(int k_eff, size_t n_vocab);
 
 struct FinalLaunch {
     CandSpace       cand;
-    bool            minp_listed; /* the exp-sum pass already listed the rows under the min-p bound */
-    bool            minp_direct; /* ... and the list walk runs straight after it: no row-final
-                                    kernel, no listing pass; a row whose list overflowed goes to
-                                    the whole-row walk */
+    WinSpace        win;
+    int             win_bins;
+    bool            win_locate;  /* a small batch: k_window finds the rows' plans itself, no row-final
+                                    kernel in front */
+    bool            minp_listed; /* the exp-sum pass has listed the rows under the min-p bound; the
+                                    row-final kernel sends those whose list holds to its walk */
+    bool            minp_direct; /* the exp-sum pass has listed the rows under the min-p bound and the
+                                    list walk runs straight after it: no row-final kernel; a row
+                                    whose list overflowed goes to the whole-row walk */
     int             mode, k, k_sel;
     bool            cap_after; /* top-k: the scan ran before the soft-cap, the row-final kernel
                                   applies it to what it keeps */
@@ -203,11 +225,13 @@ struct FinalLaunch {
  * the bit-exact expf; p at the probed token stays exact. Without penalties and without a list
  * the workgroups of a row then do not meet: each sums against its chunk's maximum and a second,
  * small launch scales the sums to the row's (k_rescale_sums).
+ * hist != NULL (no list, no slab sums): also the chunks' histograms of the masses,
+ * [rows][chunks][WIN_BINS], of which the first hist_bins bins are written.
  * Returns 0 or a hipError_t value (the launch itself is checked by the caller as usual). */
 int launch_scan_expsum(const Launch &L, float inv_t, float *tmax, uint64_t *chunk_best,
                        double *chunk_sum, const int32_t *probe_token, int probe_L, float *probe_p,
                        const CandSpace *list, int zb_list, double *slab_sum, const MeetSpace &meet,
-                       bool fast = false);
+                       bool fast = false, float *hist = nullptr, int hist_bins = 0);
 /* The temperature draw in one kernel (sampler_draw.h): out[row] = the id drawn with
  * uniforms[row]. For L.nv == 2. `meet.slots` holds 2 * rows * n_chunks zeroed words: the
  * workgroups of a row meet twice. */
@@ -276,11 +300,11 @@ void launch_cand_scan_final(const Launch &scan, const Launch &L, const FinalLaun
 int  launch_topk_general(const Launch &L, const FinalLaunch &f);
 /* Per-device kernel attributes; call once with the device current. Returns a hipError_t value. */
 int configure_device_kernels();
-/* rows flagged 1 by the sorted row-final kernel: list their candidates, then draw from the
- * list; rows the list cannot serve (and rows the row-final kernel flagged 2) take the whole-row
- * walk in the same launch: probabilities of the whole row into `probs`, then the walk over them */
+/* what follows the exp-sum pass (minp_direct: the walk over the lists it made) or the sorted
+ * row-final kernel (otherwise: rows it flagged are served by k_window); rows that neither can serve
+ * take the whole-row walk, in the same launch or spread over their chunks behind it */
 /* The whole-row walk spread over the workgroups of the row's chunks (sampler_walk_coop.h), for
- * the rows the list walk flags 2 when `spread` is set: `rows` is the workspace of
+ * the rows flagged 2 when `spread` is set: `rows` is the workspace of
  * walk_coop_bytes(max rows) bytes, zero before its first use and cleared again by this call when
  * `clear` is set; the steps of this launch are numbered from step_base + 1 on (at most 16); `hint`
  * (two words of page-locked host memory, or null): a launch in which a row was walked in full

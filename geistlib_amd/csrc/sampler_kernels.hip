@@ -33,6 +33,7 @@
 #include "sampler_device.h"
 
 #include <cmath>
+#include <cstring>
 #include <type_traits>
 
 namespace gs {
@@ -211,7 +212,7 @@ struct FusedScan {
     uint32_t  local;    /* MeetSpace::local */
     uint64_t *s_red;    /* LDS, NWAVES words */
     uint64_t *s_bb;     /* LDS, one word */
-    uint32_t *s_arrive; /* LDS, three arrival counters (and a fourth word), zero and published
+    uint32_t *s_arrive; /* LDS, four arrival counters (and a word between), zero and published
                          * before use */
 };
 
@@ -328,7 +329,7 @@ __device__ __forceinline__ float fast_expf_le0(float x) {
  * inside the pass, was measured too: the acknowledged device-scope stores and the atomic it
  * needs keep every workgroup longer than the launch costs; 50.6 against 48.6 us for the
  * verification of 32 sequences, 53.3 with the meeting.) */
-template <int NV, bool PEN, bool LISTM, bool SLABS, bool PLAIN, bool FAST, bool NOMEET>
+template <int NV, bool PEN, bool LISTM, bool SLABS, bool PLAIN, bool FAST, bool NOMEET, bool HIST>
 __device__ __forceinline__ void expsum_chunk(const RowView &rv, int row, int chunk, int n_rows,
                                              int base, int end, float inv_t,
                                              double *__restrict__ chunk_sum,
@@ -337,7 +338,8 @@ __device__ __forceinline__ void expsum_chunk(const RowView &rv, int row, int chu
                                              float *__restrict__ probe_p, const CandSpace &list,
                                              int zb_list, uint32_t *s_cnt16, double *s_sum,
                                              uint64_t *s_tab, uint64_t tabv, double *s_tr,
-                                             uint2 *s_stage, uint32_t *s_nstage,
+                                             uint2 *s_stage, uint32_t *s_nstage, uint32_t *s_hist,
+                                             float *__restrict__ hist, int hist_bins,
                                              const FusedScan &fs) {
     const int tid = threadIdx.x;
     /* with penalties the work before the meet is long, and the row's other workgroups wait for
@@ -376,8 +378,10 @@ __device__ __forceinline__ void expsum_chunk(const RowView &rv, int row, int chu
     }
     if (tid < 32)
         s_tab[tid] = tabv;
-    if (tid < 4) /* three arrival counters and the staging list's length */
+    if (tid < 5) /* four arrival counters and the staging list's length */
         fs.s_arrive[tid] = 0;
+    if (HIST && tid < WIN_BINS / 4)
+        reinterpret_cast<uint4 *>(s_hist)[tid] = make_uint4(0u, 0u, 0u, 0u);
     if (PEN) {
         history_clear<NV * TPB * 4>(s_cnt16);
         history_count(rv, row, pf, base, end, s_cnt16);
@@ -463,18 +467,33 @@ __device__ __forceinline__ void expsum_chunk(const RowView &rv, int row, int chu
     double      acc  = 0.0;
     double      accs[SLABS && !TRANSPOSED ? NV : 1];
     const float list_thr = zbin_threshold(zb_list); /* zbin(arg) <= zb_list */
+    /* the least p of the histogram's last bin: rows whose mass lies in a few peaks add little to it */
+    const float hist_least = HIST ? __uint_as_float(win_key_lo(hist_bins - 1)) : 0.0f;
     /* positions at or beyond `end` hold -inf (load_raw): they weigh exactly 0 and land in no
      * bin, so the loop carries no bound tests */
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
         double a4;
-        float  args[4];
+        float  args[4], weight[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             args[c]        = softmax_arg(f4_get(v[j], c), mx, inv_t);
-            const double p = (double) (FAST ? fast_expf_le0(args[c])
-                                            : geist_expf_glibc_le0(args[c], s_tab));
+            const float  e = FAST ? fast_expf_le0(args[c]) : geist_expf_glibc_le0(args[c], s_tab);
+            const double p = (double) e;
             a4             = c == 0 ? p : a4 + p;
+            if (HIST)
+                weight[c] = e;
+        }
+        if (HIST) {
+            /* (one test for the group: of a peaked row's elements next to none weigh anything) */
+            if (max3f(max3f(weight[0], weight[1], weight[2]), weight[3], weight[3]) >= hist_least) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const uint32_t t = WIN_TOP - __float_as_uint(weight[c]);
+                    if (weight[c] >= hist_least)
+                        atomicAdd(&s_hist[t >> WIN_SHIFT], win_weight(t));
+                }
+            }
         }
         if (LISTM) {
             /* the group's candidates go to the workgroup's staging list in LDS right away (the
@@ -568,6 +587,20 @@ __device__ __forceinline__ void expsum_chunk(const RowView &rv, int row, int chu
             chunk_sum[at] = total;
         }
     }
+    if (HIST) {
+        /* the wavefront that arrives last finds every addition performed and writes the chunk's
+         * histogram */
+        if (wave_arrives_last(fs.s_arrive + 4)) {
+            float *h = hist + ((long) row * rv.n_chunks + chunk) * WIN_BINS;
+            for (int i = 4 * (tid & (WAVE - 1)); i < hist_bins; i += 4 * WAVE) {
+                const uint4 t = *reinterpret_cast<const uint4 *>(s_hist + i);
+                /* (the four bins share an octave) */
+                const float scale = win_scale(i);
+                *reinterpret_cast<float4 *>(h + i) = make_float4(
+                    (float) t.x * scale, (float) t.y * scale, (float) t.z * scale, (float) t.w * scale);
+            }
+        }
+    }
     if (LISTM) {
         /* the wavefront that arrives last moves the staged entries to the row's list: one add to
          * the row's counter per workgroup. A workgroup with more candidates than the staging
@@ -597,7 +630,8 @@ __device__ __forceinline__ void expsum_chunk(const RowView &rv, int row, int chu
 /* The penalised list-making form needs 82 registers when left alone, two more than let a sixth
  * workgroup share a compute unit; held to 80 it spills nothing and a launch of 128 x 151936 is
  * about a microsecond shorter. (Held to 72 or 64 it spills and is slower.) */
-template <int NV, bool PEN, bool LISTM, bool SLABS, bool FAST = false, bool NOMEET = false>
+template <int NV, bool PEN, bool LISTM, bool SLABS, bool FAST = false, bool NOMEET = false,
+          bool HIST = false>
 __global__ __launch_bounds__(TPB, (NV == 8 && PEN && LISTM) ? 6 : 1) void k_scan_expsum(RowView rv, float inv_t,
                                                      float *__restrict__ tmax,
                                                      uint64_t *__restrict__ chunk_best,
@@ -605,13 +639,15 @@ __global__ __launch_bounds__(TPB, (NV == 8 && PEN && LISTM) ? 6 : 1) void k_scan
                                                      double *__restrict__ slab_sum,
                                                      const int32_t *__restrict__ probe_token,
                                                      int probe_L, float *__restrict__ probe_p,
-                                                     CandSpace list, int zb_list, MeetSpace meet) {
-    
+                                                     CandSpace list, int zb_list, MeetSpace meet,
+                                                     float *__restrict__ hist, int hist_bins) {
+    __shared__ __align__(16) uint32_t s_hist[HIST ? WIN_BINS : 4];
+    static_assert(!HIST || (!SLABS && !NOMEET), "forms with a histogram");
     __shared__ __align__(16) uint32_t s_cnt16[PEN ? NV * TPB * 2 : 1];
     __shared__ double   s_sum[SLABS ? NWAVES * NV : NWAVES];
     __shared__ uint64_t s_tab[32];
     __shared__ uint64_t s_red[NWAVES], s_bb;
-    __shared__ uint32_t s_arrive[4];
+    __shared__ uint32_t s_arrive[5];
     /* the staging list of the candidates: in the history's count table when there is one */
     __shared__ uint2 s_stage_own[(LISTM && !PEN) ? SCAN_STAGE : 1];
     static_assert(!(LISTM && PEN) || sizeof(s_cnt16) >= SCAN_STAGE * sizeof(uint2),
@@ -650,15 +686,15 @@ __global__ __launch_bounds__(TPB, (NV == 8 && PEN && LISTM) ? 6 : 1) void k_scan
     const bool plain = rv.vec_ok && end - base == NV * TPB * 4 && !(rv.softcap > 0.0f) &&
                        rv.allowed == nullptr;
     if (plain)
-        expsum_chunk<NV, PEN, LISTM, SLABS, true, FAST, NOMEET>(
+        expsum_chunk<NV, PEN, LISTM, SLABS, true, FAST, NOMEET, HIST>(
             rv, row, chunk, (int) gridDim.y, base, end, inv_t, chunk_sum, slab_sum,
             probe_token, probe_L, probe_p, list, zb_list, s_cnt16, s_sum, s_tab, tabv, s_tr, s_stage,
-            s_arrive + 3, fs);
+            s_arrive + 3, s_hist, hist, hist_bins, fs);
     else
-        expsum_chunk<NV, PEN, LISTM, SLABS, false, FAST, NOMEET>(
+        expsum_chunk<NV, PEN, LISTM, SLABS, false, FAST, NOMEET, HIST>(
             rv, row, chunk, (int) gridDim.y, base, end, inv_t, chunk_sum, slab_sum,
             probe_token, probe_L, probe_p, list, zb_list, s_cnt16, s_sum, s_tab, tabv, s_tr, s_stage,
-            s_arrive + 3, fs);
+            s_arrive + 3, s_hist, hist, hist_bins, fs);
 }
 
 /* The scaling of the form without a meeting: a wavefront per row, a lane per chunk. */
@@ -1192,13 +1228,13 @@ struct FinalArgs {
     const double   *slab_sum; /* FINAL_TEMPERATURE: [rows][chunks][SLABS_MAX] */
     const float    *tmax;
     int32_t        *out;
-    int32_t        *row_flag; /* FINAL_SORTED: 1 = the row goes on to the candidate list,
-                               * 2 = to the whole-row walk */
+    int32_t        *row_flag; /* FINAL_SORTED: 1 = the row goes on to k_window, 2 = to the
+                               * whole-row walk, 4 = to the walk over its min-p list */
     CandSpace       cand;
     double          ln_min_p; /* log(min_p), taken on the host */
-    int             zb_min_p; /* last z bin that can hold an entry passing min_p (with slack);
-                               * ZBINS - 1 when min_p is off or that deep */
-    bool            minp_listed; /* the exp-sum pass listed every row up to that bin */
+    WinSpace        win;
+    int             win_bins;
+    bool            minp_listed; /* the exp-sum pass listed the rows under the min-p bound */
     bool            cap_after;   /* top-k: the scan ran on the logits before the soft-cap (the
                                   * thread maxima, the candidates); the row-final kernel applies
                                   * it to what it keeps. The cap tanhf(x / c) * c never turns the
@@ -1453,6 +1489,7 @@ __device__ __forceinline__ bool topk_from_tmax(const RowView &rv, const FinalArg
 #include "sampler_draw.h"
 #include "sampler_sorted_prob.h"
 #include "sampler_walk_coop.h"
+#include "sampler_window.h"
 #include "sampler_spec.h"
 #include "sampler_draft.h"
 #include "sampler_cands.h"
@@ -1507,7 +1544,10 @@ template <int NV, bool PEN>
 __global__ __launch_bounds__(TPB) void k_final_sorted(RowView rv, FinalArgs a) {
     __shared__ uint64_t s_red[NWAVES];
     __shared__ uint64_t s_tab[32];
-    __shared__ __align__(16) uint8_t s_big[TMAX_LDS];
+    __shared__ union {
+        __align__(16) uint8_t slot[TMAX_LDS];
+        WinLocateShared       loc;
+    } s_big;
     __shared__ uint32_t s_mx[TPB];
     __shared__ int      s_selid[SEL_MAX];
     __shared__ __align__(16) uint32_t s_pcnt[PEN ? SEL_MAX * 4 * NV : 4];
@@ -1547,25 +1587,19 @@ __global__ __launch_bounds__(TPB) void k_final_sorted(RowView rv, FinalArgs a) {
         return;
     }
     if (a.minp_listed && a.cand.count[(long) row * CAND_COUNT_STRIDE] <= CAND_CAP) {
-        /* the exp-sum pass listed the row under the min-p bound (holding softmax arguments, not pn): the list
-         * walk serves it, top-p included -- the kept prefix is the shorter of the two */
+        /* the exp-sum pass listed the row under the min-p bound: the list walk serves it, top-p
+         * included -- the kept prefix is the shorter of the two */
         if (tid == 0) {
-            const int   B      = a.zb_min_p;
-            const float p_out  = geist_expf_glibc_le0(-(float) (B + 1) / (float) ZBIN_PER_NAT, s_tab);
-            const float pn_out = (float) ((double) p_out / sum);
-            a.cand.out_key[row]   = __float_as_uint(pn_out) + 1u;
-            a.cand.row_bound[row] = B;
-            a.cand.row_sum[row]   = sum;
-            a.row_flag[row]       = 4;
-            a.out[row]            = -1;
+            a.row_flag[row] = 4;
+            a.out[row]      = -1;
         }
         return;
     }
     if (C <= 16)
-        tok = sorted_from_tmax<NV, PEN, 16>(rv, a, row, mx, sum, u_row, s_big, s_mx, s_wt, s_selid,
+        tok = sorted_from_tmax<NV, PEN, 16>(rv, a, row, mx, sum, u_row, s_big.slot, s_mx, s_wt, s_selid,
                                             s_pcnt, s_m, s_srt, &s_n, &s_n2, s_tab);
     else if (C <= TMAX_LDS / TPB)
-        tok = sorted_from_tmax<NV, PEN, TMAX_LDS / TPB>(rv, a, row, mx, sum, u_row, s_big, s_mx,
+        tok = sorted_from_tmax<NV, PEN, TMAX_LDS / TPB>(rv, a, row, mx, sum, u_row, s_big.slot, s_mx,
                                                         s_wt, s_selid, s_pcnt, s_m, s_srt, &s_n,
                                                         &s_n2, s_tab);
     if (tok >= 0) {
@@ -1576,90 +1610,19 @@ __global__ __launch_bounds__(TPB) void k_final_sorted(RowView rv, FinalArgs a) {
         }
         return;
     }
-    /* The shortcut could not serve the row. Last z bin (z = (max - l) * inv_t) that can hold an
-     * element of the kept prefix.
-     *   top-p: estimated from ALL the row's thread maxima, binned by z with fast exponentials as
-     *   weights. Where M of the T scanning threads have their maximum above a value, about
-     *   -T ln(1 - M/T) elements lie above it if the vocabulary order is unrelated to the logits
-     *   (each element beyond a thread's first hides behind that thread's maximum), so a bin's
-     *   mass is scaled by 1 / (1 - M/T) at the bin. The first bin at which the scaled mass
-     *   passes top_p plus a quarter of the rest, and one more bin, is taken. It is an estimate:
-     *   the walk over the list sums the listed mass exactly and hands the row on to the
-     *   whole-row walk when the kept prefix is not certainly inside the list.
-     *   min-p: pn_i >= min_p * pn_0 needs z_i <= -ln(min_p), in closed form, taken with slack.
-     *   Both set: the shorter prefix, so the smaller bin. */
+    /* The shortcut could not serve the row: where its nucleus ends and its draw falls, for k_window */
     __syncthreads();
-    constexpr int COPIES = 8; /* lanes spread over copies of the bins: fewer same-address adds */
-    float        *s_zh   = reinterpret_cast<float *>(s_big);                      /* [COPIES][ZBINS] */
-    int          *s_zc   = reinterpret_cast<int *>(s_big + COPIES * ZBINS * 4);   /* [COPIES][ZBINS] */
-    static_assert(COPIES * ZBINS * 8 <= TMAX_LDS, "bins live in the slot table's space");
-    const bool want_p = a.top_p > 0.0f && a.top_p < 1.0f;
-    for (int i = tid; i < COPIES * ZBINS * 2; i += TPB)
-        reinterpret_cast<uint32_t *>(s_big)[i] = 0u;
-    __syncthreads();
-    if (want_p) {
-        const float *tm   = a.tmax + (long) row * C * TPB + tid;
-        const int    copy = (tid & (COPIES - 1)) * ZBINS;
-        const int    last = a.zb_min_p < ZBINS - 2 ? a.zb_min_p + 1 : ZBINS - 2; /* deeper bins cannot matter */
-        for (int q = 0; q < C; ++q) {
-            const float arg = softmax_arg(tm[(long) q * TPB], mx, a.inv_t);
-            const int   zb  = zbin(arg); /* NaN (a thread without an element) lands past `last` */
-            if (zb <= last) {
-                atomicAdd(&s_zc[copy + zb], 1);
-                unsafeAtomicAdd(&s_zh[copy + zb], __expf(arg));
-            }
-        }
-    }
-    __syncthreads();
-    if (tid < WAVE) {
-        int B = ZBINS - 1;
-        if (want_p) {
-            /* scanning threads that hold at least one element of the row */
-            const int rem  = rv.n_vocab - (C - 1) * rv.per_chunk;
-            const int T    = (C - 1) * TPB + ((rem + 3) / 4 < TPB ? (rem + 3) / 4 : TPB);
-            const int b0   = 2 * tid, b1 = 2 * tid + 1;
-            int       c0 = 0, c1 = 0;
-            float     w0 = 0.f, w1 = 0.f;
-#pragma unroll
-            for (int k = 0; k < COPIES; ++k) {
-                c0 += s_zc[k * ZBINS + b0];
-                c1 += s_zc[k * ZBINS + b1];
-                w0 += s_zh[k * ZBINS + b0];
-                w1 += s_zh[k * ZBINS + b1];
-            }
-            const int    before = wave_scan_i32_dpp(c0 + c1) - c0 - c1;
-            const double invT   = 1.0 / (double) (T > 0 ? T : 1);
-            const double l0     = 1.0 - ((double) before + 0.5 * (double) c0) * invT;
-            const double l1     = 1.0 - ((double) (before + c0) + 0.5 * (double) c1) * invT;
-            const double s0     = (double) w0 / (l0 > 0.05 ? l0 : 0.05);
-            const double s1     = (double) w1 / (l1 > 0.05 ? l1 : 0.05);
-            const double incl   = wave_scan_f64_dpp(s0 + s1);
-            const double need   = ((double) a.top_p + 0.25 * (1.0 - (double) a.top_p)) * sum;
-            const uint64_t h0   = __ballot(incl - s1 >= need && b0 < ZBINS - 1);
-            const uint64_t h1   = __ballot(incl >= need && b1 < ZBINS - 1);
-            int            first = ZBINS;
-            if (h0)
-                first = 2 * (__ffsll((long long) h0) - 1);
-            if (h1) {
-                const int f1 = 2 * (__ffsll((long long) h1) - 1) + 1;
-                first        = f1 < first ? f1 : first;
-            }
-            if (first < ZBINS - 1)
-                B = first + 1 < ZBINS - 1 ? first + 1 : first; /* one more bin for the estimate */
-        }
-        B = a.zb_min_p < B ? a.zb_min_p : B;
-        if (tid == 0) {
-            /* an element outside the list has z >= (B + 1) / ZBIN_PER_NAT (the product in zbin()
-             * is exact), so its p is at most expf of minus that; one step up covers any
-             * non-monotonic last bit of expf or of the division */
-            const float p_out  = geist_expf_glibc_le0(-(float) (B + 1) / (float) ZBIN_PER_NAT, s_tab);
-            const float pn_out = (float) ((double) p_out / sum);
-            a.cand.out_key[row]   = __float_as_uint(pn_out) + 1u;
-            a.cand.row_bound[row] = B;
-            a.cand.count[(long) row * CAND_COUNT_STRIDE]     = 0;
-            a.row_flag[row]       = B < ZBINS - 1 ? 1 : 2;
-            a.out[row]            = -1;
-        }
+    const bool    finite = sum > 0.0 && sum < __builtin_inf() && mx > -__builtin_inff() && mx < __builtin_inff();
+    double        h[4];
+    window_sum_hist(a.win.hist + (long) row * C * WIN_BINS, C, a.win_bins, s_big.loc, h);
+    const WinPlan plan = window_locate(h, a.win_bins, sum, a.top_p, a.min_p, u_row, s_big.loc);
+    if (tid == 0) {
+        WinRow *wr      = static_cast<WinRow *>(a.win.row) + row;
+        wr->plan        = plan;
+        wr->mx          = mx;
+        wr->sum         = sum;
+        a.row_flag[row] = finite && plan.ok ? 1 : 2;
+        a.out[row]      = -1;
     }
 }
 
@@ -1911,13 +1874,30 @@ static void dispatch(int nv, bool pen, F &&f) {
 int launch_scan_expsum(const Launch &L, float inv_t, float *tmax, uint64_t *chunk_best,
                         double *chunk_sum, const int32_t *probe_token, int probe_L, float *probe_p,
                         const CandSpace *list, int zb_list, double *slab_sum, const MeetSpace &meet,
-                        bool fast) {
+                        bool fast, float *hist, int hist_bins) {
     const dim3 grid(L.rv.n_chunks, L.rows), block(TPB);
     auto go = [&](auto kernel) {
         kernel<<<grid, block, 0, L.stream>>>(L.rv, inv_t, tmax, chunk_best, chunk_sum,
                                              list ? nullptr : slab_sum, probe_token, probe_L, probe_p,
-                                             list ? *list : CandSpace{}, list ? zb_list : 0, meet);
+                                             list ? *list : CandSpace{}, list ? zb_list : 0, meet, hist,
+                                             hist_bins);
     };
+    if (hist && list) { /* (rows in chunks of 8192) */
+        if (L.pen)
+            fast ? go(k_scan_expsum<8, true, true, false, true, false, true>)
+                 : go(k_scan_expsum<8, true, true, false, false, false, true>);
+        else
+            fast ? go(k_scan_expsum<8, false, true, false, true, false, true>)
+                 : go(k_scan_expsum<8, false, true, false, false, false, true>);
+        return 0;
+    }
+    if (hist) {
+        dispatch(L.nv, L.pen, [&](auto nv, auto pen) {
+            fast ? go(k_scan_expsum<GS_NV, GS_PEN, false, false, true, false, true>)
+                 : go(k_scan_expsum<GS_NV, GS_PEN, false, false, false, false, true>);
+        });
+        return 0;
+    }
     if (fast && !list && !L.pen) { /* the tolerance mode's form without a meeting */
         if (L.nv == 8)
             slab_sum ? go(k_scan_expsum<8, false, false, true, true, true>)
@@ -1949,6 +1929,23 @@ int launch_scan_expsum(const Launch &L, float inv_t, float *tmax, uint64_t *chun
                  : go(k_scan_expsum<GS_NV, GS_PEN, false, false>);
     });
     return 0;
+}
+
+int win_bins_for(float top_p, float min_p, size_t n_vocab) {
+    /* Elements below (1 - top_p) / n_vocab of the largest weigh less than 1 - top_p together (the
+     * row's sum is at least 1), so the nucleus ends above; min-p keeps nothing below min_p. One bin
+     * more for the roundings in between. */
+    double p = 0.0;
+    if (top_p > 0.0f && top_p < 1.0f)
+        p = (1.0 - (double) top_p) / (double) n_vocab;
+    if (min_p > 0.0f && (double) min_p > p)
+        p = min_p < 1.0f ? (double) min_p : 1.0;
+    const float pf = (float) (p * (1.0 - 1e-5));
+    uint32_t    key;
+    memcpy(&key, &pf, sizeof(key));
+    const int last = (int) ((0x3f800000u - key) >> WIN_SHIFT);
+    const int n    = (last + 2 + 3) & ~3;
+    return n < WIN_BINS ? n : WIN_BINS;
 }
 
 int zbin_of_min_p(float min_p) {
@@ -2045,7 +2042,8 @@ static FinalArgs final_args(const FinalLaunch &f) {
     a.out        = f.out;
     a.cand       = f.cand;
     a.ln_min_p   = f.min_p > 0.0f ? std::log((double) f.min_p) : 0.0;
-    a.zb_min_p    = zbin_of_min_p(f.min_p);
+    a.win         = f.win;
+    a.win_bins    = f.win_bins;
     a.minp_listed = f.minp_listed;
     a.cap_after   = f.cap_after;
     return a;
@@ -2249,9 +2247,7 @@ void launch_write_probs(const Launch &L, float inv_t, const uint64_t *chunk_best
 int configure_device_kernels() {
     /* k_sorted_candidates keeps a whole candidate list in LDS: more than the static limit */
     const int   dyn = CAND_CAP * (int) sizeof(uint32_t);
-    const void *kernels[] = {(const void *) k_sorted_candidates<2, false>,
-                             (const void *) k_sorted_candidates<2, true>,
-                             (const void *) k_sorted_candidates<8, false>,
+    const void *kernels[] = {(const void *) k_sorted_candidates<8, false>,
                              (const void *) k_sorted_candidates<8, true>};
     for (const void *k : kernels) {
         const hipError_t e =
@@ -2276,25 +2272,32 @@ void launch_candidates(const Launch &L, const FinalLaunch &f, float *probs, long
     g.ld_probs   = ld_probs;
     /* the cooperative whole-row walk holds a chunk of 8192 in registers */
     const int defer = wc.rows != nullptr && wc.spread && L.nv == 8 ? 1 : 0;
-    if (f.minp_direct) {
-        /* the exp-sum pass has listed every row: no row-final kernel, no listing pass. An
-         * unlisted element lies in z bin zb + 1 or beyond; the same expf as on the device. */
+    if (!f.minp_direct) {
+        /* a few rounds of workgroups at most: of a batch whose rows the shortcut has served, one that
+         * leaves at once still costs its start (8192 of them 5.7 us, 2048 2.5) */
+        const int per_wg = f.win_locate ? 1 : (int) (((long) L.rows * L.rv.n_chunks + 2047) / 2048);
+        const dim3 win_grid((L.rv.n_chunks + per_wg - 1) / per_wg, L.rows);
+        auto go = [&](auto kernel) {
+            kernel<<<win_grid, block, 0, L.stream>>>(L.rv, g, f.win, f.win_bins, per_wg, f.top_p, f.min_p,
+                                                     f.uniforms, f.row_flag, f.out, f.cand.path, wc.spread ? 4 : 3,
+                                                 defer, wc.hint, wc.call);
+        };
+        if (f.win_locate)
+            L.pen ? go(k_window<true, true>) : go(k_window<false, true>);
+        else
+            L.pen ? go(k_window<true, false>) : go(k_window<false, false>);
+    }
+    if (f.minp_direct || f.minp_listed) {
+        /* An unlisted element lies in z bin zb + 1 or beyond; the same expf as on the device. */
         static const uint64_t tab[32] = GEIST_EXPF_TABLE_INIT;
         const int             zb      = zbin_of_min_p(f.min_p);
         const float p_out = geist_expf_glibc_le0(-(float) (zb + 1) / (float) ZBIN_PER_NAT, tab);
-        dispatch(L.nv, L.pen, [&](auto nv, auto pen) {
-            k_sorted_candidates<GS_NV, GS_PEN><<<dim3(L.rows), block, dyn, L.stream>>>(
+        auto go = [&](auto kernel) {
+            kernel<<<dim3(L.rows), block, dyn, L.stream>>>(
                 L.rv, g, f.cand, f.top_p, f.min_p, f.uniforms, f.row_flag, f.out, f.chunk_sum,
-                L.rv.n_chunks, p_out, defer, wc.hint, wc.call);
-        });
-    } else {
-        dispatch(L.nv, L.pen, [&](auto nv, auto pen) {
-            k_list_candidates<GS_NV, GS_PEN><<<grid, block, 0, L.stream>>>(
-                L.rv, f.inv_t, f.chunk_best, f.chunk_sum, f.row_flag, f.cand);
-            k_sorted_candidates<GS_NV, GS_PEN><<<dim3(L.rows), block, dyn, L.stream>>>(
-                L.rv, g, f.cand, f.top_p, f.min_p, f.uniforms, f.row_flag, f.out, nullptr, 0, 0.0f,
-                defer, wc.hint, wc.call);
-        });
+                L.rv.n_chunks, p_out, f.minp_direct ? 0 : 1, defer, wc.hint, wc.call);
+        };
+        L.pen ? go(k_sorted_candidates<8, true>) : go(k_sorted_candidates<8, false>);
     }
     if (defer) {
         /* the rows flagged 2, a workgroup per chunk */
@@ -2312,11 +2315,11 @@ void launch_candidates(const Launch &L, const FinalLaunch &f, float *probs, long
                 wc.wait_limit, wc.hint, wc.call);
         /* rows that are still flagged 2 (a wait ran out, sums that are not finite): one workgroup
          * each, as without the spread walk */
-        dispatch(L.nv, L.pen, [&](auto nv, auto pen) {
-            k_sorted_candidates<GS_NV, GS_PEN><<<dim3(L.rows), block, dyn, L.stream>>>(
-                L.rv, g, f.cand, f.top_p, f.min_p, f.uniforms, f.row_flag, f.out, nullptr, 0, 0.0f,
-                0, nullptr, 0u);
-        });
+        auto go = [&](auto kernel) {
+            kernel<<<dim3(L.rows), block, 0, L.stream>>>(L.rv, g, f.cand, f.top_p, f.min_p, f.uniforms,
+                                                         f.row_flag, f.out);
+        };
+        L.pen ? go(k_whole_row<8, true>) : go(k_whole_row<8, false>);
     }
 }
 

@@ -9,10 +9,12 @@
  *   shortcut (k_final_sorted)    thread maxima -> a logit bound below which nothing of the kept
  *                                prefix can lie -> re-read the threads above it -> order those
  *                                entries -> walk. Kept prefixes of up to about a hundred.
- *   list (flag 1 or 4: k_list_candidates / the exp-sum pass, k_sorted_candidates)
- *                                every element up to a z bin is listed with its normalised
- *                                probability; one mass histogram over the list locates the
- *                                nucleus edge and the draw. Kept prefixes of thousands.
+ *   window (k_window, sampler_window.h)  the exp-sum pass's histogram of the masses tells in which
+ *                                narrow ranges the nucleus ends and the draw falls; one pass sums
+ *                                exactly what lies above them and lists what lies inside.
+ *   list (min-p of a few percent: k_sorted_candidates)  every element the min-p floor can keep is
+ *                                listed by the exp-sum pass; one mass histogram over the list
+ *                                locates the nucleus edge and the draw.
  *   whole row (flag 2: sorted_general_row)  the row's probabilities are written once, then a
  *                                mass-weighted radix descent over their bit patterns finds the
  *                                edge and the drawn entry. Anything else.
@@ -500,7 +502,7 @@ __device__ __forceinline__ void sg_select_digit(SortedGenShared &sh, uint64_t ta
  * limit_key = 0, limit_ties = 0 with `limited` false for no restriction.
  * Out: kappa (key bits), cnt_above / mass_above (strictly greater keys), ties_total.
  * Returns false when the whole (restricted) list weighs less than the target. */
-__device__ bool sg_descent(const float *pn, int n, uint64_t target, bool limited,
+__device__ __forceinline__ bool sg_descent(const float *pn, int n, uint64_t target, bool limited,
                            uint32_t limit_key, uint32_t limit_ties, SortedGenShared &sh,
                            uint32_t &kappa, uint32_t &cnt_above, uint64_t &mass_above,
                            uint32_t &ties_total) {
@@ -553,7 +555,7 @@ __device__ bool sg_descent(const float *pn, int n, uint64_t target, bool limited
 
 /* The j-th smallest id among the list entries whose key equals `key`, ids < 2^21: two counting
  * passes over the bits of the id (the list is in no particular order). */
-__device__ int list_jth_id(const float *pn, const uint32_t *ids, int n, uint32_t key, int j,
+__device__ __forceinline__ int list_jth_id(const float *pn, const uint32_t *ids, int n, uint32_t key, int j,
                            SortedGenShared &sh, int *s_scan, int *s_pick) {
     const int tid    = threadIdx.x;
     uint32_t  prefix = 0u;
@@ -614,7 +616,7 @@ __device__ int list_jth_id(const float *pn, const uint32_t *ids, int n, uint32_t
  * threads together having written all of them), or SEEN_NONE to have the maximum looked for. */
 constexpr uint32_t SEEN_NONE = 0xffffffffu;
 template <bool LIST>
-__device__ int sorted_descend(const float *pn, const uint32_t *ids, int n, float top_p, float min_p,
+__device__ __forceinline__ int sorted_descend(const float *pn, const uint32_t *ids, int n, float top_p, float min_p,
                               float u, uint32_t kout, SortedGenShared &sh, int *s_scan,
                               int *s_pick, uint32_t seen_max = SEEN_NONE) {
     const int  tid   = threadIdx.x;
@@ -855,113 +857,6 @@ __device__ __forceinline__ int sorted_general_row(const RowView &rv, int row, in
 }
 
 /* ============================================================================================
- * k_list_candidates: third pass over the rows flagged 1. Every element whose z bin is at or
- * before the row's bound is appended, in no particular order, to the row's list as (bits of its
- * normalised probability pn = (float)((double)p / sum), vocabulary id). A list longer than
- * CAND_CAP keeps counting; the row-final kernel then hands the row on.
- * ========================================================================================== */
-constexpr int LIST_STAGE = 2048; /* candidates of one chunk staged in LDS */
-
-template <int NV, bool PEN>
-__global__ __launch_bounds__(TPB) void k_list_candidates(RowView rv, float inv_t,
-                                                         const uint64_t *__restrict__ chunk_best,
-                                                         const double *__restrict__ chunk_sum,
-                                                         const int32_t *__restrict__ row_flag,
-                                                         CandSpace cand) {
-    static_assert(4 * NV <= 32, "one mask bit per element of a thread");
-    __shared__ __align__(16) uint32_t s_cnt16[PEN ? NV * TPB * 2 : 1];
-    __shared__ uint64_t s_red[NWAVES];
-    __shared__ uint64_t s_tab[32];
-    __shared__ double   s_total;
-    __shared__ int      s_count, s_base;
-    __shared__ float    s_arg[LIST_STAGE];
-    __shared__ uint32_t s_id[LIST_STAGE];
-    int                 row, chunk;
-    xcd_row_chunk(row, chunk);
-    const int tid = threadIdx.x;
-    if (row_flag[row] != 1)
-        return;
-    if (tid < 32)
-        s_tab[tid] = g_expf_tab[tid];
-    if (tid == 0) {
-        double t = 0.0;
-        for (int c = 0; c < rv.n_chunks; ++c)
-            t += chunk_sum[(long) row * rv.n_chunks + c];
-        s_total = t;
-        s_count = 0;
-    }
-    int base, end;
-    chunk_bounds<NV>(rv, chunk, base, end);
-    float4 v[NV];
-    fetch_chunk<NV, PEN>(rv, row, (int) gridDim.y, base, end, s_cnt16, v);
-    const float  mx  = key2f(best_key(row_best_from_chunks(chunk_best, row, rv.n_chunks, s_red)));
-    const double tot = s_total;
-    const int    B   = cand.row_bound[row];
-    const float  thr = zbin_threshold(B); /* zbin(arg) <= B */
-    uint32_t     mask = 0u;
-#pragma unroll
-    for (int j = 0; j < NV; ++j) {
-        const int e = base + 4 * (j * TPB + tid);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const bool in = e + c < end && softmax_arg(f4_get(v[j], c), mx, inv_t) > thr;
-            mask |= (uint32_t) in << (4 * j + c);
-        }
-    }
-    /* places: inside the workgroup through LDS, one global add for the workgroup */
-    int pos = wave_reserve(__popc(mask), &s_count);
-    __syncthreads();
-    const int n_blk = s_count;
-    if (tid == 0)
-        s_base = n_blk ? atomicAdd(&cand.count[(long) row * CAND_COUNT_STRIDE], n_blk) : 0;
-    uint32_t *ck = cand.key + (long) row * CAND_CAP;
-    uint32_t *ci = cand.idx + (long) row * CAND_CAP;
-    if (n_blk <= LIST_STAGE) {
-        /* stage (softmax argument, id) densely, then one exponential per staged entry */
-#pragma unroll
-        for (int j = 0; j < NV; ++j) {
-            const int e = base + 4 * (j * TPB + tid);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                if ((mask >> (4 * j + c)) & 1u) {
-                    s_arg[pos] = softmax_arg(f4_get(v[j], c), mx, inv_t);
-                    s_id[pos]  = (uint32_t) (e + c);
-                    ++pos;
-                }
-            }
-        }
-        __syncthreads();
-        const int gbase = s_base;
-        for (int i = tid; i < n_blk; i += TPB) {
-            if (gbase + i < CAND_CAP) {
-                const float p   = geist_expf_glibc_le0(s_arg[i], s_tab);
-                ck[gbase + i]   = __float_as_uint((float) ((double) p / tot));
-                ci[gbase + i]   = s_id[i];
-            }
-        }
-    } else {
-        __syncthreads();
-        pos += s_base;
-#pragma unroll
-        for (int j = 0; j < NV; ++j) {
-            const int e = base + 4 * (j * TPB + tid);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                if ((mask >> (4 * j + c)) & 1u) {
-                    if (pos < CAND_CAP) {
-                        const float p =
-                            geist_expf_glibc_le0(softmax_arg(f4_get(v[j], c), mx, inv_t), s_tab);
-                        ck[pos] = __float_as_uint((float) ((double) p / tot));
-                        ci[pos] = (uint32_t) (e + c);
-                    }
-                    ++pos;
-                }
-            }
-        }
-    }
-}
-
-/* ============================================================================================
  * list_walk_fast: the walk over a candidate list with ONE histogram. The keys that can matter lie
  * in (kout, kmax]; that range is cut into SG_BINS bins of equal width in key space, descending,
  * and the mass per bin is accumulated once (2^-62 fixed point, so exact and order-independent).
@@ -982,18 +877,6 @@ struct ListWalkShared {
     uint64_t res_before, res_before_edge, out_pack, out_mass;
     int      res_bin, n_small;
 };
-
-__device__ __forceinline__ uint64_t wave_scan_u64(uint64_t v) {
-    const int lane = threadIdx.x & (WAVE - 1);
-#pragma unroll
-    for (int d = 1; d < WAVE; d <<= 1) {
-        const uint64_t o = ((uint64_t) (uint32_t) __shfl_up((int) (v >> 32), d, WAVE) << 32) |
-                           (uint32_t) __shfl_up((int) (uint32_t) v, d, WAVE);
-        if (lane >= d)
-            v += o;
-    }
-    return v;
-}
 
 /* Orders and walks the entries of bin `b` that belong to the kept set (pack >= edge_pack): the
  * first one at which `before` plus the running mass reaches `target` goes to sh.out_pack, the
@@ -1188,14 +1071,36 @@ __device__ __forceinline__ int list_walk_fast(const float *pn, const uint32_t *i
     return (int) best_idx(sh.out_pack);
 }
 
-/* k_sorted_candidates: one workgroup per row flagged 1 or 4 walks the row's list (staged in LDS
- * when it fits; flag 4: listed by the exp-sum pass, holding p). On success the flag is cleared; a row the list cannot serve -- too long, or a kept
- * prefix that may reach past the list -- takes the whole-row walk (flag 2).
- * direct_sum != NULL: every row was listed by the exp-sum pass under the min-p bound (the list
- * holds softmax arguments, not pn) and no other kernel ran in between: the row's sum is taken from the chunk
- * sums here (in chunk order, as everywhere), the bound on an unlisted element's pn from
- * direct_p_out = expf of the first z bin outside the list, and the flag is written for every
- * row.
+/* The rows flagged 2, a workgroup each: the whole-row walk. */
+template <int NV, bool PEN>
+__global__ __launch_bounds__(TPB) void k_whole_row(RowView rv, SortedRowArgs g, CandSpace cand,
+                                                   float top_p, float min_p,
+                                                   const float *__restrict__ uniforms,
+                                                   const int32_t *__restrict__ row_flag,
+                                                   int32_t *__restrict__ out) {
+    __shared__ SortedGenShared sh;
+    __shared__ __align__(16) uint32_t s_cnt16[PEN ? NV * TPB * 2 : 1];
+    __shared__ uint64_t s_tab[32];
+    __shared__ double   s_total;
+    __shared__ int      s_scan[NWAVES];
+    __shared__ int      s_pick;
+    const int row = blockIdx.x;
+    if (row_flag[row] != 2)
+        return;
+    const int tok = sorted_general_row<NV, PEN>(rv, row, rv.n_rows, g, top_p, min_p, uniforms[row], sh,
+                                                s_cnt16, s_tab, s_scan, &s_pick, &s_total);
+    if (threadIdx.x == 0) {
+        out[row]       = tok;
+        cand.path[row] = 3;
+    }
+}
+
+/* k_sorted_candidates: one workgroup per row.
+ * The rows were listed by the exp-sum pass under the min-p bound (the list holds softmax
+ * arguments, not pn): all of them (only_flagged 0), or those flagged 4. The row's sum is taken from
+ * the chunk sums here (in chunk order, as everywhere), the bound on an unlisted element's pn from
+ * p_out = expf of the first z bin outside the list, and the flag is written. A row the list cannot
+ * serve -- too long, or a kept prefix that may reach past the list -- takes the whole-row walk.
  * walk_hint (page-locked host memory, or null): set to walk_call, the call's number, when a row
  * of the launch needs the whole-row walk -- the host then sends the next calls' such rows to
  * k_whole_row_coop, which spreads the walk over the row's chunks: this launch is told so by
@@ -1206,9 +1111,9 @@ __global__ __launch_bounds__(TPB) void k_sorted_candidates(RowView rv, SortedRow
                                                            const float *__restrict__ uniforms,
                                                            int32_t *__restrict__ row_flag,
                                                            int32_t *__restrict__ out,
-                                                           const double *__restrict__ direct_sum,
-                                                           int n_chunks, float direct_p_out,
-                                                           int defer_walk,
+                                                           const double *__restrict__ chunk_sum,
+                                                           int n_chunks, float p_out,
+                                                           int only_flagged, int defer_walk,
                                                            uint32_t *__restrict__ walk_hint,
                                                            uint32_t walk_call) {
     extern __shared__ uint32_t s_key[]; /* CAND_CAP keys: every list is walked from LDS */
@@ -1228,12 +1133,13 @@ __global__ __launch_bounds__(TPB) void k_sorted_candidates(RowView rv, SortedRow
      * the row's flag, the length of its list, the table of expf, the chunk sums (a thread each)
      * and the first two list entries of every thread (within the row's CAND_CAP places whatever
      * the length turns out to be) */
-    const int       flag = direct_sum ? 5 : row_flag[row];
+    if (only_flagged && row_flag[row] != 4)
+        return;
     const uint64_t  tabv = g_expf_tab[tid & 31];
     const int       n    = cand.count[(long) row * CAND_COUNT_STRIDE];
     const uint32_t *gk   = cand.key + (long) row * CAND_CAP;
     const uint32_t *gi   = cand.idx + (long) row * CAND_CAP;
-    const double    csum = direct_sum && tid < n_chunks ? direct_sum[(long) row * n_chunks + tid] : 0.0;
+    const double    csum = tid < n_chunks ? chunk_sum[(long) row * n_chunks + tid] : 0.0;
     const float     u_row = uniforms[row];
     uint32_t        kpre[2];
 #pragma unroll
@@ -1244,47 +1150,23 @@ __global__ __launch_bounds__(TPB) void k_sorted_candidates(RowView rv, SortedRow
     if (tid < MAX_CHUNKS)
         s_csum[tid] = csum;
     __syncthreads();
-    if (flag == 2) { /* sent past the list by the row-final kernel */
-        if (tid == 0 && walk_hint)
-            *walk_hint = walk_call;
-        if (defer_walk)
-            return; /* k_whole_row_coop follows and serves the rows flagged 2 */
-        const int t = sorted_general_row<NV, PEN>(rv, row, rv.n_rows, g, top_p, min_p,
-                                                  u_row, sh.gen, s_cnt16, s_tab, s_scan,
-                                                  &s_pick, &s_total);
-        if (tid == 0) {
-            out[row]       = t;
-            cand.path[row] = 3;
-        }
-        return;
-    }
-    if (flag != 1 && flag != 4 && flag != 5)
-        return;
-    int       tok = -1;
-    double   sum  = 1.0;
-    uint32_t kout = 0u;
-    if (direct_sum) {
-        /* every thread adds the chunk sums in chunk order */
-        sum = 0.0;
-        for (int c = 0; c < n_chunks; ++c)
-            sum += s_csum[c];
-        kout = __float_as_uint((float) ((double) direct_p_out / sum)) + 1u;
-    } else {
-        kout = cand.out_key[row];
-        if (flag == 4)
-            sum = cand.row_sum[row];
-    }
+    int    tok = -1;
+    double sum = 0.0; /* every thread adds the chunk sums in chunk order */
+    for (int c = 0; c < n_chunks; ++c)
+        sum += s_csum[c];
+    const uint32_t kout = __float_as_uint((float) ((double) p_out / sum)) + 1u;
     if (n >= 1 && n <= CAND_CAP) {
-        /* flags 4, 5: the list holds the softmax arguments; p = expf(argument),
+        /* the list holds the softmax arguments; p = expf(argument),
          * pn = (float)((double)p / sum), sampler.c:80, 251-253 */
+        auto pn_of = [&](uint32_t arg) {
+            return __float_as_uint(
+                (float) ((double) geist_expf_glibc_le0(__uint_as_float(arg), s_tab) / sum));
+        };
 #pragma unroll
         for (int q = 0; q < 2; ++q) { /* the entries asked for at the start */
             const int i = q * TPB + tid;
             if (i < n)
-                s_key[i] = flag >= 4 ? __float_as_uint((float) ((double) geist_expf_glibc_le0(
-                                                                    __uint_as_float(kpre[q]), s_tab) /
-                                                                sum))
-                                     : kpre[q];
+                s_key[i] = pn_of(kpre[q]);
         }
         for (int i0 = 2 * TPB; i0 < n; i0 += 8 * TPB) { /* eight independent loads in flight per thread */
             uint32_t k[8];
@@ -1295,10 +1177,7 @@ __global__ __launch_bounds__(TPB) void k_sorted_candidates(RowView rv, SortedRow
             for (int q = 0; q < 8; ++q) {
                 const int i = i0 + q * TPB + tid;
                 if (i < n)
-                    s_key[i] = flag >= 4 ? __float_as_uint((float) ((double) geist_expf_glibc_le0(
-                                                                        __uint_as_float(k[q]), s_tab) /
-                                                                    sum))
-                                         : k[q];
+                    s_key[i] = pn_of(k[q]);
             }
         }
         if (n <= CAND_LDS) {

@@ -177,9 +177,9 @@ int geist_hip_sampler_set_wait_limit(geist_hip_sampler *s, uint32_t polls);
  * negative on error. */
 int geist_hip_sampler_one_launch_topk(geist_hip_sampler *s, int enable);
 
-/* No counterpart in the reference. A top-p / min-p row whose kept prefix is too long for the
- * candidate list (tens of thousands of entries: a flat row at a high temperature) is walked in
- * full, as sampler.c:246-304 sorts and walks it. One workgroup takes 275 to 300 us for a row of
+/* No counterpart in the reference. A top-p / min-p row whose token neither a list nor the narrow
+ * ranges of its mass histogram can certify (long runs of equal values, a min-p list that overflows) is
+ * walked in full, as sampler.c:246-304 sorts and walks it. One workgroup takes 275 to 300 us for a row of
  * 128 k logits; spread over the workgroups of the row's chunks, which keep their part of the row
  * in registers and meet after every pass, the walk takes a fifth of that -- at the price of one
  * more launch per call.
@@ -189,7 +189,9 @@ int geist_hip_sampler_one_launch_topk(geist_hip_sampler *s, int enable);
  *   GEIST_HIP_WHOLE_ROW_WALK_SPREAD         always send it
  *   GEIST_HIP_WHOLE_ROW_WALK_ONE_WORKGROUP  never
  * Tokens are the same in every mode. geist_hip_sampler_row_paths reports 3 for a row walked by
- * one workgroup, 4 for a row walked by its chunks' workgroups. The waits of the spread form are
+ * one workgroup, 4 for a row walked by its chunks' workgroups; rows with more than 16384 kept
+ * entries that needed no such walk are reported as 3 in a call that would not have spread it, as 4
+ * in one that would. The waits of the spread form are
  * bounded by geist_hip_sampler_set_wait_limit like those of the one-pass kernels: a row whose
  * workgroups do not all turn up in time is walked by its first workgroup alone. */
 #define GEIST_HIP_WHOLE_ROW_WALK_ADAPTIVE 0
@@ -354,8 +356,9 @@ int geist_hip_host_malloc(geist_hip_sampler *s, size_t bytes, void **h_ptr);
 int geist_hip_host_free(geist_hip_sampler *s, void *h_ptr);
 
 /* Diagnostics (no reference counterpart): after a full-vocabulary top-p / min-p call, which walk
- * served each row: 1 = shortcut over the per-thread maxima, 2 = candidate list, 3 = the whole
- * row. Synchronous; h_paths receives `rows` entries. */
+ * served each row: 1 = the shortcut over the per-thread maxima (in small batches: at most 128 kept
+ * entries), 2 = a list, or narrow ranges of a kept prefix of at most 16384 entries, 3 and 4 = the
+ * whole row, or a longer prefix (geist_hip_sampler_set_whole_row_walk). Synchronous; h_paths receives `rows` entries. */
 int geist_hip_sampler_row_paths(geist_hip_sampler *s, int32_t *h_paths, size_t rows);
 
 /* Diagnostics (no reference counterpart): after a top-k call, which path served each row:

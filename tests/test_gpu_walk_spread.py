@@ -158,3 +158,41 @@ def test_waits_that_run_out(oracle, P):
             assert hs.row_paths(rows).tolist() == [4] * rows
     finally:
         hs.close()
+
+
+def window_rows(g, rows, n):
+    """Nuclei from a few entries to most of the row, and crowds where ranges of bins end or overflow."""
+    x = (g.standard_normal((rows, n)) * g.choice([0.5, 1.5, 2.0, 3.0], (rows, 1))).astype(np.float32)
+    x[1, : n // 2] = x[1].max() - 1.0 + 1e-3 * g.random(n // 2).astype(np.float32)  # one bin, over one chunk's stage
+    x[2] = np.round(x[2] * 16) / 16                     # runs of equal values, a few hundred each
+    x[3, 0], x[3, n - 1] = x[3].max() + 6.0, x[3].max() + 5.5   # first and last element lead
+    return x
+
+
+# 24 x 2047..50257: the plan found by the window pass itself; 96 rows: with a row-final kernel in front;
+# 260 x 66000: several chunks to a workgroup
+@pytest.mark.parametrize("rows,n", [(8, 2047), (8, 2048), (24, 2049), (5, 8193), (24, 50257), (96, 33001),
+                                    (96, 32768), (260, 66000)])
+@pytest.mark.parametrize("kw", [dict(top_p=0.95), dict(top_p=0.5, min_p=1e-3), dict(min_p=1e-4),
+                                dict(top_p=0.999)])
+def test_edge_and_draw_found_in_narrow_ranges(oracle, P, rows, n, kw):
+    """The token of rows served through the histogram of the masses: every size at which the launch
+    changes, draws at both ends, against the oracle's sorted walk. At most one row may lie within the
+    contract's 1e-6 of a slot's edge."""
+    from geistlib_amd import HipSampler
+    print(f"window rows={rows} n={n} {kw}", flush=True)
+    g = np.random.default_rng(rows * 100003 + n)
+    base = window_rows(g, 6, n)
+    x = np.ascontiguousarray(base[np.arange(rows) % 6])
+    ub = g.random(6).astype(np.float32)
+    ub[0], ub[5] = 0.0, np.float32(1.0 - 2.0 ** -24)
+    u = ub[np.arange(rows) % 6]
+    want, infos = want_of(oracle, base, ub, temperature=1.0, **kw)
+    hs = HipSampler(max_rows=rows, max_vocab=n)
+    try:
+        for call in range(2):                           # (the second may spread its whole-row walks)
+            got = run_rows(hs, torch, x, u, P(temperature=1.0, **kw))
+            assert compare_ids(got[:6], want[:len(got[:6])], infos[:len(got[:6])], f"{rows}x{n} {kw}") <= 1
+            assert all(got[r] == got[r % 6] for r in range(rows))
+    finally:
+        hs.close()
