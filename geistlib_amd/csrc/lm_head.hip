@@ -279,6 +279,190 @@ __global__ __launch_bounds__(LM_TPB) void k_q8w_gemv(const int8_t *__restrict__ 
                          y, ld_y, fuse);
 }
 
+/* q8w_gemv_m1 for three to eight activation rows, on the matrix cores. v_mfma_f32_4x4x1 performs, for
+ * sixteen blocks of four lanes, one fused multiply-add per output, rounded once (subnormals kept:
+ * compared with fmaf over every range of exponents), so a chain stays a chain: an accumulator per
+ * chain takes the columns 16 t + j in order as the reference's do. A lane holds a table row (its
+ * weight is the instruction's second operand); of the first operand one block of four activations
+ * is broadcast to all blocks, so one register carries sixteen columns of four activation rows and
+ * the instruction's block selector picks the column. Output register i of a lane: activation row i
+ * against the lane's table row.
+ *
+ * A workgroup has 64 table rows, a wavefront of it four of the sixteen chains (its quarter of every
+ * sixteen columns): four times the wavefronts that whole chains would give, which a table of 32000
+ * rows needs to fill the chip. 256 columns are staged in LDS as dwords [column / 4][row] -- written and
+ * read without bank conflicts --, two stages take turns, and two more are on their way in registers.
+ *
+ * What bounds it: the table's bytes, and from five rows on the matrix cores (256 operations in eight
+ * cycles; twice the vector unit's rate). The vector form, with an LDS read for every four
+ * multiply-adds, waited for LDS. */
+typedef float mfma_f4 __attribute__((ext_vector_type(4)));
+template <int J>
+__device__ __forceinline__ void chain_mfma(float x, float w, mfma_f4 &acc) {
+    acc = __builtin_amdgcn_mfma_f32_4x4x1f32(x, w, acc, 4, J, 0);
+}
+/* Four columns, one of each of the wavefront's chains: d holds the lane's weights, x[g] the activations
+ * of rows 4 g .. 4 g + 3 of four such steps, of which this is number U. */
+template <int G, int U>
+__device__ __forceinline__ void chains_step(uint32_t d, const float (&x)[G], mfma_f4 (&acc)[G][4]) {
+    float w[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        w[e] = (float) (int) (int8_t) (d >> (8 * e));
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        chain_mfma<4 * U + 0>(x[g], w[0], acc[g][0]);
+        chain_mfma<4 * U + 1>(x[g], w[1], acc[g][1]);
+        chain_mfma<4 * U + 2>(x[g], w[2], acc[g][2]);
+        chain_mfma<4 * U + 3>(x[g], w[3], acc[g][3]);
+    }
+}
+constexpr int MF_ROWS  = 64;  /* table rows of a workgroup */
+constexpr int MF_COLS  = 256; /* columns of a stage */
+constexpr int MF_PITCH = MF_ROWS + 1; /* dwords: rows 4 apart of 16 column groups fall on 64 banks */
+__device__ __forceinline__ void mf_barrier() { /* orders LDS only: loads stay on their way */
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+template <int G>
+__global__ __launch_bounds__(LM_TPB, 4) void k_q8w_gemv_mfma(const int8_t *__restrict__ wq,
+                                                             const float *__restrict__ scales,
+                                                             long n_out, int n_in,
+                                                             const float *__restrict__ x, long ld_x,
+                                                             int n_m, float *__restrict__ y, long ld_y) {
+    __shared__ union {
+        uint32_t tile[2][MF_COLS / 4][MF_PITCH];
+        float    chain[4][16][MF_ROWS]; /* the chains of four activation rows, at the end */
+    } s;
+    const int  tid = threadIdx.x, lane = tid & (LM_WAVE - 1);
+    const int  wave = __builtin_amdgcn_readfirstlane(tid / LM_WAVE);
+    const long row0 = (long) blockIdx.x * MF_ROWS;
+    mfma_f4    acc[G][4];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            acc[g][e] = mfma_f4{0.0f, 0.0f, 0.0f, 0.0f};
+    /* Rows beyond the table repeat its last, activation rows beyond n_m theirs, columns past the row's
+     * end (n_in is a multiple of 16) its last sixteen: none of them is used. */
+    const int     seg = tid & 15;
+    const int8_t *wp[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const long r = row0 + 16 * i + (tid >> 4);
+        wp[i]        = wq + (r < n_out ? r : n_out - 1) * n_in;
+    }
+    const float *xp[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const int m = 4 * g + (lane & 3);
+        xp[g]       = x + (m < n_m ? m : n_m - 1) * ld_x + 4 * wave + ((lane >> 2) & 3);
+    }
+    struct Regs {
+        uint4 w[4];
+    } r0, r1;
+    auto load = [&](int st, Regs &r) {
+        int col = st * MF_COLS + 16 * seg;
+        col     = col < n_in ? col : n_in - 16;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            typedef uint32_t nt_u4 __attribute__((ext_vector_type(4)));
+            const nt_u4 t = __builtin_nontemporal_load(reinterpret_cast<const nt_u4 *>(wp[i] + col));
+            r.w[i]        = make_uint4(t.x, t.y, t.z, t.w);
+        }
+    };
+    float xc[4][G], xn[4][G];
+    auto  load_x = [&](int st) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            int col = st * MF_COLS + 64 * q + 16 * (lane >> 4);
+            col     = col < n_in ? col : n_in - 16;
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+                xn[q][g] = xp[g][col];
+        }
+    };
+    auto store = [&](int st, const Regs &r) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            uint32_t *t = &s.tile[st & 1][4 * seg][16 * i + (tid >> 4)];
+            t[0 * MF_PITCH] = r.w[i].x;
+            t[1 * MF_PITCH] = r.w[i].y;
+            t[2 * MF_PITCH] = r.w[i].z;
+            t[3 * MF_PITCH] = r.w[i].w;
+        }
+    };
+    const int n_stage = (n_in + MF_COLS - 1) / MF_COLS;
+    load(0, r0);
+    if (n_stage > 1)
+        load(1, r1);
+    load_x(0);
+    store(0, r0);
+    if (n_stage > 2)
+        load(2, r0);
+    mf_barrier();
+    /* Stage st is in LDS; `next` holds the one behind it, the other registers the one after. */
+    auto stage = [&](int st, Regs &next) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+                xc[q][g] = xn[q][g];
+        if (st + 1 < n_stage) {
+            load_x(st + 1);
+            store(st + 1, next); /* (read last before the barrier behind the stage before this) */
+        }
+        if (st + 3 < n_stage)
+            load(st + 3, next);
+        const uint32_t *t    = &s.tile[st & 1][wave][lane];
+        const int       left = n_in - st * MF_COLS;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            /* (a branch per 64 columns: the compiler would convert a whole stage ahead) */
+            if (64 * q >= left)
+                break;
+            chains_step<G, 0>(t[(16 * q + 0) * MF_PITCH], xc[q], acc);
+            if (64 * q + 16 < left)
+                chains_step<G, 1>(t[(16 * q + 4) * MF_PITCH], xc[q], acc);
+            if (64 * q + 32 < left)
+                chains_step<G, 2>(t[(16 * q + 8) * MF_PITCH], xc[q], acc);
+            if (64 * q + 48 < left)
+                chains_step<G, 3>(t[(16 * q + 12) * MF_PITCH], xc[q], acc);
+        }
+        mf_barrier();
+    };
+    for (int st = 0; st < n_stage; st += 2) {
+        stage(st, r1);
+        if (st + 1 < n_stage)
+            stage(st + 1, r0);
+    }
+    /* wavefront i folds activation row i's chains: (chain j + chain j+8), (i + i+4),
+     * ((0+1) + (2+3)), as gemv_body */
+    const long  row   = row0 + lane;
+    const float scale = row < n_out ? scales[row] : 0.0f;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        if (g)
+            mf_barrier();
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                s.chain[i][4 * wave + e][lane] = acc[g][e][i];
+        mf_barrier();
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            v[j] = dadd(s.chain[wave][j][lane], s.chain[wave][j + 8][lane]);
+        const float q0 = dadd(v[0], v[4]), q1 = dadd(v[1], v[5]);
+        const float q2 = dadd(v[2], v[6]), q3 = dadd(v[3], v[7]);
+        const float sum = __fmul_rn(dadd(dadd(q0, q1), dadd(q2, q3)), scale);
+        if (row < n_out && 4 * g + wave < n_m)
+            y[(4 * g + wave) * ld_y + row] = sum;
+    }
+}
+
 /* The projection for several activation rows. Here a lane owns all sixteen chains of one weight
  * row (a wavefront works on 64 rows), so the activations of a step are the same for every lane
  * and come from scalar registers: each converted weight feeds n_m multiply-adds whose second
@@ -529,10 +713,13 @@ void launch_q8w_gemv(hipStream_t stream, const int8_t *wq, const float *scales, 
                                                          fuse ? *fuse : none);
     else if (n_m <= 2)
         k_q8w_gemv<2, false><<<grid, block, 0, stream>>>(wq, scales, n_out, n_in, x, ld_x, n_m, y, ld_y, none);
-    else if (n_m <= 4)
-        k_q8w_gemv<4, false><<<grid, block, 0, stream>>>(wq, scales, n_out, n_in, x, ld_x, n_m, y, ld_y, none);
-    else
-        k_q8w_gemv<8, false><<<grid, block, 0, stream>>>(wq, scales, n_out, n_in, x, ld_x, n_m, y, ld_y, none);
+    else {
+        const dim3 grid_m((unsigned) ((n_out + MF_ROWS - 1) / MF_ROWS));
+        if (n_m <= 4)
+            k_q8w_gemv_mfma<1><<<grid_m, block, 0, stream>>>(wq, scales, n_out, n_in, x, ld_x, n_m, y, ld_y);
+        else
+            k_q8w_gemv_mfma<2><<<grid_m, block, 0, stream>>>(wq, scales, n_out, n_in, x, ld_x, n_m, y, ld_y);
+    }
 }
 
 } // namespace gs

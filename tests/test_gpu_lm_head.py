@@ -258,6 +258,27 @@ def test_q8w_quantise_and_gemv_bit_exact(hs, oracle, n_out, n_in, m):
     assert (bits(got) == bits(want)).all(), np.argwhere(bits(got) != bits(want))[:5]
 
 
+@pytest.mark.parametrize("n_out,n_in", [(1, 16), (63, 240), (64, 256), (65, 272), (130, 1040), (257, 752),
+                                        (200, 1536)])
+@pytest.mark.parametrize("m,tiny", [(3, False), (4, True), (5, False), (7, True), (8, False), (13, False)])
+def test_q8w_gemv_of_several_rows(hs, oracle, n_out, n_in, m, tiny):
+    """Batches of three and more rows, by chains on the matrix cores: remainders of a workgroup's 64 table
+    rows, of a stage's 256 columns and of four activation rows, and sums among the subnormals. Every
+    chain is the oracle's, so every result is equal in every bit."""
+    print(f"q8w rows n_out={n_out} n_in={n_in} m={m} tiny={tiny}", flush=True)
+    g = np.random.default_rng(n_out * 31 + n_in + m)
+    wq = g.integers(-127, 128, (n_out, n_in)).astype(np.int8)
+    sc = g.random(n_out).astype(np.float32)
+    x = g.standard_normal((m, n_in)).astype(np.float32)
+    if tiny:
+        x *= np.float32(1e-40)
+        sc[:] = 1.0
+    y = torch.empty((m, n_out + 3), dtype=torch.float32, device="cuda")
+    hs.q8w_gemv(to_dev(wq, torch), to_dev(sc, torch), to_dev(x, torch), y[:, :n_out])
+    hs.sync()
+    assert np.array_equal(y[:, :n_out].cpu().numpy().view(np.uint32), oracle.q8w_gemv(wq, sc, x).view(np.uint32))
+
+
 @pytest.mark.parametrize("rows,vocab,d_model", [(1, 40000, 256), (1, 20000, 2560), (2, 9000, 512),
                                                 (3, 8200, 128), (9, 5000, 64)])
 def test_project_sample_rows_q8w_equals_the_separate_steps(hs, oracle, rows, vocab, d_model):
