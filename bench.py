@@ -1043,9 +1043,9 @@ def bench_lm_head_spec(args):
 
 
 def bench_whole_row_walk(args):
-    """Workload whole_row_walk: top-p rows whose kept prefix is tens of thousands of entries (flat
-    rows at temperature 1: logits N(0, 0.5^2), top-p 0.9), which neither the thread-maxima
-    shortcut nor the candidate list can serve: every row is walked in full
+    """Workload whole_row_walk: top-p rows of long runs of equal values (flat rows at temperature 1:
+    logits N(0, 0.5^2) rounded to halves, top-p 0.9), which neither the thread-maxima shortcut
+    nor the narrow ranges of the mass histogram can serve: every row is walked in full
     (src/engine/sampler.c:246-304 sorts and walks it). Timed per step for 1, 16 and 64 rows of
     128256 with the walk by one workgroup per row and spread over the workgroups of the row's
     chunks (geist_hip_sampler_set_whole_row_walk), the steps reading four copies of the batch in
@@ -1062,7 +1062,7 @@ def bench_whole_row_walk(args):
         hs = HipSampler(max_rows=rows, max_vocab=n)
         g = torch.Generator(device=dev)
         g.manual_seed(100 + rows)
-        xs = [torch.randn((rows, n), device=dev, generator=g) * 0.5 for _ in range(4)]
+        xs = [torch.round(torch.randn((rows, n), device=dev, generator=g)) * 0.5 for _ in range(4)]
         u = torch.rand(rows, device=dev, generator=g)
         out = torch.empty(rows, dtype=torch.int32, device=dev)
         got = {}
@@ -1091,7 +1091,7 @@ def bench_whole_row_walk(args):
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f32",
         "data": "synthetic",
         "config": {"workload": "whole_row_walk_b16_v128256", "rows": 16, "n_vocab": n,
-                   "temperature": 1.0, "top_p": 0.9, "logits": "N(0, 0.5^2)"},
+                   "temperature": 1.0, "top_p": 0.9, "logits": "N(0, 0.5^2) in halves"},
         "legs": legs,
     }
     if not args.no_cpu:

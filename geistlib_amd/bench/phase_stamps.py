@@ -12,7 +12,7 @@ times (--rows N: the same on N rows, e.g. 1 for the decode step of one session).
 closer to the uninstrumented kernel's than those of a dense one.
 
 --walk: the same for k_whole_row_coop (the whole-row top-p walk spread over the row's chunks) on
-ROWS (default 16) flat rows of 128256, top-p 0.9: the stamps of the first row's workgroups."""
+ROWS (default 16) flat rows of 128256 in halves, top-p 0.9: the stamps of the first row's workgroups."""
 import ctypes as C
 import os
 import sys
@@ -47,7 +47,7 @@ def walk_main(rows):
     hs = HipSampler(rows, vocab)
     g = torch.Generator(device="cuda")
     g.manual_seed(1)
-    xs = [torch.randn(rows, vocab, device="cuda", generator=g) * 0.5 for _ in range(4)]
+    xs = [torch.round(torch.randn(rows, vocab, device="cuda", generator=g)) * 0.5 for _ in range(4)]
     u = torch.rand(rows, device="cuda", generator=g)
     out = torch.zeros(rows, dtype=torch.int32, device="cuda")
     prm = SampleParams.make(temperature=1.0, top_p=0.9)

@@ -268,7 +268,8 @@ __global__ __launch_bounds__(LM_TPB) void k_f16_gemv(const uint16_t *__restrict_
 }
 
 /* q8w_gemv_m1 (kernel_f16_gemv.c:95-127): the same chains over int8 weights, times the row's
- * scale. Half the bytes per weight, so twice the columns per stage. */
+ * scale. Half the bytes per weight, so twice the columns per stage. One and two activation rows; more
+ * go to the matrix cores (k_q8w_gemv_mfma: two rows 65 us there, 58 here, for 128256 x 2560). */
 template <int MT, bool SL>
 __global__ __launch_bounds__(LM_TPB) void k_q8w_gemv(const int8_t *__restrict__ wq,
                                                      const float *__restrict__ scales, long n_out,
@@ -293,9 +294,11 @@ __global__ __launch_bounds__(LM_TPB) void k_q8w_gemv(const int8_t *__restrict__ 
  * rows needs to fill the chip. 256 columns are staged in LDS as dwords [column / 4][row] -- written and
  * read without bank conflicts --, two stages take turns, and two more are on their way in registers.
  *
- * What bounds it: the table's bytes, and from five rows on the matrix cores (256 operations in eight
- * cycles; twice the vector unit's rate). The vector form, with an LDS read for every four
- * multiply-adds, waited for LDS. */
+ * What bounds it: the table's bytes (128256 x 2560, 4 rows 66 us, 5.0 TB/s), and from five rows on the
+ * matrix cores too (63e12 of these multiply-adds a second in a loop of nothing else: 42 of the 93 us
+ * of 8 rows; the vector unit's rate is half that). The vector form, with an LDS read for every four
+ * multiply-adds and eight rows' work for five, waited for LDS: 92 us for 4 rows, 152 for 8;
+ * 32000 x 3072, 3 rows 44 -> 25, 8 rows 78 -> 30. */
 typedef float mfma_f4 __attribute__((ext_vector_type(4)));
 template <int J>
 __device__ __forceinline__ void chain_mfma(float x, float w, mfma_f4 &acc) {

@@ -583,9 +583,10 @@ static int reserve_sorted_workspace(geist_hip_sampler *s) {
         return GEIST_HIP_OK;
     const size_t R = s->max_rows;
     /* chunks of 8192 logits, or, in small batches, of 2048 */
-    size_t wgs = R * ((s->max_vocab + 8191) / 8192);
+    const size_t small = R * ((s->max_vocab + 2047) / 2048);
+    size_t       wgs   = R * ((s->max_vocab + 8191) / 8192);
     if (wgs < (size_t) gs::WIN_SMALL)
-        wgs = (size_t) gs::WIN_SMALL;
+        wgs = small < (size_t) gs::WIN_SMALL ? small : (size_t) gs::WIN_SMALL;
     /* one allocation, cut into parts of whole cache lines; those that start at zero come first */
     size_t size = 0;
     auto   part = [&](size_t bytes) {
@@ -594,10 +595,9 @@ static int reserve_sorted_workspace(geist_hip_sampler *s) {
         return at;
     };
     const size_t win_row = part(R * gs::WIN_ROW_BYTES), walk = part(gs::walk_coop_bytes(R)), zeroed = size;
-    const size_t win_list = part(R * gs::WIN_CAP * sizeof(uint64_t));
     const size_t win_chunk = part(wgs * gs::WIN_CHUNK_BYTES);
     const size_t win_hist = part(wgs * gs::WIN_BINS * sizeof(float));
-    const size_t key = part(R * CAND_CAP * sizeof(uint32_t)), idx = part(R * CAND_CAP * sizeof(uint32_t));
+    const size_t lists = part(R * gs::CAND_ROW * sizeof(uint32_t));
     const size_t count = part(R * gs::CAND_COUNT_STRIDE * sizeof(int32_t));
     const size_t path = part(R * sizeof(int32_t)), probs = part(R * s->max_vocab * sizeof(float));
     char        *base = nullptr;
@@ -616,11 +616,11 @@ static int reserve_sorted_workspace(geist_hip_sampler *s) {
     walk_hint[0] = walk_hint[1] = 0u;
     s->sorted_base = base;
     s->win.row     = base + win_row;
-    s->win.list    = reinterpret_cast<uint64_t *>(base + win_list);
+    s->win.list    = reinterpret_cast<uint64_t *>(base + lists);
     s->win.chunk   = base + win_chunk;
     s->win.hist    = reinterpret_cast<float *>(base + win_hist);
-    s->cand.key    = reinterpret_cast<uint32_t *>(base + key);
-    s->cand.idx    = reinterpret_cast<uint32_t *>(base + idx);
+    s->cand.key    = reinterpret_cast<uint32_t *>(base + lists);
+    s->cand.idx    = s->cand.key + CAND_CAP;
     s->cand.count  = reinterpret_cast<int32_t *>(base + count);
     s->cand.path   = reinterpret_cast<int32_t *>(base + path);
     s->walk_rows   = base + walk;

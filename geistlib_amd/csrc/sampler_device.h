@@ -600,17 +600,9 @@ __device__ __forceinline__ float softmax_arg(float l, float mx, float inv_t) {
     return __fmul_rn(__fsub_rn(l, mx), inv_t);
 }
 
-/* z bin of an element: z = -(softmax argument) >= 0 in steps of 1/ZBIN_PER_NAT, truncated;
- * -inf and everything past the last bin land in ZBINS - 1 or above (callers clamp or skip). The
- * exp-sum pass and the candidate pass must agree on it bit for bit, hence one function. */
-__device__ __forceinline__ int zbin(float arg) {
-    const float z = __fmul_rn(arg, -(float) ZBIN_PER_NAT);
-    return z < (float) (ZBINS - 1) ? (int) z : ZBINS - 1;
-}
-
-/* zbin(arg) <= b, as one comparison: the scaling in zbin() is by a power of two, hence exact,
- * and truncation keeps z < b + 1, so the test is arg > -(b + 1) / ZBIN_PER_NAT (false for NaN,
- * as zbin's last bin is). */
+/* The elements up to z bin b -- z = -(softmax argument) in steps of 1/ZBIN_PER_NAT, truncated -- are
+ * those with a softmax argument above this (false for NaN): the scaling is by a power of two, hence
+ * exact, and truncation keeps z < b + 1. */
 __device__ __forceinline__ float zbin_threshold(int b) {
     return -(float) (b + 1) / (float) ZBIN_PER_NAT;
 }

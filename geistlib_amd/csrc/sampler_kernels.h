@@ -88,11 +88,12 @@ struct Launch {
 constexpr int ZBINS        = 128;
 constexpr int ZBIN_PER_NAT = 4;
 constexpr int CAND_CAP     = 16384; /* list entries per row */
+constexpr int CAND_ROW     = 2 * CAND_CAP; /* words of a row: its keys, then its ids */
 constexpr int CAND_LDS     = 4096;  /* lists up to this length are staged in LDS */
 constexpr int CAND_COUNT_STRIDE = 32;
 struct CandSpace {
-    uint32_t *key;       /* [rows][CAND_CAP] bits of the softmax argument */
-    uint32_t *idx;       /* [rows][CAND_CAP] vocabulary ids */
+    uint32_t *key;       /* [rows][CAND_CAP], rows CAND_ROW apart: bits of the softmax argument */
+    uint32_t *idx;       /* ... vocabulary ids */
     int32_t  *count;     /* [rows * CAND_COUNT_STRIDE]: a row's counter has a cache line to itself
                           * (the appending wavefronts' atomic adds to one line serialise) */
     int32_t  *path;      /* [rows] which walk served the row (geist_hip_sampler_row_paths) */
@@ -110,9 +111,10 @@ constexpr int WIN_CAP   = 16384; /* list entries per row */
  * 63 x 63 reads) 39.3 / 43.5; 8 x 262144 (8 x 128 x 128) 58 / 54, 48 x 100000 (2352 chunks) 48 / 21. */
 constexpr int WIN_SMALL       = 1024;
 constexpr int WIN_SMALL_READS = 65536;
+static_assert(WIN_CAP * 2 == CAND_ROW, "a row's list takes the place of its min-p list");
 struct WinSpace {
     float    *hist;  /* [rows][chunks][WIN_BINS], by the launch's chunks */
-    uint64_t *list;  /* [rows][WIN_CAP] */
+    uint64_t *list;  /* [rows][WIN_CAP], where a row's min-p list would lie: a row has one or the other */
     void     *chunk; /* [rows][chunks] x WIN_CHUNK_BYTES */
     void     *row;   /* [rows] x WIN_ROW_BYTES, zero before the first use */
 };

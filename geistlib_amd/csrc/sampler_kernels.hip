@@ -15,9 +15,11 @@
  *   k_cand_scan, k_final_cand (sampler_cands.h)   the top-k path for plain rows: the scan hands
  *                    each wavefront's leading groups on, the row-final kernel gathers nothing
  *                                                                              sampler.c:178-228
- *   k_list_candidates, k_sorted_candidates (sampler_sorted_prob.h)
+ *   k_window (sampler_window.h), k_sorted_candidates, k_whole_row (sampler_sorted_prob.h),
+ *   k_whole_row_coop (sampler_walk_coop.h)
  *                    full-vocabulary top-p / min-p for kept prefixes the shortcut cannot
- *                    serve: candidate list, then the whole row                 sampler.c:246-304
+ *                    serve: narrow ranges of a mass histogram, the min-p list, the whole row
+ *                                                                              sampler.c:246-304
  *   k_write_probs    normalised probabilities of a row                        sampler.c:246-253
  *   k_chunk_lse, k_final_logprob   log-softmax of chosen tokens               tools/eval_geist.c:63-73
  *   k_penalties      in-place penalties                                       (no reference counterpart)
@@ -466,7 +468,7 @@ __device__ __forceinline__ void expsum_chunk(const RowView &rv, int row, int chu
     volatile double *tr = s_tr + (tid / WAVE) * (8 * WAVE);
     double      acc  = 0.0;
     double      accs[SLABS && !TRANSPOSED ? NV : 1];
-    const float list_thr = zbin_threshold(zb_list); /* zbin(arg) <= zb_list */
+    const float list_thr = zbin_threshold(zb_list);
     /* the least p of the histogram's last bin: rows whose mass lies in a few peaks add little to it */
     const float hist_least = HIST ? __uint_as_float(win_key_lo(hist_bins - 1)) : 0.0f;
     /* positions at or beyond `end` hold -inf (load_raw): they weigh exactly 0 and land in no
@@ -614,8 +616,8 @@ __device__ __forceinline__ void expsum_chunk(const RowView &rv, int row, int chu
             if (lane == 0 && total)
                 at = atomicAdd(&list.count[(long) row * CAND_COUNT_STRIDE], (int) total);
             at = __builtin_amdgcn_readfirstlane(at);
-            uint32_t *ck = list.key + (long) row * CAND_CAP;
-            uint32_t *ci = list.idx + (long) row * CAND_CAP;
+            uint32_t *ck = list.key + (long) row * CAND_ROW;
+            uint32_t *ci = list.idx + (long) row * CAND_ROW;
             for (uint32_t i = lane; i < n && i < SCAN_STAGE; i += WAVE) {
                 const uint2 t = s_stage[i];
                 if (at + (int) i < CAND_CAP) {
@@ -2193,11 +2195,16 @@ void launch_row_final(const Launch &L, const FinalLaunch &f) {
         k_final_argmax<<<grid, block, 0, L.stream>>>(L.rv, a);
         return;
     }
+    if (f.mode == FINAL_SORTED) { /* (rows in chunks of 8192: smaller batches have no such launch) */
+        if (L.pen)
+            k_final_sorted<8, true><<<grid, block, 0, L.stream>>>(L.rv, a);
+        else
+            k_final_sorted<8, false><<<grid, block, 0, L.stream>>>(L.rv, a);
+        return;
+    }
     dispatch(L.nv, L.pen, [&](auto nv, auto pen) {
         if (f.mode == FINAL_TEMPERATURE)
             k_final_temperature<GS_NV, GS_PEN><<<grid, block, 0, L.stream>>>(L.rv, a);
-        else if (f.mode == FINAL_SORTED)
-            k_final_sorted<GS_NV, GS_PEN><<<grid, block, 0, L.stream>>>(L.rv, a);
         else if (L.rv.allowed)
             k_final_topk<GS_NV, GS_PEN, true><<<grid, block, 0, L.stream>>>(L.rv, a);
         else

@@ -1137,8 +1137,8 @@ __global__ __launch_bounds__(TPB) void k_sorted_candidates(RowView rv, SortedRow
         return;
     const uint64_t  tabv = g_expf_tab[tid & 31];
     const int       n    = cand.count[(long) row * CAND_COUNT_STRIDE];
-    const uint32_t *gk   = cand.key + (long) row * CAND_CAP;
-    const uint32_t *gi   = cand.idx + (long) row * CAND_CAP;
+    const uint32_t *gk   = cand.key + (long) row * CAND_ROW;
+    const uint32_t *gi   = cand.idx + (long) row * CAND_ROW;
     const double    csum = tid < n_chunks ? chunk_sum[(long) row * n_chunks + tid] : 0.0;
     const float     u_row = uniforms[row];
     uint32_t        kpre[2];
