@@ -631,7 +631,8 @@ class HipSampler:
 
     def row_paths(self, rows):
         """Which walk served each row of the last full-vocabulary top-p / min-p call
-        (1 shortcut, 2 a list or narrow ranges, 3 / 4 the whole row or a longer prefix)."""
+        (1 shortcut, 2 min-p list, 3 / 4 the whole row by one workgroup / by its chunks',
+        5 narrow ranges of the mass histogram)."""
         import numpy as np
         out = np.zeros(int(rows), dtype=np.int32)
         self._check(self.lib.geist_hip_sampler_row_paths(self.h, out.ctypes.data_as(C.c_void_p),

@@ -91,12 +91,20 @@ constexpr int CAND_CAP     = 16384; /* list entries per row */
 constexpr int CAND_ROW     = 2 * CAND_CAP; /* words of a row: its keys, then its ids */
 constexpr int CAND_LDS     = 4096;  /* lists up to this length are staged in LDS */
 constexpr int CAND_COUNT_STRIDE = 32;
+/* What geist_hip_sampler_row_paths reports: the walk that has run and given the token. */
+enum RowPath : int32_t {
+    PATH_SHORTCUT      = 1, /* the thread maxima (or a row whose sum is NaN: no walk) */
+    PATH_LIST          = 2, /* the list under the min-p bound */
+    PATH_ONE_WORKGROUP = 3, /* the whole row, by one workgroup */
+    PATH_SPREAD        = 4, /* the whole row, by the workgroups of its chunks */
+    PATH_WINDOW        = 5, /* narrow ranges of the mass histogram (k_window) */
+};
 struct CandSpace {
     uint32_t *key;       /* [rows][CAND_CAP], rows CAND_ROW apart: bits of the softmax argument */
     uint32_t *idx;       /* ... vocabulary ids */
     int32_t  *count;     /* [rows * CAND_COUNT_STRIDE]: a row's counter has a cache line to itself
                           * (the appending wavefronts' atomic adds to one line serialise) */
-    int32_t  *path;      /* [rows] which walk served the row (geist_hip_sampler_row_paths) */
+    int32_t  *path;      /* [rows] which walk served the row, a RowPath */
 };
 
 /* Workspace of the rows of the top-p / min-p modes that the thread-maxima shortcut does not serve

@@ -1584,7 +1584,7 @@ __global__ __launch_bounds__(TPB) void k_final_sorted(RowView rv, FinalArgs a) {
         if (tid == 0) {
             a.row_flag[row]  = 0;
             a.out[row]       = rv.n_vocab - 1;
-            a.cand.path[row] = 1;
+            a.cand.path[row] = PATH_SHORTCUT;
         }
         return;
     }
@@ -1608,7 +1608,7 @@ __global__ __launch_bounds__(TPB) void k_final_sorted(RowView rv, FinalArgs a) {
         if (tid == 0) {
             a.row_flag[row]  = 0;
             a.out[row]       = tok;
-            a.cand.path[row] = 1;
+            a.cand.path[row] = PATH_SHORTCUT;
         }
         return;
     }
@@ -2286,8 +2286,8 @@ void launch_candidates(const Launch &L, const FinalLaunch &f, float *probs, long
         const dim3 win_grid((L.rv.n_chunks + per_wg - 1) / per_wg, L.rows);
         auto go = [&](auto kernel) {
             kernel<<<win_grid, block, 0, L.stream>>>(L.rv, g, f.win, f.win_bins, per_wg, f.top_p, f.min_p,
-                                                     f.uniforms, f.row_flag, f.out, f.cand.path, wc.spread ? 4 : 3,
-                                                 defer, wc.hint, wc.call);
+                                                     f.uniforms, f.row_flag, f.out, f.cand.path, defer,
+                                                     wc.hint, wc.call);
         };
         if (f.win_locate)
             L.pen ? go(k_window<true, true>) : go(k_window<false, true>);

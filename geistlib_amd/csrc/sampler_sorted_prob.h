@@ -1091,7 +1091,7 @@ __global__ __launch_bounds__(TPB) void k_whole_row(RowView rv, SortedRowArgs g, 
                                                 s_cnt16, s_tab, s_scan, &s_pick, &s_total);
     if (threadIdx.x == 0) {
         out[row]       = tok;
-        cand.path[row] = 3;
+        cand.path[row] = PATH_ONE_WORKGROUP;
     }
 }
 
@@ -1197,7 +1197,7 @@ __global__ __launch_bounds__(TPB) void k_sorted_candidates(RowView rv, SortedRow
     }
     /* what the list cannot certify takes the whole-row walk here and now (tok is the same in
      * every thread) */
-    int path = 2;
+    RowPath path = PATH_LIST;
     if (tok < 0) {
         if (tid == 0 && walk_hint)
             *walk_hint = walk_call;
@@ -1208,10 +1208,10 @@ __global__ __launch_bounds__(TPB) void k_sorted_candidates(RowView rv, SortedRow
         }
         tok  = sorted_general_row<NV, PEN>(rv, row, rv.n_rows, g, top_p, min_p, u_row,
                                            sh.gen, s_cnt16, s_tab, s_scan, &s_pick, &s_total);
-        path = 3;
+        path = PATH_ONE_WORKGROUP;
     }
     if (tid == 0) {
-        row_flag[row]  = path == 3 ? 2 : 0;
+        row_flag[row]  = path == PATH_ONE_WORKGROUP ? 2 : 0;
         out[row]       = tok;
         cand.path[row] = path;
     }

@@ -656,7 +656,7 @@ __global__ __launch_bounds__(TPB, 2) void k_whole_row_coop(RowView rv, SortedRow
             for (int c = 0; c < 4; ++c) {
                 if (key[4 * q + c] == kd && ++seen == want) {
                     out[row]       = base + 4 * (q * TPB + tid) + c;
-                    cand.path[row] = 4;
+                    cand.path[row] = PATH_SPREAD;
                     row_flag[row]  = 0; /* served */
                 }
             }

@@ -198,9 +198,8 @@ struct WinRow {
     uint32_t pad[18];
 };
 static_assert(sizeof(WinRow) == 128, "a cache line per row");
-struct WinChunk { /* what a workgroup reports */
+struct alignas(32) WinChunk { /* what a workgroup reports, within a cache line: */
     uint64_t above_e, above_d, above_m; /* mass before the edge's bins, the draw's, of the min-p prefix */
-    uint64_t kept;                      /* entries up to the plan's last bin */
 };
 
 constexpr int WIN_SUB = 512; /* sub-bins of a range's keys: a few entries each */
@@ -300,8 +299,8 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
                                                 const float *__restrict__ uniforms,
                                                 int32_t *__restrict__ row_flag,
                                                 int32_t *__restrict__ out,
-                                                int32_t *__restrict__ path, int wide_path,
-                                                int defer_walk, uint32_t *__restrict__ walk_hint,
+                                                int32_t *__restrict__ path, int defer_walk,
+                                                uint32_t *__restrict__ walk_hint,
                                                 uint32_t walk_call) {
     constexpr int NV = LOCATE ? 2 : 8;
     /* LDS in two parts: the plan's words, then the list's staging, or the whole-row walk's words; and
@@ -319,8 +318,8 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
         __align__(16) uint32_t cnt16[PEN ? NV * TPB * 2 : 1];
     } sb;
     __shared__ uint64_t s_tab[32];
-    __shared__ uint64_t s_part[NWAVES][4];
-    __shared__ uint64_t s_sum[4];
+    __shared__ uint64_t s_part[NWAVES][3];
+    __shared__ uint64_t s_sum[3];
     __shared__ uint32_t s_n, s_base;
     __shared__ int      s_last;
     __shared__ double   s_total;
@@ -360,7 +359,7 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
             if (wg == 0 && tid == 0) {
                 row_flag[row] = 0;
                 out[row]      = rv.n_vocab - 1;
-                path[row]     = 1;
+                path[row]     = PATH_WINDOW;
             }
             return;
         }
@@ -383,7 +382,6 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
         const float floor_w = __fmul_rn(min_p, pn_0);
         const int   e0 = plan.need_p ? plan.e0 : 0, e1 = plan.need_p ? plan.e1 : -1;
         uint64_t    a_e = 0, a_d = 0, a_m = 0;
-        uint32_t    kept = 0;
         const int last_chunk = (wg + 1) * per_wg < C ? (wg + 1) * per_wg : C;
 #pragma unroll 1
         for (int chunk = wg * per_wg;;) {
@@ -404,7 +402,6 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
                         a_e += d < e0 ? fx : 0ull;
                         a_d += d < plan.d0 ? fx : 0ull;
                         a_m += pn >= floor_w ? fx : 0ull;
-                        kept += d <= plan.last;
                         const bool re = d >= e0 && d <= e1, rd = d >= plan.d0 && d <= plan.d1;
                         if (re || rd) {
                             const uint32_t at = __hip_atomic_fetch_add(&s_n, 1u, __ATOMIC_RELAXED,
@@ -426,12 +423,10 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
         a_e = wave_scan_u64(a_e);
         a_d = wave_scan_u64(a_d);
         a_m = wave_scan_u64(a_m);
-        const uint64_t kw = (uint64_t) (uint32_t) wave_scan_i32_dpp((int) kept);
         if (lane == WAVE - 1) {
             s_part[tid / WAVE][0] = a_e;
             s_part[tid / WAVE][1] = a_d;
             s_part[tid / WAVE][2] = a_m;
-            s_part[tid / WAVE][3] = kw;
         }
         __syncthreads();
         const uint32_t n = s_n;
@@ -439,7 +434,7 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
             s_base = __hip_atomic_fetch_add(&wr->count, n > (uint32_t) WIN_STAGE ? (uint32_t) WIN_CAP + 1u : n,
                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         WinChunk *slots = static_cast<WinChunk *>(win.chunk) + (long) row * W;
-        if (tid < 4) {
+        if (tid < 3) {
             uint64_t t = 0;
 #pragma unroll
             for (int w = 0; w < NWAVES; ++w)
@@ -468,17 +463,17 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
         constexpr int EARLY = 4;
         /* (a thread per workgroup; the list's first entries are asked for before its length is known) */
         const uint32_t total = coop_ld32(&wr->count);
-        uint64_t       part[4], first[EARLY];
+        uint64_t       part[3], first[EARLY];
         static_assert(WIN_CAP >= EARLY * TPB, "the list has places for the early loads");
         const int slot = tid < W ? tid : W - 1;
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+        for (int q = 0; q < 3; ++q)
             part[q] = coop_ld64(&slots[slot].above_e + q);
 #pragma unroll
         for (int q = 0; q < EARLY; ++q)
             first[q] = coop_ld64(rl + q * TPB + tid);
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+        for (int q = 0; q < 3; ++q)
             part[q] = tid < W ? part[q] : 0ull;
         /* most lists are in registers with that; the rest of a long one is read each time */
         auto each = [&](auto &&f) {
@@ -490,7 +485,7 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
                 f(coop_ld64(rl + i));
         };
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < 3; ++q) {
             const uint64_t t = wave_scan_u64(part[q]);
             if (lane == WAVE - 1)
                 s_part[tid / WAVE][q] = t;
@@ -505,7 +500,7 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
             sb.find.n_small = 0;
             sb.find.found   = 0;
         }
-        if (tid < 4) {
+        if (tid < 3) {
             uint64_t t = 0;
 #pragma unroll
             for (int w = 0; w < NWAVES; ++w)
@@ -513,7 +508,7 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
             s_sum[tid] = t;
         }
         __syncthreads();
-        const uint64_t above_e = s_sum[0], above_d = s_sum[1], above_m = s_sum[2], n_kept = s_sum[3];
+        const uint64_t above_e = s_sum[0], above_d = s_sum[1], above_m = s_sum[2];
         auto pn_bits = [&](uint32_t key) {
             return __float_as_uint((float) ((double) __uint_as_float(key) / tot));
         };
@@ -594,7 +589,7 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
                     ok = best_key(got) < key_over(plan.d0) && best_key(got) > key_under(plan.d1);
                     if (ok && tid == 0) {
                         out[row]  = (int32_t) best_idx(got);
-                        path[row] = LOCATE && n_kept <= 128ull ? 1 : n_kept <= (uint64_t) CAND_CAP ? 2 : wide_path;
+                        path[row] = PATH_WINDOW;
                         row_flag[row] = 0;
                     }
                 }
@@ -618,7 +613,7 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
                                                 s_tab, s_scan, &s_pick, &s_total);
     if (tid == 0) {
         out[row]  = tok;
-        path[row] = 3;
+        path[row] = PATH_ONE_WORKGROUP;
     }
 }
 

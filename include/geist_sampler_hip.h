@@ -189,9 +189,7 @@ int geist_hip_sampler_one_launch_topk(geist_hip_sampler *s, int enable);
  *   GEIST_HIP_WHOLE_ROW_WALK_SPREAD         always send it
  *   GEIST_HIP_WHOLE_ROW_WALK_ONE_WORKGROUP  never
  * Tokens are the same in every mode. geist_hip_sampler_row_paths reports 3 for a row walked by
- * one workgroup, 4 for a row walked by its chunks' workgroups; rows with more than 16384 kept
- * entries that needed no such walk are reported as 3 in a call that would not have spread it, as 4
- * in one that would. The waits of the spread form are
+ * one workgroup, 4 for a row walked by its chunks' workgroups. The waits of the spread form are
  * bounded by geist_hip_sampler_set_wait_limit like those of the one-pass kernels: a row whose
  * workgroups do not all turn up in time is walked by its first workgroup alone. */
 #define GEIST_HIP_WHOLE_ROW_WALK_ADAPTIVE 0
@@ -356,9 +354,9 @@ int geist_hip_host_malloc(geist_hip_sampler *s, size_t bytes, void **h_ptr);
 int geist_hip_host_free(geist_hip_sampler *s, void *h_ptr);
 
 /* Diagnostics (no reference counterpart): after a full-vocabulary top-p / min-p call, which walk
- * served each row: 1 = the shortcut over the per-thread maxima (in small batches: at most 128 kept
- * entries), 2 = a list, or narrow ranges of a kept prefix of at most 16384 entries, 3 and 4 = the
- * whole row, or a longer prefix (geist_hip_sampler_set_whole_row_walk). Synchronous; h_paths receives `rows` entries. */
+ * served each row: 1 = the shortcut over the per-thread maxima, 2 = the list under the min-p bound,
+ * 3 and 4 = the whole row, by one workgroup or by its chunks' (geist_hip_sampler_set_whole_row_walk),
+ * 5 = narrow ranges of the row's mass histogram. Synchronous; h_paths receives `rows` entries. */
 int geist_hip_sampler_row_paths(geist_hip_sampler *s, int32_t *h_paths, size_t rows);
 
 /* Diagnostics (no reference counterpart): after a top-k call, which path served each row:

@@ -30,6 +30,21 @@ def pack_allowed(allowed):
     return np.ascontiguousarray(packed).view(np.uint32).reshape(rows, words).view(np.int32)
 
 
+def crowded_rows(g, rows, n):
+    """Flat rows of which most elements crowd at one place: more of them in a single bin of the mass
+    histogram than its lists hold, so that a nucleus that ends there, or a draw that falls there, takes
+    the whole-row walk (n of 20000 and more; top-p 0.5 to 0.95 end there). Row 1 is quantised (index
+    order among equal probabilities), row 2 has a few tiny probabilities, row 3 is all equal."""
+    x = (g.standard_normal((rows, n)) * 0.4).astype(np.float32)
+    crowd = g.random((rows, n)) < 0.85
+    x[crowd] = (-0.5 + 0.0005 * g.standard_normal(int(crowd.sum()))).astype(np.float32)
+    x[1] = np.round(x[1] * 4) / 4
+    x[2, g.integers(0, n, 50)] = -90.0
+    if rows > 3:
+        x[3] = 1.0
+    return x
+
+
 def run_rows(sampler, torch, logits, uniforms, params, history=None, history_len=None,
              pad=0, lead=0, allowed=None):
     """pad: extra elements between rows; lead: elements before the first row (an unaligned base).

@@ -6,7 +6,7 @@ between its steps run out and a row's first workgroup has to walk it alone."""
 import numpy as np
 import pytest
 
-from gpu_util import compare_ids, run_rows
+from gpu_util import compare_ids, crowded_rows, run_rows
 
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
@@ -18,15 +18,6 @@ ADAPTIVE, SPREAD, ONE = 0, 1, 2
 def P():
     from geistlib_amd import SampleParams
     return SampleParams.make
-
-
-def flat_rows(g, rows, n):
-    x = (g.standard_normal((rows, n)) * 0.4).astype(np.float32)
-    x[1] = np.round(x[1] * 4) / 4             # many equal probabilities: index order decides
-    x[2, g.integers(0, n, 50)] = -90.0        # a few tiny probabilities
-    if rows > 3:
-        x[3] = 1.0                            # all equal
-    return x
 
 
 def want_of(oracle, x, u, **kw):
@@ -45,7 +36,7 @@ def test_spread_walk_gives_the_oracles_tokens(oracle, P, n):
         hs.set_whole_row_walk(SPREAD)
         for kw in (dict(temperature=1.0, top_p=0.9), dict(temperature=0.8, top_p=0.95, min_p=1e-4),
                    dict(temperature=1.3, min_p=1e-5), dict(temperature=1.0, top_p=0.5)):
-            x = flat_rows(g, rows, n)
+            x = crowded_rows(g, rows, n)
             u = g.random(rows).astype(np.float32)
             u[4] = 0.0
             u[5] = np.float32(1.0 - 2.0 ** -24)
@@ -54,9 +45,9 @@ def test_spread_walk_gives_the_oracles_tokens(oracle, P, n):
             want, infos = want_of(oracle, x, u, **kw)
             near = compare_ids(got, want, infos, f"spread walk n={n} {kw}")
             assert near <= 1
-            # (short rows and narrow nuclei are within the list's reach: path 2)
-            assert set(paths) <= {2, 4}, (paths, kw)
-            if n >= 50001 and kw.get("top_p", 1.0) >= 0.9:
+            # (short rows, and draws beside the crowd without a nucleus, need no such walk)
+            assert set(paths) <= {2, 4, 5}, (paths, kw)
+            if n >= 20000 and "top_p" in kw:
                 assert paths == [4] * rows, (paths, kw)
     finally:
         hs.close()
@@ -66,7 +57,7 @@ def test_spread_walk_with_penalties_cap_and_mask(oracle, P):
     from geistlib_amd import HipSampler
     n, rows = 70001, 5
     g = np.random.default_rng(7)
-    x = flat_rows(g, rows, n)
+    x = crowded_rows(g, rows, n)
     u = g.random(rows).astype(np.float32)
     hist = g.integers(0, n, (rows, 300)).astype(np.int32)
     hlen = np.array([300, 0, 17, 300, 128], dtype=np.int32)
@@ -99,15 +90,16 @@ def test_spread_walk_with_penalties_cap_and_mask(oracle, P):
 def test_modes_agree_and_the_adaptive_one_follows_the_rows(oracle, P):
     """One workgroup, spread, adaptive: the same ids. In the adaptive mode the first call with
     such rows is served by one workgroup per row (path 3) and says so; the following calls are
-    spread (path 4), until 64 calls in a row have had no such row."""
+    spread (path 4), until 64 calls in a row have had no such row. The other rows are served by the
+    shortcut in a call that spreads, through the mass histogram (path 5) in one that does not."""
     from geistlib_amd import HipSampler
     n, rows = 100000, 8
     g = np.random.default_rng(3)
     kw = dict(temperature=1.0, top_p=0.9, precedence=0)
     hs = HipSampler(max_rows=8, max_vocab=n)
     try:
-        flat = [flat_rows(g, rows, n) for _ in range(3)]
-        peaked = (g.standard_normal((rows, n)) * 6).astype(np.float32)
+        flat = [crowded_rows(g, rows, n) for _ in range(3)]
+        peaked = (g.standard_normal((rows, n)) * 8).astype(np.float32)
         u = g.random(rows).astype(np.float32)
         ids = {}
         for mode in (ONE, SPREAD):
@@ -127,7 +119,7 @@ def test_modes_agree_and_the_adaptive_one_follows_the_rows(oracle, P):
                 k = [i for i, f in enumerate(flat) if f is x][0]
                 assert got == ids[ONE][k]
         # a call counts for the 64 that follow it
-        assert seen == [[1]] * 65 + [[3], [4], [4], [1], [4]] + [[1]] * 65 + [[3], [4]], seen
+        assert seen == [[1]] * 64 + [[5], [3], [4], [4], [1], [4]] + [[1]] * 64 + [[5], [3], [4]], seen
     finally:
         hs.close()
 
@@ -143,7 +135,7 @@ def test_waits_that_run_out(oracle, P):
     hs = HipSampler(max_rows=8, max_vocab=n)
     try:
         hs.set_whole_row_walk(SPREAD)
-        x = flat_rows(g, rows, n)
+        x = crowded_rows(g, rows, n)
         u = g.random(rows).astype(np.float32)
         want, infos = want_of(oracle, x, u, **kw)
         hs.set_wait_limit(0)
@@ -178,7 +170,8 @@ def window_rows(g, rows, n):
 def test_edge_and_draw_found_in_narrow_ranges(oracle, P, rows, n, kw):
     """The token of rows served through the histogram of the masses: every size at which the launch
     changes, draws at both ends, against the oracle's sorted walk. At most one row may lie within the
-    contract's 1e-6 of a slot's edge."""
+    contract's 1e-6 of a slot's edge. The rows without crowds are served there (path 5), or in larger
+    batches by the shortcut or the min-p list in front; never by the whole-row walk."""
     from geistlib_amd import HipSampler
     print(f"window rows={rows} n={n} {kw}", flush=True)
     g = np.random.default_rng(rows * 100003 + n)
@@ -194,5 +187,8 @@ def test_edge_and_draw_found_in_narrow_ranges(oracle, P, rows, n, kw):
             got = run_rows(hs, torch, x, u, P(temperature=1.0, **kw))
             assert compare_ids(got[:6], want[:len(got[:6])], infos[:len(got[:6])], f"{rows}x{n} {kw}") <= 1
             assert all(got[r] == got[r % 6] for r in range(rows))
+            small = rows * -(-n // 2048) <= 1024 and call == 0
+            paths = hs.row_paths(rows).tolist()
+            assert {paths[r] for r in range(rows) if r % 6 not in (1, 2)} <= ({5} if small else {1, 2, 5}), paths
     finally:
         hs.close()
