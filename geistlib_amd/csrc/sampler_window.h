@@ -20,6 +20,8 @@
 #ifndef GEIST_SAMPLER_WINDOW_H
 #define GEIST_SAMPLER_WINDOW_H
 
+#include "sampler_window_range.h"
+
 namespace gs {
 
 /* Where to look in a row: the bins [e0, e1] hold the entry at which the nucleus reaches top_p
@@ -90,7 +92,7 @@ __device__ __forceinline__ void window_sum_hist(const float *__restrict__ hist, 
 }
 
 /* The plan of a row from window_sum_hist's bins; every thread of the workgroup calls and receives
- * the same. */
+ * the same, and so does every other workgroup that reads the same bins. */
 __device__ __forceinline__ WinPlan window_locate(const double (&h)[4], int nb, double sum, float top_p,
                                                  float min_p, float u, WinLocateShared &sh) {
     const int  tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
@@ -113,7 +115,9 @@ __device__ __forceinline__ WinPlan window_locate(const double (&h)[4], int nb, d
         sh.cum[4 * tid + i] = run;
     }
     __syncthreads();
-    /* hit[slot], hit[slot + 1]: the first bins at which the running mass reaches a and b */
+    /* hit[slot], hit[slot + 1]: the first bins at which the running mass reaches a and b. The first: a
+     * thread's masses and its neighbour's are rounded on their own ways, so the running mass can
+     * step back by a last bit between them, and a target within that bit is reached twice. */
     auto find = [&](int slot, double a, double b) {
         double before = tid ? sh.cum[4 * tid - 1] : -1.0; /* (a target of 0 is reached in bin 0) */
         if (tid == 0) {
@@ -123,9 +127,9 @@ __device__ __forceinline__ WinPlan window_locate(const double (&h)[4], int nb, d
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             if (before < a && cum[i] >= a)
-                sh.hit[slot] = 4 * tid + i;
+                atomicMin(&sh.hit[slot], 4 * tid + i);
             if (before < b && cum[i] >= b)
-                sh.hit[slot + 1] = 4 * tid + i;
+                atomicMin(&sh.hit[slot + 1], 4 * tid + i);
             before = cum[i];
         }
     };
@@ -202,31 +206,17 @@ struct alignas(32) WinChunk { /* what a workgroup reports, within a cache line: 
     uint64_t above_e, above_d, above_m; /* mass before the edge's bins, the draw's, of the min-p prefix */
 };
 
-constexpr int WIN_SUB = 512; /* sub-bins of a range's keys: a few entries each */
 struct WinFindShared {
     uint64_t mass[2][WIN_SUB]; /* of the edge's range, of the draw's */
     uint64_t small[TPB];
     uint64_t scan[2][NWAVES];
     uint64_t res_before, out_pack, out_mass;
-    int      res_bin, n_small, found;
+    int      res_bin, n_small, found, stray;
 };
 
 /* a list entry: pack_best(pn, id) with its two leading id bits replaced by the roles */
 constexpr uint64_t WIN_ROLE_E = 0x80000000ull, WIN_ROLE_D = 0x40000000ull;
 __device__ __forceinline__ uint64_t win_pack(uint64_t entry) { return entry | WIN_ROLE_E | WIN_ROLE_D; }
-
-/* The keys klo .. khi of a range of bins, cut into sub-bins from the greatest down. */
-struct WinRange {
-    uint32_t khi;
-    int      shift;
-    __device__ __forceinline__ WinRange(uint32_t klo, uint32_t hi) : khi(hi) {
-        const uint32_t span = hi - klo;
-        const int      bits = span ? 32 - __clz((int) span) : 0;
-        shift               = bits > 9 ? bits - 9 : 0;
-        static_assert(WIN_SUB == 1 << 9, "nine bits of the range");
-    }
-    __device__ __forceinline__ int sub(uint32_t key) const { return (int) ((khi - key) >> shift); }
-};
 
 /* The first entry of the list with role `role` and pack >= lim, in the order of the packs from the
  * greatest down, at which the running mass reaches `target`: sh.out_pack, and sh.out_mass, the
@@ -254,7 +244,7 @@ __device__ __forceinline__ bool window_find(Each each, uint64_t role, uint64_t l
     if (b < 0)
         return false;
     each([&](uint64_t e) {
-        if ((e & role) && range.sub(best_key(e)) == b && win_pack(e) >= lim) {
+        if ((e & role) && win_sub(range, best_key(e)) == b && win_pack(e) >= lim) {
             const int at = atomicAdd(&sh.n_small, 1);
             if (at < TPB)
                 sh.small[at] = win_pack(e);
@@ -499,6 +489,7 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
             sb.find.res_bin = -1;
             sb.find.n_small = 0;
             sb.find.found   = 0;
+            sb.find.stray   = 0;
         }
         if (tid < 3) {
             uint64_t t = 0;
@@ -521,17 +512,19 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
         uint64_t edge_pack = 0ull, mass_keep = 0ull;
         if (ok) {
             /* both ranges' masses by sub-bin (the words were cleared before the last barrier) */
-            const WinRange re(pn_bits(win_key_lo(plan.need_p ? plan.e1 : 0)),
-                              pn_bits(win_key_hi(plan.need_p ? plan.e0 : 0)));
-            const WinRange rd(pn_bits(win_key_lo(plan.d1)), pn_bits(win_key_hi(plan.d0)));
+            const WinRange re = win_range(pn_bits(win_key_lo(plan.need_p ? plan.e1 : 0)),
+                                          pn_bits(win_key_hi(plan.need_p ? plan.e0 : 0)));
+            const WinRange rd = win_range(pn_bits(win_key_lo(plan.d1)), pn_bits(win_key_hi(plan.d0)));
             each([&](uint64_t e) {
                 const uint64_t fx = pn_fx_bits(best_key(e));
-                if (e & WIN_ROLE_E)
-                    atomicAdd((unsigned long long *) &sb.find.mass[0][re.sub(best_key(e))],
-                              (unsigned long long) fx);
-                if (e & WIN_ROLE_D)
-                    atomicAdd((unsigned long long *) &sb.find.mass[1][rd.sub(best_key(e))],
-                              (unsigned long long) fx);
+                const int      be = e & WIN_ROLE_E ? win_sub(re, best_key(e)) : 0;
+                const int      bd = e & WIN_ROLE_D ? win_sub(rd, best_key(e)) : 0;
+                if ((be | bd) < 0) /* (in no list of a workgroup with this plan) */
+                    sb.find.stray = 1;
+                if ((e & WIN_ROLE_E) && be >= 0)
+                    atomicAdd((unsigned long long *) &sb.find.mass[0][be], (unsigned long long) fx);
+                if ((e & WIN_ROLE_D) && bd >= 0)
+                    atomicAdd((unsigned long long *) &sb.find.mass[1][bd], (unsigned long long) fx);
             });
             __syncthreads();
             static_assert(WIN_SUB == 2 * TPB, "two sub-bins to a thread");
@@ -552,7 +545,8 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
                     run[k] += sb.find.scan[k][w];
                 run[k] += k == 0 ? above_e : above_d;
             }
-            if (plan.need_p) {
+            ok = sb.find.stray == 0;
+            if (ok && plan.need_p) {
                 const uint64_t target = (uint64_t) __double2ull_ru((double) top_p * 0x1p62);
                 ok = above_e < target && window_find(each, WIN_ROLE_E, 0ull, re, run[0],
                                                      m[0][0], m[0][1], target, sb.find);
