@@ -14,8 +14,9 @@
  *
  * The histogram decides where to look, never the token: the last workgroup checks that the exact
  * masses put the edge and the draw inside their ranges, and that neither is tied with an entry
- * outside. A row that fails (runs of equal values beyond the list's length, sums that are not
- * finite, prefixes that end below p = 2^-32) takes the whole-row walk.
+ * outside. A row that fails (ranges with more entries than WIN_MANY by their masses or than the list
+ * by their number, sums that are not finite, prefixes that end below p = 2^-32) takes the whole-row
+ * walk. Runs of equal values are cut by their ids (window_long).
  */
 #ifndef GEIST_SAMPLER_WINDOW_H
 #define GEIST_SAMPLER_WINDOW_H
@@ -23,6 +24,10 @@
 #include "sampler_window_range.h"
 
 namespace gs {
+
+constexpr int WIN_STAGE = 2048; /* entries a workgroup stages in LDS */
+constexpr int WIN_MANY  = 8192; /* a crowd of more entries is sooner walked than listed: 24 rows of 50257 in
+                                 * halves 99 us so, 229 with lists of up to 16384 */
 
 /* Where to look in a row: the bins [e0, e1] hold the entry at which the nucleus reaches top_p
  * (need_p), [d0, d1] the entry drawn; `last` is the last bin that can hold a kept entry. thr: every
@@ -180,6 +185,20 @@ __device__ __forceinline__ WinPlan window_locate(const double (&h)[4], int nb, d
     __syncthreads();
     r.d0 = sh.hit[2] < r.last ? sh.hit[2] : r.last;
     r.d1 = sh.hit[3] < r.last ? sh.hit[3] : r.last;
+    /* a range of which the masses alone tell that its entries are too many -- more than the list's (weights
+     * are rounded down, so the number is), or a crowd, far above the ranges beside it --: the row is
+     * walked in full, and its workgroups need not find that out */
+    auto below    = [&](int d) { return d >= 0 ? sh.cum[d < nb ? d : nb - 1] : 0.0; };
+    auto too_many = [&](int a, int b) {
+        const double mass = below(b) - below(a - 1), p = (double) __uint_as_float(win_key_hi(a));
+        if (mass <= (double) WIN_MANY * p)
+            return false;
+        const int    w      = b - a + 1;
+        const double beside = (below(a - 1) - below(a - 1 - w)) + (below(b + w) - below(b));
+        return mass > (double) (WIN_CAP + 1) * p || mass > 2.0 * beside;
+    };
+    if (r.ok && (too_many(r.d0, r.d1) || (r.need_p && too_many(r.e0, r.e1))))
+        r.ok = 0;
     int deep = r.d1;
     if (r.need_p && r.e1 > deep)
         deep = r.e1;
@@ -190,8 +209,6 @@ __device__ __forceinline__ WinPlan window_locate(const double (&h)[4], int nb, d
     __syncthreads(); /* the shared words may be used again */
     return r;
 }
-
-constexpr int WIN_STAGE = 2048; /* entries a workgroup stages in LDS */
 
 /* A row of the pass's workspace; `arrive` and `count` are zero between launches. */
 struct WinRow {
@@ -212,33 +229,58 @@ struct WinFindShared {
     uint64_t scan[2][NWAVES];
     uint64_t res_before, out_pack, out_mass;
     int      res_bin, n_small, found, stray;
+    uint32_t kmin, kmax;
 };
 
 /* a list entry: pack_best(pn, id) with its two leading id bits replaced by the roles */
 constexpr uint64_t WIN_ROLE_E = 0x80000000ull, WIN_ROLE_D = 0x40000000ull;
+__device__ __forceinline__ uint64_t win_entry(uint32_t key, uint32_t id, bool edge, bool draw) {
+    return (pack_best(key, id) & ~(WIN_ROLE_E | WIN_ROLE_D)) | (edge ? WIN_ROLE_E : 0ull) |
+           (draw ? WIN_ROLE_D : 0ull);
+}
 __device__ __forceinline__ uint64_t win_pack(uint64_t entry) { return entry | WIN_ROLE_E | WIN_ROLE_D; }
+
+/* Of the c entries in sh.small, at most one per thread, the one at which the running mass, sh.res_before
+ * before them, reaches `target`. */
+__device__ __forceinline__ void window_pick(int c, uint64_t target, WinFindShared &sh) {
+    const int tid = threadIdx.x;
+    if (tid < c) {
+        /* the running mass up to this entry: no order needed, the entries are few */
+        const uint64_t me = sh.small[tid], fx = pn_fx_bits(best_key(me));
+        uint64_t       r = sh.res_before;
+        for (int j = 0; j < c; ++j) {
+            const uint64_t o = sh.small[j];
+            r += o >= me ? pn_fx_bits(best_key(o)) : 0ull;
+        }
+        if (r >= target && r - fx < target) {
+            sh.out_pack = me;
+            sh.out_mass = r;
+            sh.found    = 1;
+        }
+    }
+}
 
 /* The first entry of the list with role `role` and pack >= lim, in the order of the packs from the
  * greatest down, at which the running mass reaches `target`: sh.out_pack, and sh.out_mass, the
  * mass with it. each(f): f(entry) for every entry of the list, the workgroup's threads sharing them.
  * run: the running mass before this thread's two sub-bins, m0 and m1 their masses. False when it is
- * not reached, or a sub-bin holds too many entries (equal values). Entries below lim leave the
- * sub-bins' masses too great from the sub-bin of lim on, where no target lies beyond lim.
- * sh.res_bin is -1 and sh.n_small, sh.found are 0 on entry (behind a barrier). */
+ * not reached, or a sub-bin holds more entries than the workgroup has threads (window_long's).
+ * Entries below lim leave the sub-bins' masses too great from the sub-bin of lim on, where no target
+ * lies beyond lim. sh.res_bin is -1 and sh.n_small, sh.found are 0 on entry (behind a barrier). */
 template <typename Each>
 __device__ __forceinline__ bool window_find(Each each, uint64_t role, uint64_t lim,
                                             const WinRange &range, uint64_t run, uint64_t m0,
                                             uint64_t m1, uint64_t target, WinFindShared &sh) {
-    const int tid = threadIdx.x;
-    if (m0 && run < target && run + m0 >= target) {
-        sh.res_bin    = 2 * tid;
-        sh.res_before = run;
-    }
-    run += m0;
-    if (m1 && run < target && run + m1 >= target) {
-        sh.res_bin    = 2 * tid + 1;
-        sh.res_before = run;
-    }
+    const int tid  = threadIdx.x;
+    auto      here = [&](int b, uint64_t m) { /* (a mass can tell that the entries are too many) */
+        if (m && run < target && run + m >= target && m <= TPB * pn_fx_bits(range.khi - ((uint32_t) b << range.shift))) {
+            sh.res_bin    = b;
+            sh.res_before = run;
+        }
+        run += m;
+    };
+    here(2 * tid, m0);
+    here(2 * tid + 1, m1);
     __syncthreads();
     const int b = sh.res_bin;
     if (b < 0)
@@ -254,22 +296,213 @@ __device__ __forceinline__ bool window_find(Each each, uint64_t role, uint64_t l
     const int c = sh.n_small;
     if (c > TPB)
         return false;
-    if (tid < c) {
-        /* the running mass up to this entry: no order needed, the entries are few */
-        const uint64_t me = sh.small[tid], fx = pn_fx_bits(best_key(me));
-        uint64_t       r = sh.res_before;
-        for (int j = 0; j < c; ++j) {
-            const uint64_t o = sh.small[j];
-            r += o >= me ? pn_fx_bits(best_key(o)) : 0ull;
-        }
-        if (r >= target && r - fx < target) {
-            sh.out_pack = me;
-            sh.out_mass = r;
-            sh.found    = 1;
-        }
-    }
+    window_pick(c, target, sh);
     __syncthreads();
     return sh.found != 0;
+}
+
+/* The running masses before thread tid's two words 2 tid, 2 tid + 1 of mass[], itself without them;
+ * m0, m1: the two. The words are complete (a barrier behind their additions). */
+__device__ __forceinline__ uint64_t window_scan_subs(const uint64_t *mass, uint64_t *scan, uint64_t &m0,
+                                                     uint64_t &m1) {
+    static_assert(WIN_SUB == 2 * TPB, "two sub-bins to a thread");
+    const int tid = threadIdx.x;
+    m0            = mass[2 * tid];
+    m1            = mass[2 * tid + 1];
+    uint64_t run  = wave_scan_u64(m0 + m1);
+    if ((tid & (WAVE - 1)) == WAVE - 1)
+        scan[tid / WAVE] = run;
+    __syncthreads();
+    run -= m0 + m1;
+    for (int w = 0; w < tid / WAVE; ++w)
+        run += scan[w];
+    return run;
+}
+
+/* An entry's mass to word `at` of mass[], -1: none; every lane of the wavefront calls. The lanes with
+ * the first one's word and key are one addition: a run of equal values would queue up at its word. */
+__device__ __forceinline__ void window_add(uint64_t *mass, int at, uint32_t key) {
+    const uint64_t any = __ballot(at >= 0);
+    if (!any)
+        return;
+    const int      lead = __ffsll((long long) any) - 1;
+    const uint32_t k0   = readlane_u32(key, lead);
+    const int      at0  = (int) readlane_u32((uint32_t) at, lead);
+    const uint64_t same = __ballot(at == at0 && key == k0);
+    const bool     one  = (int) (threadIdx.x & (WAVE - 1)) == lead;
+    const uint64_t fx   = pn_fx_bits(key) * (one ? (uint64_t) __popcll(same) : 1ull);
+    if (one || (at >= 0 && !(at == at0 && key == k0)))
+        atomicAdd((unsigned long long *) &mass[at], (unsigned long long) fx);
+}
+
+/* The same for lists that window_find does not serve, with a crowd in one sub-bin: edge and draw, the checks of k_window included; the token, or -1. A sub-bin with more
+ * entries than threads is cut into sub-bins in turn, from its least key to its greatest, and where
+ * these are one, by the ids (below n_ids), so runs of equal values end as any others do. Called by the
+ * whole workgroup; sh.mass[0] is used again. */
+template <typename Over, typename Under>
+__device__ __forceinline__ int window_long(const uint64_t *list, uint32_t total, const WinPlan &plan,
+                                           const WinRange &re, const WinRange &rd, uint64_t above_e,
+                                           uint64_t above_d, uint64_t above_m, int n_ids, float top_p,
+                                           uint32_t floor_key, float u, Over key_over, Under key_under,
+                                           WinFindShared &sh) {
+    const int     tid = threadIdx.x;
+    constexpr int PER = 8; /* entries of a thread that stay in registers, and loads in flight for the rest */
+    uint64_t      first[PER];
+    auto load = [&](uint32_t i0, uint64_t (&e)[PER]) {
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const uint32_t i = i0 + q * TPB + tid;
+            e[q]             = coop_ld64(list + (i < total ? i : total - 1u));
+            e[q]             = i < total ? e[q] : 0ull;
+        }
+    };
+    load(0, first);
+    auto each = [&](auto &&f) {
+        uint64_t e[PER], next[PER];
+#pragma unroll
+        for (int q = 0; q < PER; ++q)
+            e[q] = first[q];
+#pragma unroll 1
+        for (uint32_t i0 = 0; i0 < total; i0 += PER * TPB) {
+            if (i0 + PER * TPB < total)
+                load(i0 + PER * TPB, next);
+#pragma unroll
+            for (int q = 0; q < PER; ++q)
+                f(e[q]);
+#pragma unroll
+            for (int q = 0; q < PER; ++q)
+                e[q] = next[q];
+        }
+    };
+    uint64_t edge_pack = 0ull, mass_keep = 0ull;
+#pragma unroll 1
+    for (int draw = plan.need_p ? 0 : 1; draw < 2; ++draw) {
+        if (draw && plan.need_m && (!plan.need_p || floor_key > best_key(edge_pack))) {
+            edge_pack = (uint64_t) floor_key << 32;
+            mass_keep = above_m;
+        }
+        const uint64_t target = draw ? (uint64_t) __double2ull_rd((double) u * (double) mass_keep) + 1ull
+                                     : (uint64_t) __double2ull_ru((double) top_p * 0x1p62);
+        const uint64_t role   = draw ? WIN_ROLE_D : WIN_ROLE_E;
+        uint64_t       before = draw ? above_d : above_e;
+        if (before >= target || (draw && target > mass_keep))
+            return -1;
+        WinRange range = draw ? rd : re;
+        uint32_t key   = 0u; /* with by_id: the key whose (complemented) ids the range holds */
+        bool     by_id = false, whole = true;
+        auto     sub   = [&](uint64_t e) {
+            if (!(e & role))
+                return -1;
+            if (!by_id)
+                return win_sub(range, best_key(e));
+            return best_key(e) == key ? win_sub(range, (uint32_t) win_pack(e)) : -1;
+        };
+        int c;
+#pragma unroll 1
+        for (;;) {
+            __syncthreads(); /* the words are read */
+            for (int i = tid; i < WIN_SUB; i += TPB)
+                sh.mass[0][i] = 0ull;
+            if (tid == 0) {
+                sh.res_bin = -1;
+                sh.n_small = 0;
+                sh.found   = 0;
+                sh.kmin    = 0xffffffffu;
+                sh.kmax    = 0u;
+            }
+            __syncthreads();
+            uint32_t kmin = 0xffffffffu, kmax = 0u;
+            auto     span = [&](uint64_t e) {
+                const uint32_t k = best_key(e);
+                kmin             = k < kmin ? k : kmin;
+                kmax             = k > kmax ? k : kmax;
+            };
+            auto spans = [&]() { /* (behind a barrier) */
+                if (kmin <= kmax) {
+                    atomicMin(&sh.kmin, kmin);
+                    atomicMax(&sh.kmax, kmax);
+                }
+            };
+            auto ids_of = [&](uint32_t k) { /* the entries of one key, by their ids */
+                key   = k;
+                by_id = true;
+                range = win_range(0xffffffffu - (uint32_t) (n_ids - 1), 0xffffffffu);
+            };
+            each([&](uint64_t e) {
+                const int at = sub(e);
+                if ((e & role) && at < 0 && whole)
+                    sh.stray = 1; /* (in no list of a workgroup with this plan) */
+                if (at >= 0)
+                    span(e);
+                window_add(sh.mass[0], at, best_key(e));
+            });
+            if (!by_id)
+                spans();
+            __syncthreads();
+            if (!by_id && sh.kmin == sh.kmax && !sh.stray) {
+                whole = false;
+                ids_of(sh.kmax);
+                continue;
+            }
+            uint64_t m0, m1, run = before + window_scan_subs(sh.mass[0], sh.scan[0], m0, m1);
+            if (m0 && run < target && run + m0 >= target) {
+                sh.res_bin    = 2 * tid;
+                sh.res_before = run;
+            }
+            run += m0;
+            if (m1 && run < target && run + m1 >= target) {
+                sh.res_bin    = 2 * tid + 1;
+                sh.res_before = run;
+            }
+            __syncthreads();
+            const int b = sh.res_bin;
+            if (b < 0 || sh.stray)
+                return -1;
+            const uint64_t run_b = sh.res_before;
+            __syncthreads(); /* the words are read */
+            if (tid == 0) {
+                sh.kmin = 0xffffffffu;
+                sh.kmax = 0u;
+            }
+            kmin = 0xffffffffu;
+            kmax = 0u;
+            __syncthreads();
+            each([&](uint64_t e) {
+                if (sub(e) == b && win_pack(e) >= edge_pack) {
+                    span(e);
+                    const int at = atomicAdd(&sh.n_small, 1);
+                    if (at < TPB)
+                        sh.small[at] = win_pack(e);
+                }
+            });
+            spans();
+            __syncthreads();
+            c = sh.n_small;
+            if (c <= TPB)
+                break;
+            before = run_b;
+            whole  = false;
+            if (by_id)
+                range = win_range_of_sub(range, b); /* (2^20 ids: four to a sub-bin at the second turn) */
+            else if (sh.kmin == sh.kmax)
+                ids_of(sh.kmax);
+            else
+                range = win_range(sh.kmin, sh.kmax);
+        }
+        window_pick(c, target, sh);
+        __syncthreads();
+        if (!sh.found)
+            return -1;
+        const uint64_t got = sh.out_pack;
+        if (best_key(got) >= key_over(draw ? plan.d0 : plan.e0) ||
+            best_key(got) <= key_under(draw ? plan.d1 : plan.e1))
+            return -1;
+        if (draw)
+            return (int) best_idx(got);
+        edge_pack = got;
+        mass_keep = sh.out_mass;
+    }
+    return -1;
 }
 
 /* LOCATE: every workgroup finds its row's plan for itself (small batches: one launch less, and no
@@ -397,8 +630,7 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
                             const uint32_t at = __hip_atomic_fetch_add(&s_n, 1u, __ATOMIC_RELAXED,
                                                                        __HIP_MEMORY_SCOPE_WORKGROUP);
                             if (at < (uint32_t) WIN_STAGE)
-                                sa.list[at] = (pack_best(k, (uint32_t) (id + c)) & ~(WIN_ROLE_E | WIN_ROLE_D)) |
-                                              (re ? WIN_ROLE_E : 0ull) | (rd ? WIN_ROLE_D : 0ull);
+                                sa.list[at] = win_entry(k, (uint32_t) (id + c), re, rd);
                         }
                     }
                 }
@@ -421,8 +653,7 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
         __syncthreads();
         const uint32_t n = s_n;
         if (tid == 0 && n)
-            s_base = __hip_atomic_fetch_add(&wr->count, n > (uint32_t) WIN_STAGE ? (uint32_t) WIN_CAP + 1u : n,
-                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            s_base = __hip_atomic_fetch_add(&wr->count, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         WinChunk *slots = static_cast<WinChunk *>(win.chunk) + (long) row * W;
         if (tid < 3) {
             uint64_t t = 0;
@@ -435,8 +666,41 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
         if (n) {
             __syncthreads();
             const uint32_t b = s_base;
-            for (uint32_t i = tid; i < n && i < (uint32_t) WIN_STAGE && b + i < (uint32_t) WIN_CAP; i += TPB)
-                coop_st64(rl + b + i, sa.list[i]);
+            if (n <= (uint32_t) WIN_STAGE) {
+                for (uint32_t i = tid; i < n && b + i < (uint32_t) WIN_CAP; i += TPB)
+                    coop_st64(rl + b + i, sa.list[i]);
+            } else if (b + n <= (uint32_t) WIN_CAP) {
+                /* more entries than the stage holds -- they crowd in one place of the row, or share a
+                 * value -- but counted: a second time over the chunks, 1024 elements at a time, and
+                 * straight to their places in the row's list */
+                if (tid == 0)
+                    s_n = 0;
+                const int from = wg * per_wg * rv.per_chunk;
+                const int to   = last_chunk * rv.per_chunk < rv.n_vocab ? last_chunk * rv.per_chunk : rv.n_vocab;
+#pragma unroll 1
+                for (int b0 = from; b0 < to; b0 += 4 * TPB) {
+                    float4 w[1];
+                    __syncthreads(); /* the history table is rebuilt; s_n */
+                    fetch_chunk<1, PEN>(rv, row, rv.n_rows, b0, b0 + 4 * TPB < to ? b0 + 4 * TPB : to,
+                                        sb.cnt16, w);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        const float arg = softmax_arg(f4_get(w[0], c), mx, g.inv_t);
+                        if (arg > plan.thr) {
+                            const float p  = geist_expf_glibc_le0(arg, s_tab);
+                            const int   d  = win_bin(__float_as_uint(p));
+                            const bool  re = d >= e0 && d <= e1, rd = d >= plan.d0 && d <= plan.d1;
+                            if (re || rd) {
+                                const uint32_t at = __hip_atomic_fetch_add(&s_n, 1u, __ATOMIC_RELAXED,
+                                                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+                                coop_st64(rl + b + at,
+                                          win_entry(__float_as_uint((float) ((double) p / tot)),
+                                                    (uint32_t) (b0 + 4 * tid + c), re, rd));
+                            }
+                        }
+                    }
+                }
+            }
         }
         /* everything reported is performed before the arrival is */
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -471,8 +735,17 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
             for (int q = 0; q < EARLY; ++q)
                 if ((uint32_t) (q * TPB + tid) < total)
                     f(first[q]);
-            for (uint32_t i = EARLY * TPB + tid; i < total; i += TPB)
-                f(coop_ld64(rl + i));
+#pragma unroll 1
+            for (uint32_t i0 = EARLY * TPB + tid; i0 < total; i0 += 8 * TPB) {
+                uint64_t e[8]; /* eight loads in flight */
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+                    e[q] = coop_ld64(rl + (i0 + q * TPB < total ? i0 + q * TPB : total - 1u));
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+                    if (i0 + q * TPB < total)
+                        f(e[q]);
+            }
         };
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
@@ -510,11 +783,11 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
         bool     ok = total <= (uint32_t) WIN_CAP;
         bool     have_p = false;
         uint64_t edge_pack = 0ull, mass_keep = 0ull;
+        const WinRange re = win_range(pn_bits(win_key_lo(plan.need_p ? plan.e1 : 0)),
+                                      pn_bits(win_key_hi(plan.need_p ? plan.e0 : 0)));
+        const WinRange rd = win_range(pn_bits(win_key_lo(plan.d1)), pn_bits(win_key_hi(plan.d0)));
         if (ok) {
             /* both ranges' masses by sub-bin (the words were cleared before the last barrier) */
-            const WinRange re = win_range(pn_bits(win_key_lo(plan.need_p ? plan.e1 : 0)),
-                                          pn_bits(win_key_hi(plan.need_p ? plan.e0 : 0)));
-            const WinRange rd = win_range(pn_bits(win_key_lo(plan.d1)), pn_bits(win_key_hi(plan.d0)));
             each([&](uint64_t e) {
                 const uint64_t fx = pn_fx_bits(best_key(e));
                 const int      be = e & WIN_ROLE_E ? win_sub(re, best_key(e)) : 0;
@@ -590,8 +863,23 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
             }
         }
         served = ok;
-    } else if (wg != 0) {
-        return;
+        if (!ok && total <= (uint32_t) WIN_CAP) {
+            const int tok = window_long(rl, total, plan, re, rd, above_e, above_d, above_m, rv.n_vocab, top_p,
+                                        __float_as_uint(floor_w), u, key_over, key_under, sb.find);
+            served = tok >= 0;
+            if (served && tid == 0) {
+                out[row]      = tok;
+                path[row]     = PATH_WINDOW;
+                row_flag[row] = 0;
+            }
+        }
+    } else {
+        /* a row without a plan, walked by one workgroup: another from row to row. These alone stay, and as
+         * every W-th of an XCD's launch order they would share a quarter of its compute units (64 rows
+         * of 128256 in halves 1487 us with the first of each row, 638 so) */
+        const int r = row >> 3;
+        if (wg != (r + r / W) % W)
+            return;
     }
     if (served)
         return;

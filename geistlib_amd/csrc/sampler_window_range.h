@@ -30,6 +30,13 @@ GEIST_HD int win_sub(const WinRange &r, uint32_t key) {
     const uint32_t at = r.khi - key; /* (wraps beyond span for a key above khi) */
     return at <= r.span ? (int) (at >> r.shift) : -1;
 }
+/* The range of the keys of sub-bin b. */
+GEIST_HD WinRange win_range_of_sub(const WinRange &r, int b) {
+    const uint32_t off  = (uint32_t) b << r.shift; /* of its greatest key */
+    const uint32_t own  = (1u << r.shift) - 1u, left = r.span - off;
+    const uint32_t span = own < left ? own : left;
+    return win_range(r.khi - off - span, r.khi - off);
+}
 
 } // namespace gs
 #endif

@@ -33,7 +33,8 @@ def pack_allowed(allowed):
 def crowded_rows(g, rows, n):
     """Flat rows of which most elements crowd at one place: more of them in a single bin of the mass
     histogram than its lists hold, so that a nucleus that ends there, or a draw that falls there, takes
-    the whole-row walk (n of 20000 and more; top-p 0.5 to 0.95 end there). Row 1 is quantised (index
+    the whole-row walk (n of 50000 and more, also where a bin's end cuts the crowd; top-p 0.5 to
+    0.95 end there). Row 1 is quantised (index
     order among equal probabilities), row 2 has a few tiny probabilities, row 3 is all equal."""
     x = (g.standard_normal((rows, n)) * 0.4).astype(np.float32)
     crowd = g.random((rows, n)) < 0.85

@@ -19,6 +19,12 @@ int main() {
             bad += s < 0 || s >= gs::WIN_SUB;
             if (k > lo) /* the next lower key: the same sub-bin or the next */
                 bad += gs::win_sub(r, k - 1) - s != 0 && gs::win_sub(r, k - 1) - s != 1;
+            /* the sub-bin's own range: this key, and the next ones of the same sub-bin alone */
+            const gs::WinRange in = gs::win_range_of_sub(r, s);
+            bad += gs::win_sub(in, k) < 0;
+            bad += k > lo && (gs::win_sub(in, k - 1) >= 0) != (gs::win_sub(r, k - 1) == s);
+            bad += k < hi && (gs::win_sub(in, k + 1) >= 0) != (gs::win_sub(r, k + 1) == s);
+            bad += in.span >= r.span && r.span != 0;
             ++total;
         };
         auto outside = [&](uint32_t k) {

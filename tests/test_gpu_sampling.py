@@ -320,7 +320,7 @@ def test_whole_row_walk_with_penalties_cap_and_mask(hs, oracle, n, lead, pad):
             infos.append(i)
         near = compare_ids(got, want, infos, f"whole-row walk n={n} {kw}")
         assert near <= 1
-        assert set(paths) <= {3, 4}, paths
+        assert set(paths) <= ({3, 4} if n >= 50000 else {3, 4, 5}), paths   # (a short row's crowd may fit a list)
 
 
 def test_ids_and_draws_in_page_locked_host_memory(hs):

@@ -45,9 +45,10 @@ def test_spread_walk_gives_the_oracles_tokens(oracle, P, n):
             want, infos = want_of(oracle, x, u, **kw)
             near = compare_ids(got, want, infos, f"spread walk n={n} {kw}")
             assert near <= 1
-            # (short rows, and draws beside the crowd without a nucleus, need no such walk)
+            # (short rows, whose crowd fits a list, and draws beside the crowd without a nucleus, need no
+            # such walk)
             assert set(paths) <= {2, 4, 5}, (paths, kw)
-            if n >= 20000 and "top_p" in kw:
+            if n >= 50000 and "top_p" in kw:
                 assert paths == [4] * rows, (paths, kw)
     finally:
         hs.close()
@@ -190,5 +191,44 @@ def test_edge_and_draw_found_in_narrow_ranges(oracle, P, rows, n, kw):
             small = rows * -(-n // 2048) <= 1024 and call == 0
             paths = hs.row_paths(rows).tolist()
             assert {paths[r] for r in range(rows) if r % 6 not in (1, 2)} <= ({5} if small else {1, 2, 5}), paths
+    finally:
+        hs.close()
+
+
+def runs_of_equal_values(g, rows, n):
+    """Rows whose edge or draw falls in a crowd of more entries than a workgroup has threads, all of it
+    within the 16384 places of a row's list."""
+    x = (g.standard_normal((rows, n)) * 2).astype(np.float32)
+    top = x.max()
+    x[0] = np.round(x[0] * 4) / 4                                         # quantised
+    x[1, g.permutation(n)[:1000]] = top + 3                               # one value, all over the row
+    x[2, n // 3 : n // 3 + 5000] = top + 2                                # one value, more than a workgroup's stage
+    x[3] = np.round(x[3] * 8) / 8
+    x[4, g.permutation(n)[:700]] = np.float32(top + 3) + np.float32(2.0 ** -20) * np.arange(700, dtype=np.float32)
+    x[5, g.permutation(n)[:900]] = np.float32(top + 3) + np.float32(2.0 ** -20) * (np.arange(900) % 2).astype(np.float32)
+    return x
+
+
+@pytest.mark.parametrize("rows,n", [(8, 12000), (24, 50257), (96, 33001), (260, 66000)])
+@pytest.mark.parametrize("kw", [dict(top_p=0.9), dict(top_p=0.5, min_p=1e-3), dict(top_p=0.03)])
+def test_runs_of_equal_values_need_no_whole_row_walk(oracle, P, rows, n, kw):
+    """Quantised logits, runs of one value and of neighbouring ones, at every form of the window's
+    launch: the oracle's token, without a walk over the whole row."""
+    from geistlib_amd import HipSampler
+    print(f"equal values rows={rows} n={n} {kw}", flush=True)
+    g = np.random.default_rng(rows + n)
+    base = runs_of_equal_values(g, 6, n)
+    x = np.ascontiguousarray(base[np.arange(rows) % 6])
+    u = g.random(rows).astype(np.float32)
+    u[0:2], u[2:4] = 0.0, np.float32(1.0 - 2.0 ** -24)
+    check = min(rows, 36)
+    want, infos = want_of(oracle, x[:check], u, temperature=1.0, **kw)
+    hs = HipSampler(max_rows=rows, max_vocab=n)
+    try:
+        for _ in range(2):
+            got = run_rows(hs, torch, x, u, P(temperature=1.0, **kw))
+            assert compare_ids(got[:check], want, infos, f"{rows}x{n} {kw}") <= 1
+            paths = hs.row_paths(rows).tolist()
+            assert set(paths) <= ({5} if rows * -(-n // 2048) <= 1024 else {1, 2, 5}), paths
     finally:
         hs.close()
