@@ -93,7 +93,8 @@ struct geist_hip_sampler {
     uint32_t  walk_calls = 0;       /* calls of the top-p / min-p path so far */
     uint32_t  walk_cleared = 0;     /* ... the one before which the workspace was last cleared */
     int       walk_mode  = 0;       /* geist_hip_sampler_set_whole_row_walk */
-    bool      walk_spread = false;  /* the last call of that path sends the spread walk */
+    bool      walk_spread = false;  /* the last call of that path sends the spread walk, */
+    bool      walk_behind = false;  /* ... or a launch for its walked rows, a workgroup each */
     bool      walk_clear = false;   /* clear the workspace before its next use */
     void    *q6k_ws      = nullptr; /* scratch of the Q6_K projection, sized like f64_ws */
     size_t   q6k_in = 0, q6k_out = 0;
@@ -842,6 +843,11 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
     if (L.rv.n_chunks > s->max_chunks)
         return fail(s, GEIST_HIP_E_UNSUPPORTED, "n_vocab %zu needs more than %d chunks",
                     rows->n_vocab, s->max_chunks);
+    /* A min-p of a few percent bounds the kept prefix to a short list on any plausible row, by the
+     * row maximum alone: the exp-sum pass lists the candidates on its way and the list walk
+     * follows it at once. Otherwise the pass leaves histograms of the masses. */
+    const int zb_m = zbin_of_min_p(rs.min_p);
+    f.minp_direct = rs.use_m && zb_m < ZBINS - 1 && rs.min_p >= 0.02f;
     /* Rows that nothing shorter can serve are walked in full: by one workgroup each, or spread over
      * the workgroups of their chunks by a kernel of its own. That kernel is a launch more for every
      * call, so it is sent only while such rows keep turning up: the kernels say so in a page-locked
@@ -864,10 +870,15 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
          * rows' own workgroups, all at once, are the faster way */
         const bool fits = rows->rows * (size_t) L.rv.n_chunks <= 1280;
         if (do_stream)
-            s->walk_spread = s->walk_mode == GEIST_HIP_WHOLE_ROW_WALK_SPREAD ||
-                             (s->walk_mode == GEIST_HIP_WHOLE_ROW_WALK_ADAPTIVE && fits &&
-                              walked != 0u && call - walked <= 64u);
+        {
+            const bool recent = walked != 0u && call - walked <= 64u;
+            s->walk_spread    = s->walk_mode == GEIST_HIP_WHOLE_ROW_WALK_SPREAD ||
+                             (s->walk_mode == GEIST_HIP_WHOLE_ROW_WALK_ADAPTIVE && fits && recent);
+            /* (the min-p lists' kernel keeps such rows to a compute unit each by itself) */
+            s->walk_behind = !fits && !s->walk_spread && recent && !f.minp_direct;
+        }
         wc.spread = s->walk_spread;
+        wc.behind = s->walk_behind;
         if (wc.spread && do_tail) {
             wc.clear = (ranout != 0u && (int32_t) (ranout - s->walk_cleared) >= 0) ||
                        s->walk_clear;
@@ -879,19 +890,16 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
         }
     }
     draws();
-    /* A min-p of a few percent bounds the kept prefix to a short list on any plausible row, by the
-     * row maximum alone: the exp-sum pass lists the candidates on its way and the list walk
-     * follows it at once. Otherwise the pass leaves histograms of the masses. */
-    const int zb_m = zbin_of_min_p(rs.min_p);
-    f.cand         = s->cand;
-    f.minp_direct  = rs.use_m && zb_m < ZBINS - 1 && rs.min_p >= 0.02f;
-    f.win          = s->win;
-    f.win_bins     = win_bins_for(rs.use_p ? rs.top_p : 0.0f, rs.min_p, rows->n_vocab);
+    f.cand     = s->cand;
+    f.win      = s->win;
+    f.win_bins = win_bins_for(rs.use_p ? rs.top_p : 0.0f, rs.min_p, rows->n_vocab);
     /* A small batch is a chain of waits, not of bytes: chunks of 2048 logits put four times the
      * workgroups to work on it, and reading the rows again costs less than the launch of the
-     * row-final kernel that spares most rows the reading. (The spread walk wants chunks of 8192.) */
+     * row-final kernel that spares most rows the reading. A rule on the batch's size alone: the chunks
+     * decide in which order a row's exponentials are added up, and the last bit of that sum must not
+     * hang on the calls before. */
     const size_t small_chunks = (rows->n_vocab + 2047) / 2048;
-    f.win_locate = !f.minp_direct && !wc.spread && small_chunks <= (size_t) s->max_chunks &&
+    f.win_locate = !f.minp_direct && small_chunks <= (size_t) s->max_chunks &&
                    small_chunks <= (size_t) MAX_CHUNKS &&
                    rows->rows * small_chunks <= (size_t) WIN_SMALL &&
                    rows->rows * small_chunks * small_chunks <= (size_t) WIN_SMALL_READS;

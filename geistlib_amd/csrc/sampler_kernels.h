@@ -323,6 +323,7 @@ int configure_device_kernels();
 struct WalkCoop {
     void     *rows;
     bool      spread;
+    bool      behind; /* no spreading, but a launch of its own, one workgroup per row */
     bool      clear;
     uint32_t  step_base;
     uint32_t  wait_limit;

@@ -2255,7 +2255,8 @@ int configure_device_kernels() {
     /* k_sorted_candidates keeps a whole candidate list in LDS: more than the static limit */
     const int   dyn = CAND_CAP * (int) sizeof(uint32_t);
     const void *kernels[] = {(const void *) k_sorted_candidates<8, false>,
-                             (const void *) k_sorted_candidates<8, true>};
+                             (const void *) k_sorted_candidates<8, true>,
+                             (const void *) k_whole_row<8, false>, (const void *) k_whole_row<8, true>};
     for (const void *k : kernels) {
         const hipError_t e =
             hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, dyn);
@@ -2269,16 +2270,16 @@ size_t walk_coop_bytes(size_t rows) { return rows * sizeof(CoopRow); }
 
 void launch_candidates(const Launch &L, const FinalLaunch &f, float *probs, long ld_probs,
                        const WalkCoop &wc) {
-    const dim3 grid(L.rv.n_chunks, L.rows), block(TPB);
+    const dim3 block(TPB);
     const int  dyn = CAND_CAP * (int) sizeof(uint32_t); /* see configure_device_kernels() */
     SortedRowArgs g;
     g.inv_t      = f.inv_t;
+    g.n_sums     = L.rv.n_chunks;
     g.chunk_best = f.chunk_best;
     g.chunk_sum  = f.chunk_sum;
     g.probs      = probs;
     g.ld_probs   = ld_probs;
-    /* the cooperative whole-row walk holds a chunk of 8192 in registers */
-    const int defer = wc.rows != nullptr && wc.spread && L.nv == 8 ? 1 : 0;
+    const int defer = wc.rows != nullptr && (wc.spread || wc.behind) ? 1 : 0;
     if (!f.minp_direct) {
         /* a few rounds of workgroups at most: of a batch whose rows the shortcut has served, one that
          * leaves at once still costs its start (8192 of them 5.7 us, 2048 2.5) */
@@ -2307,24 +2308,30 @@ void launch_candidates(const Launch &L, const FinalLaunch &f, float *probs, long
         L.pen ? go(k_sorted_candidates<8, true>) : go(k_sorted_candidates<8, false>);
     }
     if (defer) {
-        /* the rows flagged 2, a workgroup per chunk */
-        if (wc.clear)
+        /* the rows flagged 2, a workgroup per chunk; the walks' own chunks are of 8192 */
+        RowView rv   = L.rv;
+        rv.per_chunk = 8192;
+        rv.n_chunks  = (rv.n_vocab + 8191) / 8192;
+        const dim3 grid(rv.n_chunks, L.rows);
+        if (wc.spread && wc.clear)
             launch_zero_words(L.stream, static_cast<uint64_t *>(wc.rows),
                               (uint32_t) (walk_coop_bytes((size_t) L.rows) / sizeof(uint64_t)));
         CoopRow *cr = static_cast<CoopRow *>(wc.rows);
-        if (L.pen)
+        if (wc.spread && L.pen)
             k_whole_row_coop<8, true><<<grid, block, 0, L.stream>>>(
-                L.rv, g, f.cand, f.top_p, f.min_p, f.uniforms, f.row_flag, f.out, cr, wc.step_base,
+                rv, g, f.cand, f.top_p, f.min_p, f.uniforms, f.row_flag, f.out, cr, wc.step_base,
                 wc.wait_limit, wc.hint, wc.call);
-        else
+        else if (wc.spread)
             k_whole_row_coop<8, false><<<grid, block, 0, L.stream>>>(
-                L.rv, g, f.cand, f.top_p, f.min_p, f.uniforms, f.row_flag, f.out, cr, wc.step_base,
+                rv, g, f.cand, f.top_p, f.min_p, f.uniforms, f.row_flag, f.out, cr, wc.step_base,
                 wc.wait_limit, wc.hint, wc.call);
-        /* rows that are still flagged 2 (a wait ran out, sums that are not finite): one workgroup
-         * each, as without the spread walk */
+        /* rows that are still flagged 2 (a wait ran out, sums that are not finite; all of them without
+         * the spread walk): one workgroup each. The additions of a walk queue up in LDS, so that two
+         * on a compute unit take twice the time of one: a batch of them asks for more LDS than two
+         * could have (256 rows of 128256 in halves 633 us so, 1634 inside k_window) */
         auto go = [&](auto kernel) {
-            kernel<<<dim3(L.rows), block, 0, L.stream>>>(L.rv, g, f.cand, f.top_p, f.min_p, f.uniforms,
-                                                         f.row_flag, f.out);
+            kernel<<<dim3(L.rows), block, wc.spread ? 0 : dyn, L.stream>>>(
+                rv, g, f.cand, f.top_p, f.min_p, f.uniforms, f.row_flag, f.out);
         };
         L.pen ? go(k_whole_row<8, true>) : go(k_whole_row<8, false>);
     }

@@ -790,6 +790,7 @@ __device__ __forceinline__ int sorted_descend(const float *pn, const uint32_t *i
  * more workgroups. Called by every thread of a 256-thread workgroup. */
 struct SortedRowArgs {
     float           inv_t;
+    int             n_sums; /* chunks of the pass that left the maxima and sums: a walk's may be others */
     const uint64_t *chunk_best;
     const double   *chunk_sum;
     float          *probs;
@@ -807,11 +808,11 @@ __device__ __forceinline__ int sorted_general_row(const RowView &rv, int row, in
         s_tab[tid] = g_expf_tab[tid];
     if (tid == 0) {
         double t = 0.0;
-        for (int c = 0; c < rv.n_chunks; ++c)
-            t += g.chunk_sum[(long) row * rv.n_chunks + c];
+        for (int c = 0; c < g.n_sums; ++c)
+            t += g.chunk_sum[(long) row * g.n_sums + c];
         *s_total = t;
     }
-    const float  mx = key2f(best_key(row_best_from_chunks(g.chunk_best, row, rv.n_chunks, sh.red64)));
+    const float  mx = key2f(best_key(row_best_from_chunks(g.chunk_best, row, g.n_sums, sh.red64)));
     const double tot = *s_total;
     float       *pn  = g.probs + (long) row * g.ld_probs;
     const float *rowp = rv.logits + (long) row * rv.ld;

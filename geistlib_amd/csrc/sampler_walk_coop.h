@@ -444,11 +444,11 @@ __global__ __launch_bounds__(TPB, 2) void k_whole_row_coop(RowView rv, SortedRow
         s_tab[tid] = g_expf_tab[tid];
     if (tid == 0) {
         double t = 0.0;
-        for (int c = 0; c < rv.n_chunks; ++c)
-            t += g.chunk_sum[(long) row * rv.n_chunks + c];
+        for (int c = 0; c < g.n_sums; ++c)
+            t += g.chunk_sum[(long) row * g.n_sums + c];
         s_total = t;
     }
-    const float mx = key2f(best_key(row_best_from_chunks(g.chunk_best, row, rv.n_chunks, sh.red64)));
+    const float mx = key2f(best_key(row_best_from_chunks(g.chunk_best, row, g.n_sums, sh.red64)));
     __syncthreads();
     const double tot = s_total;
     if (!(tot > 0.0 && tot < __builtin_inf() && mx > -__builtin_inff() && mx < __builtin_inff())) {

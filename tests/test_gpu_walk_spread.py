@@ -91,8 +91,8 @@ def test_spread_walk_with_penalties_cap_and_mask(oracle, P):
 def test_modes_agree_and_the_adaptive_one_follows_the_rows(oracle, P):
     """One workgroup, spread, adaptive: the same ids. In the adaptive mode the first call with
     such rows is served by one workgroup per row (path 3) and says so; the following calls are
-    spread (path 4), until 64 calls in a row have had no such row. The other rows are served by the
-    shortcut in a call that spreads, through the mass histogram (path 5) in one that does not."""
+    spread (path 4), until 64 calls in a row have had no such row. The other rows are served
+    through the mass histogram (path 5) in all of them."""
     from geistlib_amd import HipSampler
     n, rows = 100000, 8
     g = np.random.default_rng(3)
@@ -120,7 +120,7 @@ def test_modes_agree_and_the_adaptive_one_follows_the_rows(oracle, P):
                 k = [i for i, f in enumerate(flat) if f is x][0]
                 assert got == ids[ONE][k]
         # a call counts for the 64 that follow it
-        assert seen == [[1]] * 64 + [[5], [3], [4], [4], [1], [4]] + [[1]] * 64 + [[5], [3], [4]], seen
+        assert seen == [[5]] * 65 + [[3], [4], [4], [5], [4]] + [[5]] * 65 + [[3], [4]], seen
     finally:
         hs.close()
 
