@@ -599,6 +599,7 @@ static int reserve_sorted_workspace(geist_hip_sampler *s) {
     const size_t win_chunk = part(wgs * gs::WIN_CHUNK_BYTES);
     const size_t win_hist = part(wgs * gs::WIN_BINS * sizeof(float));
     const size_t lists = part(R * gs::CAND_ROW * sizeof(uint32_t));
+    const size_t win_list = part(R * gs::win_cap_for(s->max_vocab) * sizeof(uint64_t));
     const size_t count = part(R * gs::CAND_COUNT_STRIDE * sizeof(int32_t));
     const size_t path = part(R * sizeof(int32_t)), probs = part(R * s->max_vocab * sizeof(float));
     char        *base = nullptr;
@@ -617,7 +618,8 @@ static int reserve_sorted_workspace(geist_hip_sampler *s) {
     walk_hint[0] = walk_hint[1] = 0u;
     s->sorted_base = base;
     s->win.row     = base + win_row;
-    s->win.list    = reinterpret_cast<uint64_t *>(base + lists);
+    s->win.list    = reinterpret_cast<uint64_t *>(base + win_list);
+    s->win.cap     = gs::win_cap_for(s->max_vocab);
     s->win.chunk   = base + win_chunk;
     s->win.hist    = reinterpret_cast<float *>(base + win_hist);
     s->cand.key    = reinterpret_cast<uint32_t *>(base + lists);

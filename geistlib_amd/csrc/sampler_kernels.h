@@ -112,17 +112,21 @@ struct CandSpace {
  * per row a record and the list of the entries around its nucleus edge and its draw. */
 constexpr int WIN_SHIFT = 19;   /* a bin of the histogram spans 2^19 neighbouring binary32 p: ... */
 constexpr int WIN_BINS  = 512;  /* ... 16 bins to a factor of two, down from 1 to 2^-32 */
-constexpr int WIN_CAP   = 16384; /* list entries per row */
+/* List entries per row, n the sampler's longest vocabulary: an eighth of it, as both ranges may hold a
+ * sixteenth of an octave in the middle of a flat row, 9000 elements each of 262144 at scale 0.5 (256 such
+ * rows, top-p 0.5: with 16384 a fifth of them were walked, 969 us a call; 392 so). */
+constexpr int WIN_CAP_MIN = 16384;
+inline int    win_cap_for(size_t n) { return n / 8 > WIN_CAP_MIN ? (int) ((n / 8 + 255) / 256 * 256) : WIN_CAP_MIN; }
 /* Launches of up to WIN_SMALL chunks of 2048, and of so many chunks' histograms read (every
  * workgroup reads all of its row's), find their plans in k_window. One row of 128256 (63 x 63) 22.5
  * us against 38 by chunks of 8192 with a row-final kernel, one of 262144 26 / 35, 16 x 128256 (16 x
  * 63 x 63 reads) 39.3 / 43.5; 8 x 262144 (8 x 128 x 128) 58 / 54, 48 x 100000 (2352 chunks) 48 / 21. */
 constexpr int WIN_SMALL       = 1024;
 constexpr int WIN_SMALL_READS = 65536;
-static_assert(WIN_CAP * 2 == CAND_ROW, "a row's list takes the place of its min-p list");
 struct WinSpace {
     float    *hist;  /* [rows][chunks][WIN_BINS], by the launch's chunks */
-    uint64_t *list;  /* [rows][WIN_CAP], where a row's min-p list would lie: a row has one or the other */
+    uint64_t *list;  /* [rows][cap] */
+    int       cap;
     void     *chunk; /* [rows][chunks] x WIN_CHUNK_BYTES */
     void     *row;   /* [rows] x WIN_ROW_BYTES, zero before the first use */
 };

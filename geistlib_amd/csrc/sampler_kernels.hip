@@ -1617,7 +1617,7 @@ __global__ __launch_bounds__(TPB) void k_final_sorted(RowView rv, FinalArgs a) {
     const bool    finite = sum > 0.0 && sum < __builtin_inf() && mx > -__builtin_inff() && mx < __builtin_inff();
     double        h[4];
     window_sum_hist(a.win.hist + (long) row * C * WIN_BINS, C, a.win_bins, s_big.loc, h);
-    const WinPlan plan = window_locate(h, a.win_bins, sum, a.top_p, a.min_p, u_row, s_big.loc);
+    const WinPlan plan = window_locate(h, a.win_bins, sum, a.top_p, a.min_p, u_row, a.win.cap, s_big.loc);
     if (tid == 0) {
         WinRow *wr      = static_cast<WinRow *>(a.win.row) + row;
         wr->plan        = plan;

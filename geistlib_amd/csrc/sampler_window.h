@@ -6,8 +6,8 @@
  * The exp-sum pass leaves, per chunk, a histogram of the masses p = expf((l - max) inv_t) over
  * WIN_BINS bins (16 to a factor of two of p, from p = 1 down). From their sum over the row's chunks
  * (window_locate) the bins are known in which the kept prefix ends and in which the draw falls; the
- * histogram's masses are binary32 sums, so each place is a range of bins wide enough for their
- * rounding. One pass over the row then (k_window, a workgroup per chunk or few) adds up the exact masses
+ * histogram's masses are sums of weights cut to 19 bits, so each place is a range of bins wide enough
+ * for what was cut. One pass over the row then (k_window, a workgroup per chunk or few) adds up the exact masses
  * of the normalised probabilities above each range and lists the entries inside them, a few
  * hundred; the workgroup that arrives last orders what little of the list it needs and walks it.
  * Masses are integers (2^-62), so they do not depend on the order of the additions.
@@ -99,7 +99,7 @@ __device__ __forceinline__ void window_sum_hist(const float *__restrict__ hist, 
 /* The plan of a row from window_sum_hist's bins; every thread of the workgroup calls and receives
  * the same, and so does every other workgroup that reads the same bins. */
 __device__ __forceinline__ WinPlan window_locate(const double (&h)[4], int nb, double sum, float top_p,
-                                                 float min_p, float u, WinLocateShared &sh) {
+                                                 float min_p, float u, int cap, WinLocateShared &sh) {
     const int  tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
     const bool use_p = top_p > 0.0f && top_p < 1.0f, use_m = min_p > 0.0f;
     const double own = (h[0] + h[1]) + (h[2] + h[3]);
@@ -138,8 +138,11 @@ __device__ __forceinline__ WinPlan window_locate(const double (&h)[4], int nb, d
             before = cum[i];
         }
     };
-    /* a chunk's bin is a binary32 sum of at most 8192 terms: relative error about 3e-6 at most
-     * in practice, the checks of k_window decide */
+    /* A bin is an integer sum of weights of 19 bits (win_weight), each cut by less than 2^-17 of itself,
+     * scaled with one rounding: too small by at most 7.7e-6 of its mass, never too large by more than
+     * 6e-8. With the roundings of pn and of the tolerance mode's exponentials (some 1e-7) twice
+     * and a half fits the margin. k_window checks where edge and draw lie; which of top-p and min-p
+     * ends the prefix first rests on this bound alone. */
     const double m = 2e-5 * sum, t = (double) top_p * sum;
     if (use_p)
         find(0, t - m, t + m);
@@ -195,7 +198,7 @@ __device__ __forceinline__ WinPlan window_locate(const double (&h)[4], int nb, d
             return false;
         const int    w      = b - a + 1;
         const double beside = (below(a - 1) - below(a - 1 - w)) + (below(b + w) - below(b));
-        return mass > (double) (WIN_CAP + 1) * p || mass > 2.0 * beside;
+        return mass > (double) (cap + 1) * p || mass > 2.0 * beside;
     };
     if (r.ok && (too_many(r.d0, r.d1) || (r.need_p && too_many(r.e0, r.e1))))
         r.ok = 0;
@@ -586,7 +589,7 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
             }
             return;
         }
-        plan = window_locate(h, win_bins, tot, top_p, min_p, u, sa.first.loc);
+        plan = window_locate(h, win_bins, tot, top_p, min_p, u, win.cap, sa.first.loc);
         const bool finite = tot > 0.0 && tot < __builtin_inf() && mx > -__builtin_inff() && mx < __builtin_inff();
         flag = finite && plan.ok ? 1 : 2;
     } else {
@@ -662,14 +665,15 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
                 t += s_part[w][tid];
             coop_st64(&slots[wg].above_e + tid, t);
         }
-        uint64_t *rl = win.list + (long) row * WIN_CAP;
+        uint64_t      *rl  = win.list + (long) row * win.cap;
+        const uint32_t cap = (uint32_t) win.cap;
         if (n) {
             __syncthreads();
             const uint32_t b = s_base;
             if (n <= (uint32_t) WIN_STAGE) {
-                for (uint32_t i = tid; i < n && b + i < (uint32_t) WIN_CAP; i += TPB)
+                for (uint32_t i = tid; i < n && b + i < cap; i += TPB)
                     coop_st64(rl + b + i, sa.list[i]);
-            } else if (b + n <= (uint32_t) WIN_CAP) {
+            } else if (b + n <= cap) {
                 /* more entries than the stage holds -- they crowd in one place of the row, or share a
                  * value -- but counted: a second time over the chunks, 1024 elements at a time, and
                  * straight to their places in the row's list */
@@ -718,7 +722,7 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
         /* (a thread per workgroup; the list's first entries are asked for before its length is known) */
         const uint32_t total = coop_ld32(&wr->count);
         uint64_t       part[3], first[EARLY];
-        static_assert(WIN_CAP >= EARLY * TPB, "the list has places for the early loads");
+        static_assert(WIN_CAP_MIN >= EARLY * TPB, "the list has places for the early loads");
         const int slot = tid < W ? tid : W - 1;
 #pragma unroll
         for (int q = 0; q < 3; ++q)
@@ -780,7 +784,7 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
          * first or of at most the second */
         auto key_over  = [&](int d) { return d > 0 ? pn_bits(win_key_hi(d) + 1u) : 0xffffffffu; };
         auto key_under = [&](int d) { return pn_bits(win_key_lo(d) - 1u); };
-        bool     ok = total <= (uint32_t) WIN_CAP;
+        bool     ok = total <= cap;
         bool     have_p = false;
         uint64_t edge_pack = 0ull, mass_keep = 0ull;
         const WinRange re = win_range(pn_bits(win_key_lo(plan.need_p ? plan.e1 : 0)),
@@ -863,7 +867,7 @@ __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, 
             }
         }
         served = ok;
-        if (!ok && total <= (uint32_t) WIN_CAP) {
+        if (!ok && total <= cap) {
             const int tok = window_long(rl, total, plan, re, rd, above_e, above_d, above_m, rv.n_vocab, top_p,
                                         __float_as_uint(floor_w), u, key_over, key_under, sb.find);
             served = tok >= 0;

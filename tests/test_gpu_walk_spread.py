@@ -232,3 +232,64 @@ def test_runs_of_equal_values_need_no_whole_row_walk(oracle, P, rows, n, kw):
             assert set(paths) <= ({5} if rows * -(-n // 2048) <= 1024 else {1, 2, 5}), paths
     finally:
         hs.close()
+
+
+@pytest.mark.parametrize("rows,n", [(24, 50257), (260, 66001)])
+def test_narrow_ranges_with_penalties_cap_and_mask(oracle, P, rows, n):
+    """The window pass with everything it has to apply to the logits once more, in its small-batch form and
+    with several chunks to a workgroup, whose history table is rebuilt from chunk to chunk; rows off a
+    16-byte boundary, draws of their own for every row. Wide nuclei, so none is left to the shortcut."""
+    from geistlib_amd import HipSampler
+    print(f"window, transforms, rows={rows} n={n}", flush=True)
+    g = np.random.default_rng(n)
+    base = (g.standard_normal((5, n)) * 1.5).astype(np.float32)
+    base[4] = np.round(base[4] * 4) / 4
+    hist = g.integers(0, n, (rows, 400)).astype(np.int32)
+    hist[:, 100:200] = base[np.arange(rows) % 5].argsort(axis=1)[:, -100:]   # the likeliest tokens among them
+    hlen = g.integers(0, 401, rows).astype(np.int32)
+    hlen[0], hlen[1] = 0, 400
+    allowed = g.random((rows, n)) < 0.8
+    allowed[3] = True
+    x = np.ascontiguousarray(base[np.arange(rows) % 5])
+    u = g.random(rows).astype(np.float32)
+    rep, freq, pres, cap = 1.3, 0.05, 0.1, 6.0
+    check = list(range(15)) + list(range(rows - 5, rows))
+    hs = HipSampler(max_rows=rows, max_vocab=n)
+    try:
+        for lead, pad in ((0, 0), (1, 2)):
+            for kw in (dict(temperature=1.0, top_p=0.9), dict(temperature=0.8, top_p=0.95, min_p=1e-4)):
+                got = run_rows(hs, torch, x, u, P(rep=rep, freq=freq, pres=pres, softcap=cap, **kw),
+                               history=hist, history_len=hlen, lead=lead, pad=pad, allowed=allowed)
+                paths = hs.row_paths(rows).tolist()
+                want, infos = [], []
+                for r in check:
+                    row = oracle.softcap(oracle.penalties(x[r], hist[r, :hlen[r]], rep, freq, pres), cap)
+                    row[~allowed[r]] = -np.inf
+                    t, i = oracle.chain_u(row, float(u[r]), **kw)
+                    want.append(t)
+                    infos.append(i)
+                near = compare_ids(got[check], want, infos, f"window, transforms, {kw} lead {lead}")
+                assert near <= 1
+                assert set(paths) <= ({5} if rows < 100 or "min_p" not in kw else {2, 5}), paths
+    finally:
+        hs.close()
+
+
+def test_flat_rows_of_a_large_vocabulary_need_no_whole_row_walk(oracle, P):
+    """Ranges of some 9000 entries each around the middle of a flat row, with and without overlap."""
+    from geistlib_amd import HipSampler
+    rows, n = 6, 262144
+    g = np.random.default_rng(5)
+    x = (g.standard_normal((rows, n)) * 0.5).astype(np.float32)
+    u = np.linspace(0.05, 0.95, rows).astype(np.float32)
+    kw = dict(temperature=1.0, top_p=0.5)
+    want, infos = want_of(oracle, x, u, **kw)
+    for max_rows in (rows, 64):
+        hs = HipSampler(max_rows=max_rows, max_vocab=n)
+        try:
+            got = run_rows(hs, torch, np.ascontiguousarray(x[np.arange(max_rows) % rows]),
+                           u[np.arange(max_rows) % rows], P(**kw))
+            assert compare_ids(got[:rows], want, infos, f"flat rows, {max_rows}") <= 1
+            assert hs.row_paths(max_rows).tolist() == [5] * max_rows
+        finally:
+            hs.close()
