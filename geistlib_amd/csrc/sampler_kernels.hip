@@ -1540,8 +1540,8 @@ __global__ __launch_bounds__(TPB) void k_final_temperature(RowView rv, FinalArgs
         a.out[row] = tok;
 }
 
-/* top-p / min-p over the whole vocabulary (sampler.c:232-305): the thread-maxima shortcut; a
- * row it cannot serve raises its flag for the whole-row walk. */
+/* top-p / min-p over the whole vocabulary (sampler.c:232-305): the thread-maxima shortcut; a row it
+ * cannot serve is given a plan and flagged for k_window, or, without a plan, for the whole-row walk. */
 template <int NV, bool PEN>
 __global__ __launch_bounds__(TPB) void k_final_sorted(RowView rv, FinalArgs a) {
     __shared__ uint64_t s_red[NWAVES];

@@ -14,9 +14,8 @@
  *
  * The histogram decides where to look, never the token: the last workgroup checks that the exact
  * masses put the edge and the draw inside their ranges, and that neither is tied with an entry
- * outside. A row that fails (ranges with more entries than WIN_MANY by their masses or than the list
- * by their number, sums that are not finite, prefixes that end below p = 2^-32) takes the whole-row
- * walk. Runs of equal values are cut by their ids (window_long).
+ * outside. A row that fails (a range with more entries than the list, a crowd of more than WIN_MANY,
+ * sums that are not finite, prefixes that end below p = 2^-32) takes the whole-row walk. Runs of equal values are cut by their ids (window_long).
  */
 #ifndef GEIST_SAMPLER_WINDOW_H
 #define GEIST_SAMPLER_WINDOW_H
@@ -516,9 +515,13 @@ __device__ __forceinline__ int window_long(const uint64_t *list, uint32_t total,
  * 1.0 to read the reports, 3.0 to find edge and draw --, in a large one the exponentials and exact
  * divisions of the kept elements (256 rows of 262144 with half of each kept: 200 us). The exp-sum pass pays
  * for the histogram with 32-bit integer additions in LDS, 8.2 -> 10.4 us for those 24 rows in chunks
- * of 8192; binary32 additions took it to 17.0. 24 rows of 50257, top-p 0.95, nuclei from ten entries
+ * of 8192; binary32 additions took it to 17.0. A large batch whose rows keep some hundreds pays more than
+ * the list of the kept entries took that this replaces (256 rows of 100000, scale 3, T 0.8, top-p 0.9: the
+ * pass 34 -> 40 us, list and list walk 41 -> k_window 52, the call 88 -> 99). 24 rows of 50257, top-p 0.95, nuclei from ten entries
  * to ten thousand: 152 -> 26 us a call (four to six launches before, half of the rows walked in
- * full); 64 rows of 128256 normal logits 163 -> 63, one 80 -> 23. */
+ * full); 64 rows of 128256 normal logits 163 -> 63, one 80 -> 23.
+ * The whole-row walk is in the small form and for the first calls with such rows in a large one; that and
+ * penalties cost the large form 64 bytes of scratch. */
 template <bool PEN, bool LOCATE>
 __global__ __launch_bounds__(TPB, 3) void k_window(RowView rv, SortedRowArgs g, WinSpace win, int win_bins, int per_wg,
                                                 float top_p, float min_p,

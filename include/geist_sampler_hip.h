@@ -178,9 +178,9 @@ int geist_hip_sampler_set_wait_limit(geist_hip_sampler *s, uint32_t polls);
 int geist_hip_sampler_one_launch_topk(geist_hip_sampler *s, int enable);
 
 /* No counterpart in the reference. A top-p / min-p row whose token neither a list nor the narrow
- * ranges of its mass histogram can certify (long runs of equal values, a min-p list that overflows) is
- * walked in full, as sampler.c:246-304 sorts and walks it. One workgroup takes 275 to 300 us for a row of
- * 128 k logits; spread over the workgroups of the row's chunks, which keep their part of the row
+ * ranges of its mass histogram can certify (a crowd of many thousands of entries within a sixteenth of
+ * an octave, a min-p list that overflows) is walked in full, as sampler.c:246-304 sorts and walks it. One
+ * workgroup takes 275 to 300 us for a row of 128 k logits, 530 to 820 where they are of few values; spread over the workgroups of the row's chunks, which keep their part of the row
  * in registers and meet after every pass, the walk takes a fifth of that -- at the price of one
  * more launch per call.
  *   GEIST_HIP_WHOLE_ROW_WALK_ADAPTIVE       (default) the extra launch is sent while such rows
@@ -188,7 +188,9 @@ int geist_hip_sampler_one_launch_topk(geist_hip_sampler *s, int enable);
  *                                           page-locked word that the next call looks at
  *   GEIST_HIP_WHOLE_ROW_WALK_SPREAD         always send it
  *   GEIST_HIP_WHOLE_ROW_WALK_ONE_WORKGROUP  never
- * Tokens are the same in every mode. geist_hip_sampler_row_paths reports 3 for a row walked by
+ * (Batches of more than 1280 chunks of 8192 have one workgroup to a row unless it is fixed, in a
+ * launch of their own while such rows keep turning up.) Tokens are the same in every mode, and after
+ * any calls: how a row's exponentials are added up follows from the batch's sizes and options. geist_hip_sampler_row_paths reports 3 for a row walked by
  * one workgroup, 4 for a row walked by its chunks' workgroups. The waits of the spread form are
  * bounded by geist_hip_sampler_set_wait_limit like those of the one-pass kernels: a row whose
  * workgroups do not all turn up in time is walked by its first workgroup alone. */
