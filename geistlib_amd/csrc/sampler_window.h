@@ -275,7 +275,8 @@ __device__ __forceinline__ bool window_find(Each each, uint64_t role, uint64_t l
                                             uint64_t m1, uint64_t target, WinFindShared &sh) {
     const int tid  = threadIdx.x;
     auto      here = [&](int b, uint64_t m) { /* (a mass can tell that the entries are too many) */
-        if (m && run < target && run + m >= target && m <= TPB * pn_fx_bits(range.khi - ((uint32_t) b << range.shift))) {
+        if (m && run < target && run + m >= target &&
+            m / TPB <= pn_fx_bits(range.khi - ((uint32_t) b << range.shift))) {
             sh.res_bin    = b;
             sh.res_before = run;
         }
