@@ -1542,8 +1542,9 @@ __global__ __launch_bounds__(TPB) void k_final_temperature(RowView rv, FinalArgs
 
 /* top-p / min-p over the whole vocabulary (sampler.c:232-305): the thread-maxima shortcut; a row it
  * cannot serve is given a plan and flagged for k_window, or, without a plan, for the whole-row walk. */
-template <int NV, bool PEN>
+template <bool PEN>
 __global__ __launch_bounds__(TPB) void k_final_sorted(RowView rv, FinalArgs a) {
+    constexpr int NV = 8; /* rows in chunks of 8192 */
     __shared__ uint64_t s_red[NWAVES];
     __shared__ uint64_t s_tab[32];
     __shared__ union {
@@ -2197,9 +2198,9 @@ void launch_row_final(const Launch &L, const FinalLaunch &f) {
     }
     if (f.mode == FINAL_SORTED) { /* (rows in chunks of 8192: smaller batches have no such launch) */
         if (L.pen)
-            k_final_sorted<8, true><<<grid, block, 0, L.stream>>>(L.rv, a);
+            k_final_sorted<true><<<grid, block, 0, L.stream>>>(L.rv, a);
         else
-            k_final_sorted<8, false><<<grid, block, 0, L.stream>>>(L.rv, a);
+            k_final_sorted<false><<<grid, block, 0, L.stream>>>(L.rv, a);
         return;
     }
     dispatch(L.nv, L.pen, [&](auto nv, auto pen) {
@@ -2254,9 +2255,9 @@ void launch_write_probs(const Launch &L, float inv_t, const uint64_t *chunk_best
 int configure_device_kernels() {
     /* k_sorted_candidates keeps a whole candidate list in LDS: more than the static limit */
     const int   dyn = CAND_CAP * (int) sizeof(uint32_t);
-    const void *kernels[] = {(const void *) k_sorted_candidates<8, false>,
-                             (const void *) k_sorted_candidates<8, true>,
-                             (const void *) k_whole_row<8, false>, (const void *) k_whole_row<8, true>};
+    const void *kernels[] = {(const void *) k_sorted_candidates<false>,
+                             (const void *) k_sorted_candidates<true>,
+                             (const void *) k_whole_row<false>, (const void *) k_whole_row<true>};
     for (const void *k : kernels) {
         const hipError_t e =
             hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, dyn);
@@ -2305,7 +2306,7 @@ void launch_candidates(const Launch &L, const FinalLaunch &f, float *probs, long
                 L.rv, g, f.cand, f.top_p, f.min_p, f.uniforms, f.row_flag, f.out, f.chunk_sum,
                 L.rv.n_chunks, p_out, f.minp_direct ? 0 : 1, defer, wc.hint, wc.call);
         };
-        L.pen ? go(k_sorted_candidates<8, true>) : go(k_sorted_candidates<8, false>);
+        L.pen ? go(k_sorted_candidates<true>) : go(k_sorted_candidates<false>);
     }
     if (defer) {
         /* the rows flagged 2, a workgroup per chunk; the walks' own chunks are of 8192 */
@@ -2333,7 +2334,7 @@ void launch_candidates(const Launch &L, const FinalLaunch &f, float *probs, long
             kernel<<<dim3(L.rows), block, wc.spread ? 0 : dyn, L.stream>>>(
                 rv, g, f.cand, f.top_p, f.min_p, f.uniforms, f.row_flag, f.out);
         };
-        L.pen ? go(k_whole_row<8, true>) : go(k_whole_row<8, false>);
+        L.pen ? go(k_whole_row<true>) : go(k_whole_row<false>);
     }
 }
 

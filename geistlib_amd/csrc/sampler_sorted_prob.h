@@ -1073,12 +1073,13 @@ __device__ __forceinline__ int list_walk_fast(const float *pn, const uint32_t *i
 }
 
 /* The rows flagged 2, a workgroup each: the whole-row walk. */
-template <int NV, bool PEN>
+template <bool PEN>
 __global__ __launch_bounds__(TPB) void k_whole_row(RowView rv, SortedRowArgs g, CandSpace cand,
                                                    float top_p, float min_p,
                                                    const float *__restrict__ uniforms,
                                                    const int32_t *__restrict__ row_flag,
                                                    int32_t *__restrict__ out) {
+    constexpr int NV = 8; /* rows in chunks of 8192 */
     __shared__ SortedGenShared sh;
     __shared__ __align__(16) uint32_t s_cnt16[PEN ? NV * TPB * 2 : 1];
     __shared__ uint64_t s_tab[32];
@@ -1106,7 +1107,7 @@ __global__ __launch_bounds__(TPB) void k_whole_row(RowView rv, SortedRowArgs g, 
  * of the launch needs the whole-row walk -- the host then sends the next calls' such rows to
  * k_whole_row_coop, which spreads the walk over the row's chunks: this launch is told so by
  * defer_walk and only flags them 2. */
-template <int NV, bool PEN>
+template <bool PEN>
 __global__ __launch_bounds__(TPB) void k_sorted_candidates(RowView rv, SortedRowArgs g,
                                                            CandSpace cand, float top_p, float min_p,
                                                            const float *__restrict__ uniforms,
@@ -1117,6 +1118,7 @@ __global__ __launch_bounds__(TPB) void k_sorted_candidates(RowView rv, SortedRow
                                                            int only_flagged, int defer_walk,
                                                            uint32_t *__restrict__ walk_hint,
                                                            uint32_t walk_call) {
+    constexpr int NV = 8; /* rows in chunks of 8192 */
     extern __shared__ uint32_t s_key[]; /* CAND_CAP keys: every list is walked from LDS */
     __shared__ union {
         SortedGenShared gen;
