@@ -518,7 +518,7 @@ __device__ __forceinline__ int window_long(const uint64_t *list, uint32_t total,
  * for the histogram with 32-bit integer additions in LDS, 8.2 -> 10.4 us for those 24 rows in chunks
  * of 8192; binary32 additions took it to 17.0. A large batch whose rows keep some hundreds pays more than
  * the list of the kept entries took that this replaces (256 rows of 100000, scale 3, T 0.8, top-p 0.9: the
- * pass 34 -> 40 us, list and list walk 41 -> k_window 52, the call 88 -> 99). 24 rows of 50257, top-p 0.95, nuclei from ten entries
+ * pass 34 -> 40 us, list and list walk 41 -> k_window 48, the call 88 -> 99). 24 rows of 50257, top-p 0.95, nuclei from ten entries
  * to ten thousand: 152 -> 26 us a call (four to six launches before, half of the rows walked in
  * full); 64 rows of 128256 normal logits 163 -> 63, one 80 -> 23.
  * The whole-row walk is in the small form and for the first calls with such rows in a large one; that and
