@@ -692,19 +692,9 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
         return after_launch(s, "argmax");
     }
     if (rs.use_k) {
-        if (rs.k > TOPK_FAST_MAX) {
-            draws();
-            f.mode         = FINAL_TOPK;
-            f.k            = rs.k;
-            *stream_kernel = "k_topk_general";
-            const int e    = do_stream ? launch_topk_general(L, f) : 0;
-            if (e != 0)
-                return fail(s, GEIST_HIP_E_BACKEND, "top-k (general) launch: %s",
-                            hipGetErrorString((hipError_t) e));
-            return after_launch(s, "top-k (general)");
-        }
-        /* the thread-maxima path wants the large chunks whatever the batch size: the final
-         * kernel holds one key per scanning thread in LDS */
+        Launch       large = L; /* the geometry of the selection over whole rows */
+        /* the thread-maxima paths want the large chunks whatever the batch size: the final
+         * kernel holds one key per scanning thread */
         L.nv           = 8;
         L.rv.per_chunk = 8192;
         L.rv.n_chunks  = (int) ((rows->n_vocab + 8191) / 8192);
@@ -715,15 +705,37 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
          * belong to the top k. A margin on the rank of the bound keeps that check from failing
          * when several leading logits are penalised away; a row that still fails takes the
          * general path. */
-        Launch scan = L;
-        f.k_sel     = rs.k;
-        if (L.pen && L.rv.rep >= 1.0f && L.rv.freq >= 0.0f && L.rv.pres >= 0.0f) {
+        Launch     scan   = L;
+        int        margin = 0;
+        const bool lazy   = L.pen && L.rv.rep >= 1.0f && L.rv.freq >= 0.0f && L.rv.pres >= 0.0f;
+        if (lazy) {
             scan.pen         = false;
             scan.rv.hist     = nullptr;
             scan.rv.hist_len = nullptr;
-            const int margin = rs.k / 2 > 8 ? rs.k / 2 : 8;
-            f.k_sel          = rs.k + margin < TOPK_FAST_MAX ? rs.k + margin : TOPK_FAST_MAX;
+            margin           = rs.k / 2 > 8 ? rs.k / 2 : 8;
         }
+        /* k_topk_wide's path (WIDE_RANK_MIN says for which ranks). The soft-cap makes neighbouring
+         * logits equal and only what lies strictly above the capped bound counts: a few ranks more.
+         * Where a row has fewer than twice as many maxima of 32 as the bound's rank, the bound
+         * would let too many elements pass. */
+        const int  rank   = rs.k + margin, cap_margin = L.rv.softcap > 0.0f ? 8 : 0;
+        const int  k_wide = rank + cap_margin < WIDE_K_SEL_MAX ? rank + cap_margin : WIDE_K_SEL_MAX;
+        const bool wide   = (lazy || !L.pen) && rs.k <= WIDE_K_SEL_MAX &&
+                          (rank > WIDE_RANK_MIN ||
+                           (cap_margin && (rank > WIDE_RANK_MIN_CAPPED || L.rv.n_chunks <= 16))) &&
+                          L.rv.n_chunks <= WIDE_CHUNKS_MAX && rows->n_vocab / 32 >= 2 * (size_t) k_wide;
+        f.mode = FINAL_TOPK;
+        f.k    = rs.k;
+        if (rs.k > TOPK_FAST_MAX && !wide) {
+            draws();
+            *stream_kernel = "k_topk_general";
+            const int e    = do_stream ? launch_topk_general(large, f) : 0;
+            if (e != 0)
+                return fail(s, GEIST_HIP_E_BACKEND, "top-k (general) launch: %s",
+                            hipGetErrorString((hipError_t) e));
+            return after_launch(s, "top-k (general)");
+        }
+        f.k_sel = rank < TOPK_FAST_MAX ? rank : TOPK_FAST_MAX;
         scan.rv.stream_loads = s->logits_streamed; /* the one pass over the rows */
         /* The soft-cap keeps the order of the logits, so the scan runs on the logits as they are
          * and the row-final kernel caps what it keeps (with the thread maxima already there from
@@ -731,8 +743,6 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
         f.cap_after = L.rv.softcap > 0.0f;
         if (f.cap_after)
             scan.rv.softcap = 0.0f;
-        f.mode = FINAL_TOPK;
-        f.k    = rs.k;
         /* Plain rows (aligned, no mask, penalties absent or left to the final kernel)
          * take the candidate path: the scan's wavefronts hand their leading groups on and the
          * row-final kernel gathers nothing. */
@@ -798,8 +808,9 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
         *stream_kernel     = "k_tmax_scan";
         if (!s->tmax_ready && do_stream)
             launch_tmax_scan(scan, s->tmax, nullptr);
+        f.k_sel = wide ? k_wide : rank + cap_margin / 4 < TOPK_FAST_MAX ? rank + cap_margin / 4 : TOPK_FAST_MAX;
         if (do_tail)
-            launch_row_final(L, f);
+            wide ? launch_topk_wide(L, f) : launch_row_final(L, f);
         return after_launch(s, "top-k");
     }
     if (!rs.use_p && !rs.use_m) {

@@ -13,6 +13,18 @@ constexpr int MAX_CHUNKS     = 128;  /* chunks per row */
 constexpr int TMAX_LDS       = 8192; /* thread maxima of one row the final kernel holds in LDS */
 constexpr int SEL_MAX        = 192;  /* threads whose elements the final kernel re-reads */
 constexpr int TOPK_FAST_MAX  = 128;  /* largest k served by the candidate path */
+constexpr int WIDE_K_SEL_MAX = 1024; /* largest rank of the bound of k_topk_wide's path ... */
+constexpr int WIDE_CHUNKS_MAX = 32;  /* ... whose rows have at most so many chunks of 8192 logits */
+/* Above this rank (k, and half of it again with penalties) rows that no scan hands candidates on for
+ * take k_topk_wide, below it k_final_topk, whose 256 threads have the shorter chain while few elements
+ * are read again: rank 40 2 x 50001 11.9 against 10.9 us, 200 x 60001 23.9 / 23.1; rank 48 11.2 / 11.3
+ * and 23.5 / 24.2; 56 11.1 / 12.1 and 23.6 / 24.8; 72 12.5 / 14.7 and 25.3 / 26.8. From rank 90 on
+ * k_final_topk's list of 192 threads starts to overflow: 16 x 128255, k = 128, 14.0 / 163. With a
+ * soft-cap, which that kernel applies to every element it reads again, from rank 17 on (rank 20 12.0 /
+ * 12.9, rank 40 12.4 / 16.6), in rows of up to 16 chunks from the first (rank 5 2 x 50001 11.7 / 12.4, 51 x
+ * 223709 23.3 / 22.3). */
+constexpr int WIDE_RANK_MIN        = 48;
+constexpr int WIDE_RANK_MIN_CAPPED = 16;
 constexpr int TOPK_MAX       = 8192; /* the reference caps top_k here (sampler.c:213-215) */
 constexpr int HISTORY_MAX    = 65535;
 
@@ -310,6 +322,9 @@ int probe_workgroup_placement(hipStream_t stream, bool *same_xcd);
 void launch_cand_scan_final(const Launch &scan, const Launch &L, const FinalLaunch &f, float *tmax,
                             const WgCands &wc, int r_w, int r_last, uint32_t *arrive,
                             bool far_always, const Notify &nt, int wgs_per_row, int groups);
+/* k_topk_wide behind launch_tmax_scan(chunks of 8192, raw where the penalties can only lower a
+ * logit and before the soft-cap): k and k_sel up to WIDE_K_SEL_MAX */
+void launch_topk_wide(const Launch &L, const FinalLaunch &f);
 /* returns a hipError_t value */
 int  launch_topk_general(const Launch &L, const FinalLaunch &f);
 /* Per-device kernel attributes; call once with the device current. Returns a hipError_t value. */

@@ -1496,6 +1496,7 @@ __device__ __forceinline__ bool topk_from_tmax(const RowView &rv, const FinalArg
 #include "sampler_draft.h"
 #include "sampler_cands.h"
 #include "sampler_cands_one_launch.h"
+#include "sampler_topk_wide.h"
 namespace gs {
 
 /* ============================================================================================
@@ -2211,6 +2212,22 @@ void launch_row_final(const Launch &L, const FinalLaunch &f) {
         else
             k_final_topk<GS_NV, GS_PEN, false><<<grid, block, 0, L.stream>>>(L.rv, a);
     });
+}
+
+void launch_topk_wide(const Launch &L, const FinalLaunch &f) {
+    const FinalArgs a = final_args(f);
+    auto go = [&](auto kernel) { kernel<<<dim3(L.rows), dim3(WK_THREADS), 0, L.stream>>>(L.rv, a); };
+    auto pick = [&](auto kpt) {
+        constexpr int K = decltype(kpt)::value;
+        if (L.pen)
+            L.rv.allowed ? go(k_topk_wide<true, true, K>) : go(k_topk_wide<true, false, K>);
+        else
+            L.rv.allowed ? go(k_topk_wide<false, true, K>) : go(k_topk_wide<false, false, K>);
+    };
+    if (L.rv.n_chunks <= 16)
+        pick(std::integral_constant<int, 4>{});
+    else
+        pick(std::integral_constant<int, WIDE_CHUNKS_MAX * TPB / WK_THREADS>{});
 }
 
 int launch_topk_general(const Launch &L, const FinalLaunch &f) {
