@@ -663,11 +663,19 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
     HIPCHK(s, hipSetDevice(s->device));
 
     /* a generator per row: the one-launch kernels take the draw themselves (a launch of its own is
-     * 4.7 us of a step of 13 to 19); every other path has the draws written in front of it */
-    const bool own_rng = rng.states && s->row_arrive && (!rng.shared || rows->rows == 1);
+     * 4.7 us of a step of 13 to 19); the scans of the other paths write the draws for the launches
+     * behind them. Where there is no such scan, or one generator for all rows, they are written in
+     * front. */
+    const bool per_row = rng.states && (!rng.shared || rows->rows == 1), own_rng = per_row && s->row_arrive;
     auto       draws   = [&] {
         if (rng.states)
             launch_rng_units(s->stream, rng.states, rng.shared, (int) rows->rows, s->uniforms);
+    };
+    auto draws_by = [&](Launch &scan) {
+        if (!per_row)
+            return draws();
+        scan.rv.draw_states = rng.states;
+        scan.rv.draws       = s->uniforms;
     };
     FinalLaunch f{};
     f.inv_t      = rs.inv_t;
@@ -792,7 +800,10 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
                                        s->handoff_far, nt, (int) wgs_row, halves ? 4 : 8);
             return after_launch(s, "top-k");
         }
-        draws();
+        if (s->tmax_ready)
+            draws();
+        else
+            draws_by(scan);
         if (m) {
             const WaveCands wc = wave_cands_at(s->wcands, row_waves);
             f.row_flag         = s->row_flag;
@@ -833,7 +844,7 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
                                         meet_space(s, scan, 2, true));
             return after_launch(s, "temperature");
         }
-        draws();
+        draws_by(scan);
         *stream_kernel = "k_scan_expsum";
         if (do_stream &&
             launch_scan_expsum(scan, rs.inv_t, nullptr, s->chunk_best, s->chunk_sum, nullptr, 0,
@@ -902,7 +913,6 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
             s->walk_steps += 16u;
         }
     }
-    draws();
     f.cand     = s->cand;
     f.win      = s->win;
     f.win_bins = win_bins_for(rs.use_p ? rs.top_p : 0.0f, rs.min_p, rows->n_vocab);
@@ -926,6 +936,7 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
     *stream_kernel = "k_scan_expsum";
     Launch scan          = L;
     scan.rv.stream_loads = s->logits_streamed; /* the one pass over whole rows */
+    draws_by(scan);
     if (do_stream &&
         /* (the thread maxima are the row-final kernel's: not wanted where none follows) */
         launch_scan_expsum(scan, rs.inv_t, f.minp_direct || f.win_locate ? nullptr : s->tmax,

@@ -132,6 +132,8 @@ __global__ __launch_bounds__(TPB) void k_cand_scan(RowView rv, float *__restrict
     int row, chunk;
     xcd_row_chunk(row, chunk);
     cand_scan_chunk<NV>(rv, tmax, wc, m, row, chunk, (int) threadIdx.x);
+    if (rv.draw_states && chunk == rv.n_chunks - 1 && threadIdx.x == 0)
+        take_row_draw(rv, row);
 }
 
 struct CandShared {

@@ -49,6 +49,10 @@ struct RowView {
     int            n_rows; /* rows of the batch (hist_len has that many entries) */
     const uint32_t *allowed;   /* NULL = no mask; bit e of a row's mask set = token e allowed */
     long            allowed_ld; /* words between rows, 0 = one mask for all rows */
+    uint64_t       *draw_states = nullptr; /* the rows' generators, when this scan (launch_tmax_scan,
+                                    launch_cand_scan, launch_scan_expsum) takes a draw of each and
+                                    leaves it in draws[row] for the launches behind; or NULL */
+    float          *draws       = nullptr;
 };
 
 /* Where the workgroups of a row meet in the one-pass exp-sum kernel (k_scan_expsum): one 64-bit

@@ -241,7 +241,7 @@ __device__ __forceinline__ void meet_store(uint64_t *slot, uint64_t v, uint32_t 
     else
         __hip_atomic_store(slot, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-template <int NV, bool PEN>
+template <int NV, bool PEN, bool DRAW = false>
 __device__ __forceinline__ uint64_t row_best_meet(const RowView &rv, int row, int chunk,
                                                   int n_rows, uint64_t mine, bool reporter,
                                                   const FusedScan &fs, uint32_t *s_cnt16,
@@ -253,6 +253,8 @@ __device__ __forceinline__ uint64_t row_best_meet(const RowView &rv, int row, in
     if (reporter) { /* one wavefront, all its lanes */
         if (lane == 0)
             meet_store(row_slots + chunk, mine, fs.local);
+        if (DRAW && rv.draw_states && chunk == C - 1 && lane == 0)
+            take_row_draw(rv, row); /* while the others are waited for */
         uint64_t a = 0, b = 0;
         uint32_t polls = 0;
         bool     met   = fs.wait_limit != 0;
@@ -431,12 +433,15 @@ __device__ __forceinline__ void expsum_chunk(const RowView &rv, int row, int chu
                 fs.chunk_best[(long) row * rv.n_chunks + chunk] = best;
         }
         if (NOMEET) {
-            if (last && (tid & (WAVE - 1)) == 0)
+            if (last && (tid & (WAVE - 1)) == 0) {
                 *fs.s_bb = best; /* the chunk's own */
+                if (rv.draw_states && chunk == rv.n_chunks - 1)
+                    take_row_draw(rv, row);
+            }
             lds_barrier();
             bb = *fs.s_bb;
         } else {
-            bb = row_best_meet<NV, PEN>(rv, row, chunk, n_rows, best, last, fs, s_cnt16);
+            bb = row_best_meet<NV, PEN, true>(rv, row, chunk, n_rows, best, last, fs, s_cnt16);
         }
     }
     if (PEN)
@@ -798,6 +803,8 @@ __global__ __launch_bounds__(TPB) void k_tmax_scan(RowView rv, float *__restrict
     if (base + 4 * tid >= end)
         tm = __builtin_nanf("");
     tmax[((long) row * rv.n_chunks + chunk) * TPB + tid] = tm;
+    if (!BEST && rv.draw_states && chunk == rv.n_chunks - 1 && tid == 0)
+        take_row_draw(rv, row);
     if (BEST) {
         /* the chunk's maximum and the first index holding it (sampler.c:52-62): only threads
          * whose own maximum equals the chunk's look for the index */
