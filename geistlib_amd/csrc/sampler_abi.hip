@@ -2320,7 +2320,7 @@ void geist_hip_spec_head_destroy(geist_hip_sampler *s, geist_hip_spec_head *sh) 
     (void) hipSetDevice(sh->device);
     gs::SpecHeadDev &d = sh->d;
     void *ptrs[] = {d.sketch, d.row_scale, d.w_drop, d.w_l1, d.dims, d.kept, d.act, d.rough,
-                    d.gmax, d.sc, d.fin_idx, d.fin_exact};
+                    d.gmax, d.sc, d.part_n, d.cand};
     for (void *p : ptrs)
         if (p)
             (void) hipFree(p);
@@ -2350,6 +2350,7 @@ int geist_hip_spec_head_build(geist_hip_sampler *s, const uint16_t *d_embed_f16,
     d.vocab = (long) n_vocab, d.d_model = (int) d_model, d.sketch_dim = (int) sd;
     d.topk = (int) topk, d.n_groups = (int) ((n_vocab + 31) / 32);
     d.list_cap = (int) (2 * topk);
+    d.slots    = gs::spec_slots(d.list_cap);
     d.w        = d_embed_f16;
     float *d_var = nullptr;
     auto   alloc = [&](auto &p, size_t bytes) {
@@ -2359,9 +2360,10 @@ int geist_hip_spec_head_build(geist_hip_sampler *s, const uint16_t *d_embed_f16,
               alloc(d.w_drop, n_vocab * 4) && alloc(d.w_l1, n_vocab * 4) && alloc(d.dims, sd * 4) &&
               alloc(d.kept, d_model) && alloc(d.act, sd * 4) && alloc(d.rough, (size_t) ((n_vocab + 31) / 32) * 32 * 4) &&
               alloc(d.gmax, (size_t) d.n_groups * 4) && alloc(d.sc, sizeof(gs::SpecScalars)) &&
-              alloc(d.fin_idx, topk * 4) && alloc(d.fin_exact, topk * 4) &&
+              alloc(d.part_n, gs::SPEC_PARTS * sizeof(int)) &&
+              alloc(d.cand, (size_t) gs::SPEC_PARTS * d.slots * sizeof(uint4)) &&
               alloc(d_var, d_model * 4);
-    int err = ok ? 0 : GEIST_HIP_E_OOM;
+    int err = !ok ? GEIST_HIP_E_OOM : gs::configure_spec_kernels() ? GEIST_HIP_E_BACKEND : 0;
     std::vector<float>    var;
     std::vector<uint32_t> dims;
     std::vector<uint8_t>  kept;

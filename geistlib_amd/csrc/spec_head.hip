@@ -13,13 +13,13 @@
  *                     sums below 2^24 (sketch_dim <= 1040), so the scores equal the reference's
  *                     integer dot bit for bit. Its epilogue leaves the maximum of every group
  *                     of 32 consecutive scores (the rows one wavefront computes).
- *   k_spec_select     the topk-th largest of those maxima: at least topk scores reach it, so
- *                     the topk best rows are among the rows >= it (about 1.1 topk rows); it
- *                     reads those groups again and keeps the topk best (the reference's heap)
- *   k_spec_exact      their exact logits, one wavefront per row, in the order of summation of
- *                     f16_gemv_m1 (16 chains, fixed tree), so that a finalist's logit is the
- *                     dense head's in every bit
- *   k_spec_final      the best exact logit among them, lowest index first
+ *   k_spec_score      the topk-th largest of those maxima: at least topk scores reach it, so
+ *                     the topk best rows are among the rows >= it (about 1.2 topk rows); those
+ *                     groups are read again, and the candidates' exact logits formed, one wavefront
+ *                     per row, in the order of summation of f16_gemv_m1 (16 chains, fixed tree), so
+ *                     that a finalist's logit is the dense head's in every bit
+ *   k_spec_final      the topk best candidates (the reference's heap) and among them the best exact
+ *                     logit, lowest index first
  *   k_spec_verify     (optional, GEIST_SPEC_VERIFY) the upper bound of every excluded row
  *                     against the winner; any row that could have won withdraws the answer
  *
@@ -32,6 +32,7 @@
 
 #include "lm_head_kernels.h"
 #include "rmsnorm_device.h"
+#include "sampler_device.h"
 
 #include <hip/hip_fp16.h>
 
@@ -59,6 +60,13 @@ __device__ __forceinline__ float key_to_float(uint32_t k) {
     return __uint_as_float((k >> 31) ? (k & 0x7fffffffu) : ~k);
 }
 
+/* orders the LDS traffic of one wavefront: what its lanes wrote before is what they read after */
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1)
@@ -70,82 +78,6 @@ __device__ __forceinline__ float wave_max(float v) {
     for (int d = 32; d >= 1; d >>= 1)
         v = __builtin_fmaxf(v, __shfl_xor(v, d, SP_WAVE));
     return v;
-}
-
-/* One count for this lane's digit (if valid). Keys that order like floats share their leading
- * digits, and atomics of one wavefront on one LDS word are serialised: the lanes that hold the
- * digit of the first valid lane add their count in one operation, the others one by one. */
-__device__ __forceinline__ void hist_add(int *s_hist, uint32_t digit, bool valid) {
-    const unsigned long long todo = __ballot(valid);
-    if (todo == 0)
-        return;
-    const int                leader = __builtin_ctzll(todo);
-    const uint32_t           dl = (uint32_t) __builtin_amdgcn_readlane((int) digit, leader);
-    const unsigned long long m  = __ballot(valid && digit == dl);
-    if ((int) (threadIdx.x & 63) == leader)
-        atomicAdd(&s_hist[dl], __builtin_popcountll(m));
-    if (valid && digit != dl)
-        atomicAdd(&s_hist[digit], 1);
-}
-
-/* The k-th largest (1 <= k <= n) of the keys the workgroup's threads hold in registers (thread t
- * holds keys[e] for the elements e * blockDim.x + t < n), by four 8-bit radix passes;
- * need_ties = how many of the keys equal to it belong to the k largest. s_hist is [4][256].
- * With PASSES < 4 only the leading 8 * PASSES bits are resolved: the result is the k-th largest
- * key with its other bits cleared (a lower bound of it that at least k keys reach).
- * Each pass costs two workgroup barriers: all wavefronts count their digits, then the first
- * wavefront alone finds the digit that holds the k-th key (lane l owns the digits 255 - 4 l ..
- * 252 - 4 l, so that a scan over the lanes runs from the largest digit down). */
-template <int EPT, int PASSES = 4>
-__device__ uint32_t block_kth_largest(const uint32_t (&keys)[EPT], int n, int k, int (*s_hist)[256],
-                                      int *s_sel, int &need_ties) {
-    const int tid = threadIdx.x, lane = tid & 63;
-    for (int i = tid; i < 4 * 256; i += (int) blockDim.x)
-        (&s_hist[0][0])[i] = 0;
-    __syncthreads();
-    uint32_t prefix = 0, mask = 0;
-    int      remaining = k;
-#pragma unroll
-    for (int pass = 0; pass < PASSES; ++pass) {
-        const int shift = 24 - 8 * pass;
-#pragma unroll
-        for (int e = 0; e < EPT; ++e)
-            hist_add(s_hist[pass], (keys[e] >> shift) & 255u,
-                     e * (int) blockDim.x + tid < n && (keys[e] & mask) == prefix);
-        __syncthreads();
-        if (tid < SP_WAVE) {
-            int c[4], local = 0;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                c[j] = s_hist[pass][255 - 4 * lane - j];
-                local += c[j];
-            }
-            int incl = local;
-#pragma unroll
-            for (int d = 1; d < SP_WAVE; d <<= 1) {
-                const int y = __shfl_up(incl, d, SP_WAVE);
-                if (lane >= d)
-                    incl += y;
-            }
-            int r = remaining - (incl - local);
-            if (r >= 1 && r <= local) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    if (r >= 1 && r <= c[j]) {
-                        s_sel[0] = 255 - 4 * lane - j;
-                        s_sel[1] = r;
-                    }
-                    r -= c[j];
-                }
-            }
-        }
-        __syncthreads();
-        prefix |= (uint32_t) s_sel[0] << shift;
-        mask |= 255u << shift;
-        remaining = s_sel[1];
-    }
-    need_ties = remaining;
-    return prefix;
 }
 
 /* ---- build ------------------------------------------------------------------------------- */
@@ -275,204 +207,177 @@ __global__ __launch_bounds__(NORM_TPB) void k_spec_act(SpecHeadDev d, const floa
     }
 }
 
-constexpr int SP_SEL_TPB = 1024; /* the two selection kernels: keys live in registers */
+constexpr int SP_SEL_TPB = 1024; /* the two selection kernels */
+constexpr int SP_WAVES   = SP_SEL_TPB / SP_WAVE;
+constexpr int SP_BINS    = 2 * SP_SEL_TPB; /* a digit of up to eleven bits */
+constexpr int SP_LDS     = 150 * 1024;     /* most dynamic LDS of a launch */
 
-/* Phase 2 of the head (spec_head.c:728-770), one workgroup of 1024 threads:
+struct SelectShared {
+    uint32_t bins[SP_BINS];
+    int      scan[SP_WAVES];
+    int      digit, left;
+    int      n_cand;
+};
+
+/* Inclusive sums over the workgroup in thread order, and the total: ends behind a barrier. */
+__device__ __forceinline__ int select_scan(SelectShared &s, int v, int &total) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    v = wave_scan_i32_dpp(v);
+    if (lane == SP_WAVE - 1)
+        s.scan[wv] = v;
+    __syncthreads();
+    const int totals = wave_scan_i32_dpp(lane < SP_WAVES ? s.scan[lane] : 0);
+    total            = (int) readlane_u32((uint32_t) totals, SP_WAVES - 1);
+    return v + (wv ? (int) readlane_u32((uint32_t) totals, wv - 1) : 0);
+}
+/* The digit in which the `need`-th largest of the counted keys lies, and its rank among that digit's;
+ * false when fewer were counted. The bins are counted and published; ends behind a barrier. */
+__device__ __forceinline__ bool select_digit(SelectShared &s, int &need, uint32_t &digit) {
+    const int tid = threadIdx.x;
+    const int b1 = (int) s.bins[SP_BINS - 1 - 2 * tid], b0 = (int) s.bins[SP_BINS - 2 - 2 * tid];
+    if (tid == 0)
+        s.digit = -1;
+    int       total;
+    const int incl = select_scan(s, b0 + b1, total), before = incl - b0 - b1;
+    if (before < need && incl >= need) {
+        const bool low = before + b1 < need;
+        s.digit        = SP_BINS - 1 - 2 * tid - (low ? 1 : 0);
+        s.left         = need - before - (low ? b1 : 0);
+    }
+    __syncthreads();
+    digit = (uint32_t) s.digit;
+    need  = s.left;
+    return s.digit >= 0;
+}
+__device__ __forceinline__ void clear_digits(SelectShared &s) {
+    reinterpret_cast<uint2 *>(s.bins)[threadIdx.x] = make_uint2(0u, 0u);
+    __syncthreads();
+}
+
+/* Phases 2 and 3 of the head (spec_head.c:728-770 and 802-826) up to the exact logits, SPEC_PARTS
+ * workgroups of 1024 threads:
  *   1. the topk-th largest group maximum (group g = rows 32 g .. 32 g + 31, written by the
  *      projection's epilogue), to 16 bits: at least topk rough scores reach it, so the topk
- *      best rows are among the rows >= it;
- *   2. only the groups whose maximum reaches that threshold are read again, their rows >= it
- *      are the candidates (about 1.1 topk, at most 2 topk);
- *   3. the topk-th largest candidate is the reference's cutoff (its heap's smallest entry); the
- *      finalists are the candidates above it and, of those equal to it, as many as complete
- *      topk rows -- the lowest indices first.
- * Thread t holds the maxima e * 1024 + t and later the candidates e * 1024 + t. */
-template <int EPT, int EPT2, int IT>
-__global__ __launch_bounds__(SP_SEL_TPB) void k_spec_select(SpecHeadDev d) {
+ *      best rows are among the rows >= it. Every workgroup finds it for itself, from the same maxima.
+ *   2. the groups whose maximum reaches that threshold (topk of them or a few more), dealt out to the
+ *      workgroups in index order, are read again; their rows >= it are the candidates (about
+ *      1.2 topk, at most 2 topk);
+ *   3. the candidates' exact logits, one wavefront per row, in f16_gemv_m1's order of summation
+ *      (src/backends/cpu_x86/kernel_f16_gemv.c:25-32, 40-59): sixteen chains of fused multiply-adds,
+ *      element k in chain k % 16, folded as (j + j+8), (i + i+4), ((0+1) + (2+3)). Lane c < 16 runs
+ *      chain c. Row and activations are laid out in LDS by chain (element k at (k % 16) * pitch +
+ *      k / 16), so that a lane reads its chain's next eight weights with one 16-byte load. d_model
+ *      is a multiple of 16. `rows_wg` wavefronts of the workgroup have a row's place in LDS.
+ * Which of the candidates are the finalists is left to k_spec_final: the cutoff needs all of them.
+ *
+ * A chain of waits: maxima 1.3 us, their count 1.4, the digits 1.3, then two trips to memory and the
+ * sums. One workgroup that did the first two steps took 16.3 us, 7.8 of them to fetch the 1036 groups'
+ * 128 bytes each, which one compute unit's share of the memory system cannot do faster; the finalists'
+ * logits took a launch of 8 us behind it. 128256 x 2560, topk 1024: the three launches behind the
+ * projection 28.1 us, the two now 18.3 (this one 12.3); the step 48.1 -> 39.9, 199992 x 1536 63.8 -> 52.7,
+ * 66544 x 2048 47.4 -> 40.8. */
+template <int EPT>
+__global__ __launch_bounds__(SP_SEL_TPB) void k_spec_score(SpecHeadDev d, const float *__restrict__ h,
+                                                           int rows_wg) {
     extern __shared__ __align__(16) uint8_t smem[];
-    int      *s_ent = reinterpret_cast<int *>(smem); /* [list_cap] groups to read again */
-    int32_t  *s_ci  = s_ent + d.list_cap;             /* [list_cap] candidate rows */
-    uint32_t *s_ck  = reinterpret_cast<uint32_t *>(s_ci + d.list_cap); /* ... and their keys */
-    __shared__ int s_hist[4][256], s_w[16], s_sel[2], s_n[3];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int n   = d.n_groups;
+    __shared__ __align__(16) SelectShared s;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = d.n_groups, part = blockIdx.x;
+    const int per   = d.d_model >> 4; /* elements per chain */
+    const int pitch = (per + 7) & ~7;
+    int      *s_ent = reinterpret_cast<int *>(smem);                   /* [slots / 32] groups */
+    int32_t  *s_ci  = s_ent + ((d.slots / 32 + 3) & ~3);               /* [slots] candidate rows */
+    uint32_t *s_ck  = reinterpret_cast<uint32_t *>(s_ci + d.slots);    /* ... and their keys */
+    float    *s_x   = reinterpret_cast<float *>(s_ck + d.slots);       /* [16][pitch] */
+    uint16_t *s_row = reinterpret_cast<uint16_t *>(s_x + 16 * pitch) + (size_t) wv * 16 * pitch;
     uint32_t  keys[EPT];
 #pragma unroll
     for (int e = 0; e < EPT; ++e) {
         const int i = e * SP_SEL_TPB + tid;
         keys[e]     = i < n ? ordered_key(d.gmax[i]) : 0u;
     }
-    if (tid < 3)
-        s_n[tid] = 0;
-    /* (16 bits of the threshold are enough: it only has to be reached by at least topk maxima
-     * and by few more rows than topk; the exact cutoff comes from the candidates below) */
-    int            ties;
-    const uint32_t tkey = block_kth_largest<EPT, 2>(keys, n, d.topk, s_hist, s_sel, ties);
-    const float    thr  = key_to_float(tkey);
-    /* 2a. the groups that reach the threshold */
-#pragma unroll
-    for (int e = 0; e < EPT; ++e) {
-        const int  i   = e * SP_SEL_TPB + tid;
-        const bool hit = i < n && keys[e] >= tkey && keys[e] != 0u;
-        const unsigned long long m = __ballot(hit);
-        if (m == 0)
-            continue;
-        int base = 0;
-        if (lane == 0)
-            base = atomicAdd(&s_n[0], __builtin_popcountll(m));
-        base = __builtin_amdgcn_readfirstlane(base);
-        const int slot = base + __builtin_popcountll(m & ((1ull << lane) - 1ull));
-        if (hit && slot < d.list_cap)
-            s_ent[slot] = i;
-    }
-    __syncthreads();
-    const int n_ent = s_n[0] < d.list_cap ? s_n[0] : d.list_cap;
-    /* 2b. their rows that reach it, into the candidate list in LDS: IT groups per thread and
-     * round with all their loads in flight together. A thread keeps which of a group's 32 rows
-     * reach it as bits -- hardly more than one does -- and stores their indices, in places from a
-     * scan over the lanes and one atomic per wavefront; the keys are fetched again below. (A ballot
-     * per row position to place the hits, and the values stored beside the indices, was 700
-     * instructions a wavefront for about 70 hits: the kernel 20.5 us of a cold step, now 16.8.) */
-    for (int round = 0; round < n_ent; round += IT * SP_SEL_TPB) { /* (uniform) */
-        float v[IT][32];
-        long  base[IT];
-#pragma unroll
-        for (int u = 0; u < IT; ++u) {
-            const int  it   = round + u * SP_SEL_TPB + tid;
-            const bool live = it < n_ent;
-            const int  i    = live ? s_ent[it] : 0;
-            base[u]         = (long) i * 32;
-            /* (no branch around a load, so that all of them are in flight together: rough is
-             * allocated in whole groups, rows beyond the vocabulary are masked afterwards) */
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const long   r0 = base[u] + 4 * j;
-                const float4 f  = *reinterpret_cast<const float4 *>(d.rough + r0);
-                v[u][4 * j]     = live && r0 + 0 < d.vocab ? f.x : -__builtin_inff();
-                v[u][4 * j + 1] = live && r0 + 1 < d.vocab ? f.y : -__builtin_inff();
-                v[u][4 * j + 2] = live && r0 + 2 < d.vocab ? f.z : -__builtin_inff();
-                v[u][4 * j + 3] = live && r0 + 3 < d.vocab ? f.w : -__builtin_inff();
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < IT; ++u) {
-            if (round + u * SP_SEL_TPB + tid - lane >= n_ent)
-                continue; /* (whole wavefronts) */
-            uint32_t hits = 0;
-#pragma unroll
-            for (int j = 0; j < 32; ++j)
-                hits |= v[u][j] >= thr ? 1u << j : 0u;
-            const int mine = __builtin_popcount(hits);
-            int       incl = mine;
-#pragma unroll
-            for (int dist = 1; dist < SP_WAVE; dist <<= 1) {
-                const int y = __shfl_up(incl, dist, SP_WAVE);
-                incl += lane >= dist ? y : 0;
-            }
-            int wbase = 0;
-            if (lane == SP_WAVE - 1)
-                wbase = atomicAdd(&s_n[1], incl);
-            int slot = __builtin_amdgcn_readlane(wbase, SP_WAVE - 1) + incl - mine;
-            for (; hits != 0u; hits &= hits - 1u, ++slot)
-                if (slot < d.list_cap)
-                    s_ci[slot] = (int32_t) (base[u] + __builtin_ctz(hits));
-        }
-    }
-    __syncthreads();
-    const int n_cand = s_n[1];
-    if (s_n[0] > d.list_cap || n_cand > d.list_cap || n_cand < d.topk) { /* (uniform) */
-        if (tid == 0) {
-            d.sc->threshold = thr, d.sc->cutoff = thr, d.sc->n_cand = n_cand, d.sc->n_final = 0;
-        }
-        return;
-    }
-    /* 3. the cutoff and the finalists */
-    uint32_t ck[EPT2];
-    int32_t  ci[EPT2];
-#pragma unroll
-    for (int e = 0; e < EPT2; ++e) {
-        const int i = e * SP_SEL_TPB + tid;
-        ci[e]       = i < n_cand ? s_ci[i] : -1;
-        ck[e]       = ci[e] >= 0 ? ordered_key(d.rough[ci[e]]) : 0u;
-    }
-#pragma unroll
-    for (int e = 0; e < EPT2; ++e)
-        if (ci[e] >= 0)
-            s_ck[e * SP_SEL_TPB + tid] = ck[e]; /* for the ties (the barriers below stand between) */
-    int            need_ties;
-    const uint32_t ckey = block_kth_largest<EPT2>(ck, n_cand, d.topk, s_hist, s_sel, need_ties);
-    int tie_cnt = 0;
-#pragma unroll
-    for (int e = 0; e < EPT2; ++e)
-        tie_cnt += (ci[e] >= 0 && ck[e] == ckey) ? 1 : 0;
-#pragma unroll
-    for (int sft = 32; sft >= 1; sft >>= 1)
-        tie_cnt += __shfl_xor(tie_cnt, sft, SP_WAVE);
-    if (lane == 0)
-        s_w[tid >> 6] = tie_cnt;
-    __syncthreads();
-    tie_cnt = 0;
-    for (int i = 0; i < SP_SEL_TPB / SP_WAVE; ++i)
-        tie_cnt += s_w[i];
-#pragma unroll
-    for (int e = 0; e < EPT2; ++e) {
-        bool in = ci[e] >= 0 && ck[e] > ckey;
-        if (ci[e] >= 0 && ck[e] == ckey) {
-            in = true;
-            if (tie_cnt > need_ties) { /* the lowest indices among the rows that tie */
-                int before = 0;
-                for (int j = 0; j < n_cand; ++j)
-                    before += (s_ci[j] < ci[e] && s_ck[j] == ckey) ? 1 : 0;
-                in = before < need_ties;
-            }
-        }
-        const unsigned long long m = __ballot(in);
-        if (m == 0)
-            continue;
-        int base = 0;
-        if (lane == 0)
-            base = atomicAdd(&s_n[2], __builtin_popcountll(m));
-        base = __builtin_amdgcn_readfirstlane(base);
-        const int slot = base + __builtin_popcountll(m & ((1ull << lane) - 1ull));
-        if (in && slot < d.topk)
-            d.fin_idx[slot] = ci[e];
-    }
-    __syncthreads();
-    if (tid == 0) {
-        d.sc->threshold = thr;
-        d.sc->cutoff    = key_to_float(ckey);
-        d.sc->n_cand    = n_cand;
-        d.sc->n_final   = s_n[2]; /* == topk */
-    }
-}
-
-/* Phase 3 (spec_head.c:802-826): the exact logit of every finalist, one wavefront per row, in
- * f16_gemv_m1's order of summation (src/backends/cpu_x86/kernel_f16_gemv.c:25-32, 40-59):
- * sixteen chains of fused multiply-adds, element k in chain k % 16, folded as (j + j+8),
- * (i + i+4), ((0+1) + (2+3)). Lane c < 16 runs chain c. Row and activations are laid out in LDS
- * by chain (element k at (k % 16) * pitch + k / 16), so that a lane reads its chain's next
- * eight weights with one 16-byte load. d_model is a multiple of 16. */
-__global__ __launch_bounds__(SP_TPB) void k_spec_exact(SpecHeadDev d, const float *__restrict__ h) {
-    extern __shared__ __align__(16) uint8_t smem[];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int per   = d.d_model >> 4;     /* elements per chain */
-    const int pitch = (per + 7) & ~7;
-    float    *s_x   = reinterpret_cast<float *>(smem);                       /* [16][pitch] */
-    uint16_t *s_row = reinterpret_cast<uint16_t *>(smem + (size_t) 16 * pitch * 4) +
-                      (size_t) wv * 16 * pitch;                              /* [16][pitch] */
-    const int n_final = d.sc->n_final;
-    if ((int) blockIdx.x * (SP_TPB / SP_WAVE) >= n_final)
-        return; /* (uniform) */
-    /* the activations are requested first and stored last, so that their latency and the row's
-     * overlap */
-    constexpr int X_PER_THREAD = SPEC_D_MODEL_MAX / SP_TPB;
+    /* the activations are asked for with the maxima and put into LDS below */
+    constexpr int X_PER_THREAD = SPEC_D_MODEL_MAX / SP_SEL_TPB;
     float         xv[X_PER_THREAD];
 #pragma unroll
     for (int i = 0; i < X_PER_THREAD; ++i)
-        xv[i] = i * SP_TPB + tid < d.d_model ? h[i * SP_TPB + tid] : 0.0f;
-    const int slot = (int) blockIdx.x * (SP_TPB / SP_WAVE) + wv;
-    if (slot < n_final) {
-        const uint16_t *src = d.w + (long) d.fin_idx[slot] * d.d_model;
+        xv[i] = i * SP_SEL_TPB + tid < d.d_model ? h[i * SP_SEL_TPB + tid] : 0.0f;
+    if (tid == 0)
+        s.n_cand = 0;
+    clear_digits(s);
+    /* 1. (16 bits of the threshold are enough: it only has to be reached by at least topk maxima
+     * and by few more rows than topk; the exact cutoff comes from the candidates) */
+#pragma unroll
+    for (int e = 0; e < EPT; ++e)
+        if (keys[e]) /* (a NaN, or beyond the groups: never counted) */
+            atomicAdd(&s.bins[keys[e] >> 21], 1u);
+    __syncthreads();
+    int      need = d.topk;
+    uint32_t d1, d2, tkey = 0u;
+    if (select_digit(s, need, d1)) {
+        clear_digits(s);
+#pragma unroll
+        for (int e = 0; e < EPT; ++e)
+            if (keys[e] && keys[e] >> 21 == d1)
+                atomicAdd(&s.bins[keys[e] >> 16 & 31u], 1u);
+        __syncthreads();
+        (void) select_digit(s, need, d2);
+        tkey = d1 << 21 | d2 << 16;
+    }
+    const float thr = key_to_float(tkey); /* (too few maxima that are numbers: NaN, nothing reaches it) */
+#pragma unroll
+    for (int i = 0; i < X_PER_THREAD; ++i) {
+        const int k = i * SP_SEL_TPB + tid;
+        if (k < d.d_model)
+            s_x[(k & 15) * pitch + (k >> 4)] = xv[i];
+    }
+    /* 2. this workgroup's share of the groups that reach the threshold */
+    int cnt = 0, n_ent;
+#pragma unroll
+    for (int e = 0; e < EPT; ++e)
+        cnt += keys[e] >= tkey && keys[e] != 0u;
+    int at = select_scan(s, cnt, n_ent) - cnt;
+    if (part == 0 && tid == 0)
+        d.sc->threshold = thr;
+    if (n_ent > d.list_cap) { /* (uniform) more around the cutoff than the list holds */
+        if (tid == 0)
+            d.part_n[part] = part == 0 ? n_ent : 0;
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < EPT; ++e)
+        if (keys[e] >= tkey && keys[e] != 0u) {
+            if (at % SPEC_PARTS == part)
+                s_ent[at / SPEC_PARTS] = e * SP_SEL_TPB + tid;
+            ++at;
+        }
+    __syncthreads();
+    const int mine = (n_ent - part + SPEC_PARTS - 1) / SPEC_PARTS; /* groups, at most slots / 32 */
+    for (int t0 = wv * SP_WAVE; t0 < mine * 8; t0 += SP_SEL_TPB) { /* (whole wavefronts) */
+        const int    t    = t0 + lane;
+        const int    r0   = t < mine * 8 ? s_ent[t >> 3] * 32 + 4 * (t & 7) : 0;
+        const long   left = t < mine * 8 ? d.vocab - r0 : 0; /* rows of the vocabulary */
+        const float4 f    = *reinterpret_cast<const float4 *>(d.rough + r0); /* (allocated in whole groups) */
+        const uint32_t m  = (uint32_t) (left > 0 && f.x >= thr) | (uint32_t) (left > 1 && f.y >= thr) << 1 |
+                           (uint32_t) (left > 2 && f.z >= thr) << 2 | (uint32_t) (left > 3 && f.w >= thr) << 3;
+        int slot = wave_reserve(__popc(m), &s.n_cand);
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            if (m >> c & 1u) {
+                s_ci[slot] = r0 + c;
+                s_ck[slot] = ordered_key(f4_get(f, c));
+                ++slot;
+            }
+    }
+    __syncthreads();
+    const int n_cand = s.n_cand;
+    if (tid == 0)
+        d.part_n[part] = n_cand;
+    /* 3. (no workgroup barrier below) */
+    if (wv >= rows_wg)
+        return;
+    for (int c = wv; c < n_cand; c += rows_wg) {
+        const uint16_t *src = d.w + (long) s_ci[c] * d.d_model;
         for (int o = lane * 8; o < d.d_model; o += SP_WAVE * 8) {
             const nt_u4 q = __builtin_nontemporal_load(reinterpret_cast<const nt_u4 *>(src + o));
             /* elements o .. o+7: chains (o & 15) .. (o & 15) + 7 at position o / 16 */
@@ -483,80 +388,131 @@ __global__ __launch_bounds__(SP_TPB) void k_spec_exact(SpecHeadDev d, const floa
                 dst[(2 * i + 1) * pitch] = (uint16_t) (q[i] >> 16);
             }
         }
-    }
-#pragma unroll
-    for (int i = 0; i < X_PER_THREAD; ++i) {
-        const int k = i * SP_TPB + tid;
-        if (k < d.d_model)
-            s_x[(k & 15) * pitch + (k >> 4)] = xv[i];
-    }
-    __syncthreads();
-    if (slot >= n_final)
-        return; /* (no workgroup barrier below) */
-    float acc = 0.0f;
-    if (lane < 16) {
-        const uint16_t *wr = s_row + lane * pitch;
-        const float    *xr = s_x + lane * pitch;
-        int             p  = 0;
-        for (; p + 8 <= per; p += 8) {
-            const uint4  q  = *reinterpret_cast<const uint4 *>(wr + p);
-            const float4 xa = *reinterpret_cast<const float4 *>(xr + p);
-            const float4 xb = *reinterpret_cast<const float4 *>(xr + p + 4);
-            acc = __builtin_fmaf(h2f((uint16_t) (q.x & 0xffffu)), xa.x, acc);
-            acc = __builtin_fmaf(h2f((uint16_t) (q.x >> 16)), xa.y, acc);
-            acc = __builtin_fmaf(h2f((uint16_t) (q.y & 0xffffu)), xa.z, acc);
-            acc = __builtin_fmaf(h2f((uint16_t) (q.y >> 16)), xa.w, acc);
-            acc = __builtin_fmaf(h2f((uint16_t) (q.z & 0xffffu)), xb.x, acc);
-            acc = __builtin_fmaf(h2f((uint16_t) (q.z >> 16)), xb.y, acc);
-            acc = __builtin_fmaf(h2f((uint16_t) (q.w & 0xffffu)), xb.z, acc);
-            acc = __builtin_fmaf(h2f((uint16_t) (q.w >> 16)), xb.w, acc);
+        wave_lds_order();
+        float acc = 0.0f;
+        if (lane < 16) {
+            const uint16_t *wr = s_row + lane * pitch;
+            const float    *xr = s_x + lane * pitch;
+            int             p  = 0;
+            for (; p + 8 <= per; p += 8) {
+                const uint4  q  = *reinterpret_cast<const uint4 *>(wr + p);
+                const float4 xa = *reinterpret_cast<const float4 *>(xr + p);
+                const float4 xb = *reinterpret_cast<const float4 *>(xr + p + 4);
+                acc = __builtin_fmaf(h2f((uint16_t) (q.x & 0xffffu)), xa.x, acc);
+                acc = __builtin_fmaf(h2f((uint16_t) (q.x >> 16)), xa.y, acc);
+                acc = __builtin_fmaf(h2f((uint16_t) (q.y & 0xffffu)), xa.z, acc);
+                acc = __builtin_fmaf(h2f((uint16_t) (q.y >> 16)), xa.w, acc);
+                acc = __builtin_fmaf(h2f((uint16_t) (q.z & 0xffffu)), xb.x, acc);
+                acc = __builtin_fmaf(h2f((uint16_t) (q.z >> 16)), xb.y, acc);
+                acc = __builtin_fmaf(h2f((uint16_t) (q.w & 0xffffu)), xb.z, acc);
+                acc = __builtin_fmaf(h2f((uint16_t) (q.w >> 16)), xb.w, acc);
+            }
+            for (; p < per; ++p)
+                acc = __builtin_fmaf(h2f(wr[p]), xr[p], acc);
         }
-        for (; p < per; ++p)
-            acc = __builtin_fmaf(h2f(wr[p]), xr[p], acc);
+        wave_lds_order(); /* the next row comes to the same place */
+        const float v   = __fadd_rn(acc, __shfl_down(acc, 8, SP_WAVE));
+        const float q   = __fadd_rn(v, __shfl_down(v, 4, SP_WAVE));
+        const float a   = __fadd_rn(q, __shfl_down(q, 1, SP_WAVE));
+        const float sum = __fadd_rn(a, __shfl_down(a, 2, SP_WAVE));
+        if (lane == 0)
+            d.cand[(long) part * d.slots + c] =
+                make_uint4(s_ck[c], (uint32_t) s_ci[c], __float_as_uint(sum), 0u);
     }
-    const float v   = __fadd_rn(acc, __shfl_down(acc, 8, SP_WAVE));
-    const float q   = __fadd_rn(v, __shfl_down(v, 4, SP_WAVE));
-    const float a   = __fadd_rn(q, __shfl_down(q, 1, SP_WAVE));
-    const float sum = __fadd_rn(a, __shfl_down(a, 2, SP_WAVE));
-    if (lane == 0)
-        d.fin_exact[slot] = sum;
 }
 
-/* The best exact logit among the finalists, the lowest index among equals (spec_head.c:827),
- * one workgroup. */
+/* The topk-th largest candidate's rough score is the reference's cutoff (its heap's smallest entry); the
+ * finalists are the candidates above it and, of those equal to it, as many as complete topk rows -- the
+ * lowest indices first. The best exact logit among them, the lowest index among equals
+ * (spec_head.c:827). One workgroup: four threads to a part of the candidates, whose entries are asked
+ * for before their number is known (a part holds four or five; beyond sixteen a loop of its own). */
 __global__ __launch_bounds__(SP_SEL_TPB) void k_spec_final(SpecHeadDev d, SpecResult *__restrict__ res) {
-    __shared__ uint64_t s_best[SP_SEL_TPB / SP_WAVE];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int n_final = d.sc->n_final;
-    if (n_final == 0) { /* (uniform) more candidates around the cutoff than the list holds */
+    extern __shared__ __align__(16) uint8_t smem[];
+    uint32_t *s_ck = reinterpret_cast<uint32_t *>(smem); /* [list_cap] keys of the rough scores, */
+    int32_t  *s_ci = reinterpret_cast<int32_t *>(s_ck + d.list_cap); /* rows, */
+    float    *s_ex = reinterpret_cast<float *>(s_ci + d.list_cap);   /* exact logits */
+    __shared__ __align__(16) SelectShared s;
+    __shared__ uint64_t s_best[SP_WAVES];
+    constexpr int       AHEAD = 4;
+    static_assert(SP_SEL_TPB == 4 * SPEC_PARTS && 4 * AHEAD <= 32, "a part has places for a group at least");
+    const int    tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const uint4 *mine = d.cand + (long) (tid >> 2) * d.slots;
+    const int    own  = d.part_n[tid >> 2];
+    uint4        ahead[AHEAD];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i)
+        ahead[i] = mine[(tid & 3) + 4 * i];
+    const float thr = d.sc->threshold;
+    int         n_cand;
+    (void) select_scan(s, (tid & 3) ? 0 : own, n_cand);
+    if (tid == 0)
+        s.n_cand = 0;
+    if (n_cand > d.list_cap || n_cand < d.topk) { /* (uniform) none, or more around the cutoff than the
+                                                   * list holds */
         if (tid == 0) {
-            res->token = -1, res->answered = 0, res->n_finalists = 0, res->n_listed = d.sc->n_cand;
-            res->cutoff = d.sc->cutoff, res->best_exact = 0.0f;
+            res->token = -1, res->answered = 0, res->n_finalists = 0, res->n_listed = n_cand;
+            res->cutoff = thr, res->best_exact = 0.0f;
         }
         return;
     }
-    uint64_t best = 0;
-    for (int i = tid; i < n_final; i += SP_SEL_TPB) {
-        const uint64_t p = ((uint64_t) ordered_key(d.fin_exact[i]) << 32) |
-                           (uint32_t) (0x7fffffff - d.fin_idx[i]);
-        best = p > best ? p : best;
-    }
+    clear_digits(s);
+    const int some = (tid & 3) < own ? (own - (tid & 3) + 3) / 4 : 0;
+    int       at   = wave_reserve(some, &s.n_cand);
+    auto put = [&](const uint4 &c) {
+        s_ck[at] = c.x;
+        s_ci[at] = (int32_t) c.y;
+        s_ex[at] = __uint_as_float(c.z);
+        ++at;
+    };
 #pragma unroll
-    for (int s = 32; s >= 1; s >>= 1) {
-        const uint64_t o = __shfl_xor(best, s, SP_WAVE);
-        best             = o > best ? o : best;
+    for (int i = 0; i < AHEAD; ++i)
+        if (i < some)
+            put(ahead[i]);
+    for (int i = AHEAD; i < some; ++i)
+        put(mine[(tid & 3) + 4 * i]);
+    __syncthreads();
+    uint32_t prefix = 0, digit = 0;
+    int      need = d.topk;
+#pragma unroll
+    for (int pass = 0; pass < 3; ++pass) { /* digits of 11, 11 and 10 bits */
+        const int shift = pass == 0 ? 21 : pass == 1 ? 10 : 0, bits = pass == 2 ? 10 : 11;
+        if (pass)
+            clear_digits(s);
+        for (int i = tid; i < n_cand; i += SP_SEL_TPB) {
+            const uint32_t k = s_ck[i];
+            if (pass == 0 || k >> (shift + bits) == prefix)
+                atomicAdd(&s.bins[k >> shift & ((1u << bits) - 1u)], 1u);
+        }
+        __syncthreads();
+        (void) select_digit(s, need, digit); /* (n_cand >= topk keys were counted) */
+        prefix = prefix << bits | digit;
     }
+    const uint32_t ckey      = prefix;
+    const int      need_ties = need, tie_cnt = (int) s.bins[digit];
+    uint64_t       best      = 0;
+    for (int i = tid; i < n_cand; i += SP_SEL_TPB) {
+        bool in = s_ck[i] >= ckey;
+        if (s_ck[i] == ckey && tie_cnt > need_ties) { /* the lowest indices among the rows that tie */
+            int before = 0;
+            for (int j = 0; j < n_cand; ++j)
+                before += (s_ci[j] < s_ci[i] && s_ck[j] == ckey) ? 1 : 0;
+            in = before < need_ties;
+        }
+        const uint64_t p = ((uint64_t) ordered_key(s_ex[i]) << 32) | (uint32_t) (0x7fffffff - s_ci[i]);
+        best             = in && p > best ? p : best;
+    }
+    best = wave_max_u64(best);
     if (lane == 0)
         s_best[wv] = best;
     __syncthreads();
     if (tid == 0) {
-        for (int i = 1; i < SP_SEL_TPB / SP_WAVE; ++i)
+        for (int i = 1; i < SP_WAVES; ++i)
             best = s_best[i] > best ? s_best[i] : best;
         res->token       = 0x7fffffff - (int32_t) (uint32_t) (best & 0xffffffffu);
         res->answered    = 1;
-        res->n_finalists = n_final;
-        res->n_listed    = d.sc->n_cand;
-        res->cutoff      = d.sc->cutoff;
+        res->n_finalists = d.topk;
+        res->n_listed    = n_cand;
+        res->cutoff      = key_to_float(ckey);
         res->best_exact  = key_to_float((uint32_t) (best >> 32));
     }
 }
@@ -594,6 +550,19 @@ void launch_spec_sketch_rows(hipStream_t stream, const SpecHeadDev &d) {
                          stream>>>(d);
 }
 
+int configure_spec_kernels() {
+    const void *kernels[] = {reinterpret_cast<const void *>(k_spec_score<4>),
+                             reinterpret_cast<const void *>(k_spec_score<8>),
+                             reinterpret_cast<const void *>(k_spec_score<SPEC_TMAX_EPT_MAX>),
+                             reinterpret_cast<const void *>(k_spec_final)};
+    for (const void *k : kernels) {
+        const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, SP_LDS);
+        if (e != hipSuccess)
+            return (int) e;
+    }
+    return 0;
+}
+
 void launch_spec_try(hipStream_t stream, const SpecHeadDev &d, const float *h, bool verify,
                      SpecResult *result, const float *norm_w, float eps, float *h_normed) {
     const dim3 one(1), block(SP_TPB), sel(SP_SEL_TPB);
@@ -608,28 +577,21 @@ void launch_spec_try(hipStream_t stream, const SpecHeadDev &d, const float *h, b
     f.gmax = d.gmax;
     launch_q8w_gemv(stream, d.sketch, d.row_scale, d.vocab, d.sketch_dim, d.act, d.sketch_dim, 1,
                     d.rough, d.vocab, &f);
-    /* group maxima: one per 32 rows; candidates: at most 2 topk */
-    const size_t lds_sel = (size_t) d.list_cap * 3 * sizeof(int);
-    if (d.n_groups <= 4 * SP_SEL_TPB && d.list_cap <= 2 * SP_SEL_TPB) {
-        k_spec_select<4, 2, 2><<<one, sel, lds_sel, stream>>>(d);
-    } else { /* up to 96 KB of LDS, above what a launch may take by default */
-        if (d.n_groups <= 8 * SP_SEL_TPB) {
-            (void) hipFuncSetAttribute(
-                reinterpret_cast<const void *>(k_spec_select<8, SPEC_LIST_EPT_MAX, 1>),
-                hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds_sel);
-            k_spec_select<8, SPEC_LIST_EPT_MAX, 1><<<one, sel, lds_sel, stream>>>(d);
-        } else {
-            (void) hipFuncSetAttribute(
-                reinterpret_cast<const void *>(
-                    k_spec_select<SPEC_TMAX_EPT_MAX, SPEC_LIST_EPT_MAX, 1>),
-                hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds_sel);
-            k_spec_select<SPEC_TMAX_EPT_MAX, SPEC_LIST_EPT_MAX, 1><<<one, sel, lds_sel, stream>>>(d);
-        }
-    }
-    const int    pitch = ((d.d_model >> 4) + 7) & ~7;
-    const size_t lds   = (size_t) 16 * pitch * (sizeof(float) + (SP_TPB / SP_WAVE) * sizeof(uint16_t));
-    k_spec_exact<<<dim3((unsigned) ((d.topk + 3) / 4)), block, lds, stream>>>(d, h);
-    k_spec_final<<<one, sel, 0, stream>>>(d, result);
+    /* as many rows at a time as LDS has room for beside the activations and the candidates (twelve of
+     * 5120 columns, sixteen up to 4096) */
+    const size_t pitch = (size_t) (((d.d_model >> 4) + 7) & ~7);
+    const size_t fixed = (size_t) ((d.slots / 32 + 3) & ~3) * 4 + (size_t) d.slots * 8 + 16 * pitch * sizeof(float);
+    const size_t row   = 16 * pitch * sizeof(uint16_t), room = SP_LDS - fixed;
+    const int    rows_wg = room / row < (size_t) SP_WAVES ? (int) (room / row) : SP_WAVES;
+    const size_t lds_score = fixed + (size_t) rows_wg * row, lds_final = (size_t) d.list_cap * 12;
+    auto score = [&](auto kernel) { kernel<<<dim3(SPEC_PARTS), sel, lds_score, stream>>>(d, h, rows_wg); };
+    if (d.n_groups <= 4 * SP_SEL_TPB)
+        score(k_spec_score<4>);
+    else if (d.n_groups <= 8 * SP_SEL_TPB)
+        score(k_spec_score<8>);
+    else
+        score(k_spec_score<SPEC_TMAX_EPT_MAX>);
+    k_spec_final<<<one, sel, lds_final, stream>>>(d, result);
     if (verify)
         k_spec_verify<<<rows, block, 0, stream>>>(d, result);
 }

@@ -17,9 +17,6 @@ struct SpecScalars {
     float h_l1_kept;  /* L1 norm of h over the kept dimensions */
     float h_l2_drop;  /* L2 norm of h over the dropped dimensions */
     float threshold;  /* a lower bound of the topk-th largest group maximum: the topk best rows are >= it */
-    float cutoff;     /* the topk-th largest rough score */
-    int   n_cand;     /* rows >= threshold */
-    int   n_final;    /* topk, or 0 when the candidates did not fit the list */
 };
 
 /* What a call answers (mirrors struct geist_hip_spec_result). */
@@ -37,6 +34,7 @@ struct SpecHeadDev {
     int  d_model, sketch_dim, topk;
     int  n_groups; /* ceil(vocab / 32): groups of consecutive rows whose maximum the projection leaves */
     int  list_cap; /* 2 topk candidates */
+    int  slots;    /* candidates a part has places for (spec_slots) */
     const uint16_t *w; /* [vocab, d_model] binary16, not owned */
     /* built once */
     int8_t   *sketch;    /* [vocab, sketch_dim] */
@@ -50,14 +48,17 @@ struct SpecHeadDev {
     float       *rough; /* [vocab], allocated up to a multiple of 32 */
     float       *gmax;  /* [n_groups] maxima of the rough scores of 32 consecutive rows */
     SpecScalars *sc;
-    int32_t     *fin_idx;    /* [topk] the finalists, any order */
-    float       *fin_exact;  /* [topk] their exact logits */
+    int     *part_n; /* [SPEC_PARTS] a part's candidates, or more than list_cap: nobody's fit */
+    uint4   *cand;   /* [SPEC_PARTS][slots] key of the rough score, row, bits of the exact logit */
 };
 
-/* The selection kernels hold their keys in registers, 1024 threads: up to 32 group maxima each
- * (a vocabulary of 2^20 rows) and up to 8 candidates each (2 x 4096). */
+/* The groups that reach the threshold, at most list_cap, are dealt out to this many workgroups. */
+constexpr int SPEC_PARTS = 256;
+inline int    spec_slots(int list_cap) { return (list_cap + SPEC_PARTS - 1) / SPEC_PARTS * 32; }
+
+/* The selection kernel holds the group maxima in registers, 1024 threads: up to 32 each (a vocabulary of
+ * 2^20 rows). */
 constexpr int SPEC_TMAX_EPT_MAX = 32;
-constexpr int SPEC_LIST_EPT_MAX = 8;
 constexpr int SPEC_VOCAB_MAX    = SPEC_TMAX_EPT_MAX * 1024 * 32;
 constexpr int SPEC_TOPK_MAX     = 4096;
 /* Largest d_model the finalist kernel stages in LDS. */
@@ -72,6 +73,9 @@ void launch_spec_dim_stats(hipStream_t stream, const uint16_t *w, long vocab, in
                            long vstep, float *dvar);
 /* sketch, row_scale, w_drop, w_l1 from w, dims and kept (spec_head.c:563-603). */
 void launch_spec_sketch_rows(hipStream_t stream, const SpecHeadDev &d);
+/* Per-device attributes of the kernels of launch_spec_try: more LDS than a launch may take by default.
+ * Call once with the device current, before the first. Returns a hipError_t value. */
+int configure_spec_kernels();
 /* transformer_spec_head_try for one normed hidden row h [d_model] (spec_head.c:624-889). With
  * norm_w != NULL, h is the hidden row before the output norm: the norm (weights norm_w, eps) runs
  * in the first kernel and h_normed [d_model] receives the normed row. */

@@ -305,3 +305,34 @@ def test_try_hidden_norms_in_the_same_launch(hs, oracle):
         want = want_sh.try_row(want_normed)
         assert (got.token, got.cutoff, got.answered) == (want["token"], want["cutoff"], 1)
     hs.spec_head_destroy(sh)
+
+
+@pytest.mark.parametrize("vocab,d_model,topk", [(20000, 5120, 256), (66001, 1280, 1024), (8192, 1280, 16),
+                                                (66000, 4096, 300)])
+def test_candidates_crowded_into_few_groups(hs, oracle, vocab, d_model, topk):
+    """Many of the best rows are consecutive: a group of 32 hands all of its rows on, the workgroup it
+    is dealt to forms several times its share of exact logits, others (topk of 16) none at all."""
+    print(f"spec crowded vocab={vocab} d_model={d_model} topk={topk}", flush=True)
+    g = np.random.default_rng(vocab + topk)
+    w16 = table(g, vocab, d_model)
+    lean = (0.02 * g.standard_normal(d_model)).astype(np.float32)
+    at = 32 * 7 + 5
+    n = topk // 2
+    w16[at:at + n] = (w16[at:at + n].astype(np.float32) + lean).astype(np.float16)
+    want_sh = oracle.spec_head_build(w16.view(np.uint16), topk=topk)
+    sh = hs.spec_head_build(torch.from_numpy(w16.view(np.int16)).cuda(), topk=topk)
+    res = torch.zeros(6, dtype=torch.int32, device="cuda")
+    answered = 0
+    for strength in (0.0, 20.0, 60.0):
+        h = (g.standard_normal(d_model) + strength * lean).astype(np.float32)
+        want = want_sh.try_row(h)
+        hs.spec_head_try(sh, torch.from_numpy(h).cuda(), res)
+        hs.sync()
+        got = result_of(res)
+        if not got.answered:                 # more candidates than the list: the head declines
+            assert got.token == -1 and got.n_listed > 2 * topk
+            continue
+        answered += 1
+        assert (got.token, got.cutoff, got.n_finalists) == (want["token"], want["cutoff"], topk)
+    assert answered >= 1
+    hs.spec_head_destroy(sh)
