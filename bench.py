@@ -158,8 +158,8 @@ def reference_top_k_baseline(w, cores, budget_s):
 def topk_path_counts(hs, row_sets, prm, d_u, d_out, n_rows):
     """Which path served the rows of a top-k configuration, over every input copy once
     (geist_hip_sampler_topk_paths after each call): the candidates handed on by the scan, the
-    per-thread maxima, the selection over the whole row; fallback_rate = the share of rows that
-    did not take the first."""
+    per-thread maxima (the first path of large batches), the selection over the whole row;
+    fallback_rate = the share of rows that did not take the first path of such a call."""
     counts = {"scan_candidates": 0, "thread_maxima": 0, "whole_row": 0, "other": 0}
     for rs in row_sets:
         hs.sample(rs, prm, d_u, d_out)
@@ -167,7 +167,8 @@ def topk_path_counts(hs, row_sets, prm, d_u, d_out, n_rows):
             counts[{0: "scan_candidates", 1: "thread_maxima", 2: "whole_row"}.get(p, "other")] += 1
     total = max(1, sum(counts.values()))
     counts["rows"] = total
-    counts["fallback_rate"] = round(1.0 - counts["scan_candidates"] / total, 6)
+    first = counts["scan_candidates"] or counts["thread_maxima"]
+    counts["fallback_rate"] = round(1.0 - first / total, 6)
     return counts
 
 

@@ -729,7 +729,7 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
         const int  rank   = rs.k + margin, cap_margin = L.rv.softcap > 0.0f ? 8 : 0;
         const int  k_wide = rank + cap_margin < WIDE_K_SEL_MAX ? rank + cap_margin : WIDE_K_SEL_MAX;
         const bool wide   = (lazy || !L.pen) && rs.k <= WIDE_K_SEL_MAX &&
-                          (rank > WIDE_RANK_MIN ||
+                          (rank > WIDE_RANK_MIN || rows->rows * rows->n_vocab >= WIDE_LOGITS ||
                            (cap_margin && (rank > WIDE_RANK_MIN_CAPPED || L.rv.n_chunks <= 16))) &&
                           L.rv.n_chunks <= WIDE_CHUNKS_MAX && rows->n_vocab / 32 >= 2 * (size_t) k_wide;
         f.mode = FINAL_TOPK;
@@ -804,7 +804,9 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
             draws();
         else
             draws_by(scan);
-        if (m) {
+        /* (rows that could be handed on, in a batch where that is the slower way: WIDE_LOGITS) */
+        const bool large_wide = wide && rows->rows * rows->n_vocab >= WIDE_LOGITS;
+        if (m && !large_wide) {
             const WaveCands wc = wave_cands_at(s->wcands, row_waves);
             f.row_flag         = s->row_flag;
             s->topk_paths_rows = rows->rows;
@@ -815,7 +817,8 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
                 launch_final_cand(L, f, wc);
             return after_launch(s, "top-k");
         }
-        s->topk_paths_rows = 0;
+        f.row_flag         = m ? s->row_flag : nullptr;
+        s->topk_paths_rows = m ? rows->rows : 0;
         *stream_kernel     = "k_tmax_scan";
         if (!s->tmax_ready && do_stream)
             launch_tmax_scan(scan, s->tmax, nullptr);

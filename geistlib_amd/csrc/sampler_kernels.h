@@ -25,6 +25,11 @@ constexpr int WIDE_CHUNKS_MAX = 32;  /* ... whose rows have at most so many chun
  * 223709 23.3 / 22.3). */
 constexpr int WIDE_RANK_MIN        = 48;
 constexpr int WIDE_RANK_MIN_CAPPED = 16;
+/* Batches of at least so many logits take that path whatever the rank, rows whose scan could hand
+ * candidates on (k_cand_scan, k_final_cand) too: their scan leaves the maxima alone, 45.6 against 53.9 us
+ * for 256 x 262144. 256 x 262144, k = 64, 56.3 / 63.9; 192 x 262144, k = 40, 43.7 / 48.8; 152 x 128512 22.4 /
+ * 24.2; 96 x 121168 16.1 / 15.8; 100 x 100000 15.3 / 14.4; 51 x 223712 16.3 / 16.2. */
+constexpr size_t WIDE_LOGITS = (size_t) 1 << 24;
 constexpr int TOPK_MAX       = 8192; /* the reference caps top_k here (sampler.c:213-215) */
 constexpr int HISTORY_MAX    = 65535;
 

@@ -84,3 +84,32 @@ def test_top_k_of_hundreds_matches_oracle(hs, oracle, n, k, form):
         want.append(t)
         infos.append(i)
     assert compare_ids(got, want, infos, f"wide n={n} k={k} {form}") <= 1
+
+
+@pytest.mark.parametrize("k", [2, 40, 64])
+@pytest.mark.parametrize("pen", [False, True])
+def test_large_batches_select_from_the_thread_maxima(oracle, k, pen):
+    """From 2^24 logits on, plain rows of any k: the call says that the thread maxima served it."""
+    from geistlib_amd import HipSampler, SampleParams
+    n, rows = 262144, 64
+    g = np.random.default_rng(k + pen)
+    x = np.tile((g.standard_normal((16, n)) * 2).astype(np.float32), (4, 1))
+    x[1] = -np.sort(-x[1])
+    x[2] = np.round(x[2])
+    x[3] = 1.5
+    u = (g.integers(0, 1 << 24, rows) / np.float32(1 << 24)).astype(np.float32)
+    kw = dict(temperature=0.7, top_k=k, top_p=0.9)
+    hist = g.integers(0, n, (rows, 700)).astype(np.int32)
+    hist[:, :20] = np.argsort(-x[5])[:20]
+    hl = np.full(rows, 700, dtype=np.int32)
+    s = HipSampler(max_rows=rows, max_vocab=n)
+    s.one_launch_topk(False)
+    got = run_rows(s, torch, x, u, SampleParams.make(**kw, **(dict(rep=1.1, freq=0.5, pres=0.2) if pen else {})),
+                   hist if pen else None, hl if pen else None)
+    paths = s.topk_paths(rows).tolist()
+    s.close()
+    check = list(range(0, 20)) + [rows - 1]
+    want = [oracle.chain_u(oracle.penalties(x[r], hist[r], 1.1, 0.5, 0.2) if pen else x[r], float(u[r]), **kw)
+            for r in check]
+    compare_ids([got[r] for r in check], [t for t, _ in want], [i for _, i in want], f"large k={k} {pen}")
+    assert set(paths) <= {1, 2} and paths.count(1) >= rows - 8, paths
