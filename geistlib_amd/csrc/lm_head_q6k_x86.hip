@@ -446,15 +446,27 @@ __device__ __forceinline__ void q6x_group_rows(const uint32_t (&z)[8], float ws0
  * fence that opens the step (an empty asm that loads may not pass and that needs the sums so
  * far: hoisted to the top of the block the rows' activations would not fit the scalar
  * registers). */
-template <int M, bool LANES>
+template <int M, bool LANES, bool SLICED>
 __global__ __launch_bounds__(Q6X_TPB, 4) void k_q6k_packed_gemm_x86(
     const uint32_t *__restrict__ packed, long n_out, int nb, const uint32_t *__restrict__ act,
-    float *__restrict__ y, long ld_y) {
+    float *__restrict__ y, long ld_y, int n_m, int slices) {
     typedef q8s_u8v u8v;
     constexpr int   G  = M < 4 ? M : 4;
     constexpr int NG = (M + G - 1) / G;
     const int     r  = threadIdx.x & 63;
-    const long    g  = (long) blockIdx.x * (Q6X_TPB / 64) + threadIdx.x / 64;
+    long wg = blockIdx.x;
+    if (SLICED) {
+        /* Slice i of a workgroup's table rows takes the activation rows from i M on (the last slice M
+         * rows that end with the batch's: what it shares with the one before comes out the same). The
+         * slices have ids that are equal modulo 8 and next to each other: one XCD, whose L2 has the
+         * table's rows for the later ones. */
+        const int slot = blockIdx.x >> 3, i = slot % slices;
+        const int m0   = i * M + M <= n_m ? i * M : n_m - M;
+        wg             = (long) (slot / slices) * 8 + (blockIdx.x & 7);
+        act += (long) m0 * ((long) nb * Q8K_ACT_DWORDS + Q8S_ACT_TAIL);
+        y += m0 * ld_y;
+    }
+    const long g = wg * (Q6X_TPB / 64) + threadIdx.x / 64;
     if (g * 64 >= n_out)
         return;
     const long row    = g * 64 + r;
@@ -612,17 +624,47 @@ void launch_rmsnorm_q8s_rows(hipStream_t stream, const float *x, long ld_x, cons
                                                                   act);
 }
 
+/* Activation rows that a workgroup takes of a batch of m over a table of `groups` x 64 rows. A wavefront
+ * owns 64 table rows and goes through their blocks in order, so a table of few rows leaves the device's
+ * 1024 SIMDs a wavefront each or none, and every wait of its is exposed: several workgroups then share
+ * the same table rows and take a slice of the batch each, which unpacks the rows once per slice but
+ * has more wavefronts in flight and shorter chains. Projection and tail of 8 rows, us, whole / slices
+ * of 4 / of 2 (of 1): 33000 x 1536 73.5 / 40.2 / 36.2 (44.5), 43680 x 3072 140 / 68.2 / 64.8 (93), 59584 x
+ * 1024 53.3 / 32.4 / 34.3, 105176 x 2816 134 / 97.7 / 117, 150000 x 1536 80.0 / 71.9 / 93, 262144 x 1536 90.2 /
+ * 112; of 5 rows 43680 x 3072 108 / 66.6 / 60.4, 150000 x 1536 65.2 / 69.8; of 4 rows 59584 x 1024 28.4 / - /
+ * 25.4, 92224 x 1024 30.2 / - / 30.7; of 2 rows 59584 x 1024 26.1 / - / - (23.7), 92224 x 1024 26.6 (28.2).
+ * Hence limits on the wavefronts that slicing makes. */
+static int q6x_rows_per_slice(long groups, int m) {
+    auto waves = [&](int rows) { return groups * ((m + rows - 1) / rows); };
+    if (m > 1 && m <= 3 && waves(1) <= 2000)
+        return 1;
+    if (m > 2 && waves(2) <= 2800)
+        return 2;
+    if (m > 4 && waves(4) <= (m > 6 ? 6000 : 4096))
+        return 4;
+    return m;
+}
+
 template <int M>
 static void q6x_gemm_launch(hipStream_t stream, const void *table, bool packed, long n_out, int nb,
                             const uint32_t *act, bool lanes, float *y, long ld_y) {
     if (packed) {
         const uint32_t *p      = static_cast<const uint32_t *>(table);
         const long      groups = (n_out + 63) / 64;
-        const dim3      grid((unsigned) ((groups + 3) / 4)), block(Q6X_TPB);
-        if (lanes)
-            k_q6k_packed_gemm_x86<M, true><<<grid, block, 0, stream>>>(p, n_out, nb, act, y, ld_y);
+        const int  rows_wg = q6x_rows_per_slice(groups, M), slices = (M + rows_wg - 1) / rows_wg;
+        const long wgs     = (groups + 3) / 4;
+        const dim3 grid((unsigned) (slices > 1 ? (wgs + 7) / 8 * 8 * slices : wgs)), block(Q6X_TPB);
+        auto       go = [&](auto kernel) {
+            kernel<<<grid, block, 0, stream>>>(p, n_out, nb, act, y, ld_y, M, slices);
+        };
+        if (slices == 1)
+            lanes ? go(k_q6k_packed_gemm_x86<M, true, false>) : go(k_q6k_packed_gemm_x86<M, false, false>);
+        else if (rows_wg == 4)
+            lanes ? go(k_q6k_packed_gemm_x86<4, true, true>) : go(k_q6k_packed_gemm_x86<4, false, true>);
+        else if (rows_wg == 2)
+            lanes ? go(k_q6k_packed_gemm_x86<2, true, true>) : go(k_q6k_packed_gemm_x86<2, false, true>);
         else
-            k_q6k_packed_gemm_x86<M, false><<<grid, block, 0, stream>>>(p, n_out, nb, act, y, ld_y);
+            lanes ? go(k_q6k_packed_gemm_x86<1, true, true>) : go(k_q6k_packed_gemm_x86<1, false, true>);
     } else {
         const uint8_t *p = static_cast<const uint8_t *>(table);
         const dim3     grid((unsigned) ((n_out + Q6X_TPB - 1) / Q6X_TPB)), block(Q6X_TPB);

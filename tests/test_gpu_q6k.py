@@ -317,3 +317,26 @@ def test_head_over_the_gemma_table_with_the_soft_cap(host, oracle):
             want = oracle.finalize_batch(sess, logits, softcap=cap).tolist()
             assert list(out) == want, (T, p, top_k, k)
         host.geist_hip_head_destroy(h)
+
+
+@pytest.mark.parametrize("groups", [40, 666, 667, 700, 934, 1000, 1001, 1400, 2048, 2049, 3001])
+@pytest.mark.parametrize("ragged", [0, 5])
+def test_q6k_batch_in_slices_equals_the_whole(hs, groups, ragged):
+    """Tables of few rows: workgroups that share table rows take a slice of the batch each (the last
+    two may overlap). The kernel over the table as it lies in the file takes the batch whole; both give
+    the same bits, on either side of every limit, for tables of whole eights and not."""
+    g = np.random.default_rng(groups + ragged)
+    n_out, n_in = groups * 64 - ragged, 256
+    w = torch.from_numpy(g.integers(0, 256, (n_out, 210), dtype=np.uint8)).cuda()
+    w[:, 208], w[:, 209] = 0x6D, 0x0C
+    packed = torch.zeros((hs.q6k_packed_bytes(n_out, n_in),), dtype=torch.uint8, device="cuda")
+    hs.q6k_pack(w, n_in, packed)
+    for m in range(2, 9):
+        x = torch.from_numpy((g.standard_normal((m, n_in)) * 3).astype(np.float32)).cuda()
+        a = torch.full((m, n_out), 7.0, dtype=torch.float32, device="cuda")
+        b = torch.full((m + 1, n_out), 7.0, dtype=torch.float32, device="cuda")
+        hs.q6k_linear_x86(w, n_in, x, a)
+        hs.q6k_packed_linear_x86(packed, n_out, n_in, x, b[:m])
+        hs.sync()
+        assert torch.equal(a.view(torch.int32), b[:m].view(torch.int32)), (groups, ragged, m)
+        assert (b[m] == 7.0).all()                    # nothing beyond the batch
