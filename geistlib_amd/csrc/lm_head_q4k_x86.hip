@@ -29,6 +29,7 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 namespace gs {
 
@@ -157,11 +158,11 @@ __device__ __forceinline__ void q4x_load(const uint32_t *__restrict__ base, int 
     k.dd    = __builtin_nontemporal_load(base + 2304 + r);
 }
 
-/* M activation rows share a pass over the table (1 or 2, and 8 with PAIRS). PAIRS: the binary32
- * accumulators are joined once per pair of sub-blocks (the reference's 16 x 16 AVX-512 tiles,
- * kernel_q4kx8_gemm_avx512_full.c:94, 729-778) instead of once per super-block. */
-template <int M, bool PAIRS>
-__global__ __launch_bounds__(Q4X_TPB, PAIRS && M > 2 ? 3 : 4) void k_q4k_packed_gemv_x86(
+/* M activation rows share a pass over the table, and the binary32 accumulators are joined once per pair
+ * of sub-blocks (the reference's 16 x 16 AVX-512 tiles, kernel_q4kx8_gemm_avx512_full.c:94, 729-778)
+ * instead of once per super-block. */
+template <int M>
+__global__ __launch_bounds__(Q4X_TPB, 3) void k_q4k_packed_gemv_x86_pairs(
     const uint32_t *__restrict__ packed, long n_out, int nb, const uint32_t *__restrict__ act,
     float *__restrict__ y, long ld_y) {
     const int  r = threadIdx.x & 63;
@@ -205,7 +206,7 @@ __global__ __launch_bounds__(Q4X_TPB, PAIRS && M > 2 ? 3 : 4) void k_q4k_packed_
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 im += __mul24((int) ((cur.mn[j >> 2] >> (8 * (j & 3))) & 0xffu), (int) bs[j]);
-                if (PAIRS ? (j & 1) : j == 7) {
+                if (j & 1) {
                     acc_min[m] = __builtin_fmaf((float) im, dm, acc_min[m]);
                     im         = 0;
                 }
@@ -218,26 +219,22 @@ __global__ __launch_bounds__(Q4X_TPB, PAIRS && M > 2 ? 3 : 4) void k_q4k_packed_
         u8v           avc[G], avn[G];
         uint32_t      even[4], odd[4];
         int           sc = 0;
-        if (M > 1) {
 #pragma unroll
-            for (int i = 0; i < G; ++i)
-                avc[i] = *reinterpret_cast<const u8v *>(a + i * act_ld);
-        }
+        for (int i = 0; i < G; ++i)
+            avc[i] = *reinterpret_cast<const u8v *>(a + i * act_ld);
 #pragma unroll
         for (int st = 0; st < 8 * NG; ++st) {
             const int j = st / NG, grp = st % NG; /* sub-block j: elements 32 j .. 32 j + 31 */
-            if (M > 1) {
-                if (st + 1 < 8 * NG) {
-                    const int jn = (st + 1) / NG, gn = (st + 1) % NG;
+            if (st + 1 < 8 * NG) {
+                const int jn = (st + 1) / NG, gn = (st + 1) % NG;
 #pragma unroll
-                    for (int i = 0; i < G; ++i)
-                        if (gn * G + i < M)
-                            avn[i] = *reinterpret_cast<const u8v *>(a + (gn * G + i) * act_ld + 8 * jn);
-                }
-#pragma unroll
-                for (int i = 0; i < M; ++i)
-                    asm volatile("" : "+v"(iacc[i])::"memory");
+                for (int i = 0; i < G; ++i)
+                    if (gn * G + i < M)
+                        avn[i] = *reinterpret_cast<const u8v *>(a + (gn * G + i) * act_ld + 8 * jn);
             }
+#pragma unroll
+            for (int i = 0; i < M; ++i)
+                asm volatile("" : "+v"(iacc[i])::"memory");
             if (grp == 0) {
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
@@ -251,7 +248,7 @@ __global__ __launch_bounds__(Q4X_TPB, PAIRS && M > 2 ? 3 : 4) void k_q4k_packed_
                 const int m = grp * G + i;
                 if (m >= M)
                     continue;
-                const u8v av  = M > 1 ? avc[i] : *reinterpret_cast<const u8v *>(a + 8 * j);
+                const u8v av  = avc[i];
                 int       dot = 0;
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
@@ -259,21 +256,14 @@ __global__ __launch_bounds__(Q4X_TPB, PAIRS && M > 2 ? 3 : 4) void k_q4k_packed_
                     dot = __builtin_amdgcn_sdot4((int) odd[k], (int) av[2 * k + 1], dot, false);
                 }
                 iacc[m] += __mul24(sc, dot);
-                if (PAIRS && (j & 1)) {
+                if (j & 1) {
                     acc[m]  = __builtin_fmaf((float) iacc[m], __fmul_rn(d, d_a[m]), acc[m]);
                     iacc[m] = 0;
                 }
             }
-            if (M > 1) {
 #pragma unroll
-                for (int i = 0; i < G; ++i)
-                    avc[i] = avn[i];
-            }
-        }
-        if (!PAIRS) {
-#pragma unroll
-            for (int m = 0; m < M; ++m)
-                acc[m] = __builtin_fmaf((float) iacc[m], __fmul_rn(d, d_a[m]), acc[m]);
+            for (int i = 0; i < G; ++i)
+                avc[i] = avn[i];
         }
         if (b + 1 < nb)
             cur = nxt;
@@ -282,6 +272,104 @@ __global__ __launch_bounds__(Q4X_TPB, PAIRS && M > 2 ? 3 : 4) void k_q4k_packed_
 #pragma unroll
         for (int m = 0; m < M; ++m)
             y[m * ld_y + row] = __fsub_rn(acc[m], acc_min[m]);
+    }
+}
+
+constexpr int q4x_split_dwords(int m) { return (2 * m + 1) * 64; } /* LDS per block */
+constexpr int Q4X_SPLIT_BLOCKS = 32; /* of batches: what 64 KB of LDS hold of three rows */
+/* One to three activation rows: the four wavefronts of a workgroup share 64 table rows and take every fourth block
+ * each; the blocks' integers, exact whoever forms them, go through LDS, and the binary32 steps over the
+ * blocks, which have an order, are then two chains, one to a wavefront. (With 64 table rows to a
+ * wavefront, which works through their blocks one after the other, norm, projection and greedy draw of
+ * 43680 x 3072 took 31.2 us, 24.2 so, 68320 x 2048 27.4 / 24.0, 150552 x 2304 46.7 / 41.8, 262144 x 1536
+ * 47.4 / 45.5, 100000 x 6144 67.1 / 68.5.) */
+template <int M>
+__global__ __launch_bounds__(Q4X_TPB, 4) void k_q4k_packed_gemv_x86(
+    const uint32_t *__restrict__ packed, long n_out, int nb, const uint32_t *__restrict__ act,
+    float *__restrict__ y, long ld_y) {
+    constexpr int W = Q4X_TPB / 64, PART = q4x_split_dwords(M);
+    extern __shared__ __align__(16) uint32_t s_part[]; /* [nb]: I and M per row of the batch, the scales */
+    __shared__ float s_min[M][64];
+    static_assert(W % 2 == 0, "a wavefront's chains are of one kind");
+    const int       r = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const long      row    = (long) blockIdx.x * 64 + r;
+    const uint32_t *base   = packed + (long) blockIdx.x * nb * Q4X_PACK_DWORDS;
+    const long      act_ld = (long) nb * Q4X_ACT_DWORDS + Q4X_ACT_TAIL;
+    Q4xBlock        cur, nxt;
+    if (wv < nb)
+        q4x_load(base + (long) wv * Q4X_PACK_DWORDS, r, cur);
+    for (int b = wv; b < nb; b += W) {
+        if (b + W < nb)
+            q4x_load(base + (long) (b + W) * Q4X_PACK_DWORDS, r, nxt);
+        const uint32_t *a = act + (long) b * Q4X_ACT_DWORDS; /* uniform: scalar loads */
+        typedef uint32_t u8v __attribute__((ext_vector_type(8)));
+        int       im[M], iacc[M];
+        u8v       bs[M];
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            im[m] = 0, iacc[m] = 0;
+            bs[m] = *reinterpret_cast<const u8v *>(a + m * act_ld + 64);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int mn = (int) ((cur.mn[j >> 2] >> (8 * (j & 3))) & 0xffu);
+            const int sc = (int) ((cur.sc[j >> 2] >> (8 * (j & 3))) & 0xffu);
+            uint32_t  even[4], odd[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t w = cur.q[4 * j + k];
+                even[k] = w & 0x0f0f0f0fu, odd[k] = (w >> 4) & 0x0f0f0f0fu;
+            }
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                im[m] += __mul24(mn, (int) bs[m][j]);
+                const u8v av  = *reinterpret_cast<const u8v *>(a + m * act_ld + 8 * j);
+                int       dot = 0;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    dot = __builtin_amdgcn_sdot4((int) even[k], (int) av[2 * k], dot, false);
+                    dot = __builtin_amdgcn_sdot4((int) odd[k], (int) av[2 * k + 1], dot, false);
+                }
+                iacc[m] += __mul24(sc, dot);
+            }
+        }
+        uint32_t *out = s_part + b * PART + r;
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            out[(2 * m) * 64]     = __float_as_uint((float) iacc[m]);
+            out[(2 * m + 1) * 64] = __float_as_uint((float) im[m]);
+        }
+        out[2 * M * 64] = cur.dd;
+        if (b + W < nb)
+            cur = nxt;
+    }
+    __syncthreads();
+    /* chain 2 m: I and d of row m, chain 2 m + 1: M and dmin; wavefront w has chains w and w + W */
+    const int kind = wv & 1;
+    float     acc[(2 * M + W - 1) / W];
+#pragma unroll
+    for (int i = 0; i < (2 * M + W - 1) / W; ++i) {
+        const int c = wv + i * W, m = c >> 1;
+        acc[i] = 0.0f;
+        if (c >= 2 * M)
+            continue;
+        const float d_a = __uint_as_float(act[m * act_ld + (long) nb * Q4X_ACT_DWORDS]);
+#pragma unroll 4
+        for (int b = 0; b < nb; ++b) {
+            const uint32_t *in = s_part + b * PART + r;
+            const uint32_t  dd = in[2 * M * 64];
+            const float d = __half2float(__ushort_as_half((unsigned short) (kind ? dd >> 16 : dd & 0xffffu)));
+            acc[i] = __builtin_fmaf(__uint_as_float(in[64 * c]), __fmul_rn(d, d_a), acc[i]);
+        }
+        if (kind)
+            s_min[m][r] = acc[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < (2 * M + W - 1) / W; ++i) {
+        const int m = (wv + i * W) >> 1;
+        if (m < M && !kind && row < n_out)
+            y[m * ld_y + row] = __fsub_rn(acc[i], s_min[m][r]);
     }
 }
 
@@ -433,16 +521,25 @@ void launch_q4k_packed_gemv_q8k(hipStream_t stream, const void *packed, long n_o
     const int       nb = n_in / 256;
     const long      groups = (n_out + 63) / 64;
     const dim3      grid((unsigned) ((groups + 3) / 4)), block(Q4X_TPB);
-    /* One row leaves the matrix cores 15/16 idle and the vector kernel streams at the same rate; two
-     * rows of at most six super-blocks, 48.9 us by it and 50.2 by the matrix cores (262144 x 1536),
-     * of ten 48.8 and 45.6 (128256 x 2560), of sixteen 57.5 and 36.5. pairs: a tile of sixteen
-     * rows' order of accumulation, which comes in eights. */
+    auto split = [&](auto m) {
+        constexpr int M = decltype(m)::value;
+        k_q4k_packed_gemv_x86<M>
+            <<<dim3((unsigned) groups), block, (size_t) nb * q4x_split_dwords(M) * sizeof(uint32_t), stream>>>(
+                p, n_out, nb, act, y, ld_y);
+    };
+    /* Up to three rows leave the matrix cores idle for the most part and the vector kernel streams at the
+     * same rate or a better one: norm, projection and greedy draw, us, by it / by the matrix cores, 2 rows
+     * 33000 x 1024 14.6 / 17.0, 43680 x 3072 25.2 / 28.5, 262144 x 1536 47.6 / 50.5; 3 rows 15.4 / 17.3,
+     * 27.2 / 28.7, 49.3 / 51.9, 64048 x 1536 22.0 / 21.5; 4 rows 36736 x 2304 24.9 / 24.7, 124296 x 1536
+     * 34.8 / 31.3. pairs: a tile of sixteen rows' order of accumulation, which comes in eights. */
     if (pairs)
-        k_q4k_packed_gemv_x86<Q4X_M_MAX, true><<<grid, block, 0, stream>>>(p, n_out, nb, act, y, ld_y);
-    else if (n_m == 1)
-        k_q4k_packed_gemv_x86<1, false><<<grid, block, 0, stream>>>(p, n_out, nb, act, y, ld_y);
-    else if (n_m == 2 && nb <= 6)
-        k_q4k_packed_gemv_x86<2, false><<<grid, block, 0, stream>>>(p, n_out, nb, act, y, ld_y);
+        k_q4k_packed_gemv_x86_pairs<Q4X_M_MAX><<<grid, block, 0, stream>>>(p, n_out, nb, act, y, ld_y);
+    else if (n_m == 1) /* (at most 64 blocks: what the reference's kernel takes) */
+        split(std::integral_constant<int, 1>{});
+    else if (n_m == 2 && nb <= Q4X_SPLIT_BLOCKS)
+        split(std::integral_constant<int, 2>{});
+    else if (n_m == 3 && nb <= Q4X_SPLIT_BLOCKS)
+        split(std::integral_constant<int, 3>{});
     else
         k_q4k_packed_linear_x86_mfma<2, 4><<<dim3((unsigned) ((groups + 1) / 2)), block, 0, stream>>>(
             p, n_out, nb, act, n_m, y, ld_y);

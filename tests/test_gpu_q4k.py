@@ -290,3 +290,28 @@ def test_head_over_a_q4k_table_with_a_soft_cap(host, oracle):
             want = oracle.finalize_batch(sess, logits, softcap=cap).tolist()
             assert list(out) == want, (T, p, top_k, k, portable)
         host.geist_hip_head_destroy(h)
+
+
+@pytest.mark.parametrize("n_in", [256, 512, 768, 1024, 1280, 4096, 8192, 8448, 16384])
+@pytest.mark.parametrize("n_out", [8, 72, 1032])
+def test_q4k_rows_whose_blocks_are_shared_out(hs, oracle, n_out, n_in):
+    """One to three rows, whose super-blocks the wavefronts of a workgroup share: fewer blocks than
+    wavefronts, remainders, and on either side of what a batch's workgroup holds. One row against the
+    oracle, batches against their rows one by one, bit for bit."""
+    g = np.random.default_rng(n_out + n_in)
+    w = random_q4k_table(g, n_out, n_in)
+    packed = packed_copy(hs, w, n_in)
+    x = (g.standard_normal((3, n_in)) * 2).astype(np.float32)
+    d_x = torch.from_numpy(x).cuda()
+    one = torch.full((3, n_out), np.nan, dtype=torch.float32, device="cuda")
+    for m in range(3):
+        hs.q4k_packed_gemv_x86(packed, n_out, n_in, d_x[m:m + 1], one[m:m + 1])
+    hs.sync()
+    want = oracle_q4k_gemv_x86(oracle.lib, w, x[0], n_in)
+    assert np.array_equal(one[0].cpu().numpy().view(np.uint32), want.view(np.uint32))
+    for m in (2, 3):
+        y = torch.full((m + 1, n_out), 7.0, dtype=torch.float32, device="cuda")
+        hs.q4k_packed_linear_x86(packed, n_out, n_in, d_x[:m], y[:m])
+        hs.sync()
+        assert torch.equal(y[:m].view(torch.int32), one[:m].view(torch.int32)), (n_out, n_in, m)
+        assert (y[m] == 7.0).all()
