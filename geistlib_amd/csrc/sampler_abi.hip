@@ -931,7 +931,11 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
                    rows->rows * small_chunks * small_chunks <= (size_t) WIN_SMALL_READS;
     /* (a shallower min-p still makes a list that holds for most rows; the others have histograms) */
     f.minp_listed = rs.use_m && zb_m < ZBINS - 1 && !f.minp_direct && !f.win_locate;
-    if (f.win_locate) {
+    const bool minp_small = f.minp_direct && small_chunks <= (size_t) s->max_chunks &&
+                            small_chunks <= (size_t) MAX_CHUNKS &&
+                            rows->rows * small_chunks <=
+                                (size_t) (L.rv.softcap > 0.0f ? MINP_SMALL_CAPPED : MINP_SMALL);
+    if (f.win_locate || minp_small) {
         L.nv           = 2;
         L.rv.per_chunk = 2048;
         L.rv.n_chunks  = (int) small_chunks;

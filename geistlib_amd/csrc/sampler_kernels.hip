@@ -205,7 +205,8 @@ __device__ __forceinline__ uint64_t wave_first_of(const float4 (&v)[NV], uint32_
 
 /* Where the thread maxima and the chunk results go, and the slots through which the workgroups
  * of a row meet. */
-constexpr uint32_t SCAN_STAGE = 2048; /* candidates a workgroup stages in LDS */
+/* candidates a workgroup stages in LDS: a quarter of a chunk of 8192, half of one of 2048 */
+template <int NV> constexpr uint32_t SCAN_STAGE = NV == 8 ? 2048 : 1024;
 struct FusedScan {
     float    *tmax;
     uint64_t *chunk_best;
@@ -515,7 +516,7 @@ __device__ __forceinline__ void expsum_chunk(const RowView &rv, int row, int chu
                     if (c == 0 ? c0 : c == 1 ? c1 : c == 2 ? c2 : c3) {
                         const uint32_t at = __hip_atomic_fetch_add(
                             s_nstage, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                        if (at < SCAN_STAGE)
+                        if (at < SCAN_STAGE<NV>)
                             s_stage[at] = make_uint2(__float_as_uint(args[c]), (uint32_t) (e + c));
                     }
                 }
@@ -616,14 +617,14 @@ __device__ __forceinline__ void expsum_chunk(const RowView &rv, int row, int chu
         if (wave_arrives_last(fs.s_arrive + 2)) {
             const int      lane  = tid & (WAVE - 1);
             const uint32_t n     = *s_nstage;
-            const uint32_t total = n > SCAN_STAGE ? (uint32_t) CAND_CAP + 1u : n;
+            const uint32_t total = n > SCAN_STAGE<NV> ? (uint32_t) CAND_CAP + 1u : n;
             int            at    = 0;
             if (lane == 0 && total)
                 at = atomicAdd(&list.count[(long) row * CAND_COUNT_STRIDE], (int) total);
             at = __builtin_amdgcn_readfirstlane(at);
             uint32_t *ck = list.key + (long) row * CAND_ROW;
             uint32_t *ci = list.idx + (long) row * CAND_ROW;
-            for (uint32_t i = lane; i < n && i < SCAN_STAGE; i += WAVE) {
+            for (uint32_t i = lane; i < n && i < SCAN_STAGE<NV>; i += WAVE) {
                 const uint2 t = s_stage[i];
                 if (at + (int) i < CAND_CAP) {
                     ck[at + i] = t.x;
@@ -655,11 +656,10 @@ __global__ __launch_bounds__(TPB, (NV == 8 && PEN && LISTM) ? 6 : 1) void k_scan
     __shared__ uint64_t s_tab[32];
     __shared__ uint64_t s_red[NWAVES], s_bb;
     __shared__ uint32_t s_arrive[5];
-    /* the staging list of the candidates: in the history's count table when there is one */
-    __shared__ uint2 s_stage_own[(LISTM && !PEN) ? SCAN_STAGE : 1];
-    static_assert(!(LISTM && PEN) || sizeof(s_cnt16) >= SCAN_STAGE * sizeof(uint2),
-                  "the count table holds the staging list");
-    uint2 *s_stage = PEN ? reinterpret_cast<uint2 *>(s_cnt16) : s_stage_own;
+    /* the staging list of the candidates: in the history's count table when that is as large */
+    constexpr bool   STAGE_IN_CNT = PEN && sizeof(s_cnt16) >= SCAN_STAGE<NV> * sizeof(uint2);
+    __shared__ uint2 s_stage_own[(LISTM && !STAGE_IN_CNT) ? SCAN_STAGE<NV> : 1];
+    uint2 *s_stage = STAGE_IN_CNT ? reinterpret_cast<uint2 *>(s_cnt16) : s_stage_own;
     /* the table the slab sums are transposed through: the history's count table has the size
      * and is free once the row's workgroups have met */
     __shared__ __align__(16) double s_tr_own[(SLABS && NV == 8 && !PEN) ? NWAVES * 8 * WAVE : 1];
@@ -1924,11 +1924,11 @@ int launch_scan_expsum(const Launch &L, float inv_t, float *tmax, uint64_t *chun
                 L.rv, inv_t, chunk_best, chunk_sum, nullptr, probe_token, probe_L, probe_p);
         return 0;
     }
-    if (list && L.nv == 8) {
-        if (L.pen)
-            fast ? go(k_scan_expsum<8, true, true, false, true>) : go(k_scan_expsum<8, true, true, false>);
-        else
-            fast ? go(k_scan_expsum<8, false, true, false, true>) : go(k_scan_expsum<8, false, true, false>);
+    if (list) {
+        dispatch(L.nv, L.pen, [&](auto nv, auto pen) {
+            fast ? go(k_scan_expsum<GS_NV, GS_PEN, true, false, true>)
+                 : go(k_scan_expsum<GS_NV, GS_PEN, true, false>);
+        });
         return 0;
     }
     dispatch(L.nv, L.pen, [&](auto nv, auto pen) {
@@ -2325,9 +2325,12 @@ void launch_candidates(const Launch &L, const FinalLaunch &f, float *probs, long
         static const uint64_t tab[32] = GEIST_EXPF_TABLE_INIT;
         const int             zb      = zbin_of_min_p(f.min_p);
         const float p_out = geist_expf_glibc_le0(-(float) (zb + 1) / (float) ZBIN_PER_NAT, tab);
+        RowView rv   = L.rv; /* (a walk's own chunks are of 8192, whatever the pass's) */
+        rv.per_chunk = 8192;
+        rv.n_chunks  = (rv.n_vocab + 8191) / 8192;
         auto go = [&](auto kernel) {
             kernel<<<dim3(L.rows), block, dyn, L.stream>>>(
-                L.rv, g, f.cand, f.top_p, f.min_p, f.uniforms, f.row_flag, f.out, f.chunk_sum,
+                rv, g, f.cand, f.top_p, f.min_p, f.uniforms, f.row_flag, f.out, f.chunk_sum,
                 L.rv.n_chunks, p_out, f.minp_direct ? 0 : 1, defer, wc.hint, wc.call);
         };
         L.pen ? go(k_sorted_candidates<true>) : go(k_sorted_candidates<false>);
