@@ -2225,10 +2225,12 @@ int geist_hip_spec_verify(geist_hip_sampler *s, const float *d_target, size_t ld
     sp.verdict    = s->verdict;
     sp.out_tokens = d_out_tokens;
     sp.n_accepted = d_n_accepted;
-    /* the residual pass and the draw in one launch while its workgroups, at the two per compute
+    /* the residual pass and the draw in one launch while its workgroups, at the number per compute
      * unit their registers allow, run in one round; past that the two kernels are the lighter */
-    if (!greedy && s->spec_one_launch &&
-        n_seq * (size_t) La.rv.n_chunks <= (size_t) gs::SPEC_ONE_LAUNCH_WGS_PER_CU * (size_t) s->cu_count) {
+    const size_t one_round =
+        (size_t) (La.nv == 2 ? gs::SPEC_ONE_LAUNCH_WGS_PER_CU_2 : gs::SPEC_ONE_LAUNCH_WGS_PER_CU) *
+        (size_t) s->cu_count;
+    if (!greedy && s->spec_one_launch && n_seq * (size_t) La.rv.n_chunks <= one_round) {
         Launch per_seq = La;
         per_seq.rows   = (int) n_seq;
         const MeetSpace m = meet_space(s, per_seq);

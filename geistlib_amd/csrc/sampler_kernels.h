@@ -315,7 +315,13 @@ constexpr int SPEC_VERDICT_BYTES = 24;
 /* meet != NULL (stochastic verification only): the residual sums and the draw in one launch (the
  * workgroups of a sequence wait for one another); NULL: two launches */
 void launch_spec(const Launch &L, const SpecLaunch &sp, const MeetSpace *meet = nullptr);
-constexpr int SPEC_ONE_LAUNCH_WGS_PER_CU = 2; /* what the one-launch kernel's 171 registers allow */
+/* workgroups of the one-launch kernel per compute unit, by what its registers allow: 146 with
+ * chunks of 8192, 78 with chunks of 2048. Chunks of 2048, one launch / two launches:
+ * 13 sequences x 1 draft x 98432 (637 workgroups) 19.8 / 21.2 us, 28 x 2 x 36992 (532) 19.6 / 21.4,
+ * 20 x 1 x 90000 (900) 19.2 / 20.4, at T 0.8 0.4 to 1.2 us less. Four is also the most that
+ * chunks of 2048 make of a verification on 256 compute units */
+constexpr int SPEC_ONE_LAUNCH_WGS_PER_CU   = 2;
+constexpr int SPEC_ONE_LAUNCH_WGS_PER_CU_2 = 4;
 /* chunk_best may be NULL when only the thread maxima are wanted */
 void launch_tmax_scan(const Launch &L, float *tmax, uint64_t *chunk_best,
                       int32_t *zero_per_row = nullptr);

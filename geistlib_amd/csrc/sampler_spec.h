@@ -16,7 +16,7 @@
  *                  count (spec_accept_seq), then the sum of max(0, p - q) over its chunk of row j*
  *   k_spec_final   grid (n_seq): draws the last token
  *   k_spec_resid_draw  grid (chunks, n_seq): the two above in one launch, for batches of up to
- *                  two workgroups per compute unit; the chunks of a sequence meet for their
+ *                  two workgroups per compute unit (four with chunks of 2048); the chunks of a sequence meet for their
  *                  residual sums and the one in whose chunk the draw falls walks it from registers
  *   k_spec_accept  grid (n_seq): the verdicts alone, for the greedy mode (no residual)
  */

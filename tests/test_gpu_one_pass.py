@@ -176,6 +176,13 @@ def test_spec_verify_one_launch_and_two_launches_agree(hs, oracle, n_seq, L, n, 
         assert nacc[1] == L and nacc[2] == 0
 
 
+@pytest.mark.parametrize("n_seq,L,n", [(13, 1, 98432), (31, 1, 65536), (32, 1, 65536)])
+def test_spec_verify_up_to_four_short_chunks_per_compute_unit(hs, oracle, n_seq, L, n):
+    """Chunks of 2048: more than two workgroups per compute unit, the most that such chunks are
+    used for (992 workgroups), and one sequence more (chunks of 8192)."""
+    test_spec_verify_one_launch_and_two_launches_agree(hs, oracle, n_seq, L, n, 0.9)
+
+
 @pytest.mark.parametrize("pen", [False, True])
 def test_min_p_lists_of_every_size(hs, oracle, pen):
     """The exp-sum pass stages a chunk's min-p candidates in LDS (2048 places per chunk): rows whose
