@@ -687,16 +687,13 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
     f.tmax       = s->tmax;
     f.out        = d_out;
 
-    if (!rs.greedy && !rs.use_k && !(s->meet && s->meet->slots[0] && s->meet->slots[1]))
+    if ((rs.greedy || !rs.use_k) && !(s->meet && s->meet->slots[0] && s->meet->slots[1]))
         return fail(s, GEIST_HIP_E_INTERNAL, "no meeting slots for the one-pass kernel");
     if (rs.greedy) {
         L.rv.stream_loads = s->logits_streamed;
-        *stream_kernel    = "k_tmax_scan";
+        *stream_kernel    = "k_greedy";
         if (do_stream)
-            launch_tmax_scan(L, s->tmax, s->chunk_best);
-        f.mode = FINAL_ARGMAX;
-        if (do_tail)
-            launch_row_final(L, f);
+            launch_greedy(L, d_out, meet_space(s, L, 1, (L.rows & 7) == 0));
         return after_launch(s, "argmax");
     }
     if (rs.use_k) {

@@ -33,7 +33,7 @@ constexpr size_t WIDE_LOGITS = (size_t) 1 << 24;
 constexpr int TOPK_MAX       = 8192; /* the reference caps top_k here (sampler.c:213-215) */
 constexpr int HISTORY_MAX    = 65535;
 
-enum { FINAL_ARGMAX = 0, FINAL_TEMPERATURE = 1, FINAL_TOPK = 2, FINAL_SORTED = 3 };
+enum { FINAL_TEMPERATURE = 1, FINAL_TOPK = 2, FINAL_SORTED = 3 };
 
 /* One batch of logit rows as the kernels see it, with the transform applied while reading. */
 struct RowView {
@@ -322,6 +322,8 @@ void launch_spec(const Launch &L, const SpecLaunch &sp, const MeetSpace *meet = 
  * chunks of 2048 make of a verification on 256 compute units */
 constexpr int SPEC_ONE_LAUNCH_WGS_PER_CU   = 2;
 constexpr int SPEC_ONE_LAUNCH_WGS_PER_CU_2 = 4;
+/* argmax of every row in one launch (sampler_greedy.h); meet: a word per (row, chunk) */
+void launch_greedy(const Launch &L, int32_t *out, const MeetSpace &meet);
 /* chunk_best may be NULL when only the thread maxima are wanted */
 void launch_tmax_scan(const Launch &L, float *tmax, uint64_t *chunk_best,
                       int32_t *zero_per_row = nullptr);

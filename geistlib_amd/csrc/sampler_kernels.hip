@@ -2,16 +2,18 @@
  * sampler_kernels.hip -- the HIP kernels of the token-sampling path (gfx950).
  *
  * Kernel map (reference lines the arithmetic follows are cited at each kernel):
+ *   k_greedy (sampler_greedy.h)   argmax                                       sampler.c:52-62
  *   k_tmax_scan      per-thread maxima (the single pass of the top-k path) and,
  *                    on request, the per-chunk maximum with its first index       sampler.c:52-62, 202-207
  *   k_scan_expsum    the one pass of the modes that weigh every element: per (row, chunk) the
  *                    maxima as above and the sum of expf((l - max) * inv_t); on request the
  *                    sums of the chunk's slabs, or the min-p candidates of the row
  *                                                                              sampler.c:52-62, 77-83
- *   k_final_argmax / _temperature / _topk / _sorted   per-row combine of each mode: argmax,
+ *   k_final_temperature / _topk / _sorted   per-row combine of each mode:
  *                    index-order CDF draw, top-k select + sorted softmax + top-p + min-p +
  *                    draw, top-p / min-p shortcut                             sampler.c:90-102, 209-222, 272-299
- *   k_topk_general   top-k for k above 128 and degenerate rows                 sampler.c:178-228
+ *   k_topk_wide (sampler_topk_wide.h)   top-k for large k and large batches    sampler.c:178-228
+ *   k_topk_general   top-k of the rows that the paths above hand back          sampler.c:178-228
  *   k_cand_scan, k_final_cand (sampler_cands.h)   the top-k path for plain rows: the scan hands
  *                    each wavefront's leading groups on, the row-final kernel gathers nothing
  *                                                                              sampler.c:178-228
@@ -1225,7 +1227,7 @@ __device__ __forceinline__ int topk_row_general(const RowView &rv, int row, int 
 }
 
 struct FinalArgs {
-    int   mode; /* FINAL_ARGMAX, FINAL_TEMPERATURE, FINAL_TOPK */
+    int   mode; /* FINAL_TEMPERATURE, FINAL_TOPK, FINAL_SORTED */
     int   k;
     int   k_sel; /* rank of the thread maximum used as the bound (>= k) */
     float inv_t;
@@ -1504,25 +1506,12 @@ __device__ __forceinline__ bool topk_from_tmax(const RowView &rv, const FinalArg
 #include "sampler_cands.h"
 #include "sampler_cands_one_launch.h"
 #include "sampler_topk_wide.h"
+#include "sampler_greedy.h"
 namespace gs {
 
 /* ============================================================================================
  * Row-final kernels: one workgroup per row, one kernel per sampling mode.
  * ========================================================================================== */
-
-/* argmax: sampler.c:52-62 */
-__global__ __launch_bounds__(TPB) void k_final_argmax(RowView rv, FinalArgs a) {
-    __shared__ uint64_t s_red[NWAVES];
-    const int           row = blockIdx.x;
-    const uint64_t      b   = row_best_from_chunks(a.chunk_best, row, rv.n_chunks, s_red);
-    if (threadIdx.x == 0) {
-        const float first = rv.logits[(long) row * rv.ld];
-        /* a NaN at index 0 is never displaced by the strict '>' of the reference; after the
-         * transforms it stays NaN, so the raw value decides (unless token 0 is forbidden) */
-        const bool nan0 = first != first && (!rv.allowed || allowed_at(rv, row, 0));
-        a.out[row]      = nan0 ? 0 : (int32_t) best_idx(b);
-    }
-}
 
 /* temperature: sampler.c:90-102 over all n in index order: locate the chunk from the per-chunk
  * sums, then scan that chunk. */
@@ -2035,6 +2024,13 @@ void launch_tmax_scan(const Launch &L, float *tmax, uint64_t *chunk_best, int32_
     });
 }
 
+void launch_greedy(const Launch &L, int32_t *out, const MeetSpace &meet) {
+    const dim3 grid(L.rv.n_chunks, L.rows), block(TPB);
+    dispatch(L.nv, L.pen, [&](auto nv, auto pen) {
+        k_greedy<GS_NV, GS_PEN><<<grid, block, 0, L.stream>>>(L.rv, out, meet);
+    });
+}
+
 static FinalArgs final_args(const FinalLaunch &f) {
     FinalArgs a;
     a.mode       = f.mode;
@@ -2200,10 +2196,6 @@ int probe_workgroup_placement(hipStream_t stream, bool *same_xcd) {
 void launch_row_final(const Launch &L, const FinalLaunch &f) {
     const FinalArgs a = final_args(f);
     const dim3 grid(L.rows), block(TPB);
-    if (f.mode == FINAL_ARGMAX) {
-        k_final_argmax<<<grid, block, 0, L.stream>>>(L.rv, a);
-        return;
-    }
     if (f.mode == FINAL_SORTED) { /* (rows in chunks of 8192: smaller batches have no such launch) */
         if (L.pen)
             k_final_sorted<true><<<grid, block, 0, L.stream>>>(L.rv, a);
