@@ -827,21 +827,30 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
     if (!rs.use_p && !rs.use_m) {
         Launch scan          = L;
         scan.rv.stream_loads = s->logits_streamed; /* the one pass over the rows */
-        if (scan.nv == 2 && (size_t) scan.rows * (size_t) scan.rv.n_chunks <= 256) {
-            /* A few rows: the step is a chain of waits, not of bytes, and a second launch is a
-             * tenth of it. Scan, sums and the draw in one kernel (10.9 against 11.8 us for one
-             * row of 128256, 12.0 against 12.7 for four; from 16 rows on the two kernels are the
-             * faster form, their workgroups being smaller and gone sooner). The measuring
-             * stages cannot split it: the streaming stage is the whole step. */
-            *stream_kernel = "k_temperature_draw";
+        /* Chunks of 2048: the step is a chain of waits, not of bytes, and a second launch is a part
+         * of it. Scan, sums and the draw in one kernel, whose workgroups all wait for the sums
+         * (`few`) or only the one that draws. All of them, the rows each on an XCD of its own, for up
+         * to 256 workgroups whose rows an XCD's 32 compute units hold at two to three each: 1 x
+         * 32000 6.2 us against 7.5 with one that draws, 1 x 128256 7.2 / 8.5, 8 x 64000 6.8 / 8.0,
+         * 3 x 131072 7.3 / 8.3, 1 x 151936 (75 chunks) 8.6 / 8.6 and with penalties 10.3 / 10.9,
+         * 1 x 170000 (84) 8.5 / 8.8, but 1 x 200000 10.5 / 8.9, 1 x 262144 13.0 / 8.7 and with
+         * penalties 16.5 / 10.5. One that draws against two
+         * launches: 5 x 128256 9.7 / 12.9 us, 8 x 128256 8.2 / 9.6, 31 x 131072 18.3 / 19.8. (In
+         * chunks of 8192 the one that draws needs 150 registers, and the whole pass the half of
+         * its wavefronts: 64 x 128256 34 against 18.9.) The tolerance mode's sums are another
+         * kernel's. The measuring stages cannot split it: the streaming stage is the whole step. */
+        const size_t wgs = (size_t) scan.rows * (size_t) scan.rv.n_chunks;
+        const bool   few = scan.nv == 2 && wgs <= 256 && scan.rv.n_chunks <= 84;
+        if (few || (scan.nv == 2 && (!s->fast_sums || wgs <= 256))) {
+            *stream_kernel    = "k_temperature_draw";
             RowGenerators gen = {};
-            if (own_rng)
+            if (few ? own_rng : per_row)
                 gen = RowGenerators{rng.states, reinterpret_cast<uint32_t *>(s->row_arrive)};
             else
                 draws();
             if (do_stream)
                 launch_temperature_draw(scan, rs.inv_t, d_uniforms, gen, d_out,
-                                        meet_space(s, scan, 2, true));
+                                        meet_space(s, scan, 2, few || (scan.rows & 7) == 0), !few);
             return after_launch(s, "temperature");
         }
         draws_by(scan);

@@ -11,6 +11,12 @@
  * registers it still holds. Results are those of the two-kernel form bit for bit: the sums are
  * formed in the same order (chunk_slab_totals), the walk is the same code (sampler_walk.h).
  *
+ * COLLECT, for more workgroups: only the workgroup of the row's last chunk waits for the sums; the
+ * others report theirs and leave. It works the place out for the row and, unless the draw falls
+ * in its own chunk, reads the located chunk again and forms its weights and slab sums as the
+ * workgroup that summed it did. 8 x 128256 9.6 -> 8.2 us, 24 x 50257 12.0 -> 10.3, 5 x 128256 with
+ * the rows' own generators 12.9 -> 9.7, 1 x 262144 13.4 -> 8.7 (all chunks waiting on one XCD).
+ *
  * The waits are bounded like the first meet's. A workgroup that gives up a wait forms what it
  * is missing itself, from the row: the maximum as before, the other chunks' sums by running
  * the same summation over each of them (all workgroups that do so get the same bits, so they
@@ -143,7 +149,7 @@ __device__ __forceinline__ void row_sums_meet(uint64_t *row_slots, int chunk, in
     __syncthreads();
 }
 
-template <int NV, bool PEN, bool RNG, bool PLAIN>
+template <int NV, bool PEN, bool RNG, bool COLLECT, bool PLAIN>
 __device__ __forceinline__ void draw_chunk(const RowView &rv, int row, int chunk, int n_rows,
                                            int base, int end, float inv_t,
                                            const float *__restrict__ uniforms,
@@ -158,9 +164,10 @@ __device__ __forceinline__ void draw_chunk(const RowView &rv, int row, int chunk
     /* the row's draw, for the first wavefront: given, or the next of the row's generator */
     float    u_row = 0.0f;
     uint64_t state = 0;
+    const bool collects = !COLLECT || chunk == C - 1;
     if (!RNG)
         u_row = uniforms[row];
-    else if (tid < WAVE)
+    else if (tid < WAVE && collects)
         state = __hip_atomic_load(rng.states + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     HistPrefetch pf;
     if (PEN)
@@ -224,12 +231,18 @@ __device__ __forceinline__ void draw_chunk(const RowView &rv, int row, int chunk
      * row's other chunks for theirs */
     chunk_slab_totals<NV>(v, mx, inv_t, s_tab, s_tr, s_sum);
     const bool last2 = wave_arrives_last(fs.s_arrive + 1);
-    if (last2 && (tid & (WAVE - 1)) == 0)
+    if (last2 && (tid & (WAVE - 1)) == 0) {
         sh.total = combine_slab_totals<NV>(s_sum, sh.slab);
+        if (!collects) /* the slot's word as row_sums_meet writes it */
+            meet_store(sum_slots + (long) row * C + chunk,
+                       (uint64_t) __double_as_longlong(sh.total) + 1u, fs.local);
+    }
+    if (!collects)
+        return;
     /* (the reporter's lane 0 wrote sh.total: its own LDS write, read back in order) */
     row_sums_meet(sum_slots + (long) row * C, chunk, C, last2 ? sh.total : 0.0, last2, met_max,
                   fs.wait_limit, sh, fs.local);
-    const bool from_registers = sh.have_sums != 0;
+    bool from_registers = sh.have_sums != 0;
     if (!from_registers) {
         /* not met: every other chunk's sum by this workgroup, with the same summation */
         if (tid == 0)
@@ -256,7 +269,9 @@ __device__ __forceinline__ void draw_chunk(const RowView &rv, int row, int chunk
      * meetings, whose polls would wait for its answer. */
     uint32_t counted = 0;
     if (tid < WAVE) {
-        if (RNG) {
+        if (RNG && COLLECT) {
+            u_row = xorshift_unit(state);
+        } else if (RNG) {
             uint32_t most = (uint32_t) (C - 1);
             /* counted when the state has arrived, which is waited for here and not before */
             asm volatile("" : "+v"(most), "+v"(state));
@@ -283,10 +298,33 @@ __device__ __forceinline__ void draw_chunk(const RowView &rv, int row, int chunk
         }
     }
     __syncthreads();
-    if (RNG && tid == 0 && counted == (uint32_t) (C - 1))
+    if (RNG && tid == 0 && (COLLECT || counted == (uint32_t) (C - 1)))
         rng.states[row] = state;
-    if (sh.walk.chunk != chunk)
-        return; /* another workgroup's */
+    if (sh.walk.chunk != chunk) {
+        if (!COLLECT)
+            return; /* another workgroup's */
+        /* the located chunk again, its weights into the registers and its slab sums as the
+         * workgroup that summed it formed them */
+        chunk = sh.walk.chunk;
+        chunk_bounds<NV>(rv, chunk, base, end);
+        fetch_chunk<NV, PEN>(rv, row, n_rows, base, end, s_cnt16, v);
+        __syncthreads(); /* the count table and the table of the sums share their memory */
+        chunk_slab_totals<NV>(v, mx, inv_t, s_tab, s_tr, s_sum);
+        __syncthreads();
+        if (tid == 0)
+            combine_slab_totals<NV>(s_sum, sh.slab);
+        __syncthreads();
+        if (tid < WAVE) {
+            double    run = sh.walk.before;
+            const int js  = walk_locate_slab<NV>(sh.slab, sh.walk.target, &run);
+            if (tid == 0) {
+                sh.walk.slab   = js;
+                sh.walk.before = run;
+            }
+        }
+        __syncthreads();
+        from_registers = true;
+    }
     const double target = sh.walk.target;
     double       carry  = sh.walk.before;
     const int    js     = __builtin_amdgcn_readfirstlane(sh.walk.slab);
@@ -321,9 +359,9 @@ __device__ __forceinline__ void draw_chunk(const RowView &rv, int row, int chunk
         out[row] = tok;
 }
 
-/* RNG: the draws come from the rows' generators, else from `uniforms`. (As a run-time choice it cost
+/* COLLECT: see above. RNG: the draws come from the rows' generators, else from `uniforms`. (As a run-time choice it cost
  * calls with given draws 0.2-0.3 us: one row of 32000 with penalties 6.98 -> 7.17, two 6.96 -> 7.29.) */
-template <int NV, bool PEN, bool RNG>
+template <int NV, bool PEN, bool RNG, bool COLLECT>
 __global__ __launch_bounds__(TPB) void k_temperature_draw(RowView rv, int n_rows, float inv_t,
                                                           const float *__restrict__ uniforms,
                                                           RowGenerators rng,
@@ -365,10 +403,10 @@ __global__ __launch_bounds__(TPB) void k_temperature_draw(RowView rv, int n_rows
     const bool plain = rv.vec_ok && end - base == NV * TPB * 4 && !(rv.softcap > 0.0f) &&
                        rv.allowed == nullptr;
     if (plain)
-        draw_chunk<NV, PEN, RNG, true>(rv, row, chunk, n_rows, base, end, inv_t, uniforms, rng, out,
+        draw_chunk<NV, PEN, RNG, COLLECT, true>(rv, row, chunk, n_rows, base, end, inv_t, uniforms, rng, out,
                                   sum_slots, s_cnt16, s_sum, s_tab, tabv, s_tr, s_draw, fs);
     else
-        draw_chunk<NV, PEN, RNG, false>(rv, row, chunk, n_rows, base, end, inv_t, uniforms, rng, out,
+        draw_chunk<NV, PEN, RNG, COLLECT, false>(rv, row, chunk, n_rows, base, end, inv_t, uniforms, rng, out,
                                    sum_slots, s_cnt16, s_sum, s_tab, tabv, s_tr, s_draw, fs);
 }
 

@@ -276,7 +276,8 @@ int launch_scan_expsum(const Launch &L, float inv_t, float *tmax, uint64_t *chun
                        bool fast = false, float *hist = nullptr, int hist_bins = 0);
 /* The temperature draw in one kernel (sampler_draw.h): out[row] = the id drawn with
  * uniforms[row]. For L.nv == 2. `meet.slots` holds 2 * rows * n_chunks zeroed words: the
- * workgroups of a row meet twice. */
+ * workgroups of a row meet twice, the second time all of them or, with `collect`, the last chunk's
+ * alone (which then also reads and advances the row's generator alone). */
 /* The rows' generators, when a kernel takes its draws from them itself: states[row] is read by the
  * row's workgroups and advanced by the last of them; arrive: a zeroed counter per row, ARRIVE_STRIDE_INTS
  * apart, left zeroed. states == NULL: the draws are in `uniforms`. */
@@ -285,7 +286,7 @@ struct RowGenerators {
     uint32_t *arrive;
 };
 void launch_temperature_draw(const Launch &L, float inv_t, const float *uniforms,
-                             const RowGenerators &rng, int32_t *out, const MeetSpace &meet);
+                             const RowGenerators &rng, int32_t *out, const MeetSpace &meet, bool collect);
 /* last z bin that can hold an entry passing min_p (with slack); ZBINS - 1 when min_p is off or
  * that deep */
 int zbin_of_min_p(float min_p);

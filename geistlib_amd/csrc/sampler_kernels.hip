@@ -1920,10 +1920,12 @@ int launch_scan_expsum(const Launch &L, float inv_t, float *tmax, uint64_t *chun
         });
         return 0;
     }
+    if (slab_sum && !fast && L.nv != 8) /* (k_temperature_draw's) */
+        return 1;
     dispatch(L.nv, L.pen, [&](auto nv, auto pen) {
         if (slab_sum)
             fast ? go(k_scan_expsum<GS_NV, GS_PEN, false, true, true>)
-                 : go(k_scan_expsum<GS_NV, GS_PEN, false, true>);
+                 : go(k_scan_expsum<8, GS_PEN, false, true>);
         else
             fast ? go(k_scan_expsum<GS_NV, GS_PEN, false, false, true>)
                  : go(k_scan_expsum<GS_NV, GS_PEN, false, false>);
@@ -1957,18 +1959,32 @@ int zbin_of_min_p(float min_p) {
 }
 
 void launch_temperature_draw(const Launch &L, float inv_t, const float *uniforms,
-                             const RowGenerators &rng, int32_t *out, const MeetSpace &meet) {
-    /* for launches of a few rows: the geometry of 2048 elements per workgroup only. Rows in
-     * eights, so that the workgroups of a row have linear ids equal modulo 8 and share an XCD
-     * (xcd_row_chunk); the workgroups of the rows that are not there leave at once. */
-    const dim3 grid(L.rv.n_chunks, (L.rows + 7) & ~7), block(TPB);
-    auto go = [&](auto kernel) {
+                             const RowGenerators &rng, int32_t *out, const MeetSpace &meet,
+                             bool collect) {
+    /* the geometry of 2048 elements per workgroup only */
+    const dim3 block(TPB);
+    auto       go = [&](auto kernel, dim3 grid) {
         kernel<<<grid, block, 0, L.stream>>>(L.rv, L.rows, inv_t, uniforms, rng, out, meet);
     };
+    if (collect) {
+        const dim3 grid(L.rv.n_chunks, L.rows);
+        if (rng.states != nullptr)
+            L.pen ? go(k_temperature_draw<2, true, true, true>, grid)
+                  : go(k_temperature_draw<2, false, true, true>, grid);
+        else
+            L.pen ? go(k_temperature_draw<2, true, false, true>, grid)
+                  : go(k_temperature_draw<2, false, false, true>, grid);
+        return;
+    }
+    /* for launches of a few rows: rows in eights, so that the workgroups of a row have linear ids equal modulo 8 and share an XCD
+     * (xcd_row_chunk); the workgroups of the rows that are not there leave at once. */
+    const dim3 grid(L.rv.n_chunks, (L.rows + 7) & ~7);
     if (rng.states != nullptr)
-        L.pen ? go(k_temperature_draw<2, true, true>) : go(k_temperature_draw<2, false, true>);
+        L.pen ? go(k_temperature_draw<2, true, true, false>, grid)
+              : go(k_temperature_draw<2, false, true, false>, grid);
     else
-        L.pen ? go(k_temperature_draw<2, true, false>) : go(k_temperature_draw<2, false, false>);
+        L.pen ? go(k_temperature_draw<2, true, false, false>, grid)
+              : go(k_temperature_draw<2, false, false, false>, grid);
 }
 
 void launch_spec(const Launch &L, const SpecLaunch &sp, const MeetSpace *meet) {

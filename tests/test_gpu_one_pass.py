@@ -268,3 +268,52 @@ def test_temperature_draw_in_one_kernel(hs, oracle, rows, n, pen, extra, wait_li
             res.append(oracle.chain_u(row, float(u[r]), temperature=T))
         near = compare_ids(got, [t for t, _ in res], [i for _, i in res], f"call {call}")
         assert near <= 1
+
+
+@pytest.mark.parametrize("wait_limit", [None, 0, 3])
+@pytest.mark.parametrize("rows,n,pen,extra", [
+    (4, 131073, False, ""),          # 260 workgroups: the first batch large enough
+    (24, 32000, True, ""),           # rows in eights, each on an XCD
+    (5, 122901, True, "mask"),       # ragged rows
+    (9, 60000, False, "softcap"),
+    (6, 100000, False, "nan"),
+    (31, 16385, False, ""),          # short rows in a batch: 279 workgroups
+])
+def test_temperature_draw_by_the_last_chunk(hs, oracle, rows, n, pen, extra, wait_limit):
+    """Larger batches and longer rows in chunks of 2048: the workgroup of the last chunk draws,
+    and reads the located chunk again unless it is its own."""
+    test_temperature_draw_in_one_kernel(hs, oracle, rows, n, pen, extra, wait_limit)
+
+
+@pytest.mark.parametrize("n", [172032, 172033])      # 84 chunks, and one element in the 85th
+def test_temperature_draw_of_a_long_row(oracle, n):
+    from geistlib_amd import HipSampler
+    s = HipSampler(max_rows=1, max_vocab=n)
+    try:
+        for limit in (None, 0):
+            test_temperature_draw_in_one_kernel(s, oracle, 1, n, True, "", limit)
+    finally:
+        s.close()
+
+
+def test_last_chunk_draws_with_the_rows_generators(hs, oracle):
+    """The generators advance by one draw a call and row, on calls in a row."""
+    from geistlib_amd import HipSampler
+    from geistlib_amd.workloads import xorshift_units
+    rows, n, T, calls = 9, 70001, 0.9, 3
+    g = np.random.default_rng(5)
+    x = (g.standard_normal((rows, n)) * 2).astype(np.float32)
+    seeds = np.arange(1, rows + 1, dtype=np.uint64) * np.uint64(7919)
+    d = to_dev(x, torch)
+    r = HipSampler.rows(d)
+    states = torch.from_numpy(seeds.view(np.int64)).cuda()
+    out = torch.full((rows,), -7, dtype=torch.int32, device="cuda")
+    draws = [xorshift_units(int(s), calls) for s in seeds]
+    for call in range(calls):
+        hs.sample_rng(r, P(temperature=T), states, False, out)
+        hs.sync()
+        res = [oracle.chain_u(x[i], float(draws[i][0][call]), temperature=T) for i in range(rows)]
+        near = compare_ids(out.cpu().numpy(), [t for t, _ in res], [i for _, i in res], f"call {call}")
+        assert near <= 1
+    after = states.cpu().numpy().view(np.uint64)
+    assert [int(s) for s in after] == [d[1] for d in draws]
