@@ -829,19 +829,37 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
         scan.rv.stream_loads = s->logits_streamed; /* the one pass over the rows */
         /* Chunks of 2048: the step is a chain of waits, not of bytes, and a second launch is a part
          * of it. Scan, sums and the draw in one kernel, whose workgroups all wait for the sums
-         * (`few`) or only the one that draws. All of them, the rows each on an XCD of its own, for up
-         * to 256 workgroups whose rows an XCD's 32 compute units hold at two to three each: 1 x
-         * 32000 6.2 us against 7.5 with one that draws, 1 x 128256 7.2 / 8.5, 8 x 64000 6.8 / 8.0,
-         * 3 x 131072 7.3 / 8.3, 1 x 151936 (75 chunks) 8.6 / 8.6 and with penalties 10.3 / 10.9,
-         * 1 x 170000 (84) 8.5 / 8.8, but 1 x 200000 10.5 / 8.9, 1 x 262144 13.0 / 8.7 and with
-         * penalties 16.5 / 10.5. One that draws against two
-         * launches: 5 x 128256 9.7 / 12.9 us, 8 x 128256 8.2 / 9.6, 31 x 131072 18.3 / 19.8. (In
-         * chunks of 8192 the one that draws needs 150 registers, and the whole pass the half of
-         * its wavefronts: 64 x 128256 34 against 18.9.) The tolerance mode's sums are another
-         * kernel's. The measuring stages cannot split it: the streaming stage is the whole step. */
-        const size_t wgs = (size_t) scan.rows * (size_t) scan.rv.n_chunks;
-        const bool   few = scan.nv == 2 && wgs <= 256 && scan.rv.n_chunks <= 84;
-        if (few || (scan.nv == 2 && (!s->fast_sums || wgs <= 256))) {
+         * (`few`) or only the one that draws.
+         *   few: the rows each on an XCD of its own, up to 256 workgroups whose rows an XCD's 32
+         * compute units hold at two to three each. 1 x 32000 6.2 us against 7.5 with one that
+         * draws, 1 x 128256 7.2 / 8.5, 8 x 64000 6.8 / 8.0, 3 x 131072 7.3 / 8.3, 1 x 151936 (75 chunks)
+         * 8.6 / 8.6 and with penalties 10.3 / 10.9, 1 x 170000 (84) 8.5 / 8.8, but 1 x 200000 10.5 /
+         * 8.9, 1 x 262144 13.0 / 8.7 and with penalties 16.5 / 10.5.
+         *   One that draws against two launches: 5 x 128256 9.7 / 12.9 us, 8 x 128256 8.2 / 9.6, 24 x
+         * 128256 12.9 / 15.8; but each row has one that draws, and many short rows are better off
+         * with two launches: 64 x 32000 10.8 / 10.9, 72 x 32000 11.6 / 11.2, 96 x 32000 13.5 / 12.1
+         * (72 x 40000 12.0 / 12.7).
+         *   What does not start at once (1536 workgroups with penalties, 2048 without, whose last
+         * quarter has no time left to hide in) goes to chunks of 8192 and two launches, unless those
+         * end in an eighth of a chunk: 13 x 262144 15.1 us / one that draws 17.3 / two launches in
+         * chunks of 2048 17.9, 31 x 131072 14.9 / 17.7 / 19.7, 24 x 151936 with penalties 16.9 / 20.3 /
+         * 22.0, 120 x 32000 14.3 / 15.5 / 14.5; 72 x 50257 (six chunks and 1105) 16.6 / 15.1 / 17.8.
+         * Short rows from somewhat later on: 80 x 40000 (1600) 14.0 / 12.6 / 12.9, 100 x 32000 (1600)
+         * 14.6 / 14.6 / 14.0.
+         * (In chunks of 8192 the one that draws needs 150 registers, and the whole pass half of its
+         * wavefronts: 64 x 128256 34 against 18.9.)
+         *   The tolerance mode's sums are another kernel's. The measuring stages cannot split the
+         * one launch: the streaming stage is the whole step. */
+        const size_t big = (rows->n_vocab + 8191) / 8192, wgs = rows->rows * (size_t) scan.rv.n_chunks;
+        const bool   short_rows = rows->rows > 64 && scan.rv.n_chunks < 20;
+        if (scan.nv == 2 && !s->fast_sums && wgs > (scan.rv.n_chunks < 32 ? 1792 : 1536) &&
+            big * 8192 * 10 <= rows->n_vocab * 11) {
+            scan.nv = L.nv = 8;
+            scan.rv.per_chunk = L.rv.per_chunk = 8192;
+            scan.rv.n_chunks = L.rv.n_chunks = (int) big;
+        }
+        const bool few = scan.nv == 2 && wgs <= 256 && scan.rv.n_chunks <= 84;
+        if (few || (scan.nv == 2 && (s->fast_sums ? wgs <= 256 : !short_rows))) {
             *stream_kernel    = "k_temperature_draw";
             RowGenerators gen = {};
             if (few ? own_rng : per_row)

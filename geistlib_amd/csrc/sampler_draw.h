@@ -360,9 +360,12 @@ __device__ __forceinline__ void draw_chunk(const RowView &rv, int row, int chunk
 }
 
 /* COLLECT: see above. RNG: the draws come from the rows' generators, else from `uniforms`. (As a run-time choice it cost
- * calls with given draws 0.2-0.3 us: one row of 32000 with penalties 6.98 -> 7.17, two 6.96 -> 7.29.) */
+ * calls with given draws 0.2-0.3 us: one row of 32000 with penalties 6.98 -> 7.17, two 6.96 -> 7.29.) 
+ * COLLECT without penalties needs 65 registers when left alone; held to 64 an eighth workgroup shares
+ * a compute unit (100 x 32000 16.3 -> 14.6 us, 100 x 40000 16.5 -> 15.3), 16 bytes of scratch in the
+ * row's last workgroup. */
 template <int NV, bool PEN, bool RNG, bool COLLECT>
-__global__ __launch_bounds__(TPB) void k_temperature_draw(RowView rv, int n_rows, float inv_t,
+__global__ __launch_bounds__(TPB, COLLECT && !PEN ? 8 : 1) void k_temperature_draw(RowView rv, int n_rows, float inv_t,
                                                           const float *__restrict__ uniforms,
                                                           RowGenerators rng,
                                                           int32_t *__restrict__ out,

@@ -1920,12 +1920,10 @@ int launch_scan_expsum(const Launch &L, float inv_t, float *tmax, uint64_t *chun
         });
         return 0;
     }
-    if (slab_sum && !fast && L.nv != 8) /* (k_temperature_draw's) */
-        return 1;
     dispatch(L.nv, L.pen, [&](auto nv, auto pen) {
         if (slab_sum)
             fast ? go(k_scan_expsum<GS_NV, GS_PEN, false, true, true>)
-                 : go(k_scan_expsum<8, GS_PEN, false, true>);
+                 : go(k_scan_expsum<GS_NV, GS_PEN, false, true>);
         else
             fast ? go(k_scan_expsum<GS_NV, GS_PEN, false, false, true>)
                  : go(k_scan_expsum<GS_NV, GS_PEN, false, false>);

@@ -278,6 +278,10 @@ def test_temperature_draw_in_one_kernel(hs, oracle, rows, n, pen, extra, wait_li
     (9, 60000, False, "softcap"),
     (6, 100000, False, "nan"),
     (31, 16385, False, ""),          # short rows in a batch: 279 workgroups
+    (80, 32000, False, ""),          # many short rows: two launches
+    (24, 131072, False, ""),         # 1536 workgroups
+    (25, 131072, True, ""),          # more: chunks of 8192, two launches
+    (72, 50257, False, ""),          # more, but an eighth of a chunk at the end
 ])
 def test_temperature_draw_by_the_last_chunk(hs, oracle, rows, n, pen, extra, wait_limit):
     """Larger batches and longer rows in chunks of 2048: the workgroup of the last chunk draws,
