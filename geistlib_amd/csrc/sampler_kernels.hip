@@ -13,7 +13,7 @@
  *                    index-order CDF draw, top-k select + sorted softmax + top-p + min-p +
  *                    draw, top-p / min-p shortcut                             sampler.c:90-102, 209-222, 272-299
  *   k_topk_wide (sampler_topk_wide.h)   top-k for large k and large batches    sampler.c:178-228
- *   k_topk_general   top-k of the rows that the paths above hand back          sampler.c:178-228
+ *   k_topk_general   top-k for a k beyond the wide path's, and degenerate rows  sampler.c:178-228
  *   k_cand_scan, k_final_cand (sampler_cands.h)   the top-k path for plain rows: the scan hands
  *                    each wavefront's leading groups on, the row-final kernel gathers nothing
  *                                                                              sampler.c:178-228
