@@ -160,7 +160,8 @@ int geist_hip_sample_rows_static(int device, void *stream, const struct geist_hi
 
 /* No counterpart in the reference. The modes that need a row's maximum before they can sum its
  * exponentials (temperature, top-p, min-p, softmax, speculative verification) read the rows
- * once: the workgroups that share a row wait for one another inside the kernel. `polls` bounds
+ * once: the workgroups that share a row wait for one another inside the kernel; for an argmax and
+ * for larger temperature draws one of them waits for what the others report. `polls` bounds
  * that wait (default 65536 polls, tens of milliseconds); a workgroup that reaches the bound
  * finds the row's maximum by reading the row itself, so the results never depend on it. 0 makes
  * every workgroup do that at once, which is slow and meant for tests of that path. */
@@ -236,7 +237,8 @@ int geist_hip_sampler_set_sums(geist_hip_sampler *s, int mode);
 /* No counterpart in the reference. Stochastic speculative verification sums the residual
  * max(0, p - q) and draws from it in one launch (the workgroups of a sequence wait for one
  * another's sums, the wait bounded by geist_hip_sampler_set_wait_limit) when sequences x chunks
- * of 8192 logits is at most two per compute unit (512 on an MI355X), one round of that kernel's
+ * of 8192 logits is at most two per compute unit (512 on an MI355X; small batches: chunks of 2048, four per
+ * compute unit), one round of that kernel's
  * workgroups; otherwise, and with enable = 0, in two launches. Results are the same either way. Returns 1 when the one-launch
  * form is in use for batches that qualify, 0 when not, negative on error. */
 int geist_hip_sampler_one_launch_spec(geist_hip_sampler *s, int enable);
