@@ -144,12 +144,15 @@ inline int    win_cap_for(size_t n) { return n / 8 > WIN_CAP_MIN ? (int) ((n / 8
  * 63 x 63 reads) 39.3 / 43.5; 8 x 262144 (8 x 128 x 128) 58 / 54, 48 x 100000 (2352 chunks) 48 / 21. */
 constexpr int WIN_SMALL       = 1024;
 constexpr int WIN_SMALL_READS = 65536;
-/* A min-p batch of up to so many chunks of 2048 is cut into those, larger ones into chunks of 8192:
+/* A min-p batch of up to so many chunks of 2048, and so many slots polled (every workgroup polls all of
+ * its row's), is cut into those, other ones into chunks of 8192:
  * 2 x 54912 14.2 us against 16.4, 46 x 45893 (1058 chunks) 19.0 / 21.4, 21 x 110528 (1134) 19.3 /
  * 18.7, 13 x 206875 (1326) 22.0 / 22.0, 100 x
- * 60000 (3000) 27.5 / 23.3. With a soft-cap, whose tanhf makes a chunk's arithmetic the longest step,
+ * 60000 (3000) 27.5 / 23.3; 8 x 151936 (8 x 75 x 75 polls) 15.8 / 16.8, 20 x 100000 (48020) 17.9 / 18.2, 12 x
+ * 128256 (47628) 17.3 / 17.0, 11 x 152960 (61875) 17.4 / 16.4, 16 x 128256 (63504) 16.8 / 15.8. With a soft-cap, whose tanhf makes a chunk's arithmetic the longest step,
  * 2 x 54912 19.5 / 35.4, 71 x 92992 (3266) 43.2 / 50.7, 64 x 128256 (4032) 53.7 / 51.1. */
 constexpr int MINP_SMALL        = 1088;
+constexpr int MINP_SMALL_POLLS  = 46080;
 constexpr int MINP_SMALL_CAPPED = 3400;
 struct WinSpace {
     float    *hist;  /* [rows][chunks][WIN_BINS], by the launch's chunks */

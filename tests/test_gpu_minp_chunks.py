@@ -11,7 +11,7 @@ torch = pytest.importorskip("torch")
 from gpu_util import compare_ids, run_rows  # noqa: E402
 
 
-@pytest.mark.parametrize("rows,n", [(1, 2047), (3, 2049), (2, 50257), (4, 130000), (17, 131072), (17, 131073),
+@pytest.mark.parametrize("rows,n", [(1, 2047), (3, 2049), (2, 50257), (4, 130000), (11, 131072), (11, 131073), (34, 65536), (34, 65537),
                                     (10, 262144)])
 @pytest.mark.parametrize("form", ["plain", "pen", "cap", "all"])
 def test_min_p_batches_in_either_chunks(oracle, rows, n, form):
