@@ -124,7 +124,8 @@ struct CandSpace {
     uint32_t *key;       /* [rows][CAND_CAP], rows CAND_ROW apart: bits of the softmax argument */
     uint32_t *idx;       /* ... vocabulary ids */
     int32_t  *count;     /* [rows * CAND_COUNT_STRIDE]: a row's counter has a cache line to itself
-                          * (the appending wavefronts' atomic adds to one line serialise) */
+                          * (the appending wavefronts' atomic adds to one line serialise); behind it
+                          * the word of its crowded chunks of 2048, a bit for every 8192 ids */
     int32_t  *path;      /* [rows] which walk served the row, a RowPath */
 };
 

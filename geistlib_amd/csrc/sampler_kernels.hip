@@ -207,8 +207,11 @@ __device__ __forceinline__ uint64_t wave_first_of(const float4 (&v)[NV], uint32_
 
 /* Where the thread maxima and the chunk results go, and the slots through which the workgroups
  * of a row meet. */
-/* candidates a workgroup stages in LDS: a quarter of a chunk of 8192, half of one of 2048 */
-template <int NV> constexpr uint32_t SCAN_STAGE = NV == 8 ? 2048 : 1024;
+/* Candidates a workgroup stages in LDS: a quarter of a chunk of 8192, all of one of 2048. A chunk of 2048
+ * with more than SCAN_CROWDED of them is crowded; a second crowded one among the same 8192 ids sends the
+ * row to the whole-row walk, which it takes in chunks of 8192 too (together they overflow that chunk's
+ * places). One alone is listed, whatever its number. */
+constexpr uint32_t SCAN_STAGE = 2048, SCAN_CROWDED = SCAN_STAGE / 2;
 struct FusedScan {
     float    *tmax;
     uint64_t *chunk_best;
@@ -416,8 +419,10 @@ __device__ __forceinline__ void expsum_chunk(const RowView &rv, int row, int chu
         const uint32_t bk   = wave_max_u32(f2key(tm));
         uint64_t       best = wave_first_of<NV, PLAIN>(v, bk, base, end);
         uint32_t prior = 0;
-        if (LISTM && chunk == 0 && tid == 0) /* the list the second half appends to starts empty */
-            prior = (uint32_t) atomicExch(&list.count[(long) row * CAND_COUNT_STRIDE], 0);
+        if (LISTM && chunk == 0 && tid == 0) /* the list the second half appends to starts empty:
+                                              * its length and the word of the crowded chunks */
+            prior = (uint32_t) atomicExch(
+                reinterpret_cast<unsigned long long *>(&list.count[(long) row * CAND_COUNT_STRIDE]), 0ull);
         if ((tid & (WAVE - 1)) == 0) {
             /* `prior` an operand of the deposit: the exchange above has returned before this
              * wavefront arrives, so before the chunk's slot is stored */
@@ -518,7 +523,7 @@ __device__ __forceinline__ void expsum_chunk(const RowView &rv, int row, int chu
                     if (c == 0 ? c0 : c == 1 ? c1 : c == 2 ? c2 : c3) {
                         const uint32_t at = __hip_atomic_fetch_add(
                             s_nstage, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                        if (at < SCAN_STAGE<NV>)
+                        if (at < SCAN_STAGE)
                             s_stage[at] = make_uint2(__float_as_uint(args[c]), (uint32_t) (e + c));
                     }
                 }
@@ -614,19 +619,28 @@ __device__ __forceinline__ void expsum_chunk(const RowView &rv, int row, int chu
     if (LISTM) {
         /* the wavefront that arrives last moves the staged entries to the row's list: one add to
          * the row's counter per workgroup. A workgroup with more candidates than the staging
-         * list holds reports more than the row's list can hold, which sends the row to the
-         * whole-row walk. */
+         * list holds, or the second crowded one of its 8192 ids (SCAN_STAGE), reports more than
+         * the row's list can hold, which sends the row to the whole-row walk. */
         if (wave_arrives_last(fs.s_arrive + 2)) {
             const int      lane  = tid & (WAVE - 1);
             const uint32_t n     = *s_nstage;
-            const uint32_t total = n > SCAN_STAGE<NV> ? (uint32_t) CAND_CAP + 1u : n;
+            int32_t       *count = &list.count[(long) row * CAND_COUNT_STRIDE];
+            bool           over  = n > SCAN_STAGE;
             int            at    = 0;
-            if (lane == 0 && total)
-                at = atomicAdd(&list.count[(long) row * CAND_COUNT_STRIDE], (int) total);
+            if (NV == 2 && n > SCAN_CROWDED) { /* the bit of the 8192 ids, four chunks */
+                static_assert(MAX_CHUNKS / 4 <= 32, "a bit for every four chunks");
+                const uint32_t bit = 1u << (chunk >> 2);
+                uint32_t       had = 0;
+                if (lane == 0)
+                    had = (uint32_t) atomicOr(count + 1, (int) bit);
+                over = (had & bit) != 0u;
+            }
+            if (lane == 0 && n)
+                at = atomicAdd(count, over ? CAND_CAP + 1 : (int) n);
             at = __builtin_amdgcn_readfirstlane(at);
             uint32_t *ck = list.key + (long) row * CAND_ROW;
             uint32_t *ci = list.idx + (long) row * CAND_ROW;
-            for (uint32_t i = lane; i < n && i < SCAN_STAGE<NV>; i += WAVE) {
+            for (uint32_t i = lane; i < n && i < SCAN_STAGE; i += WAVE) {
                 const uint2 t = s_stage[i];
                 if (at + (int) i < CAND_CAP) {
                     ck[at + i] = t.x;
@@ -653,15 +667,16 @@ __global__ __launch_bounds__(TPB, (NV == 8 && PEN && LISTM) ? 6 : 1) void k_scan
                                                      float *__restrict__ hist, int hist_bins) {
     __shared__ __align__(16) uint32_t s_hist[HIST ? WIN_BINS : 4];
     static_assert(!HIST || (!SLABS && !NOMEET), "forms with a histogram");
-    __shared__ __align__(16) uint32_t s_cnt16[PEN ? NV * TPB * 2 : 1];
+    /* the staging list of the candidates shares the memory of the history's count table, which with
+     * chunks of 2048 is the smaller of the two */
+    __shared__ __align__(16) uint32_t s_cnt16[!PEN ? 1 : LISTM ? SCAN_STAGE * 2 : NV * TPB * 2];
     __shared__ double   s_sum[SLABS ? NWAVES * NV : NWAVES];
     __shared__ uint64_t s_tab[32];
     __shared__ uint64_t s_red[NWAVES], s_bb;
     __shared__ uint32_t s_arrive[5];
-    /* the staging list of the candidates: in the history's count table when that is as large */
-    constexpr bool   STAGE_IN_CNT = PEN && sizeof(s_cnt16) >= SCAN_STAGE<NV> * sizeof(uint2);
-    __shared__ uint2 s_stage_own[(LISTM && !STAGE_IN_CNT) ? SCAN_STAGE<NV> : 1];
-    uint2 *s_stage = STAGE_IN_CNT ? reinterpret_cast<uint2 *>(s_cnt16) : s_stage_own;
+    static_assert(SCAN_STAGE * sizeof(uint2) >= NV * TPB * 2 * sizeof(uint32_t), "room for the counts");
+    __shared__ uint2 s_stage_own[(LISTM && !PEN) ? SCAN_STAGE : 1];
+    uint2 *s_stage = PEN ? reinterpret_cast<uint2 *>(s_cnt16) : s_stage_own;
     /* the table the slab sums are transposed through: the history's count table has the size
      * and is free once the row's workgroups have met */
     __shared__ __align__(16) double s_tr_own[(SLABS && NV == 8 && !PEN) ? NWAVES * 8 * WAVE : 1];
