@@ -20,8 +20,9 @@
  * table row; a dword holds the 4-bit values of eight consecutive elements, one mask gives the
  * even ones as bytes and a shift and a mask the odd ones, and two v_dot4_i32_i8 multiply them
  * with the activations, which the quantiser lays out to match (per eight elements a dword of the
- * even ones and a dword of the odd ones) and which are scalar operands. Batches of decode rows go
- * to the matrix cores (k_q4k_packed_linear_x86_mfma).
+ * even ones and a dword of the odd ones) and which are scalar operands. Four wavefronts share 64 table
+ * rows' blocks for up to three activation rows; batches of four to eight go to the matrix cores
+ * (k_q4k_packed_linear_x86_mfma).
  */
 #include "lm_head_kernels.h"
 #include "rmsnorm_device.h"
@@ -158,11 +159,12 @@ __device__ __forceinline__ void q4x_load(const uint32_t *__restrict__ base, int 
     k.dd    = __builtin_nontemporal_load(base + 2304 + r);
 }
 
-/* M activation rows share a pass over the table, and the binary32 accumulators are joined once per pair
- * of sub-blocks (the reference's 16 x 16 AVX-512 tiles, kernel_q4kx8_gemm_avx512_full.c:94, 729-778)
- * instead of once per super-block. */
-template <int M>
-__global__ __launch_bounds__(Q4X_TPB, 3) void k_q4k_packed_gemv_x86_pairs(
+/* 64 table rows to a wavefront, which goes through their blocks in order; M activation rows share a pass
+ * over the table (1, and 8 with PAIRS). PAIRS: the binary32 accumulators are joined once per pair of
+ * sub-blocks (the reference's 16 x 16 AVX-512 tiles, kernel_q4kx8_gemm_avx512_full.c:94, 729-778) instead
+ * of once per super-block. */
+template <int M, bool PAIRS>
+__global__ __launch_bounds__(Q4X_TPB, PAIRS && M > 2 ? 3 : 4) void k_q4k_packed_gemv_x86_rows(
     const uint32_t *__restrict__ packed, long n_out, int nb, const uint32_t *__restrict__ act,
     float *__restrict__ y, long ld_y) {
     const int  r = threadIdx.x & 63;
@@ -206,7 +208,7 @@ __global__ __launch_bounds__(Q4X_TPB, 3) void k_q4k_packed_gemv_x86_pairs(
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 im += __mul24((int) ((cur.mn[j >> 2] >> (8 * (j & 3))) & 0xffu), (int) bs[j]);
-                if (j & 1) {
+                if (PAIRS ? (j & 1) : j == 7) {
                     acc_min[m] = __builtin_fmaf((float) im, dm, acc_min[m]);
                     im         = 0;
                 }
@@ -219,22 +221,26 @@ __global__ __launch_bounds__(Q4X_TPB, 3) void k_q4k_packed_gemv_x86_pairs(
         u8v           avc[G], avn[G];
         uint32_t      even[4], odd[4];
         int           sc = 0;
+        if (M > 1) {
 #pragma unroll
-        for (int i = 0; i < G; ++i)
-            avc[i] = *reinterpret_cast<const u8v *>(a + i * act_ld);
+            for (int i = 0; i < G; ++i)
+                avc[i] = *reinterpret_cast<const u8v *>(a + i * act_ld);
+        }
 #pragma unroll
         for (int st = 0; st < 8 * NG; ++st) {
             const int j = st / NG, grp = st % NG; /* sub-block j: elements 32 j .. 32 j + 31 */
-            if (st + 1 < 8 * NG) {
-                const int jn = (st + 1) / NG, gn = (st + 1) % NG;
+            if (M > 1) {
+                if (st + 1 < 8 * NG) {
+                    const int jn = (st + 1) / NG, gn = (st + 1) % NG;
 #pragma unroll
-                for (int i = 0; i < G; ++i)
-                    if (gn * G + i < M)
-                        avn[i] = *reinterpret_cast<const u8v *>(a + (gn * G + i) * act_ld + 8 * jn);
+                    for (int i = 0; i < G; ++i)
+                        if (gn * G + i < M)
+                            avn[i] = *reinterpret_cast<const u8v *>(a + (gn * G + i) * act_ld + 8 * jn);
+                }
+#pragma unroll
+                for (int i = 0; i < M; ++i)
+                    asm volatile("" : "+v"(iacc[i])::"memory");
             }
-#pragma unroll
-            for (int i = 0; i < M; ++i)
-                asm volatile("" : "+v"(iacc[i])::"memory");
             if (grp == 0) {
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
@@ -248,7 +254,7 @@ __global__ __launch_bounds__(Q4X_TPB, 3) void k_q4k_packed_gemv_x86_pairs(
                 const int m = grp * G + i;
                 if (m >= M)
                     continue;
-                const u8v av  = avc[i];
+                const u8v av  = M > 1 ? avc[i] : *reinterpret_cast<const u8v *>(a + 8 * j);
                 int       dot = 0;
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
@@ -256,14 +262,21 @@ __global__ __launch_bounds__(Q4X_TPB, 3) void k_q4k_packed_gemv_x86_pairs(
                     dot = __builtin_amdgcn_sdot4((int) odd[k], (int) av[2 * k + 1], dot, false);
                 }
                 iacc[m] += __mul24(sc, dot);
-                if (j & 1) {
+                if (PAIRS && (j & 1)) {
                     acc[m]  = __builtin_fmaf((float) iacc[m], __fmul_rn(d, d_a[m]), acc[m]);
                     iacc[m] = 0;
                 }
             }
+            if (M > 1) {
 #pragma unroll
-            for (int i = 0; i < G; ++i)
-                avc[i] = avn[i];
+                for (int i = 0; i < G; ++i)
+                    avc[i] = avn[i];
+            }
+        }
+        if (!PAIRS) {
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+                acc[m] = __builtin_fmaf((float) iacc[m], __fmul_rn(d, d_a[m]), acc[m]);
         }
         if (b + 1 < nb)
             cur = nxt;
@@ -282,7 +295,7 @@ constexpr int Q4X_SPLIT_BLOCKS = 32; /* of batches: what 64 KB of LDS hold of th
  * blocks, which have an order, are then two chains, one to a wavefront. (With 64 table rows to a
  * wavefront, which works through their blocks one after the other, norm, projection and greedy draw of
  * 43680 x 3072 took 31.2 us, 24.2 so, 68320 x 2048 27.4 / 24.0, 150552 x 2304 46.7 / 41.8, 262144 x 1536
- * 47.4 / 45.5, 100000 x 6144 67.1 / 68.5.) */
+ * 47.4 / 45.5, 32000 x 8192 60.4 / 36.6, 256000 x 8192 194 / 191; where it loses: q4x_whole_rows.) */
 template <int M>
 __global__ __launch_bounds__(Q4X_TPB, 4) void k_q4k_packed_gemv_x86(
     const uint32_t *__restrict__ packed, long n_out, int nb, const uint32_t *__restrict__ act,
@@ -515,6 +528,18 @@ void launch_rmsnorm_q8k_row_rows(hipStream_t stream, const float *x, long ld_x, 
                                                                       ties_even, act);
 }
 
+/* Whether one activation row takes k_q4k_packed_gemv_x86_rows. The form that shares the blocks has a
+ * workgroup per 64 table rows, four at a time on each of 256 compute units: just past 1536 (and 1792)
+ * a few compute units have a seventh (eighth) to wait for, while the other form's wavefronts, two to a SIMD
+ * up to 2048, run at once. Shared / not, us: 24 blocks 116500 (1821 workgroups) 75.2 / 73.9, 28 blocks 100500
+ * (1571) 77.8 / 76.7, 48 blocks 100500 127.3 / 122.4, 108000 (1688) 130.5 / 128.6, 115500 (1805) 142.2 / 136.1,
+ * 60 blocks 115500 173.7 / 167.5; elsewhere 24 blocks 100500 66.9 / 67.1, 20 blocks 118500 64.4 / 64.7, 36
+ * blocks 98000 (1532) 91.6 / 93.7, 113000 (1766) 101.5 / 103.1, 48 blocks 128000 150.0 / 150.6, 140000 163 / 193. */
+static bool q4x_whole_rows(long groups, int nb) {
+    return (nb >= 22 && groups > 1792 && groups <= (nb < 28 ? 1860 : 1888)) ||
+           (nb >= 28 && groups > 1536 && groups <= 1664);
+}
+
 void launch_q4k_packed_gemv_q8k(hipStream_t stream, const void *packed, long n_out, int n_in,
                                 const uint32_t *act, int n_m, bool pairs, float *y, long ld_y) {
     const uint32_t *p  = static_cast<const uint32_t *>(packed);
@@ -531,14 +556,20 @@ void launch_q4k_packed_gemv_q8k(hipStream_t stream, const void *packed, long n_o
      * same rate or a better one: norm, projection and greedy draw, us, by it / by the matrix cores, 2 rows
      * 33000 x 1024 14.6 / 17.0, 43680 x 3072 25.2 / 28.5, 262144 x 1536 47.6 / 50.5; 3 rows 15.4 / 17.3,
      * 27.2 / 28.7, 49.3 / 51.9, 64048 x 1536 22.0 / 21.5; 4 rows 36736 x 2304 24.9 / 24.7, 124296 x 1536
-     * 34.8 / 31.3. pairs: a tile of sixteen rows' order of accumulation, which comes in eights. */
+     * 34.8 / 31.3. Three rows of 24 blocks and more leave room for three workgroups on a compute unit,
+     * 768 on the card: what is left over waits, where the matrix cores' 512 of 128 table rows run at once
+     * -- 49600 x 6144 48.2 / 46.3, 58000 x 7168 56.6 / 54.7, 65500 x 8192 67.5 / 64.5, but 49100 x 6144
+     * (768) 42.1 / 46.1 and 66500 x 6144 55.4 / 61.9. pairs: a tile of sixteen rows' order of
+     * accumulation, which comes in eights. */
     if (pairs)
-        k_q4k_packed_gemv_x86_pairs<Q4X_M_MAX><<<grid, block, 0, stream>>>(p, n_out, nb, act, y, ld_y);
+        k_q4k_packed_gemv_x86_rows<Q4X_M_MAX, true><<<grid, block, 0, stream>>>(p, n_out, nb, act, y, ld_y);
+    else if (n_m == 1 && q4x_whole_rows(groups, nb))
+        k_q4k_packed_gemv_x86_rows<1, false><<<grid, block, 0, stream>>>(p, n_out, nb, act, y, ld_y);
     else if (n_m == 1) /* (at most 64 blocks: what the reference's kernel takes) */
         split(std::integral_constant<int, 1>{});
     else if (n_m == 2 && nb <= Q4X_SPLIT_BLOCKS)
         split(std::integral_constant<int, 2>{});
-    else if (n_m == 3 && nb <= Q4X_SPLIT_BLOCKS)
+    else if (n_m == 3 && nb <= Q4X_SPLIT_BLOCKS && !(nb >= 24 && groups > 768 && groups <= 1024))
         split(std::integral_constant<int, 3>{});
     else
         k_q4k_packed_linear_x86_mfma<2, 4><<<dim3((unsigned) ((groups + 1) / 2)), block, 0, stream>>>(
