@@ -268,6 +268,46 @@ __global__ __launch_bounds__(Q6X_TPB, 4) void k_q6k_packed_gemv_x86(
         y[row] = (s_sum[0][r] + s_sum[1][r]) + (s_sum[2][r] + s_sum[3][r]);
 }
 
+/* The same with 64 table rows to a wavefront, which goes through their blocks in order
+ * (q6x_whole_rows says for which tables). */
+__global__ __launch_bounds__(Q6X_TPB, 4) void k_q6k_packed_gemv_x86_rows(
+    const uint32_t *__restrict__ packed, long n_out, int nb, const uint32_t *__restrict__ act,
+    float *__restrict__ y) {
+    const int  r = threadIdx.x & 63;
+    const long g = (long) blockIdx.x * (Q6X_TPB / 64) + threadIdx.x / 64;
+    if (g * 64 >= n_out)
+        return;
+    const long row = g * 64 + r;
+    float      acc[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+        acc[u] = 0.0f;
+    const uint32_t *base = packed + g * nb * Q6X_PACK_DWORDS;
+    uint32_t        qa[24], qb[24], sc[4], d52;
+    q6x_load_scales(base, r, sc, d52);
+    q6x_load6(base, r, 0, qa);
+    for (int b = 0; b < nb; ++b) {
+        const uint32_t *blk = base + (long) b * Q6X_PACK_DWORDS;
+        const uint32_t *a   = act + (long) b * Q8K_ACT_DWORDS; /* uniform: scalar loads */
+        q6x_load6(blk, r, 6, qb);
+        const float d = q6x_block_scale(a, d52);
+        int         lane[8];
+        q6x_offsets(a, sc, lane);
+        uint32_t sc_now[4] = {sc[0], sc[1], sc[2], sc[3]};
+        q6x_half(qa, sc_now, 0, a, lane);
+        if (b + 1 < nb) {
+            q6x_load_scales(blk + Q6X_PACK_DWORDS, r, sc, d52);
+            q6x_load6(blk + Q6X_PACK_DWORDS, r, 0, qa);
+        }
+        q6x_half(qb, sc_now, 1, a, lane);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            acc[u] = __builtin_fmaf(d, (float) lane[u], acc[u]);
+    }
+    if (row < n_out)
+        y[row] = ((acc[0] + acc[4]) + (acc[1] + acc[5])) + ((acc[2] + acc[6]) + (acc[3] + acc[7]));
+}
+
 /* The same over the table as it lies in the file, for callers that keep no packed copy: a lane
  * owns a table row and reads its 210-byte blocks whole. There the four low bits and the two high
  * bits of an element lie apart, but in the order the dot product wants them: a dword of ql holds
@@ -740,11 +780,28 @@ void launch_rmsnorm_q8k_rows(hipStream_t stream, const float *x, long ld_x, cons
                                                                   act);
 }
 
+/* Whether a table takes k_q6k_packed_gemv_x86_rows: of rows of more than sixteen blocks (which the other
+ * form takes in turns, a barrier each), those that leave a few of 256 compute units an eighth workgroup of
+ * 64 table rows, four of which run there at a time, while this form's wavefronts, two to a SIMD up to
+ * 2048, run at once. Shared blocks / not, us: 20 blocks 114800 (1794 workgroups) 87.9 / 88.8, 116500 (1821) 90.9 /
+ * 89.7, 118500 (1852) 91.6 / 90.8, 120500 (1883) 92.1 / 92.2; 32 blocks 116500 140.3 / 137.9; 48 blocks 114800
+ * 200.7 / 197.9, 116500 206.0 / 201.3, 122500 209.2 / 211.1; elsewhere 20 blocks 101000 80.9 / 83.3, 32 blocks 32000
+ * 49.2 / 84.8, 114600 (1791) 132.3 / 135.8, 128256 147.0 / 149.9, 256000 274 / 282. */
+static bool q6x_whole_rows(long groups, int nb) {
+    return nb > Q6X_SPLIT_BLOCKS && groups > (nb < 32 ? 1804 : 1792) && groups <= 1872;
+}
+
 void launch_q6k_packed_gemv_q8k(hipStream_t stream, const void *packed, long n_out, int n_in,
                                 const uint32_t *act, float *y) {
     const int    nb  = n_in / 256;
+    const long   groups = (n_out + 63) / 64;
+    if (q6x_whole_rows(groups, nb)) {
+        k_q6k_packed_gemv_x86_rows<<<dim3((unsigned) ((groups + 3) / 4)), dim3(Q6X_TPB), 0, stream>>>(
+            static_cast<const uint32_t *>(packed), n_out, nb, act, y);
+        return;
+    }
     const size_t lds = (size_t) (nb < Q6X_SPLIT_BLOCKS ? nb : Q6X_SPLIT_BLOCKS) * Q6X_SPLIT_DWORDS * sizeof(float);
-    k_q6k_packed_gemv_x86<<<dim3((unsigned) ((n_out + 63) / 64)), dim3(Q6X_TPB), lds, stream>>>(
+    k_q6k_packed_gemv_x86<<<dim3((unsigned) groups), dim3(Q6X_TPB), lds, stream>>>(
         static_cast<const uint32_t *>(packed), n_out, nb, act, y);
 }
 

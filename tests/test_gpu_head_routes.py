@@ -55,6 +55,8 @@ def logits(hs, kind, w, n_in, x):
     ("q4k", 1, 28, 1665), ("q4k", 1, 33, 1888), ("q4k", 1, 33, 1889),
     ("q4k", 3, 23, 800), ("q4k", 3, 24, 768), ("q4k", 3, 24, 769), ("q4k", 3, 32, 1024),
     ("q4k", 3, 24, 1025),
+    ("q6k", 1, 16, 1810), ("q6k", 1, 17, 1804), ("q6k", 1, 17, 1805), ("q6k", 1, 31, 1872),
+    ("q6k", 1, 32, 1792), ("q6k", 1, 32, 1793), ("q6k", 1, 33, 1873),
 ])
 @pytest.mark.parametrize("ragged", [0, 24, 56])
 def test_parts_of_a_table_give_the_bits_of_the_whole(hs, kind, m, blocks, groups, ragged):
@@ -68,3 +70,18 @@ def test_parts_of_a_table_give_the_bits_of_the_whole(hs, kind, m, blocks, groups
     for at in range(0, n_out, part):
         few = logits(hs, kind, w[at:at + part].contiguous(), n_in, x)
         assert torch.equal(few, whole[:, at:at + part]), at
+
+
+@pytest.mark.parametrize("n_in", [512, 1536])
+@pytest.mark.parametrize("groups", [2049, 3001, 4097])
+@pytest.mark.parametrize("ragged", [0, 5])
+def test_q6k_batches_too_large_for_slices(hs, groups, n_in, ragged):
+    print(f"q6k batches, {groups} groups - {ragged}, {n_in}", flush=True)
+    n_out = groups * 64 - ragged
+    w = table("q6k", n_out, n_in, groups + n_in)
+    g = np.random.default_rng(groups)
+    for m in range(2, 9):
+        x = torch.from_numpy((g.standard_normal((m, n_in)) * 3).astype(np.float32)).cuda()
+        file = torch.full((m, n_out), 7.0, dtype=torch.float32, device="cuda")
+        hs.q6k_linear_x86(w, n_in, x, file)
+        assert torch.equal(logits(hs, "q6k", w, n_in, x), file.view(torch.int32)), m
