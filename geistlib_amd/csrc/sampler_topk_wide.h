@@ -120,8 +120,11 @@ __device__ __forceinline__ bool topk_wide_row(const RowView &rv, const FinalArgs
     __syncthreads();
     /* The bound: two digits of eleven bits; a NaN's key is 0 and is not counted. Up to a rank of a
      * quarter of the threads each enters only the largest of its maxima: at least as many reach a
-     * bound as of those do, a seventh more in the worst case, for an eighth of the additions, which
-     * queue in the few bins that a row's maxima fall into (256 x 262144, k = 64: 1.9 us). */
+     * bound as of those do, for an eighth of the additions, which queue in the few bins that a row's
+     * maxima fall into (256 x 262144, k = 64: 1.9 us). In rows without order a few more than the rank
+     * reach it (a thirtieth at 64, an eighth at 256); where the leaders share threads, ids equal modulo
+     * 1024 in chunks four apart, up to KPT times the rank do, and a row whose list that overflows selects
+     * over the whole row. */
     uint32_t key[KPT];
 #pragma unroll
     for (int q = 0; q < KPT; ++q)
