@@ -957,11 +957,7 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
     f.minp_listed = rs.use_m && zb_m < ZBINS - 1 && !f.minp_direct && !f.win_locate;
     const bool minp_small = f.minp_direct && small_chunks <= (size_t) s->max_chunks &&
                             small_chunks <= (size_t) MAX_CHUNKS &&
-                            (L.rv.softcap > 0.0f
-                                 ? rows->rows * small_chunks <= (size_t) MINP_SMALL_CAPPED
-                                 : rows->rows * small_chunks <= (size_t) MINP_SMALL &&
-                                       rows->rows * small_chunks * small_chunks <=
-                                           (size_t) MINP_SMALL_POLLS);
+                            gs::minp_small_chunks(rows->rows, small_chunks, L.pen, L.rv.softcap > 0.0f);
     if (f.win_locate || minp_small) {
         L.nv           = 2;
         L.rv.per_chunk = 2048;

@@ -145,16 +145,30 @@ inline int    win_cap_for(size_t n) { return n / 8 > WIN_CAP_MIN ? (int) ((n / 8
  * 63 x 63 reads) 39.3 / 43.5; 8 x 262144 (8 x 128 x 128) 58 / 54, 48 x 100000 (2352 chunks) 48 / 21. */
 constexpr int WIN_SMALL       = 1024;
 constexpr int WIN_SMALL_READS = 65536;
-/* A min-p batch of up to so many chunks of 2048, and so many slots polled (every workgroup polls all of
- * its row's), is cut into those, other ones into chunks of 8192:
- * 2 x 54912 14.2 us against 16.4, 46 x 45893 (1058 chunks) 19.0 / 21.4, 21 x 110528 (1134) 19.3 /
- * 18.7, 13 x 206875 (1326) 22.0 / 22.0, 100 x
- * 60000 (3000) 27.5 / 23.3; 8 x 151936 (8 x 75 x 75 polls) 15.8 / 16.8, 20 x 100000 (48020) 17.9 / 18.2, 12 x
- * 128256 (47628) 17.3 / 17.0, 11 x 152960 (61875) 17.4 / 16.4, 16 x 128256 (63504) 16.8 / 15.8. With a soft-cap, whose tanhf makes a chunk's arithmetic the longest step,
- * 2 x 54912 19.5 / 35.4, 71 x 92992 (3266) 43.2 / 50.7, 64 x 128256 (4032) 53.7 / 51.1. */
-constexpr int MINP_SMALL        = 1088;
-constexpr int MINP_SMALL_POLLS  = 46080;
-constexpr int MINP_SMALL_CAPPED = 3400;
+/* Whether a min-p batch is cut into chunks of 2048 (n of them to a row) or of 8192: us a call, those / these.
+ *   Without a soft-cap up to 1088 of them, and so many slots polled (every workgroup polls all of its
+ * row's): rows that share no XCD up to 32768 -- 2 x 54912 14.1 / 16.0, 46 x 45893 (1058 chunks) 19.8 / 22.6,
+ * 29 x 65528 (29696 polls) 18.4 / 18.3, but 21 x 80920 (33600) 17.9 / 17.7, 18 x 95256 (39762) 18.3 / 17.4, 22 x
+ * 89112 (42592) 18.3 / 17.6 -- and rows in eights, each on one XCD, or with penalties up to 46080: 8 x 151936
+ * (45000) 15.6 / 16.5, 14 x 110000 with penalties (40824) 19.6 / 22.2; beyond, the one gives and the other
+ * takes: 12 x 128256 (47628) 18.1 / 17.4 and with penalties 19.1 / 20.7, 11 x 152960 (61875) 18.8 / 17.7 and
+ * 19.7 / 20.4.
+ *   With one, whose tanhf makes a chunk's arithmetic the longest step, up to 3400 chunks: 2 x 54912 19.2 /
+ * 35.1, 52 x 131072 (3328) 44.6 / 51.6, 150 x 45000 (3300) 42.9 / 51, 64 x 128256 (4032) 54.7 / 52.4; with
+ * penalties, whose registers hold seven workgroups on a compute unit for eight, up to 3072: 37 x 162840
+ * (2960) 48.7 / 50.5, 48 x 130072 (3072) 48.6 / 50.4, 26 x 248856 (3172) 55.1 / 53.3, 67 x 101400 (3350) 54.4 /
+ * 53.3. Long rows in eights that are not all resident at once (rows / 8 x chunks on 32 compute units, which
+ * wait for the rest of their row meanwhile) keep the chunks of 8192: from 81 chunks a row on 24 x 261144
+ * 58.4 / 47.7, 40 x 171032 53.9 / 51.9, 16 x 261144 43.6 / 41.0, but 40 x 158744 (78) 4 % less; with penalties
+ * from 65 on 32 x 203800 66.9 / 50.8, 40 x 142360 53.9 / 49.8, 48 x 138264 57.5 / 51.7, but 48 x 121880 (60)
+ * 47.9 / 50.3; 1792 chunks are resident, 16 x 195608 32.0 / 41.8, 16 x 228376 42.3 / 42.2. */
+inline bool minp_small_chunks(size_t rows, size_t n, bool pen, bool capped) {
+    const bool   eights = rows % 8 == 0;
+    const size_t wgs    = rows * n;
+    if (!capped)
+        return wgs <= 1088 && wgs * n <= (eights || pen ? 46080 : 32768);
+    return wgs <= (pen ? 3072 : 3400) && (!eights || n <= (pen ? 64 : 80) || wgs <= 1792);
+}
 struct WinSpace {
     float    *hist;  /* [rows][chunks][WIN_BINS], by the launch's chunks */
     uint64_t *list;  /* [rows][cap] */
