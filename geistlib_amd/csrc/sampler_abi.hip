@@ -851,15 +851,15 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
          *   The tolerance mode's sums are another kernel's. The measuring stages cannot split the
          * one launch: the streaming stage is the whole step. */
         const size_t big = (rows->n_vocab + 8191) / 8192, wgs = rows->rows * (size_t) scan.rv.n_chunks;
-        const bool   short_rows = rows->rows > 64 && scan.rv.n_chunks < 20;
-        if (scan.nv == 2 && !s->fast_sums && wgs > (scan.rv.n_chunks < 32 ? 1792 : 1536) &&
+        const bool   short_rows = rows->rows > 64 && scan.rv.n_chunks < 20, capped = L.rv.softcap > 0.0f;
+        if (scan.nv == 2 && !s->fast_sums && !capped && wgs > (scan.rv.n_chunks < 32 ? 1792 : 1536) &&
             big * 8192 * 10 <= rows->n_vocab * 11) {
             scan.nv = L.nv = 8;
             scan.rv.per_chunk = L.rv.per_chunk = 8192;
             scan.rv.n_chunks = L.rv.n_chunks = (int) big;
         }
-        const bool few = scan.nv == 2 && wgs <= 256 && scan.rv.n_chunks <= 84;
-        if (few || (scan.nv == 2 && (s->fast_sums ? wgs <= 256 : !short_rows))) {
+        const bool few = scan.nv == 2 && wgs <= 256 && (scan.rv.n_chunks <= 84 || capped);
+        if (few || (scan.nv == 2 && (s->fast_sums ? wgs <= 256 : !short_rows && !capped))) {
             *stream_kernel    = "k_temperature_draw";
             RowGenerators gen = {};
             if (few ? own_rng : per_row)
