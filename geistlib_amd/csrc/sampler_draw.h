@@ -15,7 +15,7 @@
  * others report theirs and leave. It works the place out for the row and, unless the draw falls
  * in its own chunk, reads the located chunk again and forms its weights and slab sums as the
  * workgroup that summed it did. 8 x 128256 9.6 -> 8.2 us, 24 x 50257 12.0 -> 10.3, 5 x 128256 with
- * the rows' own generators 12.9 -> 9.7, 1 x 262144 13.4 -> 8.7 (all chunks waiting on one XCD).
+ * the rows' own generators 12.9 -> 9.7, 1 x 262144 13.0 -> 8.7 (all chunks waiting on one XCD).
  *
  * The waits are bounded like the first meet's. A workgroup that gives up a wait forms what it
  * is missing itself, from the row: the maximum as before, the other chunks' sums by running
