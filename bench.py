@@ -32,9 +32,10 @@ sys.path.insert(0, ROOT)
 sys.path.insert(0, os.path.join(ROOT, "tests"))
 
 HBM_PEAK_GBS = 8000.0
-# Logits of a batch from which a top-k call scans for thread maxima first (WIDE_LOGITS in
-# csrc/sampler_kernels.h); smaller ones have the scan hand candidates on.
-TOPK_MAXIMA_LOGITS = 1 << 24
+# Logits of a batch from which a top-k call scans for thread maxima first, of long rows and of others
+# (wide_by_size in csrc/sampler_kernels.h); smaller ones have the scan hand candidates on.
+TOPK_MAXIMA_ROW = 16 * 8192
+TOPK_MAXIMA_LOGITS = (1 << 24, 1 << 25)
 COLD_WORKING_SET = 640 * 1024 * 1024   # bytes of logits the timed loops cycle through
 
 # HBM bytes moved by one launch of the step's kernel, from rocprofv3's FETCH_SIZE and
@@ -162,8 +163,7 @@ def topk_path_counts(hs, row_sets, prm, d_u, d_out, n_rows):
     """Which path served the rows of a top-k configuration, over every input copy once
     (geist_hip_sampler_topk_paths after each call): the candidates handed on by the scan, the
     per-thread maxima, the selection over the whole row; fallback_rate = the share of rows that
-    did not take the first path of such a call, which from TOPK_MAXIMA_LOGITS logits on is the
-    thread maxima."""
+    did not take the first path of such a call, which for large batches is the thread maxima."""
     counts = {"scan_candidates": 0, "thread_maxima": 0, "whole_row": 0, "other": 0}
     for rs in row_sets:
         hs.sample(rs, prm, d_u, d_out)
@@ -171,7 +171,8 @@ def topk_path_counts(hs, row_sets, prm, d_u, d_out, n_rows):
             counts[{0: "scan_candidates", 1: "thread_maxima", 2: "whole_row"}.get(p, "other")] += 1
     total = max(1, sum(counts.values()))
     counts["rows"] = total
-    large = n_rows * row_sets[0].n_vocab >= TOPK_MAXIMA_LOGITS
+    n_vocab = row_sets[0].n_vocab
+    large = n_rows * n_vocab >= TOPK_MAXIMA_LOGITS[n_vocab <= TOPK_MAXIMA_ROW]
     first = counts["thread_maxima" if large else "scan_candidates"]
     counts["fallback_rate"] = round(1.0 - first / total, 6)
     return counts

@@ -725,13 +725,13 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
          * would let too many elements pass. */
         const int  rank   = rs.k + margin, cap_margin = L.rv.softcap > 0.0f ? 8 : 0;
         const int  k_wide = rank + cap_margin < WIDE_K_SEL_MAX ? rank + cap_margin : WIDE_K_SEL_MAX;
-        const bool wide   = (lazy || !L.pen) && rs.k <= WIDE_K_SEL_MAX &&
-                          (rank > WIDE_RANK_MIN || rows->rows * rows->n_vocab >= WIDE_LOGITS ||
-                           (cap_margin && (rank > WIDE_RANK_MIN_CAPPED || L.rv.n_chunks <= 16))) &&
-                          L.rv.n_chunks <= WIDE_CHUNKS_MAX && rows->n_vocab / 32 >= 2 * (size_t) k_wide;
+        const bool wide_fits = (lazy || !L.pen) && rs.k <= WIDE_K_SEL_MAX &&
+                               L.rv.n_chunks <= WIDE_CHUNKS_MAX && rows->n_vocab / 32 >= 2 * (size_t) k_wide;
+        const bool wide_rank = wide_fits && (rank > WIDE_RANK_MIN ||
+                                             (cap_margin && (rank > WIDE_RANK_MIN_CAPPED || L.rv.n_chunks <= 16)));
         f.mode = FINAL_TOPK;
         f.k    = rs.k;
-        if (rs.k > TOPK_FAST_MAX && !wide) {
+        if (rs.k > TOPK_FAST_MAX && !wide_rank) {
             draws();
             *stream_kernel = "k_topk_general";
             const int e    = do_stream ? launch_topk_general(large, f) : 0;
@@ -801,8 +801,9 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
             draws();
         else
             draws_by(scan);
-        /* (rows that could be handed on, in a batch where that is the slower way: WIDE_LOGITS) */
-        const bool large_wide = wide && rows->rows * rows->n_vocab >= WIDE_LOGITS;
+        /* (rows that could be handed on, in a batch where that is the slower way) */
+        const bool large_wide = m && wide_fits && wide_by_size(rows->rows * rows->n_vocab, L.rv.n_chunks);
+        const bool wide       = wide_rank || large_wide;
         if (m && !large_wide) {
             const WaveCands wc = wave_cands_at(s->wcands, row_waves);
             f.row_flag         = s->row_flag;

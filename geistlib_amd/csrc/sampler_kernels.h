@@ -25,11 +25,17 @@ constexpr int WIDE_CHUNKS_MAX = 32;  /* ... whose rows have at most so many chun
  * 223709 23.3 / 22.3). */
 constexpr int WIDE_RANK_MIN        = 48;
 constexpr int WIDE_RANK_MIN_CAPPED = 16;
-/* Batches of at least so many logits take that path whatever the rank, rows whose scan could hand
- * candidates on (k_cand_scan, k_final_cand) too: their scan leaves the maxima alone, 45.6 against 53.9 us
- * for 256 x 262144. 256 x 262144, k = 64, 56.3 / 63.9; 192 x 262144, k = 40, 43.7 / 48.8; 152 x 128512 22.4 /
- * 24.2; 96 x 121168 16.1 / 15.8; 100 x 100000 15.3 / 14.4; 51 x 223712 16.3 / 16.2. */
-constexpr size_t WIDE_LOGITS = (size_t) 1 << 24;
+/* Rows whose scan could hand candidates on (k_cand_scan, k_final_cand) take that path too, whatever the
+ * rank, in batches of 2^25 logits, rows of more than 16 chunks from 2^24 on: their scan leaves the maxima
+ * alone, 45.6 against 53.9 us for 256 x 262144. Maxima / candidates: 256 x 262144, k = 64, 56.3 / 63.9; 192 x
+ * 262144, k = 40, 43.7 / 48.5 and with penalties 45.3 / 49.2; 256 x 131072 (2^25) 30.0 / 30.6; 64 x 262144 (2^24)
+ * 19.3 / 19.3, k = 64 19.6 / 20.1, with penalties 21.0 / 19.8; 110 x 152960 k = 64 19.9 / 26.0, k = 40 with
+ * penalties 21.4 / 27.7; of fewer chunks below 2^25 128 x 131072 19.0 / 18.3 and with penalties 20.8 / 19.4, 256 x
+ * 65536 19.4 / 18.3 and 21.2 / 19.4, 256 x 100000 24.6 / 24.2 and 26.6 / 25.1. Other rows (masks, unaligned)
+ * go by the rank alone: k = 20 with a mask 64 x 262144 21.5 / 20.3, 192 x 262144 46.5 / 44.9. */
+inline bool wide_by_size(size_t logits, int n_chunks) {
+    return logits >= (size_t) 1 << (n_chunks > 16 ? 24 : 25);
+}
 constexpr int TOPK_MAX       = 8192; /* the reference caps top_k here (sampler.c:213-215) */
 constexpr int HISTORY_MAX    = 65535;
 

@@ -365,8 +365,8 @@ int geist_hip_sampler_row_paths(geist_hip_sampler *s, int32_t *h_paths, size_t r
 
 /* Diagnostics (no reference counterpart): after a top-k call, which path served each row:
  * 0 = the candidates handed on by the scan, 1 = the per-thread maxima (rows whose leading logits
- * crowd into few wavefronts' elements, runs of equal values; every row of a batch of 2^24 logits and
- * more), 2 = the selection over the whole
+ * crowd into few wavefronts' elements, runs of equal values; every row of a batch of 2^25 logits and
+ * more, 2^24 where rows have more than 131072), 2 = the selection over the whole
  * row; -1 for every row when the call did not take the candidate path at all (soft-cap, mask,
  * unaligned rows, k above 64, penalties that can raise a logit). Synchronous. */
 int geist_hip_sampler_topk_paths(geist_hip_sampler *s, int32_t *h_paths, size_t rows);

@@ -25,6 +25,8 @@ def rate(paths, rows, n_vocab):
     (64, 128256, [1] * 64, 1.0),                     # all of them fell back to the thread maxima
     (64, 128256, [0] * 48 + [1] * 12 + [2] * 4, 0.25),
     (256, 262144, [1] * 256, 0.0),                   # thread maxima first
+    (128, 131072, [1] * 128, 1.0), (256, 131072, [1] * 256, 0.0), (127, 131073, [1] * 127, 1.0),
+    (128, 131073, [1] * 128, 0.0),
     (256, 262144, [1] * 192 + [2] * 64, 0.25),
 ])
 def test_fallback_rate(rows, n_vocab, paths, want):
@@ -33,5 +35,6 @@ def test_fallback_rate(rows, n_vocab, paths, want):
 
 def test_the_limit_is_the_librarys():
     text = open(os.path.join(ROOT, "geistlib_amd", "csrc", "sampler_kernels.h")).read()
-    shift = re.search(r"constexpr size_t WIDE_LOGITS = \(size_t\) 1 << (\d+);", text).group(1)
-    assert bench.TOPK_MAXIMA_LOGITS == 1 << int(shift)
+    chunks, long_rows, others = re.search(r"1 << \(n_chunks > (\d+) \? (\d+) : (\d+)\)", text).groups()
+    assert bench.TOPK_MAXIMA_ROW == int(chunks) * 8192
+    assert bench.TOPK_MAXIMA_LOGITS == (1 << int(long_rows), 1 << int(others))

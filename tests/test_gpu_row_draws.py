@@ -18,7 +18,7 @@ CASES = [
     (80, 32000, T, "fast"), (64, 128256, T, "fast"),        # ... without a meeting
     (80, 32000, {**T, **PEN}, "fast"),
     (40, 32000, K40, "two"), (12, 131072, {**K40, **PEN}, "two"),   # k_cand_scan, k_final_cand
-    (128, 131072, K40, ""),                                 # 2^24 logits: k_tmax_scan, k_topk_wide
+    (64, 262144, K40, ""), (256, 131072, K40, ""),           # large: k_tmax_scan, k_topk_wide
     (16, 50001, K40, ""),                                   # k_tmax_scan, k_final_topk
     (4, 50001, dict(temperature=0.9, top_k=150), ""),       # k_tmax_scan, k_topk_wide
     (24, 50257, dict(temperature=1.0, top_p=0.95), ""),     # exp-sum pass, k_window
@@ -79,7 +79,7 @@ def test_draws_taken_by_a_scan(rows, n, options, form):
 
 @pytest.mark.parametrize("rows,n,options,form", [
     (9, 70001, T, ""), (24, 32000, {**T, **PEN}, ""),       # the last chunk draws
-    (80, 32000, T, ""), (80, 32000, T, "fast"), (40, 32000, K40, "two"), (128, 131072, K40, ""),
+    (80, 32000, T, ""), (80, 32000, T, "fast"), (40, 32000, K40, "two"), (64, 262144, K40, ""),
     (24, 50257, dict(temperature=1.0, top_p=0.95), ""), (6, 40000, {**T, "min_p": 0.05}, ""),
     (9, 70001, dict(temperature=0.0), ""), (8, 32000, dict(temperature=0.0, **PEN), ""),
 ])

@@ -41,3 +41,32 @@ def test_leaders_in_shared_columns(oracle, k, pen):
     want = [oracle.chain_u(oracle.penalties(x[r], hist[r], 1.2, 0.3, 0.1) if pen else x[r], float(u[r]), **kw)
             for r in range(rows)]
     assert compare_ids(got, [t for t, _ in want], [i for _, i in want], f"columns k={k}") <= 1
+
+
+@pytest.mark.parametrize("rows,n,first", [(128, 131072, 0), (255, 131072, 0), (256, 131072, 1),
+                                          (127, 131076, 0), (128, 131076, 1)])
+@pytest.mark.parametrize("pen", [False, True])
+def test_the_first_path_follows_from_the_batch(rows, n, first, pen):
+    """Candidates handed on by the scan (0) or the thread maxima (1): the same ids either way, those of
+    the rows in calls of a few."""
+    print(f"first path {rows} x {n} pen={pen}", flush=True)
+    from geistlib_amd import HipSampler, SampleParams
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(rows + n + pen)
+    x = torch.randn((rows, n), device="cuda", generator=gen) * 2
+    hist = torch.randint(0, n, (rows, 300), device="cuda", generator=gen, dtype=torch.int32)
+    hl = torch.full((rows,), 300, device="cuda", dtype=torch.int32)
+    u = torch.rand((rows,), device="cuda", generator=gen)
+    prm = SampleParams.make(temperature=0.7, top_k=40, top_p=0.9, **(dict(rep=1.1, freq=0.5, pres=0.3) if pen else {}))
+    out, few = (torch.full((rows,), -7, dtype=torch.int32, device="cuda") for _ in range(2))
+    s = HipSampler(max_rows=rows, max_vocab=n)
+    s.one_launch_topk(False)
+    s.sample(HipSampler.rows(x, hist, hl), prm, u, out)
+    paths = s.topk_paths(rows).tolist()
+    for at in range(0, rows, 16):
+        to = slice(at, at + 16)
+        s.sample(HipSampler.rows(x[to], hist[to], hl[to]), prm, u[to].contiguous(), few[to])
+    s.sync()
+    s.close()
+    assert out.tolist() == few.tolist()
+    assert paths.count(first) > rows // 2, paths    # (a few leave it: their leaders crowd)
