@@ -831,30 +831,34 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
         /* Chunks of 2048: the step is a chain of waits, not of bytes, and a second launch is a part
          * of it. Scan, sums and the draw in one kernel, whose workgroups all wait for the sums
          * (`few`) or only the one that draws.
-         *   few: (with a soft-cap whatever the row's length) the rows each on an XCD of its own, up to 256 workgroups whose rows an XCD's 32
-         * compute units hold at two to three each. 1 x 32000 6.2 us against 7.5 with one that
-         * draws, 1 x 128256 7.2 / 8.5, 8 x 64000 6.8 / 8.0, 3 x 131072 7.3 / 8.3, 1 x 151936 (75 chunks)
-         * 8.6 / 8.6 and with penalties 10.3 / 10.9, 1 x 170000 (84) 8.5 / 8.8, but 1 x 200000 10.5 /
-         * 8.9, 1 x 262144 13.0 / 8.7 and with penalties 16.5 / 10.5.
+         *   few: (with a soft-cap whatever the row's length) the rows each on an XCD of its own, up to
+         * 256 workgroups whose rows an XCD's 32 compute units hold at two to three each. 1 x 32000
+         * 6.2 us against 7.5 with one that draws, 1 x 128256 7.2 / 8.5, 8 x 64000 6.8 / 8.0, 3 x
+         * 131072 7.3 / 8.3, 1 x 151936 (75 chunks) 8.6 / 8.6 and with penalties 10.3 / 10.9, 1 x
+         * 170000 (84) 8.5 / 8.8, but 1 x 200000 10.5 / 8.9, 1 x 262144 13.0 / 8.7 and with penalties
+         * 16.5 / 10.5.
          *   One that draws against two launches: 5 x 128256 9.7 / 12.9 us, 8 x 128256 8.2 / 9.6, 24 x
          * 128256 12.9 / 15.8; but each row has one that draws, and many short rows are better off
          * with two launches: 64 x 32000 10.8 / 10.9, 72 x 32000 11.6 / 11.2, 96 x 32000 13.5 / 12.1
          * (72 x 40000 12.0 / 12.7).
-         * With a soft-cap one that draws has a chunk's tanhf at the end of its waits: two launches in chunks of
-         * 2048, 40 x 78000 25.2 / 36.3, 12 x 262144 24.2 / 30.1, 64 x 32000 19.9 / 23.7. With a mask, whose words
-         * it reads again, up to 1024 workgroups: 9 x 147456 (648) 12.1 / 13.1, 24 x 86016 (1008) 10.5 / 11.4, but 9 x
-         * 261144 (1152) 16.3 / 15.7, 23 x 131072 (1472) 17.3 / 15.8, 12 x 262144 18.1 / 16.6. Rows of 32 chunks (with
-         * a mask of 16 too) have the workgroups that draw on the same few compute units: 40 rows of them and
-         * more two launches, 48 x 65536 12.6 / 11.6, with a mask 40 x 65536 13.8 / 11.1, 64 x 32760 11.7 / 11.2, but
-         * 31 x 64536 12.1 / 12.8.
+         * With a soft-cap one that draws has a chunk's tanhf at the end of its waits: two launches in
+         * chunks of 2048, 40 x 78000 25.2 / 36.3, 12 x 262144 24.2 / 30.1, 64 x 32000 19.9 / 23.7.
+         * With a mask, whose words it reads again, up to 1344 workgroups, with penalties 1450: 9 x
+         * 147456 (648) 12.1 / 13.1, 19 x 120000 (1121) 14.1 / 15.0, 33 x 80000 (1320) 14.8 / 15.2 and
+         * with penalties 15.3 / 16.6, 9 x 261144 (1152) 15.8 / 15.4 and with penalties 16.8 / 17.0, 18
+         * x 157312 (1386) with penalties 16.1 / 17.4, but 23 x 131072 (1472) 17.2 / 15.7, 12 x 262144
+         * 18.2 / 16.7. Rows of 32 chunks (with a mask of 16 too) have the workgroups that draw on the
+         * same few compute units: 40 rows of them and more two launches, 48 x 65536 12.6 / 11.6, with
+         * a mask 40 x 65536 13.8 / 11.1, 64 x 32760 11.7 / 11.2, but 31 x 64536 12.1 / 12.8.
          *   What does not start at once (1536 workgroups with penalties, 2048 without, whose last
          * quarter has no time left to hide in) goes to chunks of 8192 and two launches, unless those
          * end in an eighth of a chunk: 13 x 262144 15.1 us / one that draws 17.3 / two launches in
          * chunks of 2048 17.9, 31 x 131072 14.9 / 17.7 / 19.7, 24 x 151936 with penalties 16.9 / 20.3 /
          * 22.0, 120 x 32000 14.3 / 15.5 / 14.5; 72 x 50257 (six chunks and 1105) 16.6 / 15.1 / 17.8.
-         * 40 rows in eights and more without penalties from 1664 on: 40 x 79872 (1560) 13.1 / 11.0 / 12.3, 48 x 69632
-         * (1632) 13.2 / 11.8 / 12.6, 40 x 90112 (1760) 12.9 / - / 13.6. Short rows from somewhat later on: 80 x 40000 (1600) 14.0 / 12.6 / 12.9, 100 x 32000 (1600)
-         * 14.6 / 14.6 / 14.0.
+         * 40 rows in eights and more without penalties from 1664 on: 40 x 79872 (1560) 13.1 / 11.0 /
+         * 12.3, 48 x 69632 (1632) 13.2 / 11.8 / 12.6, 40 x 90112 (1760) 12.9 / - / 13.6. Short rows
+         * from somewhat later on: 80 x 40000 (1600) 14.0 / 12.6 / 12.9, 100 x 32000 (1600) 14.6 / 14.6
+         * / 14.0.
          * (In chunks of 8192 the one that draws needs 150 registers, and the whole pass half of its
          * wavefronts: 64 x 128256 34 against 18.9.)
          *   The tolerance mode's sums are another kernel's. The measuring stages cannot split the
@@ -870,7 +874,7 @@ int gs_host::sample_stages(geist_hip_sampler *s, const struct geist_hip_rows *ro
         }
         const bool few = scan.nv == 2 && wgs <= 256 && (scan.rv.n_chunks <= 84 || capped);
         const bool crowd  = scan.rv.n_chunks % (L.rv.allowed ? 16 : 32) == 0 && rows->rows >= 40;
-        const bool by_one = !short_rows && !capped && !crowd && !(L.rv.allowed && wgs > 1024);
+        const bool by_one = !short_rows && !capped && !crowd && !(L.rv.allowed && wgs > (L.pen ? 1450u : 1344u));
         if (few || (scan.nv == 2 && (s->fast_sums ? wgs <= 256 : by_one))) {
             *stream_kernel    = "k_temperature_draw";
             RowGenerators gen = {};

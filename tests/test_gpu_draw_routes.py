@@ -9,7 +9,8 @@ torch = pytest.importorskip("torch")
 from gpu_util import compare_ids, run_rows  # noqa: E402
 
 TEMPERATURE = [(2, 180001, "cap"), (3, 172032, "cap"), (12, 262144, "cap"), (20, 188210, "cap pen"),
-               (64, 32000, "cap"), (8, 262144, "mask"), (9, 233472, "mask"), (40, 65536, "mask"),
+               (64, 32000, "cap"), (8, 262144, "mask"), (21, 131072, "mask"), (22, 131072, "mask"),
+               (22, 131071, "mask pen"), (23, 131071, "mask pen"), (40, 65536, "mask"),
                (64, 32760, "mask"), (39, 65536, ""), (40, 65536, ""), (48, 64001, "pen")]
 MIN_P = [(5, 165888, "pen"), (6, 149504, ""), (6, 151553, ""), (8, 151936, ""),      # 32768 and 46080 polls
          (24, 151552, "cap"), (24, 153600, "cap"), (24, 163840, "cap"), (24, 165889, "cap"),
